@@ -158,7 +158,7 @@ int ddtr_batch::enqueue(const void *const *inputs, const int *t_processed, float
         int st = AA_HIP_SUCCESS;
         for (int r = 0; r < e->nranges(); ++r, ++flat) {
             range_launch rl;
-            st = e->prepare_range(r, t_processed[flat], d_out[flat], out_pitch[flat], s, &rl);
+            st = e->prepare_range(r, t_processed[flat], d_out[flat], out_pitch[flat], s, &rl, true);
             if (st != AA_HIP_SUCCESS) return st;
             if (rl.ndms <= 0 || rl.t_processed <= 0) continue;
             const int f = rl.sample_bytes == 1 ? family_of(rl.variant, rl.row_quads) : -1;

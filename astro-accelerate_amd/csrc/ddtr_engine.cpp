@@ -26,6 +26,12 @@ int hip_fail(hipError_t e, const char *what) {
                 std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// A batched range with this many tiles fills the GPU's 256 work-groups twice
+// over and runs a matrix launch of its own; smaller ones stay in the shared
+// launches (96 beams of 64-256 channels: 1.98 ms batched, 4.27 ms with a
+// matrix launch per range).
+constexpr long kMatrixAloneTiles = 512;
+
 bool is_pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
 int log2i(int v) {
     int k = 0;
@@ -144,7 +150,7 @@ lds_params lds_params_of(const range_launch &rl) {
     p.out_pitch = rl.out_pitch;
     p.row_quads = rl.row_quads;
     p.pair_recs = rl.pair_recs;
-    lds_job_tiles(p, rl.variant);
+    if (rl.variant != kShapeMatrix) lds_job_tiles(p, rl.variant);
     return p;
 }
 
@@ -158,6 +164,7 @@ hipError_t launch_range(const range_launch &rl, hipStream_t s) {
         return launch_dedisperse_direct_u16(L, rl.pitch / 2, rl.nchans, rl.d_dmshifts, rl.ndms, rl.t_processed,
                                             rl.mstartdm, rl.mdmstep, rl.inBin, rl.out, rl.out_pitch, s);
     }
+    if (rl.variant == kShapeMatrix) return launch_dedisperse_matrix(lds_params_of(rl), rl.mat, s);
     if (rl.variant >= 0) return launch_dedisperse_lds(lds_params_of(rl), rl.variant, s);
     return launch_dedisperse_direct_u8(rl.L, rl.pitch, rl.nchans, rl.d_dmshifts, rl.ndms, rl.t_processed,
                                        rl.mstartdm, rl.mdmstep, rl.inBin, rl.out, rl.out_pitch, s);
@@ -239,6 +246,8 @@ ddtr_engine::~ddtr_engine() {
     if (m_d_err) (void)hipFree(m_d_err);
     for (const plan_tables &t : m_tables)
         if (t.ptr) (void)hipFree(t.ptr);
+    for (const matrix_tables &t : m_matrix)
+        if (t.t.ptr) (void)hipFree(t.t.ptr);
 }
 
 int ddtr_engine::set_kernel(int kernel) {
@@ -349,7 +358,7 @@ int ddtr_engine::ensure_level(int k, hipStream_t s) {
 }
 
 int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_pitch, hipStream_t s,
-                               range_launch *rl) {
+                               range_launch *rl, bool batched) {
     if (r < 0 || r >= (int)m_ranges.size()) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "bad range index");
     if (!d_out || out_pitch < (size_t)std::max(t_processed, 0))
         return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "bad output buffer");
@@ -394,6 +403,33 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
     }
     if (m_lds.size() != m_ranges.size()) m_lds.assign(m_ranges.size(), lds_choice{-2, 0});
     lds_choice &c = m_lds[(size_t)r];
+    // No shape asked for: the matrix kernel where its plan is the cheaper one.
+    if (range_variant(r) < 0 && (m_kernel == AA_HIP_KERNEL_AUTO || m_kernel == AA_HIP_KERNEL_LDS) &&
+        (!batched || matrix_tiles_at_most(rd.ndms, t_processed) >= kMatrixAloneTiles)) {
+        if (m_matrix.size() != m_ranges.size()) m_matrix.resize(m_ranges.size());
+        matrix_tables &mt = m_matrix[(size_t)r];
+        if (!mt.planned) {
+            std::vector<uint8_t> bytes;
+            const matrix_layout lay =
+                matrix_plan(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, lv.pitch, &bytes);
+            if (lay.tile_out > 0) {
+                st = keep_tables(mt.t, kShapeMatrix, bytes);
+                if (st != AA_HIP_SUCCESS) return st;
+            }
+            mt.lay = lay;
+            mt.planned = true;
+        }
+        const long tiles =
+            mt.lay.tile_out > 0 ? (long)mt.lay.n_dm_tiles * ((t_processed + mt.lay.tile_out - 1) / mt.lay.tile_out) : 0;
+        if (tiles > 0 && (!batched || tiles >= kMatrixAloneTiles)) {
+            st = resolve_launch(m_kernel, lv.ptr, lv.pitch, m_nchans, m_d_dmshifts, m_dmshifts.data(), rd.ndms,
+                                t_processed, mstartdm, mdmstep, rd.inBin, d_out, out_pitch,
+                                lds_choice{kShapeMatrix, mt.lay.tile_out}, rl);
+            rl->pair_recs = mt.t.ptr;
+            rl->mat = mt.lay;
+            return st;
+        }
+    }
     if (c.variant == -2) {
         const int want = r < (int)m_variant_pref.size() ? m_variant_pref[(size_t)r] : -1;
         c = choose_lds(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, want);
@@ -403,35 +439,40 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
     st = resolve_launch(m_kernel, lv.ptr, lv.pitch, m_nchans, m_d_dmshifts, m_dmshifts.data(), rd.ndms,
                         t_processed, mstartdm, mdmstep, rd.inBin, d_out, out_pitch, c, rl);
     if (st != AA_HIP_SUCCESS || rl->variant < 2) return st;
-    // Chunk shapes 2 and 3 read plan tables; they depend on the range and
+    // Chunk shapes from 2 on read plan tables; they depend on the range and
     // shape only, so they are built once (on the first call that needs them,
     // never while a later call is being captured into a graph).
     if (m_tables.size() != m_ranges.size()) m_tables.assign(m_ranges.size(), plan_tables{});
     plan_tables &pt = m_tables[(size_t)r];
     if (pt.variant != rl->variant) {
-        if (pt.ptr) {
-            (void)hipFree(pt.ptr);
-            m_device_bytes -= pt.bytes;
-            pt = plan_tables{};
-        }
         std::vector<uint8_t> bytes;
         if (lds_plan_tables(rl->variant, m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, lv.pitch, &bytes) !=
             rl->row_quads)
             return fail(AA_HIP_ERROR_UNSUPPORTED, "plan tables disagree with the chosen row width");
-        void *t = nullptr;
-        hipError_t e = hipMalloc(&t, bytes.size());
-        if (e == hipSuccess) e = hipMemcpy(t, bytes.data(), bytes.size(), hipMemcpyHostToDevice);
-        if (e != hipSuccess) {
-            if (t) (void)hipFree(t);
-            return hip_fail(e, "plan tables");
-        }
-        pt.variant = rl->variant;
-        pt.ptr = t;
-        pt.bytes = bytes.size();
-        m_device_bytes += bytes.size();
+        st = keep_tables(pt, rl->variant, bytes);
+        if (st != AA_HIP_SUCCESS) return st;
     }
-    void *t = pt.ptr;
-    rl->pair_recs = t;
+    rl->pair_recs = pt.ptr;
+    return AA_HIP_SUCCESS;
+}
+
+int ddtr_engine::keep_tables(plan_tables &pt, int variant, const std::vector<uint8_t> &bytes) {
+    if (pt.ptr) {
+        (void)hipFree(pt.ptr);
+        m_device_bytes -= pt.bytes;
+    }
+    pt = plan_tables{};
+    void *t = nullptr;
+    hipError_t e = hipMalloc(&t, bytes.size());
+    if (e == hipSuccess) e = hipMemcpy(t, bytes.data(), bytes.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        if (t) (void)hipFree(t);
+        return hip_fail(e, "plan tables");
+    }
+    pt.variant = variant;
+    pt.ptr = t;
+    pt.bytes = bytes.size();
+    m_device_bytes += bytes.size();
     return AA_HIP_SUCCESS;
 }
 
@@ -442,6 +483,10 @@ int ddtr_engine::set_range_variant(int r, int variant) {
     m_variant_pref[(size_t)r] = variant;
     if (m_lds.size() == m_ranges.size()) m_lds[(size_t)r] = lds_choice{-2, 0};
     return AA_HIP_SUCCESS;
+}
+
+int ddtr_engine::range_variant(int r) const {
+    return r >= 0 && r < (int)m_variant_pref.size() ? m_variant_pref[(size_t)r] : -1;
 }
 
 int ddtr_engine::autotune_range(int r, int t_processed, float *d_out, size_t out_pitch, int reps, hipStream_t s,
@@ -458,12 +503,13 @@ int ddtr_engine::autotune_range(int r, int t_processed, float *d_out, size_t out
     if (e == hipSuccess) e = hipEventCreate(&e1);
     int st = AA_HIP_SUCCESS;
     float best_ms = 0.0f;
-    for (int v = 0; v < kLdsVariants && e == hipSuccess && st == AA_HIP_SUCCESS; ++v) {
-        ms[v] = -1.0f;
+    float auto_ms = -1.0f;   // the automatic choice where that is the matrix kernel
+    for (int v = -1; v < kLdsVariants && e == hipSuccess && st == AA_HIP_SUCCESS; ++v) {
+        if (v >= 0) ms[v] = -1.0f;
         st = set_range_variant(r, v);
         range_launch rl;
         if (st == AA_HIP_SUCCESS) st = prepare_range(r, t_processed, d_out, out_pitch, s, &rl);
-        if (st != AA_HIP_SUCCESS || rl.variant != v) continue;
+        if (st != AA_HIP_SUCCESS || rl.variant != (v < 0 ? kShapeMatrix : v)) continue;
         e = launch_range(rl, s);
         if (e == hipSuccess) e = hipEventRecord(e0, s);
         for (int i = 0; i < reps && e == hipSuccess; ++i) e = launch_range(rl, s);
@@ -472,8 +518,8 @@ int ddtr_engine::autotune_range(int r, int t_processed, float *d_out, size_t out
         float t = 0.0f;
         if (e == hipSuccess) e = hipEventElapsedTime(&t, e0, e1);
         if (e != hipSuccess) break;
-        ms[v] = t / (float)reps;
-        if (*best < 0 || ms[v] < best_ms) {
+        (v < 0 ? auto_ms : ms[v]) = t / (float)reps;
+        if (v >= 0 && (*best < 0 || ms[v] < best_ms)) {
             *best = v;
             best_ms = ms[v];
         }
@@ -482,7 +528,8 @@ int ddtr_engine::autotune_range(int r, int t_processed, float *d_out, size_t out
     if (e1) (void)hipEventDestroy(e1);
     m_kernel = saved_kernel;
     if (st == AA_HIP_SUCCESS && e != hipSuccess) st = hip_fail(e, "autotune");
-    if (st == AA_HIP_SUCCESS) st = set_range_variant(r, *best);
+    const bool keep_auto = auto_ms >= 0.0f && (*best < 0 || auto_ms <= best_ms);
+    if (st == AA_HIP_SUCCESS) st = set_range_variant(r, keep_auto ? -1 : *best);
     return st;
 }
 

@@ -19,6 +19,7 @@
 
 #include "ddtr_kernels.h"
 #include "ddtr_lds.h"
+#include "ddtr_matrix.h"
 
 namespace aa_hip {
 
@@ -60,7 +61,8 @@ struct range_launch {
     size_t out_pitch = 0;
     int variant = -1;
     int row_quads = 0;
-    const void *pair_recs = nullptr;  // chunk shapes 2-4: device plan tables
+    const void *pair_recs = nullptr;  // chunk shapes 2-6 and the matrix kernel: device plan tables
+    matrix_layout mat;                // variant kShapeMatrix: layout of those tables
     int sample_bytes = 1;             // 2: u16 rows (samples wider than 8 bits; pitch still in bytes)
     long row_len = 0;                 // u16 rows: valid samples per row
     int wide_win = -1;                // u16 rows: dedisperse_u16's window, -1 = direct kernel
@@ -107,13 +109,19 @@ public:
     // Everything run_range does before the launch (binning up to the range's
     // level on `s`, validation, kernel choice); the launch itself is left to
     // the caller (launch_range, or a batched launch).
-    int prepare_range(int r, int t_processed, float *d_out, size_t out_pitch, hipStream_t s, range_launch *rl);
+    // batched: the caller puts the launches of many ranges into shared ones;
+    // the matrix kernel, which runs one launch per range, is then taken only
+    // by ranges that fill the GPU by themselves.
+    int prepare_range(int r, int t_processed, float *d_out, size_t out_pitch, hipStream_t s, range_launch *rl,
+                      bool batched = false);
     // LDS chunk shape preferred for range r (-1 = first that fits, in the
     // order of choose_lds); used when it fits the range's delay spread.
     int set_range_variant(int r, int variant);
+    int range_variant(int r) const;
     // Times every LDS chunk shape that fits range r (reps launches each, after
     // one untimed launch; output written to d_out) and keeps the fastest as
-    // the range's preference.  ms[v] = average launch time of shape v, or -1
+    // the range's preference, or none where the matrix kernel is the automatic
+    // choice and faster than all of them.  ms[v] = average launch time of shape v, or -1
     // when it does not fit.  *best = -1 when no shape fits.
     int autotune_range(int r, int t_processed, float *d_out, size_t out_pitch, int reps, hipStream_t s,
                        int *best, float *ms);
@@ -156,7 +164,16 @@ private:
         void *ptr = nullptr;
         size_t bytes = 0;
     };
-    std::vector<plan_tables> m_tables;  // per range: chunk shape 2-4 plan tables (device), built on first use
+    std::vector<plan_tables> m_tables;  // per range: plan tables (device), built on first use
+    struct matrix_tables {
+        bool planned = false;   // lay is known (tile_out 0: not this kernel)
+        matrix_layout lay;
+        plan_tables t;
+    };
+    std::vector<matrix_tables> m_matrix;  // per range: the matrix kernel's, kept beside the LDS shape's, which a
+                                          // captured batch may still read
+    // Uploads tables of `variant` in place of what pt holds.
+    int keep_tables(plan_tables &pt, int variant, const std::vector<uint8_t> &bytes);
     size_t m_device_bytes = 0;
 };
 

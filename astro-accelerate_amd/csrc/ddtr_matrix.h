@@ -1,0 +1,39 @@
+// Dedispersion on the matrix cores (see ddtr_matrix.hip for the algorithm).
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <cstddef>
+#include <cstdint>
+#include <vector>
+
+#include "ddtr_lds.h"
+
+namespace aa_hip {
+
+// Internal number of this kernel beside the LDS chunk shapes 0-6.
+constexpr int kShapeMatrix = kLdsVariants;
+
+// Where the parts of a range's plan tables lie, and the tile they are for.
+struct matrix_layout {
+    int n_dm_tiles = 0;
+    int tile_out = 0;      // output samples per tile (0: the range does not take this kernel)
+    size_t off_group = 0, off_step = 0, bytes = 0;
+};
+
+// More tiles than any plan of such a range has (tiles are at least 1024
+// samples): for callers that only want the kernel for many.
+inline long matrix_tiles_at_most(int ndms, int t_processed)
+{
+    return (long)((ndms + 15) / 16) * ((t_processed + 1023) / 1024);
+}
+
+// Plan tables of one range over rows `pitch` bytes apart: fills `bytes` (when
+// not null) as the kernel reads them and returns their layout; tile_out 0 when
+// the range does not fit or the LDS shapes are the better choice.  Host only.
+matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float mstartdm, float mdmstep, size_t pitch,
+                          std::vector<uint8_t>* bytes);
+
+// p.pair_recs: the tables on the device.
+hipError_t launch_dedisperse_matrix(const lds_params& p, const matrix_layout& lay, hipStream_t s);
+
+}  // namespace aa_hip

@@ -43,7 +43,8 @@ typedef enum {
 
 /* Kernel variants for aa_hip_dedisperse_u8 / aa_hip_ddtr_set_kernel. */
 typedef enum {
-    AA_HIP_KERNEL_AUTO = 0,     /* LDS kernel when a chunk shape fits (tuned shape if set), else direct */
+    AA_HIP_KERNEL_AUTO = 0,     /* handles: tuned LDS shape if set, else the matrix-core kernel where it is the
+                                   cheaper one; else the LDS kernel when a chunk shape fits, else direct */
     AA_HIP_KERNEL_DIRECT = 1,   /* one thread per (DM, sample), global gathers */
     AA_HIP_KERNEL_LDS = 2,      /* LDS-staged windows, packed integer sums, first shape that fits */
     AA_HIP_KERNEL_LDS_C32 = 3,  /* LDS kernel, 32-channel chunks (rows up to 2432 bytes) */
@@ -274,11 +275,14 @@ int aa_hip_ddtr_run_range(aa_hip_ddtr *h, int range, int t_processed, float *d_o
  * tiles (offsets up to 268), 5 = shape 2 on 1512-sample tiles (offsets up
  * to 520), 6 = shape 2 with 32-DM tiles (two DM trials per wave over the
  * same rows); shapes 2, 4, 5 and 6 read rows with 16-byte LDS reads.
- * set_range_variant records a preference for range r (-1 = first that
- * fits, in the order 4, 5, 2, 3, 0, 1, 6), used whenever it fits.
+ * set_range_variant records a preference for range r (-1 = automatic: the
+ * matrix-core kernel where the range's plan makes it the cheaper one, else the
+ * first shape that fits, in the order 4, 5, 2, 3, 0, 1, 6), used whenever it
+ * fits.
  * autotune_range times every shape that fits range r on `stream` (reps
- * launches each, writing d_out), keeps the fastest as the preference and
- * reports it: *best_variant (-1 if none fits) and variant_ms[0..6] (-1 =
+ * launches each, writing d_out), keeps the fastest as the preference (or -1
+ * where the matrix-core kernel is the automatic choice and faster still) and
+ * reports the fastest shape: *best_variant (-1 if none fits) and variant_ms[0..6] (-1 =
  * does not fit; the array holds 7 floats).
  * The range's level must be resident (after ingest). */
 int aa_hip_ddtr_set_range_variant(aa_hip_ddtr *h, int range, int variant);
@@ -297,7 +301,8 @@ int aa_hip_ddtr_autotune_range(aa_hip_ddtr *h, int range, int t_processed, float
  * LDS shapes in one persistent launch, the pair pre-summation shapes in one
  * launch per tile width and row width; ranges on the quad shape, or that no
  * chunk shape fits, run launches of their own after them (in the same
- * graph).  With use_graph != 0 the
+ * graph), as do ranges of at least 512 tiles that take the matrix-core kernel.
+ * With use_graph != 0 the
  * sequence is captured into a hipGraph on the first call for a given set of
  * buffers and replayed by later calls with the same buffers.  Results are
  * bit-identical to aa_hip_ddtr_execute_chunk per beam.  Calls on one batch

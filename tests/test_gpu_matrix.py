@@ -1,0 +1,75 @@
+"""The matrix-core dedispersion kernel (the automatic choice of a DdtrPlan
+range whose channel groups fit it), bit for bit against the CPU oracle at the
+edges of its tiles, groups and steps."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# name, nchans, fch1, foff, dm_low, dm_step, ndms, t_processed, inBin, fill
+GEOMS = [
+    ("one_sample_last_tile", 512, 1550.0, -0.5859, 0.0, 0.1, 64, 2 * 1888 + 1, 1, "noise"),
+    ("dm_zero_tile", 512, 1550.0, -0.5859, 0.0, 0.5, 32, 4000, 1, "noise"),         # base delays start at 0
+    ("ragged_channels", 333, 1500.0, -0.96, 12.3, 0.3, 48, 3001, 1, "noise"),       # last step part empty
+    ("ragged_trials", 512, 1550.0, -0.5859, 40.0, 0.5, 37, 2500, 1, "noise"),       # last DM tile part empty
+    ("one_trial", 1024, 1550.0, -0.29, 100.0, 0.5, 1, 1000, 1, "noise"),
+    ("saturated", 4096, 1760.0, -0.19775, 0.0, 0.1, 16, 2100, 1, "full"),           # largest sums, groups of 256
+    ("zeros", 1024, 1760.0, -0.391, 10.0, 0.2, 16, 2100, 1, "zero"),                # every byte at the signed end
+    ("two_windows", 512, 1550.0, -0.5859, 300.0, 1.0, 48, 3333, 1, "noise"),        # 8-byte windows
+    ("four_windows", 416, 1760.0, -0.96, 500.0, 1.6, 32, 3000, 2, "noise"),         # 16-byte windows, binned
+    ("many_channels", 16384, 1500.0, -0.0244140625, 0.0, 0.2, 20, 2500, 1, "noise"),
+]
+
+
+@pytest.mark.parametrize("pitch_extra", [0, 13])
+@pytest.mark.parametrize("geom", GEOMS, ids=[g[0] for g in GEOMS])
+def test_matrix_range(aa, oracle, cuda, geom, pitch_extra):
+    import torch
+    name, nchans, fch1, foff, low, step, ndms, tp, ib, fill = geom
+    print(f"matrix {name} pitch +{pitch_extra}", flush=True)
+    tsamp = 64e-6
+    ds = oracle.dmshifts(nchans, fch1, foff)
+    tsr = np.float32(np.float32(tsamp) * np.float32(ib))
+    ms, st = np.float32(np.float32(low) / tsr), np.float32(np.float32(step) / tsr)
+    maxd = int(np.trunc(np.float32(ds[-1]) * np.float32(np.float64(ndms - 1) * st + ms))) + 1
+    nsamp = (tp + maxd) * ib
+    rng = np.random.default_rng(nchans + ndms)
+    if fill == "noise":
+        data = rng.integers(0, 256, size=(nsamp, nchans), dtype=np.uint8)
+    else:
+        data = np.full((nsamp, nchans), 255 if fill == "full" else 0, dtype=np.uint8)
+        data[rng.integers(0, nsamp, 50), rng.integers(0, nchans, 50)] = 128
+    rows = oracle.corner_turn(data, nsamp, nchans)
+    for _ in range(ib.bit_length() - 1):
+        rows = oracle.bin2(rows, rows.shape[1] // 2)
+    want = oracle.dedisperse(rows[:, :tp + maxd].copy(), ds, ndms, tp, float(ms), float(st), ib)
+    plan = aa.DdtrPlan(ds, [(low, step, ndms, ib)], tsamp, maxd * ib, tp * ib)
+    d_in = torch.from_numpy(data).to(cuda)
+    for kernel in (aa.KERNEL_AUTO, aa.KERNEL_LDS):
+        plan.set_kernel(kernel)
+        out = torch.full((ndms, tp + pitch_extra), -1.0, dtype=torch.float32, device=cuda)
+        plan.ingest(d_in, tp * ib)
+        plan.run_range(0, tp, out)
+        got = out.cpu().numpy()
+        np.testing.assert_array_equal(got[:, :tp], want)
+        assert np.all(got[:, tp:] == -1.0)   # nothing written past a row's samples
+
+
+def test_matrix_choice_follows_the_kernel_setting(aa, oracle, cuda):
+    """The automatic choice, a forced shape and a preferred one, in turn on one handle."""
+    import torch
+    nchans, tsamp, tp, ndms = 512, 64e-6, 3000, 48
+    ds = oracle.dmshifts(nchans, 1550.0, -0.5859)
+    maxd = int(ds[-1] * (0.5 * ndms / tsamp)) + 2
+    data = oracle.gen_noise(5, tp + maxd, nchans)
+    plan = aa.DdtrPlan(ds, [(0.0, 0.5, ndms, 1)], tsamp, maxd, tp)
+    d_in = torch.from_numpy(data).to(cuda)
+    want = oracle.dedisperse(oracle.corner_turn(data, tp + maxd, nchans), ds, ndms, tp, 0.0,
+                             float(np.float32(0.5) / np.float32(tsamp)), 1)
+    plan.ingest(d_in, tp)
+    for kernel, variant in ((0, -1), (5, -1), (0, -1), (0, 4), (0, 1), (0, -1), (1, -1), (2, -1)):
+        plan.set_kernel(kernel)
+        plan.set_range_variant(0, variant)
+        out = torch.full((ndms, tp), -1.0, dtype=torch.float32, device=cuda)
+        plan.run_range(0, tp, out)
+        np.testing.assert_array_equal(out.cpu().numpy(), want, err_msg=f"kernel {kernel} variant {variant}")
