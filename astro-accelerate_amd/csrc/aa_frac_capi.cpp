@@ -29,11 +29,13 @@ struct aa_hip_frac {
 struct aa_hip_refine {
     int device = 0;
     int ncand = 0;
-    int grid = 0;
+    int nitems = 0;
     int loss_kind = 0;
     aa_hip::refine_cand* d_cands = nullptr;
-    int* d_order = nullptr;
-    int* d_counter = nullptr;
+    aa_hip::refine_item* d_items = nullptr;
+    aa_hip::refine_state* d_state = nullptr;
+    double* d_loss = nullptr;    // scan losses, then the gradients at the best points
+    double* d_part = nullptr;    // partial profiles of an evaluation
     double* d_power = nullptr;   // channel powers of every candidate (loss 1)
 };
 
@@ -230,7 +232,8 @@ int aa_hip_refine_create(int device, int ncand, const int64_t* x_offsets, const 
     if (ncand <= 0 || !x_offsets || !ds_offsets || !nchans || !nsamp)
         return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "invalid candidate table");
     std::vector<aa_hip::refine_cand> cands((size_t)ncand);
-    int64_t power_entries = 0;
+    int64_t power_entries = 0, part_entries = 0;
+    std::vector<aa_hip::refine_item> items;
     for (int b = 0; b < ncand; ++b) {
         if (nchans[b] <= 0 || nchans[b] > aa_hip::kRefineMaxChannels || nsamp[b] <= 0 ||
             nsamp[b] > aa_hip::kRefineMaxSamples || x_offsets[b] < 0 || ds_offsets[b] < 0)
@@ -238,14 +241,22 @@ int aa_hip_refine_create(int device, int ncand, const int64_t* x_offsets, const 
                                                       ": windows up to " + std::to_string(aa_hip::kRefineMaxChannels) +
                                                       " channels x " + std::to_string(aa_hip::kRefineMaxSamples) +
                                                       " samples, non-negative offsets");
-        cands[(size_t)b] = aa_hip::refine_cand{x_offsets[b], ds_offsets[b], power_entries, nchans[b], nsamp[b]};
+        cands[(size_t)b] =
+            aa_hip::refine_cand{x_offsets[b], ds_offsets[b], power_entries, part_entries, nchans[b], nsamp[b]};
         power_entries += nchans[b];
+        part_entries += aa_hip::refine_part_entries(nchans[b], nsamp[b]);
+        for (int c = 0; c < nchans[b]; c += aa_hip::kRefineChunk)
+            for (int g = 0; g * aa_hip::kRefineSeg < nsamp[b]; ++g)
+                items.push_back(aa_hip::refine_item{b, c / aa_hip::kRefineChunk, c,
+                                                    std::min(aa_hip::kRefineChunk, nchans[b] - c), g});
     }
-    // largest windows first (longest work items start early)
-    std::vector<int> order((size_t)ncand);
-    for (int b = 0; b < ncand; ++b) order[(size_t)b] = b;
-    std::stable_sort(order.begin(), order.end(), [&](int i, int j) {
-        return (long)cands[(size_t)i].C * cands[(size_t)i].T > (long)cands[(size_t)j].C * cands[(size_t)j].T;
+    if (items.size() > 0x7fffffffu) return fail(AA_HIP_ERROR_UNSUPPORTED, "too many windows");
+    // longest items first: the tail is made of short ones
+    std::stable_sort(items.begin(), items.end(), [&](const aa_hip::refine_item& i, const aa_hip::refine_item& j) {
+        const auto work = [&](const aa_hip::refine_item& k) {
+            return (long)k.nc * std::min(aa_hip::kRefineSeg, cands[(size_t)k.cand].T - k.seg * aa_hip::kRefineSeg);
+        };
+        return work(i) > work(j);
     });
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return fail(AA_HIP_ERROR_NO_DEVICE, "no HIP device");
@@ -257,16 +268,17 @@ int aa_hip_refine_create(int device, int ncand, const int64_t* x_offsets, const 
     int cur = 0;
     (void)hipGetDevice(&cur);
     hipError_t e = hipSetDevice(device);
-    int ncu = 0;
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device);
-    p->grid = std::max(1, ncu) * aa_hip::refine_blocks_per_cu();
+    p->nitems = (int)items.size();
     if (e == hipSuccess) e = hipMalloc(&p->d_cands, sizeof(aa_hip::refine_cand) * (size_t)ncand);
-    if (e == hipSuccess) e = hipMalloc(&p->d_order, sizeof(int) * (size_t)ncand);
-    if (e == hipSuccess) e = hipMalloc(&p->d_counter, sizeof(int));
+    if (e == hipSuccess) e = hipMalloc(&p->d_items, sizeof(aa_hip::refine_item) * items.size());
+    if (e == hipSuccess) e = hipMalloc(&p->d_state, sizeof(aa_hip::refine_state) * (size_t)ncand);
+    if (e == hipSuccess) e = hipMalloc(&p->d_loss, sizeof(double) * (size_t)ncand * (aa_hip::kRefineScan + 1));
+    if (e == hipSuccess) e = hipMalloc(&p->d_part, sizeof(double) * (size_t)part_entries);
     if (e == hipSuccess) e = hipMalloc(&p->d_power, sizeof(double) * (size_t)power_entries);
     if (e == hipSuccess)
         e = hipMemcpy(p->d_cands, cands.data(), sizeof(aa_hip::refine_cand) * (size_t)ncand, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(p->d_order, order.data(), sizeof(int) * (size_t)ncand, hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+        e = hipMemcpy(p->d_items, items.data(), sizeof(aa_hip::refine_item) * items.size(), hipMemcpyHostToDevice);
     (void)hipSetDevice(cur);
     if (e != hipSuccess) {
         const int st = from_hip(e, "aa_hip_refine_create");
@@ -280,8 +292,10 @@ int aa_hip_refine_create(int device, int ncand, const int64_t* x_offsets, const 
 int aa_hip_refine_destroy(aa_hip_refine* h) {
     if (!h) return AA_HIP_SUCCESS;
     if (h->d_cands) (void)hipFree(h->d_cands);
-    if (h->d_order) (void)hipFree(h->d_order);
-    if (h->d_counter) (void)hipFree(h->d_counter);
+    if (h->d_items) (void)hipFree(h->d_items);
+    if (h->d_state) (void)hipFree(h->d_state);
+    if (h->d_loss) (void)hipFree(h->d_loss);
+    if (h->d_part) (void)hipFree(h->d_part);
     if (h->d_power) (void)hipFree(h->d_power);
     delete h;
     return AA_HIP_SUCCESS;
@@ -307,8 +321,9 @@ int aa_hip_refine_run(aa_hip_refine* h, const float* d_x, const float* d_delay_p
     a.x = d_x;
     a.ds = d_delay_per_dm;
     a.cands = h->d_cands;
-    a.order = h->d_order;
+    a.items = h->d_items;
     a.ncand = h->ncand;
+    a.nitems = h->nitems;
     a.u = d_u;
     a.step = d_step;
     a.prev_grad = d_prev_grad;
@@ -320,10 +335,13 @@ int aa_hip_refine_run(aa_hip_refine* h, const float* d_x, const float* d_delay_p
     a.scan_n = scan_n;
     a.scan_lo = scan_lo;
     a.scan_step = scan_step;
-    a.counter = h->d_counter;
+    a.cur = h->d_state;
+    a.scan_loss = h->d_loss;
+    a.best_grad = h->d_loss + (size_t)h->ncand * aa_hip::kRefineScan;
+    a.part = h->d_part;
     a.loss_kind = h->loss_kind;
     a.power = h->d_power;
-    return from_hip(aa_hip::launch_refine(a, h->grid, (hipStream_t)stream), "refine");
+    return from_hip(aa_hip::launch_refine(a, (hipStream_t)stream), "refine");
 }
 
 }  // extern "C"

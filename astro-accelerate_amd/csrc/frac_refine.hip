@@ -24,25 +24,34 @@
 // An optional coarse scan first evaluates L (forward pass only) at scan_n
 // offsets u + scan_lo + k * scan_step and starts the steps from the best.
 //
-// One persistent launch: a work-group (1024 threads) takes candidates from a
-// queue (largest first) and runs every step of that candidate itself, so the
-// forward pass, the adjoint pass and the update are fused.  Thread layout: a
-// group of S lanes covers the window's samples, 4 consecutive samples per
-// lane (S = ceil(T / 4) rounded up to whole waves), and the work-group holds
-// G = 1024 / S such groups, each summing every G-th channel; so short windows
-// keep every lane busy.  A lane reads its 4 samples x[c][4s + i_c ..
-// 4s + i_c + 3] as one 16-byte load, 4 channels in flight; the taps that
-// reach into the next lane's samples are exchanged once per pass through
-// LDS (pass 1) or folded into per-lane weights (pass 2).
-// Pass 1 sums the groups' partial profiles in double, adds them in LDS in
-// group order, pass 2 re-reads the windows (recomputation: no shifted tile is
-// stored) and accumulates the DM derivative, and thread 0 applies a
-// sign-based adaptive step (Rprop: the step grows by 1.2 while the sign of
-// dL/du holds and halves when it flips); the result is the best point
-// visited.  Every sum runs in a fixed order: results do not depend on
-// scheduling.  Windows are read straight from global memory: with one trial
-// per candidate there is no reuse to stage, and the passes are bound by HBM
-// bandwidth.
+// One evaluation is one pass over the windows: dy/du (t) = sum_c ds[c] (x[c][t +
+// i_c + 1] - x[c][t + i_c]) does not depend on y, so the pass accumulates y and
+// dy/du together and dE/du = 2 sum_t y dy/du follows from them.  The scan's
+// points (kScan at a time) share one pass too.
+//
+// Work split: an item is up to kChunk channels x kSeg samples of one window, a
+// 256-thread work-group each, so that windows of any number and size spread
+// over the whole GPU.  A group of S lanes covers the item's samples, 4
+// consecutive ones per lane, and the work-group holds G = 256 / S such groups,
+// each summing every G-th channel.  A lane reads its 4 samples x[c][t0 + i_c ..
+// t0 + i_c + 3] as one 16-byte load; the second tap of the sample before them
+// is kept apart and added to it after the pass.  Sums are double; the groups'
+// are added in LDS and the items' by one work-group per candidate
+// (refine_combine_kernel), which also applies the sign-based adaptive step
+// (Rprop: the step grows by 1.2 while the sign of dL/du holds and halves when
+// it flips); the result is the best point visited.  Every sum runs in a fixed
+// order: results do not depend on scheduling.  An evaluation is two launches.
+//
+// Bound: HBM (each pass reads every window once; the partial profiles add 2 to
+// 3 % of that).  Measured on 256 windows (1024-4096 channels x 256-4096
+// samples, 3.64 GB; 9-point scan and 20 steps): 22.2 ms, of which a gradient
+// pass takes 0.75 ms (4.85 TB/s; a 4 GiB device copy does 4.77), its combine
+// 0.04, a scan pass of 3 points 1.45, the channel powers 1.05.  With one
+// work-group per window, two passes per evaluation and one per scan point it
+// took 178 ms (the largest windows' work-groups ran long after the others).
+// Scan points per pass: 9 in one took 6.1 ms (150 registers), 5 and 4 took
+// 2 x 2.4, 3 take 3 x 1.45; two channels in flight per lane in a scan pass 1.88
+// instead of 1.45 (the window-edge branch of each load).
 #include "frac_refine.h"
 
 #include <cmath>
@@ -51,45 +60,14 @@ namespace aa_hip {
 
 namespace {
 
-constexpr int kThreads = 1024;
+constexpr int kThreads = kRefineThreads;
 constexpr int kSpt = 4;                       // consecutive samples per lane
 constexpr int kU = 4;                         // channels in flight per lane
-constexpr int kYSlots = kThreads * kSpt;      // the groups' partial profiles (G * T <= 4096)
-static_assert(kRefineMaxSamples <= kYSlots, "a window's samples fit one lane span each");
-
-__shared__ int2 r_tab[kRefineMaxChannels];   // (i_c, f_c bits) of the current u
-__shared__ double r_y[kYSlots];
-__shared__ double r_red[32];
-__shared__ float r_u;
-__shared__ long r_item;
-
-__device__ __forceinline__ double block_sum(double v, int tid)
-{
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    __syncthreads();                        // r_red free (previous reduction read)
-    if ((tid & 63) == 0) r_red[tid >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
-    for (int i = 0; i < kThreads / 64; ++i) s += r_red[i];
-    return s;
-}
-
-struct lane_layout {
-    int G;        // groups in the work-group
-    int g, s;     // this lane's group and position in it
-    bool active;  // g < G
-};
-
-__device__ __forceinline__ lane_layout layout_of(int T, int tid)
-{
-    const int S = ((T + kSpt - 1) / kSpt + 63) / 64 * 64;   // <= 1024 for T <= 4096
-    lane_layout L;
-    L.G = kThreads / S;
-    L.g = tid / S;
-    L.s = tid - L.g * S;
-    L.active = L.g < L.G;
-    return L;
-}
+constexpr int kSeg = kRefineSeg;
+constexpr int kChunk = kRefineChunk;
+constexpr int kScan = kRefineScan;
+constexpr int kCombineThreads = 1024;
+static_assert(kSeg == kThreads * kSpt, "a segment's samples fit one lane span each");
 
 // w[m] = row[j + m], m = 0..3, zero outside [0, T).
 __device__ __forceinline__ void load4(const float* __restrict__ row, int j, int T, float (&w)[4])
@@ -115,217 +93,282 @@ __device__ __forceinline__ float load1(const float* __restrict__ row, int i, int
     return (i >= 0 && i < T) ? row[i] : 0.0f;
 }
 
-// (L, dL/du) of candidate `cd` at residual DM u; every thread gets both
-// (dL/du only when want_grad).  power: the candidate's channel powers v_c
-// (loss 1) or null (loss 0).
-__device__ void evaluate(const refine_args& a, const refine_cand& cd, const double* __restrict__ power, float u,
-                         int tid, bool want_grad, double* loss, double* grad)
+// Integer and fractional delay of a channel at residual DM u.
+__device__ __forceinline__ int2 delay_of(float ds, float u)
 {
-    const float* __restrict__ x = a.x + cd.x_off;
-    const float* __restrict__ ds = a.ds + cd.ds_off;
-    const int C = cd.C, T = cd.T;
-    double npart = 0.0, dnpart = 0.0;   // this thread's channels of N and dN/du
-    __syncthreads();  // r_tab and r_y free
-    for (int c = tid; c < C; c += kThreads) {
-        const double d = (double)ds[c];
-        const double tau = d * (double)u;
-        const double fl = fmin(fmax(floor(tau), -1073741824.0), 1073741824.0);
-        const float f32 = (float)(tau - fl);
-        const int i = (int)fl;
-        r_tab[c] = make_int2(i, __float_as_int(f32));
-        if (power) {
-            const double f = (double)f32;       // the weight the passes use
-            const double n0 = (double)max(0, T - abs(i)), n1 = (double)max(0, T - abs(i + 1));
-            const double v = power[c];
-            npart = __builtin_fma(v, (1.0 - f) * (1.0 - f) * n0 + f * f * n1, npart);
-            dnpart = __builtin_fma(v * d, 2.0 * f * n1 - 2.0 * (1.0 - f) * n0, dnpart);
-        }
-    }
-    __syncthreads();
-
-    // pass 1: this group's channels of the profile at the lane's 4 samples.
-    // A lane reads only its own 4 samples x[c][t0 + i_c + m]; the second tap
-    // of sample t0 - 1 (f x[c][t0 + i_c]) is its left neighbour's, kept in yn
-    // and added to the neighbour's sample in LDS after the pass.  The last
-    // lane of a group also reads x[c][4S + i_c] when its last sample, 4S - 1,
-    // is inside the window (T = 4S).
-    const lane_layout L = layout_of(T, tid);
-    const int t0 = kSpt * L.s;
-    const int S = kThreads / L.G;
-    const bool edge = L.active && L.s == S - 1 && kSpt * S == T;
-    double y[kSpt], yn = 0.0;
-#pragma unroll
-    for (int m = 0; m < kSpt; ++m) y[m] = 0.0;
-    if (L.active) {
-        int c = L.g;
-        for (; c + (kU - 1) * L.G < C; c += kU * L.G) {
-            float w[kU][4];
-            double f[kU];
-            int i0[kU];
-#pragma unroll
-            for (int k = 0; k < kU; ++k) {
-                const int cc = c + k * L.G;
-                const int2 e = r_tab[cc];
-                f[k] = (double)__int_as_float(e.y);
-                i0[k] = e.x;
-                load4(x + (size_t)cc * T, t0 + e.x, T, w[k]);
-            }
-#pragma unroll
-            for (int k = 0; k < kU; ++k) {
-#pragma unroll
-                for (int m = 0; m < kSpt; ++m) y[m] = __builtin_fma(1.0 - f[k], (double)w[k][m], y[m]);
-#pragma unroll
-                for (int m = 1; m < kSpt; ++m) y[m - 1] = __builtin_fma(f[k], (double)w[k][m], y[m - 1]);
-                yn = __builtin_fma(f[k], (double)w[k][0], yn);
-                if (edge) y[kSpt - 1] = __builtin_fma(f[k], (double)load1(x + (size_t)(c + k * L.G) * T, T + i0[k], T),
-                                                      y[kSpt - 1]);
-            }
-        }
-        for (; c < C; c += L.G) {
-            float w[4];
-            const int2 e = r_tab[c];
-            const double f = (double)__int_as_float(e.y);
-            load4(x + (size_t)c * T, t0 + e.x, T, w);
-#pragma unroll
-            for (int m = 0; m < kSpt; ++m) y[m] = __builtin_fma(1.0 - f, (double)w[m], y[m]);
-#pragma unroll
-            for (int m = 1; m < kSpt; ++m) y[m - 1] = __builtin_fma(f, (double)w[m], y[m - 1]);
-            yn = __builtin_fma(f, (double)w[0], yn);
-            if (edge) y[kSpt - 1] = __builtin_fma(f, (double)load1(x + (size_t)c * T, T + e.x, T), y[kSpt - 1]);
-        }
-#pragma unroll
-        for (int m = 0; m < kSpt; ++m)
-            if (t0 + m < T) r_y[L.g * T + t0 + m] = y[m];
-    }
-    __syncthreads();
-    if (L.active && t0 >= 1 && t0 - 1 < T) r_y[L.g * T + t0 - 1] += yn;   // one lane per slot
-    __syncthreads();
-    // the whole profile at the lane's samples and at t0 - 1: groups added in order
-    double l2 = 0.0, yp = 0.0;
-    if (L.active) {
-#pragma unroll
-        for (int m = 0; m < kSpt; ++m) {
-            double s = 0.0;
-            if (t0 + m < T)
-                for (int g = 0; g < L.G; ++g) s += r_y[g * T + t0 + m];
-            y[m] = s;                                   // 0 outside 0 <= t < T
-            if (L.g == 0) l2 = __builtin_fma(s, s, l2);
-        }
-        if (t0 >= 1 && t0 - 1 < T)
-            for (int g = 0; g < L.G; ++g) yp += r_y[g * T + t0 - 1];
-    }
-
-    if (!want_grad) {
-        *loss = block_sum(l2 - npart, tid);
-        *grad = 0.0;
-        return;
-    }
-    // pass 2: dE/du over this group's channels, recomputing the window reads:
-    // sum_t y(t) (x(t + i + 1) - x(t + i)) = sum_t (y(t - 1) - y(t)) x(t + i)
-    // + y(4S - 1) x(4S + i), so each lane weighs its own 4 samples by
-    // D[m] = y(t0 + m - 1) - y(t0 + m) (and the last lane, when T = 4S, its
-    // sample 4S + i by y(T - 1)).
-    double D[kSpt];
-    D[0] = yp - y[0];
-#pragma unroll
-    for (int m = 1; m < kSpt; ++m) D[m] = y[m - 1] - y[m];
-    double gs = 0.0;
-    if (L.active) {
-        int c = L.g;
-        for (; c + (kU - 1) * L.G < C; c += kU * L.G) {
-            float w[kU][4];
-            int i0[kU];
-#pragma unroll
-            for (int k = 0; k < kU; ++k) {
-                const int cc = c + k * L.G;
-                i0[k] = r_tab[cc].x;
-                load4(x + (size_t)cc * T, t0 + i0[k], T, w[k]);
-            }
-#pragma unroll
-            for (int k = 0; k < kU; ++k) {
-                double s = 0.0;
-#pragma unroll
-                for (int m = 0; m < kSpt; ++m) s = __builtin_fma(D[m], (double)w[k][m], s);
-                if (edge) s = __builtin_fma(y[kSpt - 1], (double)load1(x + (size_t)(c + k * L.G) * T, T + i0[k], T), s);
-                gs = __builtin_fma((double)ds[c + k * L.G], s, gs);
-            }
-        }
-        for (; c < C; c += L.G) {
-            float w[4];
-            const int i0 = r_tab[c].x;
-            load4(x + (size_t)c * T, t0 + i0, T, w);
-            double s = 0.0;
-#pragma unroll
-            for (int m = 0; m < kSpt; ++m) s = __builtin_fma(D[m], (double)w[m], s);
-            if (edge) s = __builtin_fma(y[kSpt - 1], (double)load1(x + (size_t)c * T, T + i0, T), s);
-            gs = __builtin_fma((double)ds[c], s, gs);
-        }
-    }
-    *loss = block_sum(l2 - npart, tid);
-    *grad = block_sum(2.0 * gs - dnpart, tid);
+    const double tau = (double)ds * (double)u;
+    const double fl = fmin(fmax(floor(tau), -1073741824.0), 1073741824.0);
+    return make_int2((int)fl, __float_as_int((float)(tau - fl)));
 }
 
-__global__ __launch_bounds__(kThreads) void refine_kernel(refine_args a)
+// Profile sample t of a window lies at t + t / kSeg of a partial profile; the
+// entry after a full segment takes the next segment's share of its last sample.
+// Sums of NP profiles `row` entries apart over the window's chunks, in order.
+template <int NP>
+__device__ __forceinline__ void profile_at(const double* __restrict__ part, size_t stride, int row, int nchunk, int t,
+                                           int T, double (&v)[NP])
 {
-    const int tid = threadIdx.x;
-    for (;;) {
-        if (tid == 0) r_item = (long)atomicAdd(a.counter, 1);
-        __syncthreads();
-        const long item = r_item;
-        __syncthreads();
-        if (item >= a.ncand) break;
-        const int b = a.order[item];
-        const refine_cand cd = a.cands[b];
-        const double* power = a.loss_kind == 1 ? a.power + cd.power_off : nullptr;
-        if (tid == 0) r_u = a.u[b];
-        __syncthreads();
-        float step = a.step[b];
-        double prev = a.prev_grad[b];
-        double loss = 0.0, grad = 0.0;
-        if (a.scan_n > 0) {  // coarse scan around u; the best offset starts the steps
-            const float u0 = r_u;
-            float best_u = u0;
-            double best_l = -INFINITY;
-            for (int k = 0; k < a.scan_n; ++k) {
-                const float uk = u0 + a.scan_lo + a.scan_step * (float)k;
-                evaluate(a, cd, power, uk, tid, false, &loss, &grad);
-                if (loss > best_l) {
-                    best_l = loss;
-                    best_u = uk;
-                }
-            }
-            if (tid == 0) r_u = best_u;
-            __syncthreads();
-        }
-        float best_u = r_u;
-        double best_l = -INFINITY, best_g = 0.0;
-        for (int s = 0; s <= a.nsteps; ++s) {
-            const float u = r_u;
-            evaluate(a, cd, power, u, tid, true, &loss, &grad);
-            if (loss > best_l) {  // the result is the best point visited
-                best_l = loss;
-                best_u = u;
-                best_g = grad;
-            }
-            if (s == a.nsteps) break;
-            if (tid == 0) {
-                if (grad * prev > 0.0) step = fminf(step * 1.2f, a.step_max);
-                else if (grad * prev < 0.0) step = fmaxf(step * 0.5f, a.step_min);
-                const float du = grad > 0.0 ? step : (grad < 0.0 ? -step : 0.0f);
-                r_u = u + du;
-                prev = grad;
-            }
-            __syncthreads();
-        }
-        if (tid == 0) {
-            a.u[b] = best_u;
-            a.step[b] = step;
-            a.prev_grad[b] = prev;
-            a.loss[b] = best_l;
-            a.grad[b] = best_g;
-        }
-        __syncthreads();
+    const double* q = part + t + t / kSeg;
+    double e[NP];
+#pragma unroll
+    for (int n = 0; n < NP; ++n) v[n] = e[n] = 0.0;
+#pragma unroll 8
+    for (int j = 0; j < nchunk; ++j)
+#pragma unroll
+        for (int n = 0; n < NP; ++n) v[n] += q[(size_t)j * stride + (size_t)n * row];
+    if ((t + 1) % kSeg == 0 && t + 1 < T) {
+        for (int j = 0; j < nchunk; ++j)
+#pragma unroll
+            for (int n = 0; n < NP; ++n) e[n] += q[(size_t)j * stride + (size_t)n * row + 1];
     }
+#pragma unroll
+    for (int n = 0; n < NP; ++n) v[n] += e[n];
+}
+
+// Partial profiles of one item.  NK = 0: y and dy/du at the candidate's current
+// u (2 arrays); NK = kScan: y at scan points k0 .. k0 + nk - 1 (nk arrays).
+template <int NK>
+__global__ __launch_bounds__(kThreads) void refine_partial_kernel(refine_args a, int k0, int nk)
+{
+    constexpr int K = NK ? NK : 1;
+    __shared__ int2 tab[K][kChunk];        // (i_c, f_c bits)
+    __shared__ float dsv[kChunk];
+    __shared__ double r_y[kSeg], r_p[NK ? 1 : kSeg + 8];
+    __shared__ double r_b[2][kThreads / 64];
+    const refine_item it = a.items[blockIdx.x];
+    const refine_cand cd = a.cands[it.cand];
+    const int tid = threadIdx.x, T = cd.T, C = it.nc, t_first = it.seg * kSeg;
+    const int nt = min(kSeg, T - t_first);
+    const bool last_seg = t_first + nt == T;
+    const float* __restrict__ x = a.x + cd.x_off + (size_t)it.c0 * T;
+    const float u0 = NK ? a.u[it.cand] : a.cur[it.cand].u;
+    for (int c = tid; c < C; c += kThreads) {
+        const float d = a.ds[cd.ds_off + it.c0 + c];
+        dsv[c] = d;
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            tab[k][c] = delay_of(d, NK ? u0 + a.scan_lo + a.scan_step * (float)(k0 + k) : u0);
+    }
+    __syncthreads();
+
+    // samples t_first .. t_first + nt - 1 and, in the window's last segment, T:
+    // its taps are the second ones of sample T - 1.  A full last segment has no
+    // lane for it: its last lane reads it in addition (edge).
+    const int ns = min(kSeg, nt + (last_seg ? 1 : 0));
+    const int S = ((ns + kSpt - 1) / kSpt + 63) / 64 * 64;
+    const int G = kThreads / S, g = tid / S, s = tid - g * S;
+    const bool active = g < G && kSpt * s < ns;
+    const int t0 = t_first + kSpt * s;
+    const bool any_edge = last_seg && nt == kSeg, edge = any_edge && s == S - 1;
+    double y[K][kSpt], yn[K], P[kSpt], pe = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        yn[k] = 0.0;
+#pragma unroll
+        for (int m = 0; m < kSpt; ++m) y[k][m] = 0.0;
+    }
+#pragma unroll
+    for (int m = 0; m < kSpt; ++m) P[m] = 0.0;
+    auto add = [&](int k, int c, const float (&w)[4]) {
+        const int2 e = tab[k][c];
+        const double f = (double)__int_as_float(e.y);
+#pragma unroll
+        for (int m = 0; m < kSpt; ++m) y[k][m] = __builtin_fma(1.0 - f, (double)w[m], y[k][m]);
+#pragma unroll
+        for (int m = 1; m < kSpt; ++m) y[k][m - 1] = __builtin_fma(f, (double)w[m], y[k][m - 1]);
+        yn[k] = __builtin_fma(f, (double)w[0], yn[k]);
+        if (!NK) {
+            const double d = (double)dsv[c];
+#pragma unroll
+            for (int m = 0; m < kSpt; ++m) P[m] = __builtin_fma(d, (double)w[m], P[m]);
+        }
+        if (any_edge && edge) {
+            const double v = (double)load1(x + (size_t)c * T, T + e.x, T);
+            y[k][kSpt - 1] = __builtin_fma(f, v, y[k][kSpt - 1]);
+            if (!NK) pe = __builtin_fma((double)dsv[c], v, pe);
+        }
+    };
+    if (active) {
+        constexpr int U = NK ? 1 : kU;
+        int c = g;
+        for (; c + (U - 1) * G < C; c += U * G) {
+            float w[U * K][4];
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    if (!NK || k < nk)
+                        load4(x + (size_t)(c + i * G) * T, t0 + tab[k][c + i * G].x, T, w[i * K + k]);
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    if (!NK || k < nk) add(k, c + i * G, w[i * K + k]);
+        }
+        for (; c < C; c += G) {
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (!NK || k < nk) {
+                    float w[4];
+                    load4(x + (size_t)c * T, t0 + tab[k][c].x, T, w);
+                    add(k, c, w);
+                }
+        }
+    }
+
+    const int row = T + (T - 1) / kSeg;              // entries of a profile
+    const int S4 = kSpt * S;                         // one group's samples in LDS (G * S4 <= kSeg)
+    double* __restrict__ out = a.part + cd.part_off + (size_t)it.chunk * (NK ? kScan : 2) * row;
+    const int o = t_first + it.seg;                  // first entry of the segment
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (NK && k >= nk) continue;   // (not break: k stays a constant in the unrolled body)
+        __syncthreads();
+        if (g < G) {
+#pragma unroll
+            for (int m = 0; m < kSpt; ++m) r_y[g * S4 + kSpt * s + m] = y[k][m];
+            if (!NK) {
+#pragma unroll
+                for (int m = 0; m < kSpt; ++m) r_p[g * S4 + kSpt * s + m] = P[m];
+            }
+        }
+        __syncthreads();
+        if (g < G) {
+            if (s > 0) r_y[g * S4 + kSpt * s - 1] += yn[k];   // one lane per entry
+            else r_b[0][g] = yn[k];
+            if (!NK && s == 0) r_b[1][g] = P[0];
+            if (!NK && G == 1 && s == S - 1) r_p[S4] = pe;    // sample T, or the next segment's
+        }
+        __syncthreads();
+        for (int t = tid; t < nt; t += kThreads) {
+            double v = 0.0, p = 0.0;
+            for (int h = 0; h < G; ++h) {
+                v += r_y[h * S4 + t];
+                if (!NK) p += r_p[h * S4 + t + 1] - r_p[h * S4 + t];
+            }
+            out[(size_t)k * row + o + t] = v;
+            if (!NK) out[(size_t)row + o + t] = p;
+        }
+        if (tid == 0 && it.seg > 0) {
+            double v = 0.0, p = 0.0;
+            for (int h = 0; h < G; ++h) {
+                v += r_b[0][h];
+                if (!NK) p += r_b[1][h];
+            }
+            out[(size_t)k * row + o - 1] = v;
+            if (!NK) out[(size_t)row + o - 1] = p;
+        }
+    }
+}
+
+__device__ __forceinline__ double block_sum(double v, double* red, int tid)
+{
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    __syncthreads();                        // red free (previous reduction read)
+    if ((tid & 63) == 0) red[tid >> 6] = v;
+    __syncthreads();
+    double s = 0.0;
+    for (int i = 0; i < kCombineThreads / 64; ++i) s += red[i];
+    return s;
+}
+
+// This thread's channels of the noise energy N (loss 1) and dN/du at u.
+__device__ __forceinline__ void noise_part(const refine_args& a, const refine_cand& cd, float u, int tid, double* n,
+                                           double* dn)
+{
+    *n = *dn = 0.0;
+    if (a.loss_kind != 1) return;
+    for (int c = tid; c < cd.C; c += kCombineThreads) {
+        const float ds = a.ds[cd.ds_off + c];
+        const int2 e = delay_of(ds, u);
+        const double f = (double)__int_as_float(e.y);       // the weight the passes use
+        const double n0 = (double)max(0, cd.T - abs(e.x)), n1 = (double)max(0, cd.T - abs(e.x + 1));
+        const double v = a.power[cd.power_off + c];
+        *n = __builtin_fma(v, (1.0 - f) * (1.0 - f) * n0 + f * f * n1, *n);
+        *dn = __builtin_fma(v * (double)ds, 2.0 * f * n1 - 2.0 * (1.0 - f) * n0, *dn);
+    }
+}
+
+// Loss at scan point k0 + blockIdx.y of candidate blockIdx.x.
+__global__ __launch_bounds__(kCombineThreads) void refine_scan_loss_kernel(refine_args a, int k0)
+{
+    __shared__ double red[kCombineThreads / 64];
+    const int b = blockIdx.x, k = blockIdx.y, tid = threadIdx.x;
+    const refine_cand cd = a.cands[b];
+    const int row = cd.T + (cd.T - 1) / kSeg, nchunk = (cd.C + kChunk - 1) / kChunk;
+    const double* part = a.part + cd.part_off + (size_t)k * row;
+    double l2 = 0.0, n, dn;
+    for (int t = tid; t < cd.T; t += kCombineThreads) {
+        double v[1];
+        profile_at(part, (size_t)kScan * row, row, nchunk, t, cd.T, v);
+        l2 = __builtin_fma(v[0], v[0], l2);
+    }
+    noise_part(a, cd, a.u[b] + a.scan_lo + a.scan_step * (float)(k0 + k), tid, &n, &dn);
+    const double l = block_sum(l2 - n, red, tid);
+    if (tid == 0) a.scan_loss[(size_t)b * kScan + k] = l;
+}
+
+// Starts the candidates' states (k0 = 0), then takes in the losses of scan
+// points k0 .. k0 + nk - 1, in order.
+__global__ void refine_start_kernel(refine_args a, int k0, int nk)
+{
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= a.ncand) return;
+    refine_state st = k0 == 0 ? refine_state{a.u[b], a.step[b], a.u[b], a.prev_grad[b], -INFINITY, 0.0} : a.cur[b];
+    for (int k = 0; k < nk; ++k) {
+        const double l = a.scan_loss[(size_t)b * kScan + k];
+        if (l > st.best_l) {
+            st.best_l = l;
+            st.best_u = a.u[b] + a.scan_lo + a.scan_step * (float)(k0 + k);
+        }
+    }
+    if (k0 + nk >= a.scan_n) {   // the steps start from the best point
+        st.u = st.best_u;
+        st.best_l = -INFINITY;
+    }
+    a.cur[b] = st;
+}
+
+// One candidate's loss and gradient from the partial profiles, and its step.
+__global__ __launch_bounds__(kCombineThreads) void refine_combine_kernel(refine_args a, int last)
+{
+    __shared__ double red[kCombineThreads / 64];
+    const int b = blockIdx.x, tid = threadIdx.x;
+    const refine_cand cd = a.cands[b];
+    const int row = cd.T + (cd.T - 1) / kSeg, nchunk = (cd.C + kChunk - 1) / kChunk;
+    const double* part = a.part + cd.part_off;
+    refine_state st = a.cur[b];
+    double l2 = 0.0, gs = 0.0, n, dn;
+    for (int t = tid; t < cd.T; t += kCombineThreads) {
+        double v[2];   // y, dy/du
+        profile_at(part, 2 * (size_t)row, row, nchunk, t, cd.T, v);
+        l2 = __builtin_fma(v[0], v[0], l2);
+        gs = __builtin_fma(v[0], v[1], gs);
+    }
+    noise_part(a, cd, st.u, tid, &n, &dn);
+    const double loss = block_sum(l2 - n, red, tid);
+    const double grad = block_sum(2.0 * gs - dn, red, tid);
+    if (tid != 0) return;
+    if (loss > st.best_l) {  // the result is the best point visited
+        st.best_l = loss;
+        st.best_u = st.u;
+        a.best_grad[b] = grad;
+    } else if (st.best_l == -INFINITY) {
+        a.best_grad[b] = 0.0;
+    }
+    if (last) {
+        a.u[b] = st.best_u;
+        a.step[b] = st.step;
+        a.prev_grad[b] = st.prev;
+        a.loss[b] = st.best_l;
+        a.grad[b] = a.best_grad[b];
+        return;
+    }
+    if (grad * st.prev > 0.0) st.step = fminf(st.step * 1.2f, a.step_max);
+    else if (grad * st.prev < 0.0) st.step = fmaxf(st.step * 0.5f, a.step_min);
+    st.u = st.u + (grad > 0.0 ? st.step : (grad < 0.0 ? -st.step : 0.0f));
+    st.prev = grad;
+    a.cur[b] = st;
 }
 
 // v_c = mean_t x[c][t]^2 of every candidate's channels: work-group (b, y)
@@ -363,29 +406,27 @@ __global__ __launch_bounds__(256) void refine_power_kernel(refine_args a)
     }
 }
 
-__global__ void refine_reset_kernel(int* counter)
-{
-    if (threadIdx.x == 0) *counter = 0;
-}
-
 }  // namespace
 
-int refine_blocks_per_cu()
-{
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, refine_kernel, kThreads, 0) != hipSuccess || n < 1) n = 1;
-    return n;
-}
-
-hipError_t launch_refine(const refine_args& a, int grid, hipStream_t s)
+hipError_t launch_refine(const refine_args& a, hipStream_t s)
 {
     if (a.ncand <= 0) return hipSuccess;
-    if (grid <= 0 || (a.loss_kind != 0 && a.loss_kind != 1) || (a.loss_kind == 1 && !a.power))
-        return hipErrorInvalidValue;
+    if (a.nitems <= 0 || (a.loss_kind != 0 && a.loss_kind != 1)) return hipErrorInvalidValue;
+    const unsigned n = (unsigned)a.ncand, ni = (unsigned)a.nitems;
     if (a.loss_kind == 1)
-        hipLaunchKernelGGL(refine_power_kernel, dim3((unsigned)a.ncand, kPowerBlocksY), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(refine_reset_kernel, dim3(1), dim3(64), 0, s, a.counter);
-    hipLaunchKernelGGL(refine_kernel, dim3((unsigned)grid), dim3(kThreads), 0, s, a);
+        hipLaunchKernelGGL(refine_power_kernel, dim3(n, kPowerBlocksY), dim3(256), 0, s, a);
+    for (int k0 = 0; k0 == 0 || k0 < a.scan_n; k0 += kScan) {
+        const int nk = a.scan_n - k0 < kScan ? a.scan_n - k0 : kScan;
+        if (nk > 0) {
+            hipLaunchKernelGGL(refine_partial_kernel<kScan>, dim3(ni), dim3(kThreads), 0, s, a, k0, nk);
+            hipLaunchKernelGGL(refine_scan_loss_kernel, dim3(n, (unsigned)nk), dim3(kCombineThreads), 0, s, a, k0);
+        }
+        hipLaunchKernelGGL(refine_start_kernel, dim3((n + 63) / 64), dim3(64), 0, s, a, k0, nk);
+    }
+    for (int i = 0; i <= a.nsteps; ++i) {
+        hipLaunchKernelGGL(refine_partial_kernel<0>, dim3(ni), dim3(kThreads), 0, s, a, 0, 0);
+        hipLaunchKernelGGL(refine_combine_kernel, dim3(n), dim3(kCombineThreads), 0, s, a, i == a.nsteps ? 1 : 0);
+    }
     return hipGetLastError();
 }
 

@@ -712,8 +712,8 @@ def bench_multibeam(args):
 def bench_refine(args):
     """Batched DM refinement: 1024 candidate windows of uneven size (1024-4096
     channels x 256-4096 float32 samples, N(0,1) + Gaussian pulse at a residual
-    DM uniform in +-1), 20 fused forward + adjoint + update steps per
-    candidate in one launch; accuracy against the injected DM and against a
+    DM uniform in +-1), 20 forward + adjoint + update steps per
+    candidate, two launches a step for all of them; accuracy against the injected DM and against a
     dense DM-grid search (448 trials, step 0.01) through the plain u8 path."""
     import torch
     import frac_ddtr
@@ -759,9 +759,9 @@ def bench_refine(args):
     log(f"[bench] refine: {ms:.2f} ms for {nsteps} steps x {n} windows; |u - r| median {np.median(err):.4f} "
         f"p90 {np.percentile(err, 90):.4f}; dense grid (plain path) {t_grid:.2f} s, median {np.median(err_grid):.4f} "
         f"p90 {np.percentile(err_grid, 90):.4f}")
-    # each of the nsteps + 1 evaluations reads every window twice (forward, recomputing
-    # adjoint), each scan point once, and the channel powers of the loss once
-    bytes_read = 4.0 * elems * (2 * (nsteps + 1) + SCAN[0] + 1)
+    # each of the nsteps + 1 evaluations reads every window once, as do every 3 scan points
+    # and the channel powers of the loss
+    bytes_read = 4.0 * elems * ((nsteps + 1) + (SCAN[0] + 2) // 3 + 1)
     gbs = bytes_read / (ms * 1e-3) / 1e9
     result = {
         "metric": "DM×sample/s bit-exact, % FP32 add roofline; batched vs per-beam speedup",

@@ -488,8 +488,8 @@ int aa_hip_frac_adjoint(aa_hip_frac *h, const float *d_x, const float *d_gy, int
  * counterpart).  Candidate b's window is float [nchans[b]][nsamp[b]] at
  * d_x + x_offsets[b] (elements), its delay-per-unit-DM table nchans[b]
  * floats at d_delay_per_dm + ds_offsets[b]; up to 4096 x 4096.  For its
- * residual DM u[b] the loss L and dL/du are evaluated by one fused forward +
- * adjoint pass (the adjoint recomputes the interpolation).  The loss
+ * residual DM u[b] the loss L and dL/du are evaluated by one pass over the
+ * windows (the profile and its derivative together).  The loss
  * (aa_hip_refine_set_loss; default AA_HIP_REFINE_LOSS_ENERGY) is
  *   ENERGY:        E = sum_t y(t)^2 of the dedispersed profile y (the
  *                  aa_hip_frac_forward transform with one trial at offset 0);
@@ -503,8 +503,8 @@ int aa_hip_frac_adjoint(aa_hip_frac *h, const float *d_x, const float *d_gy, int
  * at u + scan_lo + k * scan_step, k < scan_n, and the best point starts the
  * steps.  Then u[b] climbs L by nsteps sign-based adaptive steps:
  * step[b] grows x1.2 (up to step_max) while the sign of dL/du holds and
- * halves (down to step_min) when it flips; u += sign(dL/du) * step.  One
- * persistent launch for all candidates and steps.  u receives the best point
+ * halves (down to step_min) when it flips; u += sign(dL/du) * step.  Two
+ * launches per evaluation, for all candidates together.  u receives the best point
  * visited (largest L), loss and grad L and dL/du there; step and prev_grad
  * (initialise prev_grad to 0) carry the step state.  nsteps = 0 only
  * evaluates (after the scan, if any). */
