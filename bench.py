@@ -780,7 +780,7 @@ def bench_refine(args):
                                            "p90": float(np.percentile(err_grid, 90)), "max": float(err_grid.max()),
                                            "trials": 448, "step": 0.01, "seconds": t_grid},
         "roofline": {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS,
-                     "traffic": None, "kernel": "refine_kernel (fused forward + adjoint + update)"},
+                     "traffic": None, "kernel": "refine_partial_kernel (profile and derivative in one pass)"},
     }
     print(json.dumps(result), flush=True)
 
