@@ -22,6 +22,7 @@ struct aa_hip_frac {
     float* d_ds = nullptr;
     float* d_trials = nullptr;
     double* d_part = nullptr;
+    float* d_ypart = nullptr;    // partial profiles of a split forward pass
     size_t part_entries = 0;
     size_t bytes = 0;
 };
@@ -59,6 +60,7 @@ void release(aa_hip_frac* p) {
     if (p->d_ds) (void)hipFree(p->d_ds);
     if (p->d_trials) (void)hipFree(p->d_trials);
     if (p->d_part) (void)hipFree(p->d_part);
+    if (p->d_ypart) (void)hipFree(p->d_ypart);
     if (cur != p->device) (void)hipSetDevice(cur);
     delete p;
 }
@@ -148,10 +150,22 @@ int aa_hip_frac_create(int device, int nchans, const float* delay_per_dm, int nt
     hipError_t e = hipSetDevice(device);
     const int ttiles = (nsamp + aa_hip::kFracTile - 1) / aa_hip::kFracTile;
     const int groups = (ntrials + 16 * tq - 1) / (16 * tq);
-    p->part_entries = (size_t)max_batch * ttiles * groups;
+    // the most work-groups and partial profiles any batch up to max_batch takes
+    size_t ypart = 0;
+    for (int b = 1; b <= max_batch; ++b) {
+        const size_t g = (size_t)b * ttiles * groups;
+        const int n = aa_hip::frac_channel_split(g, nchans);
+        p->part_entries = std::max(p->part_entries, g * n);
+        if (n > 1) ypart = std::max(ypart, (size_t)n * b * ntrials * nsamp);
+        if (n == 1 && g > (size_t)aa_hip::kFracMaxSplitGroups) {   // larger batches are not split
+            p->part_entries = std::max(p->part_entries, (size_t)max_batch * ttiles * groups);
+            break;
+        }
+    }
     if (e == hipSuccess) e = hipMalloc(&p->d_ds, sizeof(float) * nchans);
     if (e == hipSuccess) e = hipMalloc(&p->d_trials, sizeof(float) * ntrials);
     if (e == hipSuccess) e = hipMalloc(&p->d_part, sizeof(double) * p->part_entries);
+    if (e == hipSuccess && ypart) e = hipMalloc(&p->d_ypart, sizeof(float) * ypart);
     if (e == hipSuccess) e = hipMemcpy(p->d_ds, ds.data(), sizeof(float) * nchans, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->d_trials, tr.data(), sizeof(float) * ntrials, hipMemcpyHostToDevice);
     (void)hipSetDevice(cur);
@@ -160,7 +174,7 @@ int aa_hip_frac_create(int device, int nchans, const float* delay_per_dm, int nt
         release(p);
         return st;
     }
-    p->bytes = sizeof(float) * (nchans + ntrials) + sizeof(double) * p->part_entries;
+    p->bytes = sizeof(float) * (nchans + ntrials) + sizeof(double) * p->part_entries + sizeof(float) * ypart;
     *out = p;
     return AA_HIP_SUCCESS;
 }
@@ -188,6 +202,8 @@ int aa_hip_frac_forward(aa_hip_frac* h, const float* d_x, int nbatch, const floa
     a.y = d_y;
     a.group_q = h->trials_per_wave;
     a.n_groups = (h->ntrials + 16 * a.group_q - 1) / (16 * a.group_q);
+    a.n_split = aa_hip::frac_channel_split((size_t)nbatch * a.n_ttiles * a.n_groups, h->nchans);
+    a.y_part = h->d_ypart;
     return from_hip(aa_hip::launch_frac_forward(a, (hipStream_t)stream), "frac forward");
 }
 
@@ -217,6 +233,7 @@ int aa_hip_frac_adjoint(aa_hip_frac* h, const float* d_x, const float* d_gy, int
         a.gdm_part = h->d_part;
         a.group_q = h->trials_per_wave;
         a.n_groups = (h->ntrials + 16 * a.group_q - 1) / (16 * a.group_q);
+        a.n_split = aa_hip::frac_channel_split((size_t)nbatch * a.n_ttiles * a.n_groups, h->nchans);
         if (aa_hip::frac_grad_dm_parts(a) > h->part_entries)
             return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "workspace too small for the batch");
         const int st = from_hip(aa_hip::launch_frac_grad_dm(a, s), "frac DM adjoint");

@@ -40,7 +40,17 @@ struct frac_args {
     int n_ttiles;          // ceil(T / kFracTile)
     int n_groups;          // trial groups (forward, dm adjoint) or channel groups (x adjoint)
     int group_q;           // trials (or channels) per wave: 1 or 2
+    int n_split;           // channel parts of the forward pass and the DM adjoint
+    float* y_part;         // [n_split][B][K][T] partial profiles (forward, n_split > 1)
 };
+
+// Channel parts for `groups` (batch x time tiles x trial groups) work-groups:
+// the number that fills the 256 CUs' rounds best, at least 8 chunks a part.
+// More than kFracMaxSplitGroups work-groups are not split further: their last
+// round weighs little, and the partial profiles would only grow.
+constexpr int kFracMaxSplit = 16;
+constexpr int kFracMaxSplitGroups = 768;
+int frac_channel_split(size_t groups, int C);
 
 // Trials per wave (1 or 2) such that a group of 16*q consecutive trials
 // keeps every staged window within a row; 0 if even q = 1 does not fit.

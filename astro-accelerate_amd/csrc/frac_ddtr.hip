@@ -158,17 +158,26 @@ __device__ __forceinline__ int ifloor(double v) { return (int)floor(v); }
 //   ds[c] * sum_t gy[b][k][t] * (x[b][c][t + i0 + 1] - x[b][c][t + i0]),
 // which is d(loss)/d(dm[b]) restricted to the group (d tau / d dm = ds[c]).
 // Rows are channels; a row's staged window starts at the smallest delay of
-// the group's trials.
+// the group's trials.  A work-group takes one of n_split parts of the channels
+// (whole chunks): a batch whose tiles and trial groups are fewer than the CUs,
+// or end on a part-filled round of them, is spread over more work-groups
+// (frac_channel_split) and the parts are added in order by frac_sum_parts_kernel
+// (forward) or frac_gdm_finalize.  32 windows of 4096 channels x 1024 samples
+// x 64 trials are 64 work-groups unsplit, 3.13 ms a pass; in 4 parts 0.80 ms.
 template <int KQ, bool GRAD>
 __global__ __launch_bounds__(kThreads) void frac_rows_kernel(frac_args a)
 {
     const int tid = threadIdx.x, lane = tid & 63, w = uni(tid >> 6);   // wave-uniform: DM or channel slots branch on it
     int blk = blockIdx.x;
+    const int sp = blk % a.n_split;
+    blk /= a.n_split;
     const int g = blk % a.n_groups;
     blk /= a.n_groups;
     const int tt = blk % a.n_ttiles;
     const int b = blk / a.n_ttiles;
-    const int C = a.C, T = a.T, K = a.K;
+    const int T = a.T, K = a.K;
+    const int part_rows = (((a.C + kCC - 1) / kCC + a.n_split - 1) / a.n_split) * kCC;
+    const int c_first = sp * part_rows, C = min(a.C, c_first + part_rows);   // this part's channels
     const int t0 = tt * kFracTile;
     const double dmb = (double)a.dm[b];
     const int kbase = g * 16 * KQ;
@@ -218,7 +227,7 @@ __global__ __launch_bounds__(kThreads) void frac_rows_kernel(frac_args a)
         }
     }
 
-    const float* xb = a.x + (size_t)b * C * T;
+    const float* xb = a.x + (size_t)b * a.C * T;
     // 4-aligned first sample of channel c's staged window
     auto row_start = [&](int c) -> int {
         const double d = (double)a.ds[c];
@@ -299,18 +308,18 @@ __global__ __launch_bounds__(kThreads) void frac_rows_kernel(frac_args a)
         }
     };
 
-    const int nch = (C + kCC - 1) / kCC;
-    load_chunk(0);
+    const int nch = C > c_first ? (C - c_first + kCC - 1) / kCC : 0;   // the last part may be empty
+    load_chunk(c_first);
     store_chunk(f_rows0, f_tab0);
     __syncthreads();
     for (int ch = 0; ch < nch; ch += 2) {
-        if (ch + 1 < nch) load_chunk((ch + 1) * kCC);
-        compute_chunk(f_rows0, f_tab0, ch * kCC);
+        if (ch + 1 < nch) load_chunk(c_first + (ch + 1) * kCC);
+        compute_chunk(f_rows0, f_tab0, c_first + ch * kCC);
         if (ch + 1 < nch) store_chunk(f_rows1, f_tab1);
         __syncthreads();
         if (ch + 1 >= nch) break;
-        if (ch + 2 < nch) load_chunk((ch + 2) * kCC);
-        compute_chunk(f_rows1, f_tab1, (ch + 1) * kCC);
+        if (ch + 2 < nch) load_chunk(c_first + (ch + 2) * kCC);
+        compute_chunk(f_rows1, f_tab1, c_first + (ch + 1) * kCC);
         if (ch + 2 < nch) store_chunk(f_rows0, f_tab0);
         __syncthreads();
     }
@@ -320,7 +329,7 @@ __global__ __launch_bounds__(kThreads) void frac_rows_kernel(frac_args a)
         for (int q = 0; q < KQ; ++q) {
             if (!act[q]) continue;
             const int k = kbase + w + 16 * q;
-            float* yk = a.y + ((size_t)b * K + k) * T;
+            float* yk = (a.n_split > 1 ? a.y_part + (size_t)sp * a.B * K * T : a.y) + ((size_t)b * K + k) * T;
 #pragma unroll
             for (int j4 = 0; j4 < kSpl / 4; ++j4) {
                 const int t = tl + 4 * j4;
@@ -339,6 +348,23 @@ __global__ __launch_bounds__(kThreads) void frac_rows_kernel(frac_args a)
             a.gdm_part[blockIdx.x] = sum;
         }
     }
+}
+
+// y = the sum of the channel parts' profiles, in order.
+__global__ __launch_bounds__(256) void frac_sum_parts_kernel(const float4* __restrict__ part, int n_split, size_t n4,
+                                                             float4* __restrict__ y)
+{
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    float4 s = part[i];
+    for (int k = 1; k < n_split; ++k) {
+        const float4 v = part[(size_t)k * n4 + i];
+        s.x += v.x;
+        s.y += v.y;
+        s.z += v.z;
+        s.w += v.w;
+    }
+    y[i] = s;
 }
 
 // gdm[b] = sum of the work-group partials of candidate b, in a fixed order.
@@ -492,7 +518,8 @@ __global__ __launch_bounds__(kThreads) void frac_grad_x_kernel(frac_args a)
 template <bool GRAD>
 hipError_t launch_rows(const frac_args& a, hipStream_t s)
 {
-    const dim3 grid((unsigned)((size_t)a.B * a.n_ttiles * a.n_groups));
+    if (a.n_split < 1 || (!GRAD && a.n_split > 1 && !a.y_part)) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((size_t)a.B * a.n_ttiles * a.n_groups * a.n_split));
     switch (a.group_q) {
     case 2: hipLaunchKernelGGL((frac_rows_kernel<2, GRAD>), grid, dim3(kThreads), 0, s, a); break;
     case 1: hipLaunchKernelGGL((frac_rows_kernel<1, GRAD>), grid, dim3(kThreads), 0, s, a); break;
@@ -522,15 +549,41 @@ int frac_trials_per_wave(const float* h_trials, int K, float ds_absmax)
     return 0;
 }
 
-hipError_t launch_frac_forward(const frac_args& a, hipStream_t s) { return launch_rows<false>(a, s); }
+// Rounds of the CUs (one work-group each: its LDS fills a CU) times the chunks
+// a round takes, 3 chunks' time of them for a tile's start and end.
+int frac_channel_split(size_t groups, int C)
+{
+    const long nch = (C + kCC - 1) / kCC;
+    int best = 1;
+    long best_cost = 0;
+    for (int n = 1; n <= kFracMaxSplit; ++n) {
+        if (n > 1 && (nch / n < 8 || groups * n > (size_t)kFracMaxSplitGroups)) break;
+        const long cost = (long)((groups * n + 255) / 256) * ((nch + n - 1) / n + 3);
+        if (n == 1 || cost < best_cost) {
+            best = n;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
 
-size_t frac_grad_dm_parts(const frac_args& a) { return (size_t)a.B * a.n_ttiles * a.n_groups; }
+hipError_t launch_frac_forward(const frac_args& a, hipStream_t s)
+{
+    const hipError_t e = launch_rows<false>(a, s);
+    if (e != hipSuccess || a.n_split == 1) return e;
+    const size_t n4 = (size_t)a.B * a.K * a.T / 4;
+    hipLaunchKernelGGL(frac_sum_parts_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s,
+                       reinterpret_cast<const float4*>(a.y_part), a.n_split, n4, reinterpret_cast<float4*>(a.y));
+    return hipGetLastError();
+}
+
+size_t frac_grad_dm_parts(const frac_args& a) { return (size_t)a.B * a.n_ttiles * a.n_groups * a.n_split; }
 
 hipError_t launch_frac_grad_dm(const frac_args& a, hipStream_t s)
 {
     const hipError_t e = launch_rows<true>(a, s);
     if (e != hipSuccess) return e;
-    const int per_b = a.n_ttiles * a.n_groups;
+    const int per_b = a.n_ttiles * a.n_groups * a.n_split;
     hipLaunchKernelGGL(frac_gdm_finalize, dim3((a.B + 255) / 256), dim3(256), 0, s, a.gdm_part, per_b, a.B, a.gdm);
     return hipGetLastError();
 }
