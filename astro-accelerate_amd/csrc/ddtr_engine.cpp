@@ -150,17 +150,24 @@ lds_params lds_params_of(const range_launch &rl) {
     p.out_pitch = rl.out_pitch;
     p.row_quads = rl.row_quads;
     p.pair_recs = rl.pair_recs;
-    if (rl.variant != kShapeMatrix) lds_job_tiles(p, rl.variant);
+    if (rl.variant >= 0 && rl.variant != kShapeMatrix) lds_job_tiles(p, rl.variant);
     return p;
 }
 
 hipError_t launch_range(const range_launch &rl, hipStream_t s) {
     if (rl.sample_bytes == 2) {
         const uint16_t *L = reinterpret_cast<const uint16_t *>(rl.L);
+        if (rl.variant == kShapeMatrix) {
+            lds_params p = lds_params_of(rl);
+            p.L = rl.planes;
+            p.pitch = rl.plane_pitch;
+            const hipError_t e = launch_dedisperse_matrix(p, rl.mat, s, rl.over, rl.flags);
+            if (e != hipSuccess) return e;
+        }
         if (rl.wide_win > 0)
             return launch_dedisperse_wide_u16(L, rl.pitch / 2, rl.row_len, rl.nchans, rl.d_dmshifts, rl.ndms,
                                               rl.t_processed, rl.mstartdm, rl.mdmstep, rl.inBin, rl.out, rl.out_pitch,
-                                              rl.wide_win, s);
+                                              rl.wide_win, s, rl.flags, rl.mat.tile_out);
         return launch_dedisperse_direct_u16(L, rl.pitch / 2, rl.nchans, rl.d_dmshifts, rl.ndms, rl.t_processed,
                                             rl.mstartdm, rl.mdmstep, rl.inBin, rl.out, rl.out_pitch, s);
     }
@@ -240,14 +247,19 @@ int ddtr_engine::create(int device, int nchans, const float *dmshifts, int nrang
 
 ddtr_engine::~ddtr_engine() {
     device_guard guard(m_device);
-    for (auto &lv : m_levels)
+    for (auto &lv : m_levels) {
         if (lv.ptr) (void)hipFree(lv.ptr);
+        if (lv.planes) (void)hipFree(lv.planes);
+        if (lv.over) (void)hipFree(lv.over);
+    }
     if (m_d_dmshifts) (void)hipFree(m_d_dmshifts);
     if (m_d_err) (void)hipFree(m_d_err);
     for (const plan_tables &t : m_tables)
         if (t.ptr) (void)hipFree(t.ptr);
-    for (const matrix_tables &t : m_matrix)
+    for (const matrix_tables &t : m_matrix) {
         if (t.t.ptr) (void)hipFree(t.t.ptr);
+        if (t.flags) (void)hipFree(t.flags);
+    }
 }
 
 int ddtr_engine::set_kernel(int kernel) {
@@ -276,10 +288,13 @@ int ddtr_engine::ingest(const void *d_input_tc, int input_bits, int t_processed0
         const hipError_t e = launch_transpose_u16_pitch((const uint16_t *)d_input_tc, len0, m_nchans,
                                                         (uint16_t *)m_levels[0].ptr, m_levels[0].pitch / 2, s);
         if (e != hipSuccess) return hip_fail(e, "corner turn");
-        for (auto &lv : m_levels) lv.len = 0;
+        for (auto &lv : m_levels) {
+            lv.len = 0;
+            lv.planes_ok = false;
+        }
         m_levels[0].len = len0;
         m_resident = 0;
-        return AA_HIP_SUCCESS;
+        return level_planes(0, s);
     }
     // The corner turn writes the binned levels the plan needs in the same
     // pass when the shapes allow it; otherwise ensure_level bins on demand.
@@ -348,11 +363,15 @@ int ddtr_engine::ensure_level(int k, hipStream_t s) {
         if (n_out > dst.capacity) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "binning level overflow");
         hipError_t e = m_sample_bytes == 2
                            ? launch_bin2_u16((const uint16_t *)src.ptr, src.pitch / 2, m_nchans, n_out,
-                                             (uint16_t *)dst.ptr, dst.pitch / 2, s)
+                                             (uint16_t *)dst.ptr, dst.pitch / 2, s, true)
                            : launch_bin2_u8(src.ptr, src.pitch, m_nchans, (int)n_out, dst.ptr, dst.pitch, s);
         if (e != hipSuccess) return hip_fail(e, "binning");
         dst.len = n_out;
         ++m_resident;
+        if (m_sample_bytes == 2) {
+            const int st = level_planes(m_resident, s);
+            if (st != AA_HIP_SUCCESS) return st;
+        }
     }
     return AA_HIP_SUCCESS;
 }
@@ -393,12 +412,21 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
         rl->out_pitch = out_pitch;
         rl->sample_bytes = 2;
         rl->row_len = i_nsamp;
-        if (m_wide_win.size() != m_ranges.size()) m_wide_win.assign(m_ranges.size(), 0);
-        int &w = m_wide_win[(size_t)r];
-        if (w == 0) w = wide_window(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep);
-        rl->wide_win = m_kernel == AA_HIP_KERNEL_DIRECT ? -1 : w;
+        rl->wide_win = m_kernel == AA_HIP_KERNEL_DIRECT ? -1 : u16_window(r);
         if (rl->wide_win < 0 && m_kernel != AA_HIP_KERNEL_AUTO && m_kernel != AA_HIP_KERNEL_DIRECT)
             return fail(AA_HIP_ERROR_UNSUPPORTED, "the 16-bit LDS kernel does not fit this range's delay spread");
+        if (rd.ndms <= 0 || !u16_matrix(r)) return AA_HIP_SUCCESS;
+        st = ensure_planes(k, s);   // (the kernel setting may have changed since the level was written)
+        if (st == AA_HIP_ERROR_OUT_OF_MEMORY) return AA_HIP_SUCCESS;
+        if (st != AA_HIP_SUCCESS) return st;
+        const matrix_tables &mt = m_matrix[(size_t)r];
+        rl->variant = kShapeMatrix;
+        rl->pair_recs = mt.t.ptr;
+        rl->mat = mt.lay;
+        rl->planes = lv.planes;
+        rl->plane_pitch = lv.plane_pitch;
+        rl->over = lv.over;
+        rl->flags = mt.flags;
         return AA_HIP_SUCCESS;
     }
     if (m_lds.size() != m_ranges.size()) m_lds.assign(m_ranges.size(), lds_choice{-2, 0});
@@ -453,6 +481,85 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
         if (st != AA_HIP_SUCCESS) return st;
     }
     rl->pair_recs = pt.ptr;
+    return AA_HIP_SUCCESS;
+}
+
+// The window of dedisperse_u16 for range r of a u16 plan (-1: direct kernel).
+int ddtr_engine::u16_window(int r) {
+    if (m_wide_win.size() != m_ranges.size()) m_wide_win.assign(m_ranges.size(), 0);
+    int &w = m_wide_win[(size_t)r];
+    if (w == 0) {
+        float mstartdm, mdmstep;
+        range_scalars(r, &mstartdm, &mdmstep);
+        w = wide_window(m_dmshifts.data(), m_nchans, m_ranges[(size_t)r].ndms, mstartdm, mdmstep);
+    }
+    return w;
+}
+
+// The automatic choice on u16 levels: the matrix kernel over the rows' byte
+// planes where its plan pays (dedisperse_u16 then computes the tiles it
+// flags).  Without the memory for its tables the range keeps dedisperse_u16.
+bool ddtr_engine::u16_matrix(int r) {
+    if (m_sample_bytes != 2 || m_kernel != AA_HIP_KERNEL_AUTO || u16_window(r) <= 0) return false;
+    if (m_matrix.size() != m_ranges.size()) m_matrix.resize(m_ranges.size());
+    matrix_tables &mt = m_matrix[(size_t)r];
+    if (mt.planned) return mt.lay.tile_out > 0;
+    mt.planned = true;
+    const range_desc &rd = m_ranges[(size_t)r];
+    const level &lv = m_levels[(size_t)log2i(rd.inBin)];
+    float mstartdm, mdmstep;
+    range_scalars(r, &mstartdm, &mdmstep);
+    std::vector<uint8_t> bytes;
+    const matrix_layout lay = matrix_plan(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep,
+                                          round_up((size_t)lv.capacity + kRowPad, kPitchAlign), &bytes, 2);
+    if (lay.tile_out <= 0 || keep_tables(mt.t, kShapeMatrix, bytes) != AA_HIP_SUCCESS) return false;
+    const size_t tiles =
+        (size_t)lay.n_dm_tiles * (size_t)((lv.capacity + lay.tile_out - 1) / lay.tile_out) * sizeof(int);
+    if (hipMalloc(&mt.flags, tiles) != hipSuccess) {
+        mt.flags = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    m_device_bytes += tiles;
+    mt.lay = lay;
+    return true;
+}
+
+// Byte planes of a u16 level that has just been written, where a range reads
+// them: on the writer's stream, so that ranges may run on others.
+int ddtr_engine::level_planes(int k, hipStream_t s) {
+    m_levels[(size_t)k].planes_ok = false;
+    for (int r = 0; r < (int)m_ranges.size(); ++r)
+        if (log2i(m_ranges[(size_t)r].inBin) == k && m_ranges[(size_t)r].ndms > 0 && u16_matrix(r)) {
+            const int st = ensure_planes(k, s);
+            return st == AA_HIP_ERROR_OUT_OF_MEMORY ? AA_HIP_SUCCESS : st;
+        }
+    return AA_HIP_SUCCESS;
+}
+
+int ddtr_engine::ensure_planes(int k, hipStream_t s) {
+    level &lv = m_levels[(size_t)k];
+    if (lv.planes_ok) return AA_HIP_SUCCESS;
+    if (!lv.planes) {
+        const size_t pitch = round_up((size_t)lv.capacity + kRowPad, kPitchAlign);
+        void *p = nullptr, *o = nullptr;
+        if (hipMalloc(&p, 2 * pitch * (size_t)m_nchans) != hipSuccess || hipMalloc(&o, 64 * sizeof(int)) != hipSuccess) {
+            (void)hipGetLastError();
+            if (p) (void)hipFree(p);
+            return AA_HIP_ERROR_OUT_OF_MEMORY;
+        }
+        lv.planes = static_cast<uint8_t *>(p);
+        lv.over = static_cast<int *>(o);
+        lv.plane_pitch = pitch;
+        m_device_bytes += 2 * pitch * (size_t)m_nchans + 64 * sizeof(int);
+    }
+    const uint16_t *rows = reinterpret_cast<const uint16_t *>(lv.ptr);
+    hipError_t e = launch_u16_sums_over(rows, lv.pitch / 2, m_nchans, lv.len, lv.over, s);
+    if (e == hipSuccess)
+        e = launch_split_u16(rows, lv.pitch / 2, m_nchans, lv.len, lv.planes,
+                             lv.planes + lv.plane_pitch * (size_t)m_nchans, lv.plane_pitch, lv.over, s);
+    if (e != hipSuccess) return hip_fail(e, "byte planes");
+    lv.planes_ok = true;
     return AA_HIP_SUCCESS;
 }
 

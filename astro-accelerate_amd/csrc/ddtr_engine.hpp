@@ -66,6 +66,12 @@ struct range_launch {
     int sample_bytes = 1;             // 2: u16 rows (samples wider than 8 bits; pitch still in bytes)
     long row_len = 0;                 // u16 rows: valid samples per row
     int wide_win = -1;                // u16 rows: dedisperse_u16's window, -1 = direct kernel
+    // u16 rows summed by the matrix kernel (variant kShapeMatrix), tiles whose
+    // sums round by dedisperse_u16:
+    const uint8_t *planes = nullptr;  // byte planes of the rows
+    size_t plane_pitch = 0;
+    const int *over = nullptr;
+    int *flags = nullptr;
 };
 
 class ddtr_engine {
@@ -142,7 +148,17 @@ private:
         size_t pitch = 0;     // bytes between rows
         long capacity = 0;    // longest row this buffer holds
         long len = 0;         // valid samples per row for the current chunk
+        // u16 levels read by the matrix kernel: their byte planes (low bytes of
+        // every row, then high bytes) and whether most sums round, both made
+        // from the chunk on first use
+        uint8_t *planes = nullptr;
+        size_t plane_pitch = 0;
+        int *over = nullptr;
+        bool planes_ok = false;
     };
+    // Byte planes of level k for the current chunk; OUT_OF_MEMORY without a
+    // message set when they cannot be allocated.
+    int ensure_planes(int k, hipStream_t s);
 
     int m_device = 0;
     int m_sample_bytes = 1;  // bytes per level sample: 1 (u8) or 2 (u16)
@@ -169,9 +185,13 @@ private:
         bool planned = false;   // lay is known (tile_out 0: not this kernel)
         matrix_layout lay;
         plan_tables t;
+        int *flags = nullptr;   // u16 levels: one entry per tile
     };
     std::vector<matrix_tables> m_matrix;  // per range: the matrix kernel's, kept beside the LDS shape's, which a
                                           // captured batch may still read
+    int u16_window(int r);
+    bool u16_matrix(int r);
+    int level_planes(int k, hipStream_t s);
     // Uploads tables of `variant` in place of what pt holds.
     int keep_tables(plan_tables &pt, int variant, const std::vector<uint8_t> &bytes);
     size_t m_device_bytes = 0;

@@ -123,13 +123,25 @@ int wide_window(const float* h_dmshifts, int nchans, int ndms, float mstartdm, f
 // wide_window.  Any even pitch and 4-byte aligned L take single dword loads.
 hipError_t launch_dedisperse_wide_u16(const uint16_t* L, size_t pitch, long row_len, int nchans,
                                       const float* d_dmshifts, int ndms, int t_processed, float mstartdm,
-                                      float mdmstep, int inBin, float* out, size_t out_pitch, int win, hipStream_t s);
+                                      float mdmstep, int inBin, float* out, size_t out_pitch, int win, hipStream_t s,
+                                      const int* flags = nullptr, int flag_tile = 0);
+// flags: only tiles that overlap a flagged one (16 trials x flag_tile samples,
+// time tile major) are computed.
+// Byte planes of u16 rows for the matrix kernel: row c of lo and hi, pitch
+// bytes apart, holds the low and high bytes of n samples (rows and pitches
+// 16-byte aligned).  over: from launch_u16_sums_over.
+hipError_t launch_split_u16(const uint16_t* in, size_t in_pitch, int nchans, long n, uint8_t* lo, uint8_t* hi,
+                            size_t out_pitch, const int* over, hipStream_t s);
+// over[k] = 1 if the channel sum at sample k n / 64 is above 2^24, else 0 (k <
+// 64): whether a chunk's float sums round.
+hipError_t launch_u16_sums_over(const uint16_t* in, size_t in_pitch, int nchans, long n, int* over, hipStream_t s);
 // [t][c] u16 -> [c][t] u16, out rows out_pitch samples apart.
 hipError_t launch_transpose_u16_pitch(const uint16_t* in_tc, long nsamp, int nchans, uint16_t* out_ct,
                                       size_t out_pitch, hipStream_t s);
-// out[c][t] = (in[c][2t] + in[c][2t+1]) >> 1, t < n_out, u16 rows.
+// out[c][t] = (in[c][2t] + in[c][2t+1]) >> 1, t < n_out, u16 rows.  padded: the
+// rows' padding may be read and written up to the next 8 outputs.
 hipError_t launch_bin2_u16(const uint16_t* in, size_t in_pitch, int nchans, long n_out, uint16_t* out,
-                           size_t out_pitch, hipStream_t s);
+                           size_t out_pitch, hipStream_t s, bool padded = false);
 
 // First single-pulse-search pass on a DM-time plane (boxcar MSD per width
 // 1..W, then best boxcar SNR and its width per start sample); `work` holds

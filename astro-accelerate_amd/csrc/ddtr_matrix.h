@@ -17,6 +17,7 @@ constexpr int kShapeMatrix = kLdsVariants;
 struct matrix_layout {
     int n_dm_tiles = 0;
     int tile_out = 0;      // output samples per tile (0: the range does not take this kernel)
+    int planes = 1;        // 2: 16-bit samples as two planes of byte rows, low bytes then high bytes
     size_t off_group = 0, off_step = 0, bytes = 0;
 };
 
@@ -29,11 +30,18 @@ inline long matrix_tiles_at_most(int ndms, int t_processed)
 
 // Plan tables of one range over rows `pitch` bytes apart: fills `bytes` (when
 // not null) as the kernel reads them and returns their layout; tile_out 0 when
-// the range does not fit or the LDS shapes are the better choice.  Host only.
+// the range does not fit or the kernel it would replace is the better choice.
+// planes 2: rows nchans .. 2 nchans - 1 hold the samples' high bytes.  Host
+// only.
 matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float mstartdm, float mdmstep, size_t pitch,
-                          std::vector<uint8_t>* bytes);
+                          std::vector<uint8_t>* bytes, int planes = 1);
 
-// p.pair_recs: the tables on the device.
-hipError_t launch_dedisperse_matrix(const lds_params& p, const matrix_layout& lay, hipStream_t s);
+// p.pair_recs: the tables on the device.  planes 2: the sums are integers; a
+// tile with a sum above 2^24, where the reference's float adds round, sets its
+// entry of flags (n_dm_tiles x time tiles, time tile major; else 0) and has to
+// be computed in channel order; more than half of over's 64 entries set flags
+// every tile and computes none.
+hipError_t launch_dedisperse_matrix(const lds_params& p, const matrix_layout& lay, hipStream_t s,
+                                    const int* over = nullptr, int* flags = nullptr);
 
 }  // namespace aa_hip

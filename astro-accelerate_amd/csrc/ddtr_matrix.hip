@@ -80,7 +80,8 @@ struct mat_tile {
 struct mat_group {
     int nsteps;
     int odd;               // bit d: trial d's first sample is the odd one of its dword
-    int pad[2];
+    int shift;             // the sums' weight: 8 for a group of high bytes
+    int pad;
     int e[kMatDms];        // dword of each trial's first sample in its LDS row
 };
 struct mat_step {
@@ -102,6 +103,8 @@ struct mat_args {
     const mat_group* groups;
     const mat_step* steps;
     int tile_out;
+    const int* over;       // 64 entries: more than half of them set: flag every tile
+    int* flags;
 };
 
 __shared__ uint32_t m_rows[2 * kMatDms * kMatRow + 512];   // the tail: reads past the last row's window
@@ -148,6 +151,8 @@ __device__ __forceinline__ void mat_step_products(const mat_raw& r, i32x4 (&acc)
     }
 }
 
+// PLANES: 16-bit samples as planes of low and high bytes.
+template <bool PLANES>
 __global__ __launch_bounds__(kMatThreads, 2) void dedisperse_matrix_kernel(mat_args a)
 {
     const lds_params& p = a.p;
@@ -158,6 +163,10 @@ __global__ __launch_bounds__(kMatThreads, 2) void dedisperse_matrix_kernel(mat_a
     const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per || tile >= ntiles) return;   // whole work-group, before any barrier
     const int t_tile = tile / p.n_dm_tiles, dm_tile = tile - t_tile * p.n_dm_tiles;
+    if (PLANES && __popcll(__ballot(a.over[threadIdx.x & 63] != 0)) > 32) {
+        if (threadIdx.x == 0) a.flags[tile] = 1;
+        return;   // whole work-group, before any barrier
+    }
     const long t0 = (long)t_tile * a.tile_out;
     const mat_tile tl = a.tiles[dm_tile];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -251,11 +260,20 @@ __global__ __launch_bounds__(kMatThreads, 2) void dedisperse_matrix_kernel(mat_a
 #pragma unroll
             for (int dd = 0; dd < 2; ++dd) {
                 const uint32_t* row = rows + (2 * wave + dd) * kMatRow + gr.e[2 * wave + dd] + lane;
+                if (PLANES && gr.shift) {
 #pragma unroll
-                for (int j = 0; j < kMatOut; ++j) {
-                    const uint32_t v = row[64 * j];
-                    lo[dd][j] += (int)(short)v;
-                    hi[dd][j] += (int)v >> 16;
+                    for (int j = 0; j < kMatOut; ++j) {
+                        const uint32_t v = row[64 * j];
+                        lo[dd][j] += (int)(short)v * 256;
+                        hi[dd][j] += ((int)v >> 16) * 256;
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < kMatOut; ++j) {
+                        const uint32_t v = row[64 * j];
+                        lo[dd][j] += (int)(short)v;
+                        hi[dd][j] += (int)v >> 16;
+                    }
                 }
             }
             ++g;
@@ -271,7 +289,8 @@ __global__ __launch_bounds__(kMatThreads, 2) void dedisperse_matrix_kernel(mat_a
     }
 
     const long t_end = t0 + a.tile_out < p.t_processed ? t0 + a.tile_out : (long)p.t_processed;
-    const int bias = 128 * p.nchans;
+    const int bias = 128 * p.nchans * (PLANES ? 257 : 1);   // what the sign flips took off every sum
+    bool above = false;   // a sum whose float adds round
 #pragma unroll
     for (int dd = 0; dd < 2; ++dd) {
         const int d = dm_tile * kMatDms + 2 * wave + dd;
@@ -281,7 +300,9 @@ __global__ __launch_bounds__(kMatThreads, 2) void dedisperse_matrix_kernel(mat_a
 #pragma unroll
         for (int j = 0; j < kMatOut; ++j) {
             const long t = t0 + 2 * (lane + 64 * j);
-            const float v0 = out_value((uint32_t)(lo[dd][j] + bias), p), v1 = out_value((uint32_t)(hi[dd][j] + bias), p);
+            const uint32_t s0 = (uint32_t)(lo[dd][j] + bias), s1 = (uint32_t)(hi[dd][j] + bias);
+            if (PLANES) above |= (t < t_end && s0 > (1u << 24)) || (t + 1 < t_end && s1 > (1u << 24));
+            const float v0 = out_value(s0, p), v1 = out_value(s1, p);
             if (aligned && t + 1 < t_end) {
                 *reinterpret_cast<float2*>(orow + t) = make_float2(v0, v1);
             } else {
@@ -289,6 +310,10 @@ __global__ __launch_bounds__(kMatThreads, 2) void dedisperse_matrix_kernel(mat_a
                 if (t + 1 < t_end) orow[t + 1] = v1;
             }
         }
+    }
+    if (PLANES) {
+        const int any = __syncthreads_or(above);
+        if (threadIdx.x == 0) a.flags[tile] = any ? 1 : 0;
     }
 }
 
@@ -403,10 +428,13 @@ double pair_cost(int nchans, int spread)
 }  // namespace
 
 matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float mstartdm, float mdmstep, size_t pitch,
-                          std::vector<uint8_t>* bytes)
+                          std::vector<uint8_t>* bytes, int planes)
 {
     matrix_layout lay;
-    if (nchans < 1 || ndms < 1 || (size_t)pitch * 17 >= (1ull << 32)) return lay;
+    if (nchans < 1 || ndms < 1 || (size_t)pitch * 17 >= (1ull << 32) || (planes == 2 && nchans > 65536)) return lay;
+    // Against the 16-bit LDS kernel (5.75 T channel-adds/s where the pair
+    // shapes do 54) any plan pays that is not 8 times the pair shapes' cost.
+    const double limit_cost = planes == 2 ? 8.0 : 1.0;
     const int ntiles = (ndms + kMatDms - 1) / kMatDms;
     std::vector<float> shift((size_t)ntiles * kMatDms);
     for (int d = 0; d < ntiles * kMatDms; ++d)   // trials past the last repeat it
@@ -456,69 +484,73 @@ matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float m
                 if (tile == 0) limit_guess = limit;
             }
         }
-        if (best.g.empty() || (tile == 0 && best_cost / kMatWin > 1.5 * pair_cost(nchans, 0))) return lay;   // far off
-        cost += best_cost;
-        mat_tile tl{(int)groups.size(), (int)best.g.size(), (int)steps.size(), (int)best.nsteps};
-        int c0 = 0;
-        for (const group_pick& pk : best.g) {
-            mat_group gr{};
-            gr.nsteps = (pk.slots + 15) / 16;
-            const int* base = d32.data() + (size_t)pk.ref * kMatDms;
-            const int w0 = *std::min_element(base, base + kMatDms);
-            for (int d = 0; d < kMatDms; ++d) {
-                gr.e[d] = (base[d] - w0) / 2;
-                gr.odd |= ((base[d] - w0) & 1) << d;
-                spread = std::max(spread, base[d] - w0);
-            }
-            int slot = 0;
-            long long addr[16];
-            auto close_step = [&]() {
-                mat_step& ms = steps.back();
-                long long lowest = addr[0];
-                for (int k = 1; k < 16; ++k) lowest = std::min(lowest, addr[k]);
-                ms.base = lowest & ~3ll;
-                for (int k = 0; k < 16; ++k) {
-                    ms.off[k] = (uint32_t)((addr[k] & ~3ll) - ms.base);
-                    ms.shift[k] = (uint32_t)(addr[k] & 3);
+        if (best.g.empty() || (tile == 0 && best_cost / kMatWin > 1.5 * limit_cost * pair_cost(nchans, 0))) return lay;   // far off
+        cost += planes * best_cost;
+        mat_tile tl{(int)groups.size(), planes * (int)best.g.size(), (int)steps.size(), planes * (int)best.nsteps};
+        for (int plane = 0; plane < planes; ++plane) {
+            int c0 = 0;
+            for (const group_pick& pk : best.g) {
+                mat_group gr{};
+                gr.shift = 8 * plane;
+                gr.nsteps = (pk.slots + 15) / 16;
+                const int* base = d32.data() + (size_t)pk.ref * kMatDms;
+                const int w0 = *std::min_element(base, base + kMatDms);
+                for (int d = 0; d < kMatDms; ++d) {
+                    gr.e[d] = (base[d] - w0) / 2;
+                    gr.odd |= ((base[d] - w0) & 1) << d;
+                    spread = std::max(spread, base[d] - w0);
                 }
-            };
-            for (int c = c0; c < c0 + pk.n; ++c) {
-                const int* row = d32.data() + (size_t)c * kMatDms;
-                int lo = row[0] - base[0], hi = lo;
-                for (int d = 1; d < kMatDms; ++d) {
-                    lo = std::min(lo, row[d] - base[d]);
-                    hi = std::max(hi, row[d] - base[d]);
-                }
-                if (hi - lo >= 16 || w0 + lo < 0) return lay;   // the 16-bit spans disagree
-                for (int part = 0; part < (hi - lo) / 4 + 1; ++part, ++slot) {
-                    const int k = slot & 15;
-                    if (k == 0) steps.emplace_back();
-                    addr[k] = (long long)c * (long long)pitch + w0 + lo + 4 * part;
-                    auto& out = steps.back().sel;
-                    for (int d = 0; d < kMatDms; ++d) {
-                        const int r = row[d] - base[d] - lo - 4 * part;
-                        // lane (d, slot / 4), dword slot % 4
-                        if (r >= 0 && r < 4) out[(k >> 2) * 16 + d][k & 3] = 1u << (8 * r);
+                int slot = 0;
+                long long addr[16];
+                auto close_step = [&]() {
+                    mat_step& ms = steps.back();
+                    long long lowest = addr[0];
+                    for (int k = 1; k < 16; ++k) lowest = std::min(lowest, addr[k]);
+                    ms.base = lowest & ~3ll;
+                    for (int k = 0; k < 16; ++k) {
+                        ms.off[k] = (uint32_t)((addr[k] & ~3ll) - ms.base);
+                        ms.shift[k] = (uint32_t)(addr[k] & 3);
                     }
-                    if (k == 15) close_step();
+                };
+                for (int c = c0; c < c0 + pk.n; ++c) {
+                    const int* row = d32.data() + (size_t)c * kMatDms;
+                    int lo = row[0] - base[0], hi = lo;
+                    for (int d = 1; d < kMatDms; ++d) {
+                        lo = std::min(lo, row[d] - base[d]);
+                        hi = std::max(hi, row[d] - base[d]);
+                    }
+                    if (hi - lo >= 16 || w0 + lo < 0) return lay;   // the 16-bit spans disagree
+                    for (int part = 0; part < (hi - lo) / 4 + 1; ++part, ++slot) {
+                        const int k = slot & 15;
+                        if (k == 0) steps.emplace_back();
+                        addr[k] = ((long long)plane * nchans + c) * (long long)pitch + w0 + lo + 4 * part;
+                        auto& out = steps.back().sel;
+                        for (int d = 0; d < kMatDms; ++d) {
+                            const int r = row[d] - base[d] - lo - 4 * part;
+                            // lane (d, slot / 4), dword slot % 4
+                            if (r >= 0 && r < 4) out[(k >> 2) * 16 + d][k & 3] = 1u << (8 * r);
+                        }
+                        if (k == 15) close_step();
+                    }
                 }
+                if (slot & 15) {   // unused slots: any readable address, zero selectors
+                    for (int k = slot & 15; k < 16; ++k) addr[k] = addr[(slot & 15) - 1];
+                    close_step();
+                }
+                groups.push_back(gr);
+                c0 += pk.n;
             }
-            if (slot & 15) {   // unused slots: any readable address, zero selectors
-                for (int k = slot & 15; k < 16; ++k) addr[k] = addr[(slot & 15) - 1];
-                close_step();
-            }
-            groups.push_back(gr);
-            c0 += pk.n;
         }
         tiles.push_back(tl);
     }
     const int tile_out = (kMatWin - spread) / 16 * 16;
     if (tile_out < kMatMinOut) return lay;
-    if (cost / ntiles / tile_out > pair_cost(nchans, spread)) return lay;
+    if (cost / ntiles / tile_out > limit_cost * pair_cost(nchans, spread)) return lay;
 
     auto align = [](size_t v) { return (v + 255) / 256 * 256; };
     lay.n_dm_tiles = ntiles;
     lay.tile_out = tile_out;
+    lay.planes = planes;
     lay.off_group = align(tiles.size() * sizeof(mat_tile));
     lay.off_step = align(lay.off_group + groups.size() * sizeof(mat_group));
     lay.bytes = lay.off_step + steps.size() * sizeof(mat_step);
@@ -531,9 +563,11 @@ matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float m
     return lay;
 }
 
-hipError_t launch_dedisperse_matrix(const lds_params& p, const matrix_layout& lay, hipStream_t s)
+hipError_t launch_dedisperse_matrix(const lds_params& p, const matrix_layout& lay, hipStream_t s, const int* over,
+                                    int* flags)
 {
     if (p.ndms <= 0 || p.t_processed <= 0) return hipSuccess;
+    if ((lay.planes == 2) != (over && flags)) return hipErrorInvalidValue;
     if (!p.pair_recs || lay.tile_out <= 0 || lay.n_dm_tiles != (p.ndms + kMatDms - 1) / kMatDms)
         return hipErrorInvalidValue;
     mat_args a{};
@@ -541,13 +575,17 @@ hipError_t launch_dedisperse_matrix(const lds_params& p, const matrix_layout& la
     a.p.n_dm_tiles = lay.n_dm_tiles;
     a.p.n_t_tiles = (p.t_processed + lay.tile_out - 1) / lay.tile_out;
     a.tile_out = lay.tile_out;
+    a.over = over;
+    a.flags = flags;
     const char* t = static_cast<const char*>(p.pair_recs);
     a.tiles = reinterpret_cast<const mat_tile*>(t);
     a.groups = reinterpret_cast<const mat_group*>(t + lay.off_group);
     a.steps = reinterpret_cast<const mat_step*>(t + lay.off_step);
     const long tiles = (long)a.p.n_dm_tiles * a.p.n_t_tiles;
     if (tiles > 0x7ffffff0L) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(dedisperse_matrix_kernel, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(kMatThreads), 0, s, a);
+    const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)));
+    if (lay.planes == 2) hipLaunchKernelGGL(dedisperse_matrix_kernel<true>, grid, dim3(kMatThreads), 0, s, a);
+    else hipLaunchKernelGGL(dedisperse_matrix_kernel<false>, grid, dim3(kMatThreads), 0, s, a);
     return hipGetLastError();
 }
 

@@ -4,8 +4,12 @@
 //   acc = 0; for c = 0 .. nchans-1: acc += (float)L[c][t + delay(c, d)];
 //   out[d][t] = (acc / nchans) / inBin
 // (src/aa_device_dedispersion_kernel.cu:422-450).  Once a sum passes 2^24
-// the float adds round, so the order is part of the result and no integer
-// or pre-summation trick applies: one float add per channel-add.
+// the float adds round, so the order is part of the result: one float add per
+// channel-add.  Below, every partial sum is exact, whatever the order: the
+// matrix kernel sums the low and high bytes and leaves the tiles with a larger
+// sum to dedisperse_u16_kernel.  1024 channels x 131,072 samples, 448 trials
+// in 2 ranges, sums below 2^24: 1.30 ms in place of 8.29 (38 against 5.9 T
+// channel-adds/s), and 0.13 ms for the byte planes.
 //
 // dedisperse_u16_kernel: a 256-thread work-group owns 16 DM trials x 512
 // samples.  Channels are staged 8 at a time in LDS (double buffered): each
@@ -52,6 +56,8 @@ struct wide_args {
     float* out;
     long out_pitch;
     int win;            // staged window: kWT + largest delay spread of a tile, even
+    const int* flags;   // tiles to compute (null: all): 16 trials x flag_tile samples, time tile major
+    int flag_tile;
 };
 
 // Aligned: rows start on 4-byte boundaries (L aligned, pitch even), so the
@@ -63,6 +69,12 @@ __global__ __launch_bounds__(256) void dedisperse_u16_kernel(wide_args a)
     __shared__ int offs[2][kWCh][kWDms];   // delay(c, d0 + k) - delay(c, d0) + parity of the window start
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const long t0 = (long)blockIdx.x * kWT;
+    if (a.flags) {
+        int any = 0;
+        const long tend = t0 + kWT < a.t_processed ? t0 + kWT : (long)a.t_processed;
+        for (long k = t0 / a.flag_tile; k * a.flag_tile < tend; ++k) any |= a.flags[k * gridDim.y + blockIdx.y];
+        if (!any) return;   // whole work-group, before any barrier
+    }
     const int d0 = blockIdx.y * kWDms;
     const int dlast = min(d0 + kWDms - 1, a.ndms - 1);
     const int ndw = a.win / 2 + 1;   // dwords staged per channel window
@@ -189,6 +201,55 @@ __global__ __launch_bounds__(256) void bin2_u16_kernel(const uint16_t* __restric
     out[(size_t)c * (size_t)out_pitch + (size_t)t] = (uint16_t)(((uint32_t)row[2 * t] + (uint32_t)row[2 * t + 1]) >> 1);
 }
 
+// The same, 8 outputs per thread with 16-byte accesses (rows and pitches
+// 16-byte aligned).  A row's last 8 reach into its padding, which the caller's
+// pitches cover.  One output per thread took 132 us for 1024 channels x
+// 65,536 outputs (3.0 TB/s), this 64 us.
+__global__ __launch_bounds__(256) void bin2_u16_vec_kernel(const uint16_t* __restrict__ in, long in_pitch, long n_out,
+                                                           uint16_t* __restrict__ out, long out_pitch)
+{
+    const long t = 8 * ((long)blockIdx.x * 256 + threadIdx.x);
+    if (t >= n_out) return;
+    const uint4* q = reinterpret_cast<const uint4*>(in + (size_t)blockIdx.y * in_pitch + 2 * t);
+    const uint4 a = q[0], b = q[1];
+    const auto mean = [](uint32_t v) { return ((v & 0xffffu) + (v >> 16)) >> 1; };
+    *reinterpret_cast<uint4*>(out + (size_t)blockIdx.y * out_pitch + t) =
+        make_uint4(mean(a.x) | mean(a.y) << 16, mean(a.z) | mean(a.w) << 16, mean(b.x) | mean(b.y) << 16,
+                   mean(b.z) | mean(b.w) << 16);
+}
+
+// Low and high bytes of u16 rows, 8 samples per thread; nothing for a chunk
+// that the matrix kernel leaves alone (more than half of over set).
+__global__ __launch_bounds__(256) void split_u16_kernel(const uint16_t* __restrict__ in, long in_pitch, long n,
+                                                        uint8_t* __restrict__ lo, uint8_t* __restrict__ hi,
+                                                        long out_pitch, const int* __restrict__ over)
+{
+    if (__popcll(__ballot(over[threadIdx.x & 63] != 0)) > 32) return;
+    const long t = 8 * ((long)blockIdx.x * 256 + threadIdx.x);
+    if (t >= n) return;   // a row's last 8 reach into its padding
+    const uint4 v = *reinterpret_cast<const uint4*>(in + (size_t)blockIdx.y * in_pitch + t);
+    const size_t o = (size_t)blockIdx.y * out_pitch + t;
+    *reinterpret_cast<uint2*>(lo + o) = make_uint2(__builtin_amdgcn_perm(v.y, v.x, 0x06040200u),
+                                                   __builtin_amdgcn_perm(v.w, v.z, 0x06040200u));
+    *reinterpret_cast<uint2*>(hi + o) = make_uint2(__builtin_amdgcn_perm(v.y, v.x, 0x07050301u),
+                                                   __builtin_amdgcn_perm(v.w, v.z, 0x07050301u));
+}
+
+// Channel sum at sample n k / 64 of the rows, k = blockIdx.x.
+__global__ __launch_bounds__(256) void u16_sums_over_kernel(const uint16_t* __restrict__ in, long in_pitch, int nchans,
+                                                            long n, int* over)
+{
+    __shared__ unsigned long long part[4];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint16_t* col = in + n * blockIdx.x / 64;
+    unsigned long long s = 0;
+    for (int c = threadIdx.x; c < nchans; c += 256) s += col[(size_t)c * in_pitch];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if (lane == 0) part[w] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) over[blockIdx.x] = part[0] + part[1] + part[2] + part[3] > (1ull << 24) ? 1 : 0;
+}
+
 inline unsigned blocks(long n, long b) { return (unsigned)((n + b - 1) / b); }
 
 }  // namespace
@@ -210,14 +271,17 @@ int wide_window(const float* h_dmshifts, int nchans, int ndms, float mstartdm, f
 
 hipError_t launch_dedisperse_wide_u16(const uint16_t* L, size_t pitch, long row_len, int nchans,
                                       const float* d_dmshifts, int ndms, int t_processed, float mstartdm,
-                                      float mdmstep, int inBin, float* out, size_t out_pitch, int win, hipStream_t s)
+                                      float mdmstep, int inBin, float* out, size_t out_pitch, int win, hipStream_t s,
+                                      const int* flags, int flag_tile)
 {
     if (!L || !d_dmshifts || !out || nchans <= 0 || ndms < 0 || t_processed < 0 || inBin <= 0 ||
         (size_t)row_len > pitch || out_pitch < (size_t)t_processed || win < 2 || win > kWRowMax || (win & 1) ||
-        ((uintptr_t)L & 1))
+        ((uintptr_t)L & 1) || (flags && flag_tile <= 0))
         return hipErrorInvalidValue;
     if (ndms == 0 || t_processed == 0) return hipSuccess;
     wide_args a{};
+    a.flags = flags;
+    a.flag_tile = flag_tile;
     a.L = L;
     a.pitch = (long)pitch;
     a.row_len = row_len;
@@ -252,12 +316,39 @@ hipError_t launch_transpose_u16_pitch(const uint16_t* in_tc, long nsamp, int nch
     return hipGetLastError();
 }
 
+hipError_t launch_split_u16(const uint16_t* in, size_t in_pitch, int nchans, long n, uint8_t* lo, uint8_t* hi,
+                            size_t out_pitch, const int* over, hipStream_t s)
+{
+    const size_t n8 = ((size_t)(n > 0 ? n : 0) + 7) / 8 * 8;
+    if (!in || !lo || !hi || !over || nchans <= 0 || n < 0 || n8 > in_pitch || n8 > out_pitch || (in_pitch & 7) ||
+        (out_pitch & 15) || (((uintptr_t)in | (uintptr_t)lo | (uintptr_t)hi) & 15))
+        return hipErrorInvalidValue;
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(split_u16_kernel, dim3(blocks(n, 2048), nchans), dim3(256), 0, s, in, (long)in_pitch, n, lo, hi,
+                       (long)out_pitch, over);
+    return hipGetLastError();
+}
+
+hipError_t launch_u16_sums_over(const uint16_t* in, size_t in_pitch, int nchans, long n, int* over, hipStream_t s)
+{
+    if (!in || !over || nchans <= 0 || n <= 0 || (size_t)n > in_pitch) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(u16_sums_over_kernel, dim3(64), dim3(256), 0, s, in, (long)in_pitch, nchans, n, over);
+    return hipGetLastError();
+}
+
 hipError_t launch_bin2_u16(const uint16_t* in, size_t in_pitch, int nchans, long n_out, uint16_t* out,
-                           size_t out_pitch, hipStream_t s)
+                           size_t out_pitch, hipStream_t s, bool padded)
 {
     if (!in || !out || nchans <= 0 || n_out < 0 || in_pitch < 2 * (size_t)n_out || out_pitch < (size_t)n_out)
         return hipErrorInvalidValue;
     if (n_out == 0) return hipSuccess;
+    const size_t n8 = ((size_t)n_out + 7) / 8 * 8;
+    if (padded && n8 <= out_pitch && 2 * n8 <= in_pitch && (in_pitch & 7) == 0 && (out_pitch & 7) == 0 &&
+        (((uintptr_t)in | (uintptr_t)out) & 15) == 0) {
+        hipLaunchKernelGGL(bin2_u16_vec_kernel, dim3(blocks(n_out, 2048), nchans), dim3(256), 0, s, in, (long)in_pitch,
+                           n_out, out, (long)out_pitch);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(bin2_u16_kernel, dim3(blocks(n_out, 256), nchans), dim3(256), 0, s, in, (long)in_pitch, n_out,
                        out, (long)out_pitch);
     return hipGetLastError();

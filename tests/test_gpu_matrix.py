@@ -73,3 +73,45 @@ def test_matrix_choice_follows_the_kernel_setting(aa, oracle, cuda):
         out = torch.full((ndms, tp), -1.0, dtype=torch.float32, device=cuda)
         plan.run_range(0, tp, out)
         np.testing.assert_array_equal(out.cpu().numpy(), want, err_msg=f"kernel {kernel} variant {variant}")
+
+
+def _u16_fill(kind, nsamp, nchans, rng):
+    x = rng.integers(0, 2001, size=(nsamp, nchans))
+    if kind == "bytes":            # low and high byte at their ends
+        x = rng.choice([0, 255, 256, 257, 65280], size=(nsamp, nchans), p=[0.3, 0.3, 0.2, 0.199, 0.001])
+    elif kind == "straddle":       # sums on both sides of 2^24 in every tile
+        x = rng.integers(2 ** 25 // nchans - 20000, 20000, size=(nsamp, nchans))
+    elif kind == "mixed":          # the end of the plane rounds, the rest does not
+        x[nsamp * 7 // 10:] += 60000
+    elif kind == "over":
+        x = rng.integers(50000, 65536, size=(nsamp, nchans))
+    elif kind == "edge":           # sums of exactly 2^24, and a few above
+        x = np.full((nsamp, nchans), 2 ** 24 // nchans)
+        x[rng.integers(0, nsamp, 3), rng.integers(0, nchans, 3)] += 1
+    return x.astype(np.uint16)
+
+
+@pytest.mark.parametrize("kind", ["low", "bytes", "straddle", "mixed", "over", "edge"])
+@pytest.mark.parametrize("nchans", [1024, 1003])
+def test_u16_byte_planes(aa, oracle, cuda, kind, nchans):
+    """16-bit plans: exact integer sums over the byte planes, and the float sums
+    in channel order wherever one passes 2^24 and the adds round."""
+    import torch
+    print(f"matrix u16 {kind} {nchans} channels", flush=True)
+    ranges = [(0, 20, 0.4, 1, 1), (20, 45, 0.8, 2, 2)]
+    tsamp, nsamp = 64e-6, 16000
+    s = oracle.strategy(ranges, nchans, nsamp, 1500.0, -300.0 / nchans, tsamp, nbits=16)
+    assert s.ok and s.num_tchunks == 1
+    x = _u16_fill(kind, nsamp, nchans, np.random.default_rng(nchans))
+    want = oracle.run(s, x)
+    plan = aa.DdtrPlan(s.dmshifts, [(s.dm[r][0], s.dm[r][2], s.ndms[r], s.dm[r][3]) for r in range(s.nranges)],
+                       tsamp, s.maxshift, s.t_processed[0][0], sample_bits=16)
+    tps = [s.t_processed[r][0] for r in range(s.nranges)]
+    d_in = torch.from_numpy(x.view(np.int16)).to(cuda)
+    for chunk in range(2):         # the second chunk finds the first one's planes and flags
+        outs = [torch.full((s.ndms[r], tps[r] + 3), -1.0, dtype=torch.float32, device=cuda) for r in range(s.nranges)]
+        plan.execute_chunk(d_in if chunk else torch.flip(d_in, (0,)).contiguous(), tps, outs)
+    for r in range(s.nranges):
+        got = outs[r].cpu().numpy()
+        np.testing.assert_array_equal(got[:, :tps[r]], want[r], err_msg=f"range {r}")
+        assert np.all(got[:, tps[r]:] == -1.0)
