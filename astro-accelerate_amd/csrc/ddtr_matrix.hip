@@ -13,8 +13,12 @@
 //
 // "Slots" generalise the channels: a slot is 4 consecutive byte positions of
 // one channel; a channel whose r spans up to 4 n values takes n slots.  A step
-// is 16 slots (K = 64).  The host plans groups, slots and selectors once per
-// range (matrix_plan).
+// is 16 slots (K = 64).  A slot is narrow if its selectors use 3 of its 4
+// positions: an odd sample can then take its even neighbour's operand and the
+// selectors a byte higher, which saves half of the operand alignments.  The
+// host plans groups, slots and selectors once per range (matrix_plan), widths
+// as even as they can be and the narrow slots of a group first; 74 to 90 % of
+// the steps of the plans below are narrow.
 //
 // Work-group: 8 waves, 16 DM trials, a window of 8 x 240 positions k.  Per step
 // a wave loads, for each of its lane's 4 slots, the 16 bytes at its own
@@ -36,19 +40,21 @@
 // loading each, and what steers the loop is read with scalar loads: a vector
 // load for it waits for the row loads before it.
 //
-// Bound: vector instruction issue.  A step is 94 vector instructions (48
-// operand alignments, 16 byte shifts, 16 sign flips, 8 lane moves) beside 16
-// products per wave; issue takes 4.3 cycles per instruction and about half of
-// a product's 16 does not overlap with it, 1120 of the 1700 cycles a step
-// takes; LDS is 13 % busy, the vector memory return path about two thirds.
+// Bound: vector instruction issue and the hand-over of the groups.  A step is
+// 60 vector instructions if narrow (32 alignments, 16 sign flips, 8 lane
+// moves, 4 selectors), 88 if not, beside 16 products per wave; issue takes 4.3
+// cycles per instruction and about half of a product's 16 does not overlap
+// with it.  With all alignments and flips left out the 8-range plan would take
+// 76 ms; LDS is 13 % busy, the vector memory return path about two thirds.
 // Tried and not kept: three row buffers (no change), the sums of a group
 // delayed into the next group's first step (99.9 against 99.2 ms), a fixed
 // interleave of products and vector instructions (99.2 against 97.6 ms).
 //
 // Measured on the 8-range plan (4096 channels x 1,048,576 samples, 6080
-// trials, 1.48e13 channel-adds): 92.7 ms for the 8 launches, 160 T adds/s,
-// against 238.6 ms with the pair shapes; the single-range plan (512 channels x
-// 131,072 samples, 1024 trials) 0.79 ms against 1.19.
+// trials, 1.48e13 channel-adds): 85 ms for the 8 launches, 174 T adds/s,
+// against 238.6 ms with the pair shapes and 92.7 ms with wide steps only; the
+// single-range plan (512 channels x 131,072 samples, 1024 trials) 0.75 ms
+// against 1.19 and 0.79.
 #include "ddtr_matrix.h"
 
 #include <algorithm>
@@ -65,7 +71,7 @@ constexpr int kMatThreads = 64 * kMatWaves;
 constexpr int kMatRun = 240;                     // window positions per wave (15 lanes of 16)
 constexpr int kMatWin = kMatRun * kMatWaves;     // window positions per tile
 constexpr int kMatRow = kMatWin / 2 + 4;         // dwords per LDS row (rows 4 banks apart modulo 32)
-constexpr int kMatOut = kMatWin / 128;             // dwords per lane of a trial's tile
+constexpr int kMatOut = kMatWin / 128;           // dwords per lane of a trial's tile
 constexpr int kMatGroupMax = 256;                // channels: 16-bit partial sums
 constexpr int kMatMinOut = 1024;                 // smallest tile worth its window
 
@@ -78,10 +84,9 @@ struct mat_tile {
     int step0, nsteps;     // their steps
 };
 struct mat_group {
-    int nsteps;
+    int nsteps, narrow;    // steps, the first ones narrow
     int odd;               // bit d: trial d's first sample is the odd one of its dword
     int shift;             // the sums' weight: 8 for a group of high bytes
-    int pad;
     int e[kMatDms];        // dword of each trial's first sample in its LDS row
 };
 struct mat_step {
@@ -124,10 +129,13 @@ struct mat_raw {
 // One step's 16 products.  Lane m of 16 holds bytes 16 m .. 16 m + 15 of its 4
 // slots; the dwords after them are the next lane's first ones (lane 15 has
 // none: its positions from 8 on are not used).
-template <bool FIRST>
+// NARROW: no slot's selectors use the last of its 4 positions, so that a pair of
+// positions 16 m + q, q even, shares an operand: the odd one takes the
+// selectors a byte higher.
+template <bool FIRST, bool NARROW>
 __device__ __forceinline__ void mat_step_products(const mat_raw& r, i32x4 (&acc)[16])
 {
-    asm volatile("; products %0" ::"n"((int)FIRST));   // keeps the two copies apart
+    asm volatile("; products %0 %1" ::"n"((int)FIRST), "n"((int)NARROW));   // keeps the copies apart
     uint32_t D[4][5];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -139,15 +147,21 @@ __device__ __forceinline__ void mat_step_products(const mat_raw& r, i32x4 (&acc)
         for (int k = 0; k < 4; ++k) D[j][k] = __builtin_amdgcn_alignbyte(R[k + 1], R[k], r.shift[j]);
         D[j][4] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)D[j][0], 0x101, 0xf, 0xf, true);   // row_shl:1
     }
-    const i32x4 b = {(int)r.sel[0], (int)r.sel[1], (int)r.sel[2], (int)r.sel[3]};
+    i32x4 b[2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        b[0][j] = (int)r.sel[j];
+        b[1][j] = (int)(r.sel[j] << 8);
+    }
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
+        const int sh = NARROW ? q & 2 : q & 3;
         i32x4 a;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            a[j] = (q & 3) ? (int)__builtin_amdgcn_alignbyte(D[j][q / 4 + 1], D[j][q / 4], q & 3) : (int)D[j][q / 4];
+            a[j] = sh ? (int)__builtin_amdgcn_alignbyte(D[j][q / 4 + 1], D[j][q / 4], sh) : (int)D[j][q / 4];
         const i32x4 zero = {0, 0, 0, 0};
-        acc[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, FIRST ? zero : acc[q], 0, 0, 0);
+        acc[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[NARROW ? q & 1 : 0], FIRST ? zero : acc[q], 0, 0, 0);
     }
 }
 
@@ -198,37 +212,49 @@ __global__ __launch_bounds__(kMatThreads, 2) void dedisperse_matrix_kernel(mat_a
         m.sel[lane] = rec_sel;
         if (lane < 8) m.off[lane] = rec_off;
     };
-    int f = 0;   // the next step to fetch
+    int f = 0;   // the next step to fetch; its addresses are at hand
     long long base = csteps[0].base;
+    u32x4m off;
+    auto meta_of = [&](int i) -> const mat_meta& { return m_meta[(i / kMatWaves) & 1][i & (kMatWaves - 1)]; };
     auto fetch = [&](mat_raw& r) {
+        const uint8_t* b = L + base;
+        base = csteps[f + 1 < S ? f + 1 : S - 1].base;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r.q[j] = *reinterpret_cast<const u32x4a*>(b + (size_t)(off[j] + vlane));
+        const mat_meta& m = meta_of(f);
+        r.sel = m.sel[lane];
+        r.shift = m.shift[kb];
+        ++f;
         if ((f & (kMatWaves - 1)) == 0) {   // a new chunk of records: the one before it has been read
             __syncthreads();
             keep_rec(f / kMatWaves + 1);
             load_rec(f / kMatWaves + 2);
         }
-        const mat_meta& m = m_meta[(f / kMatWaves) & 1][f & (kMatWaves - 1)];
-        r.sel = m.sel[lane];
-        r.shift = m.shift[kb];
-        const u32x4m off = m.off[kb];
-        const uint8_t* b = L + base;
-        base = csteps[f + 1 < S ? f + 1 : S - 1].base;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) r.q[j] = *reinterpret_cast<const u32x4a*>(b + (size_t)(off[j] + vlane));
-        ++f;
+        off = meta_of(f).off[kb];
     };
 
     load_rec(0);
     keep_rec(0);
     load_rec(1);
+    __syncthreads();
+    keep_rec(1);
+    load_rec(2);
+    off = meta_of(0).off[kb];
     mat_raw A, B;
     fetch(A);
-    int s = 0, g = 0, left = groups[0].nsteps;
+    int s = 0, g = 0, left = groups[0].nsteps, narrow = groups[0].narrow;
     bool first = true;
 
     auto body = [&](mat_raw& cur, mat_raw& fill) {
         fetch(fill);
-        if (first) mat_step_products<true>(cur, acc);
-        else mat_step_products<false>(cur, acc);
+        if (narrow > 0) {
+            if (first) mat_step_products<true, true>(cur, acc);
+            else mat_step_products<false, true>(cur, acc);
+        } else {
+            if (first) mat_step_products<true, false>(cur, acc);
+            else mat_step_products<false, false>(cur, acc);
+        }
+        --narrow;
         first = false;
         ++s;
         if (--left == 0) {
@@ -278,6 +304,7 @@ __global__ __launch_bounds__(kMatThreads, 2) void dedisperse_matrix_kernel(mat_a
             }
             ++g;
             left = s < S ? groups[g].nsteps : 0;
+            narrow = s < S ? groups[g].narrow : 0;
             first = true;
         }
     };
@@ -339,39 +366,52 @@ struct tile_delays {
     int nchans;
 };
 
+// Slots of a channel whose r spans `span` values, as even as they can be: of
+// them, wide ones (4 values; the others 3 or fewer).
+inline int slots_of(int span) { return (span + 3) / 4; }
+inline int wide_of(int span) { return std::max(0, span - 3 * slots_of(span)); }
+
 // Whether channels [c0, c0 + n) with reference channel `ref` span at most
 // `limit` values each, at non-negative row offsets.
-bool group_fits(const tile_delays& t, int c0, int n, int ref, int limit, int* slots)
+bool group_fits(const tile_delays& t, int c0, int n, int ref, int limit, int* slots, int* wide)
 {
     const int16_t* r16 = t.d16 + (size_t)ref * kMatDms;
     const int* r32 = t.d32 + (size_t)ref * kMatDms;
     int w0 = r32[0];
     for (int d = 1; d < kMatDms; ++d) w0 = std::min(w0, r32[d]);
-    int total = 0;
+    int total = 0, w = 0;
     for (int c = c0; c < c0 + n; ++c) {
         int lo, hi;
         rel_span(t.d16 + (size_t)c * kMatDms, r16, lo, hi);
         const int span = hi - lo + 1;
         if (span > limit || w0 + lo < 0) return false;
-        total += (span + 3) / 4;
+        total += slots_of(span);
+        w += wide_of(span);
     }
     *slots = total;
+    *wide = w;
     return true;
 }
 
+// Work of a plan in units of one step with wide slots (about 1600 cycles per
+// work-group); the hand-over of a group through LDS takes about 2000 cycles.
+constexpr double kNarrowCost = 0.8;
+constexpr double kGroupCost = 1.2;
+
 struct group_pick {
-    int n = 0, ref = 0, slots = 0;
+    int n = 0, ref = 0, slots = 0, wide = 0;
+    int steps() const { return (slots + 15) / 16; }
+    int narrow_steps() const { return wide ? (slots - wide) / 16 : steps(); }   // the steps without a wide slot
+    double cost() const { return steps() - (1.0 - kNarrowCost) * narrow_steps() + kGroupCost; }
 };
 
 group_pick fit(const tile_delays& t, int c0, int n, int limit)
 {
     group_pick g;
-    int slots = 0;
+    int slots = 0, wide = 0;
     for (int ref : {c0 + n / 2, c0})   // the first channel where the middle one would read before the rows
-        if (group_fits(t, c0, n, ref, limit, &slots)) {
-            g.n = n;
-            g.ref = ref;
-            g.slots = slots;
+        if (group_fits(t, c0, n, ref, limit, &slots, &wide)) {
+            g = group_pick{n, ref, slots, wide};
             break;
         }
     return g;
@@ -409,10 +449,6 @@ group_pick pick_group(const tile_delays& t, int c0, int limit, int guess)
     }
     return best;
 }
-
-// Work of a plan in units of one step (about 1700 cycles per work-group): the
-// hand-over of a group through LDS measured 1.2 of them.
-constexpr double kGroupCost = 1.2;
 
 // Cost of the pair shapes in the same units: 16 channels of one of their
 // tiles, which shorten with the trials' spread.  Break-even measured on plans
@@ -463,21 +499,22 @@ matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float m
         const tile_delays t{d32.data(), d16.data(), nchans};
         pick_list best;
         double best_cost = INFINITY;
-        for (int limit = 4; limit <= 16; limit *= 2) {
+        for (int limit : {4, 6, 8, 12, 16}) {
             if (tile > 0 && limit != limit_guess) continue;   // one limit per range: the first tile's best
             pick_list l;
             int guess = 64;
             bool ok = true;
+            double w = 0.0;
             for (int c = 0; c < nchans && ok;) {
                 const group_pick g = pick_group(t, c, limit, guess);
                 ok = g.n > 0;
                 if (!ok) break;
                 l.g.push_back(g);
-                l.nsteps += (g.slots + 15) / 16;
+                l.nsteps += g.steps();
+                w += g.cost();
                 guess = g.n;
                 c += g.n;
             }
-            const double w = (double)l.nsteps + kGroupCost * (double)l.g.size();
             if (ok && w < best_cost) {
                 best_cost = w;
                 best = l;
@@ -492,7 +529,8 @@ matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float m
             for (const group_pick& pk : best.g) {
                 mat_group gr{};
                 gr.shift = 8 * plane;
-                gr.nsteps = (pk.slots + 15) / 16;
+                gr.nsteps = pk.steps();
+                gr.narrow = pk.narrow_steps();
                 const int* base = d32.data() + (size_t)pk.ref * kMatDms;
                 const int w0 = *std::min_element(base, base + kMatDms);
                 for (int d = 0; d < kMatDms; ++d) {
@@ -502,16 +540,24 @@ matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float m
                 }
                 int slot = 0;
                 long long addr[16];
+                bool near = true;   // slots within the kernel's 32-bit offsets
                 auto close_step = [&]() {
                     mat_step& ms = steps.back();
                     long long lowest = addr[0];
                     for (int k = 1; k < 16; ++k) lowest = std::min(lowest, addr[k]);
                     ms.base = lowest & ~3ll;
                     for (int k = 0; k < 16; ++k) {
-                        ms.off[k] = (uint32_t)((addr[k] & ~3ll) - ms.base);
+                        const long long off = (addr[k] & ~3ll) - ms.base;
+                        near = near && off < (1ll << 32) - 2 * kMatWin;
+                        ms.off[k] = (uint32_t)off;
                         ms.shift[k] = (uint32_t)(addr[k] & 3);
                     }
                 };
+                // narrow slots first, then the wide ones
+                struct part {
+                    int c, start, width;   // channel, first r (from the channel's lowest delay - base), values
+                };
+                std::vector<part> narrow, wide;
                 for (int c = c0; c < c0 + pk.n; ++c) {
                     const int* row = d32.data() + (size_t)c * kMatDms;
                     int lo = row[0] - base[0], hi = lo;
@@ -519,24 +565,36 @@ matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float m
                         lo = std::min(lo, row[d] - base[d]);
                         hi = std::max(hi, row[d] - base[d]);
                     }
-                    if (hi - lo >= 16 || w0 + lo < 0) return lay;   // the 16-bit spans disagree
-                    for (int part = 0; part < (hi - lo) / 4 + 1; ++part, ++slot) {
-                        const int k = slot & 15;
-                        if (k == 0) steps.emplace_back();
-                        addr[k] = ((long long)plane * nchans + c) * (long long)pitch + w0 + lo + 4 * part;
-                        auto& out = steps.back().sel;
-                        for (int d = 0; d < kMatDms; ++d) {
-                            const int r = row[d] - base[d] - lo - 4 * part;
-                            // lane (d, slot / 4), dword slot % 4
-                            if (r >= 0 && r < 4) out[(k >> 2) * 16 + d][k & 3] = 1u << (8 * r);
-                        }
-                        if (k == 15) close_step();
+                    const int span = hi - lo + 1;
+                    if (span > 16 || w0 + lo < 0) return lay;   // the 16-bit spans disagree
+                    for (int k = 0, r = lo; k < slots_of(span); ++k) {
+                        const bool w = k < wide_of(span);
+                        const int width = std::min(w ? 4 : 3, hi + 1 - r);
+                        (w ? wide : narrow).push_back(part{c, r, width});
+                        r += width;
                     }
+                }
+                if ((int)(narrow.size() + wide.size()) != pk.slots || (int)wide.size() != pk.wide) return lay;
+                narrow.insert(narrow.end(), wide.begin(), wide.end());
+                for (const part& pt : narrow) {
+                    const int k = slot & 15;
+                    if (k == 0) steps.emplace_back();
+                    addr[k] = ((long long)plane * nchans + pt.c) * (long long)pitch + w0 + pt.start;
+                    const int* row = d32.data() + (size_t)pt.c * kMatDms;
+                    auto& out = steps.back().sel;
+                    for (int d = 0; d < kMatDms; ++d) {
+                        const int r = row[d] - base[d] - pt.start;
+                        // lane (d, slot / 4), dword slot % 4
+                        if (r >= 0 && r < pt.width) out[(k >> 2) * 16 + d][k & 3] = 1u << (8 * r);
+                    }
+                    if (k == 15) close_step();
+                    ++slot;
                 }
                 if (slot & 15) {   // unused slots: any readable address, zero selectors
                     for (int k = slot & 15; k < 16; ++k) addr[k] = addr[(slot & 15) - 1];
                     close_step();
                 }
+                if (!near) return lay;
                 groups.push_back(gr);
                 c0 += pk.n;
             }
