@@ -25,11 +25,19 @@
 // kernel centres on the plane mean c = mean_1 and divides
 // (B'_w - (mean_w - w c)) by sd_w.
 //
-// Cost per start sample and width: 2 (MSD at W = 32, else 3) or 5 (SNR)
-// VALU operations.  At W = 32 both passes read a run of consecutive start
-// samples' samples into registers once (8 in the MSD pass, 4 in the SNR
-// pass), else one LDS read per start sample and width.  VALU-bound; the
-// plane is read twice from HBM.
+// Cost per start sample and width: 2 VALU operations in the MSD pass at W =
+// 32, else 3; 3.8 in the SNR pass at W = 32, else 5.  At W = 32 both passes
+// read a run of consecutive start samples' samples into registers once (8 in
+// the MSD pass, 4 in the SNR pass), else one LDS read per start sample and
+// width.  VALU-bound; the plane is read twice from HBM.
+//
+// Measured on 1536 x 890,624 samples at W = 32 (2.4e9 instructions of a wave
+// for the 2 and 3.8 operations, 7.1 ms at 4.34 cycles each and 2.4 GHz; 19.2 GB,
+// 4.0 ms): MSD 2.76 ms, SNR 4.81 ms.  Before, MSD 4.77 ms: a third of its
+// instructions were the sums over the lanes of 32 widths one at a time, the
+// tile's staging (LDS written, read and written again to centre it) and one
+// wave's serial sum over the tile's edges.  SNR 6.37 ms, with 5 operations per
+// width and stores of one float at a stride of four.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -49,17 +57,11 @@ constexpr int kBlocks = 1024;             // persistent MSD grid
 
 struct spd_aux {              // finalize -> SNR kernel
     float c;                  // centring value: mean of width-1 sums (the plane mean)
-    float pad[3];
+    int finite;               // every off * rsd and rsd is
+    float pad[2];
     float off[kMaxW];         // mean_w - w * c
     float rsd[kMaxW];         // 1 / sd_w (0 when sd_w == 0)
 };
-
-__device__ __forceinline__ float wave_sum(float v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
 
 // v plus the value `ctrl` selects from another lane (DPP); lanes the row
 // mask leaves out, or whose source is out of range, add 0.
@@ -84,14 +86,75 @@ __device__ __forceinline__ float wave_sum_to_lane63(float v)
     return v;
 }
 
+// Sums over the wave's 64 lanes of 32 values, each lane keeping one: lane l
+// gets value spread_width(l)'s.  Half of the values go to the other half of the
+// lanes at each step (row swaps, then DPP with a select), so 70 instructions
+// where a sum to lane 63 per value takes 21 each.
+__device__ __forceinline__ int spread_width(int lane)
+{
+    return (lane >> 5) * 16 + (lane >> 4 & 1) * 8 + (lane >> 2 & 1) * 4 + (lane >> 3 & 1) * 2 + (lane >> 1 & 1);
+}
+template <int CTRL>
+__device__ __forceinline__ float spread_add(float a, float b, bool second)
+{
+    const float keep = second ? b : a, send = second ? a : b;
+    return keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(send), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float wave_spread_sum(const float (&a)[32], int lane)
+{
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[i]), __float_as_uint(a[i + 16]), false, false);
+        v[i] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 8]), false, false);
+        v[i] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+    }
+    // row_ror:4 pairs lanes of unlike bit 2 (and any bit 3), row_ror:8 of unlike bit 3
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = spread_add<0x124>(v[i], v[i + 4], lane & 4);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) v[i] = spread_add<0x128>(v[i], v[i + 2], lane & 8);
+    v[0] = spread_add<0x4E>(v[0], v[1], lane & 2);
+    return dpp_add<0xB1, 0xf>(v[0]);
+}
+
+// v plus the double `ctrl` selects from another lane of the row mask (0 from
+// beyond the row).
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ double dpp_add64(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROW_MASK, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROW_MASK, 0xf, false);
+    return v + __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+// Inclusive prefix sums over lanes 0-31.
+__device__ __forceinline__ double scan32(double v)
+{
+    v = dpp_add64<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
+    v = dpp_add64<0x112, 0xf>(v);
+    v = dpp_add64<0x114, 0xf>(v);
+    v = dpp_add64<0x118, 0xf>(v);
+    return dpp_add64<0x142, 0xa>(v);   // row_bcast15
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef f32x4 f32x4u __attribute__((aligned(4)));   // rows start at any float
+typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+
 // Chan et al.'s pairwise update: (n_a, m_a, M2_a) += (n_b, m_b, M2_b).
 __device__ __forceinline__ void chan_merge(double& na, double& ma, double& m2a, double nb, double mb, double m2b)
 {
     if (nb <= 0.0) return;
     const double n = na + nb;
-    const double delta = mb - ma;
-    ma += delta * (nb / n);
-    m2a += m2b + delta * delta * (na * nb / n);
+    const double delta = mb - ma, part = nb / n;
+    ma += delta * part;
+    m2a += m2b + delta * delta * (na * part);
     na = n;
 }
 
@@ -121,33 +184,56 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
         const long rest = (long)nsamp - t0;
         const int nout = (int)(rest < kTile ? rest : kTile);                 // start samples in the tile
         const int nload = (int)(rest < kTile + W - 1 ? rest : kTile + W - 1);  // samples staged
-        __syncthreads();   // the previous tile's readers of s and red are done
-        float part = 0.0f;
-        for (int i = tid; i < kTile + kMaxW; i += kThreads) {
-            const float v = i < nload ? row[t0 + i] : 0.0f;
-            s[i] = v;
-            if (i < nout) part += v;
+        // All 32 widths fit at every start sample (a wave-uniform case).
+        const bool fast = WC == kMaxW && nload == kTile + W - 1;
+        float c;
+        if (fast) {
+            // The tile waits in registers for its mean, so it is written to LDS
+            // once and centred.
+            f32x4 v[kK / 4];
+#pragma unroll
+            for (int k = 0; k < kK / 4; ++k)
+                v[k] = *reinterpret_cast<const f32x4u*>(row + t0 + 4 * (tid + kThreads * k));
+            const float after = tid < kMaxW - 1 ? row[t0 + kTile + tid] : 0.0f;
+            float part = 0.0f;
+#pragma unroll
+            for (int k = 0; k < kK / 4; ++k) part += (v[k].x + v[k].y) + (v[k].z + v[k].w);
+            part = wave_sum_to_lane63(part);
+            __syncthreads();   // the previous tile's readers of s, red and wsum are done
+            if (lane == 63) wsum[wv] = part;
+            __syncthreads();
+            c = (wsum[0] + wsum[1] + wsum[2] + wsum[3]) / (float)nout;
+#pragma unroll
+            for (int k = 0; k < kK / 4; ++k) *reinterpret_cast<f32x4*>(s + 4 * (tid + kThreads * k)) = v[k] - c;
+            if (tid < kMaxW) s[kTile + tid] = after - c;
+            __syncthreads();
+        } else {
+            __syncthreads();   // the previous tile's readers of s, red and wsum are done
+            float part = 0.0f;
+            for (int i = tid; i < kTile + kMaxW; i += kThreads) {
+                const float v = i < nload ? row[t0 + i] : 0.0f;
+                s[i] = v;
+                if (i < nout) part += v;
+            }
+            part = wave_sum_to_lane63(part);
+            if (lane == 63) wsum[wv] = part;
+            __syncthreads();
+            c = (wsum[0] + wsum[1] + wsum[2] + wsum[3]) / (float)nout;
+            for (int i = tid; i < nload; i += kThreads) s[i] -= c;
+            __syncthreads();
         }
-        part = wave_sum(part);
-        if (lane == 0) wsum[wv] = part;
-        __syncthreads();
-        const float c = (wsum[0] + wsum[1] + wsum[2] + wsum[3]) / (float)nout;
-        for (int i = tid; i < nload; i += kThreads) s[i] -= c;
-        __syncthreads();
         float a1[kMaxW], a2[kMaxW];
 #pragma unroll
         for (int w = 0; w < kMaxW; ++w) a1[w] = a2[w] = 0.0f;
-        // All 32 widths fit at every start sample (a wave-uniform case): the
-        // sums of B_w over the tile follow from the tile's sum C_0 and its
+        // With all widths at every start sample the sums of B_w over the tile follow from the tile's sum C_0 and its
         // edges (below), so the loop keeps only the running sum and the
         // square sums; runs of kRun consecutive start samples per thread,
         // their kRun + 31 samples read once into registers with 16-byte
         // reads (instead of one LDS read per start sample and width).
-        const bool fast = WC == kMaxW && nload == kTile + W - 1;
+        float cs = 0.0f;   // fast: this thread's part of C_0 = sum of s[0 .. kTile)
         if (fast) {
             constexpr int kRun = 8, kWin = kRun + kMaxW;   // 40 registers: s[j0 .. j0 + 39]
             static_assert(kTile % (kRun * kThreads) == 0, "whole runs per thread");
-            float cs = 0.0f;   // this thread's part of C_0 = sum of s[0 .. kTile)
 #pragma unroll 1
             for (int k = 0; k < kTile / (kRun * kThreads); ++k) {
                 const int j0 = kRun * (tid + kThreads * k);
@@ -171,7 +257,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
                     }
                 }
             }
-            a1[0] = cs;
         } else if (nload == kTile + W - 1) {   // every width fits at every start sample
 #pragma unroll 2
             for (int k = 0; k < kK; ++k) {
@@ -201,36 +286,27 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
                 }
             }
         }
-#pragma unroll
-        for (int w = 0; w < kMaxW; ++w) {
-            if (w < W) {
-                const float r1 = fast && w > 0 ? 0.0f : wave_sum_to_lane63(a1[w]);
-                const float r2 = wave_sum_to_lane63(a2[w]);
-                if (lane == 63) {
-                    red[wv][w] = r1;
-                    red[wv][kMaxW + w] = r2;
-                }
-            }
-        }
+        const float r2 = wave_spread_sum(a2, lane);
+        const float r1 = fast ? wave_sum_to_lane63(cs) : wave_spread_sum(a1, lane);
+        if ((lane & 1) == 0) red[wv][kMaxW + spread_width(lane)] = r2;
+        if (fast ? lane == 63 : (lane & 1) == 0) red[wv][fast ? 0 : spread_width(lane)] = r1;
         __syncthreads();
         if (tid < W) {
             const int w = tid + 1;
-            double S1;
+            const int w1 = fast ? 0 : tid;
+            double S1 = (double)red[0][w1] + (double)red[1][w1] + (double)red[2][w1] + (double)red[3][w1];
             if (fast) {
                 // sum over the tile's starts j of B_w(j) = sum_{m<w} C_m, with
-                // C_m = sum_{j<kTile} s[j + m] = C_{m-1} + s[kTile - 1 + m] - s[m - 1]:
-                // S1 = w C_0 + sum_{i=1}^{w-1} (w - i) (s[kTile - 1 + i] - s[i - 1])
-                S1 = (double)w * ((double)red[0][0] + (double)red[1][0] + (double)red[2][0] + (double)red[3][0]);
-                for (int i = 1; i < w; ++i) S1 += (double)(w - i) * ((double)s[kTile - 1 + i] - (double)s[i - 1]);
-            } else {
-                S1 = (double)red[0][tid] + (double)red[1][tid] + (double)red[2][tid] + (double)red[3][tid];
+                // C_m = sum_{j<kTile} s[j + m] = C_{m-1} + s[kTile - 1 + m] - s[m - 1]
+                const double e = tid > 0 ? (double)s[kTile - 1 + tid] - (double)s[tid - 1] : 0.0;
+                S1 = scan32(S1 + scan32(e));
             }
             const double S2 = (double)red[0][kMaxW + tid] + (double)red[1][kMaxW + tid] +
                               (double)red[2][kMaxW + tid] + (double)red[3][kMaxW + tid];
             const long fit = (long)nload - w + 1;               // start samples whose width-w boxcar is staged
             const double n = (double)(fit < nout ? (fit > 0 ? fit : 0) : nout);
             if (n > 0.0) {   // the tile's moments of B_w = B'_w + w c
-                const double mt = S1 / n;
+                const double mt = fast ? S1 * (1.0 / kTile) : S1 / n;
                 const double m2t = S2 - S1 * mt;
                 chan_merge(accn, accm, acc2, n, mt + (double)w * (double)c, m2t > 0.0 ? m2t : 0.0);
             }
@@ -283,12 +359,18 @@ __global__ __launch_bounds__(kFinThreads) void spd_msd_finalize_kernel(const dou
         msd[2 * w + 1] = (float)sd[w];
     }
     __syncthreads();
+    bool finite = true;
     if (w < W && i == 0) {
         const double c = (double)(float)mean[0];
+        const float off = (float)(mean[w] - (double)(w + 1) * c);
+        const float rsd = sd[w] > 0.0 ? (float)(1.0 / sd[w]) : 0.0f;
         if (w == 0) aux->c = (float)c;
-        aux->off[w] = (float)(mean[w] - (double)(w + 1) * c);
-        aux->rsd[w] = sd[w] > 0.0 ? (float)(1.0 / sd[w]) : 0.0f;
+        aux->off[w] = off;
+        aux->rsd[w] = rsd;
+        finite = fabsf(rsd) < INFINITY && fabsf(off * rsd) < INFINITY;
     }
+    finite = __syncthreads_and(finite);
+    if (threadIdx.x == 0) aux->finite = finite;
 }
 
 template <int WC>
@@ -298,7 +380,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 {
     const int W = WC > 0 ? WC : W_arg;
     __shared__ __align__(16) float s[kTile + kMaxW];
-    __shared__ float off[kMaxW], rsd[kMaxW];
+    __shared__ float off[kMaxW];
+    __shared__ __align__(16) float rsd[kMaxW], prod[kMaxW];   // prod: -off * rsd
     const int tid = threadIdx.x;
     const long per_row = ((long)nsamp + kTile - 1) / kTile;
     const long d = blockIdx.x / per_row;
@@ -311,8 +394,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
     if (tid < kMaxW) {
         off[tid] = aux->off[tid];
         rsd[tid] = aux->rsd[tid];
+        prod[tid] = -off[tid] * rsd[tid];
     }
-    for (int i = tid; i < kTile + kMaxW; i += kThreads) s[i] = i < nload ? row[t0 + i] - c : 0.0f;
+    if (WC == kMaxW && nload == kTile + W - 1) {
+        f32x4 v[kK / 4];
+#pragma unroll
+        for (int k = 0; k < kK / 4; ++k)
+            v[k] = *reinterpret_cast<const f32x4u*>(row + t0 + 4 * (tid + kThreads * k));
+        const float after = tid < kMaxW - 1 ? row[t0 + kTile + tid] : 0.0f;
+#pragma unroll
+        for (int k = 0; k < kK / 4; ++k) *reinterpret_cast<f32x4*>(s + 4 * (tid + kThreads * k)) = v[k] - c;
+        if (tid < kMaxW) s[kTile + tid] = after - c;
+    } else {
+        for (int i = tid; i < kTile + kMaxW; i += kThreads) s[i] = i < nload ? row[t0 + i] - c : 0.0f;
+    }
     __syncthreads();
     float* so = snr ? snr + d * snr_pitch + t0 : nullptr;
     uint16_t* wo = width ? width + d * width_pitch + t0 : nullptr;
@@ -322,13 +417,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 #pragma unroll
         for (int w = 0; w < kMaxW; ++w) {
             r[w] = rsd[w];
-            p[w] = -off[w] * r[w];
+            p[w] = WC == kMaxW ? __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(prod[w]))) : prod[w];
         }
-        if constexpr (WC == kMaxW) {
-            // runs of kRun consecutive start samples per thread, their
-            // kRun + 31 samples read into registers once
+        // Finite: no SNR is a NaN (the offsets hold the plane's mean, so every
+        // sample is finite as well), which the maxima below would pass over.
+        if (WC == kMaxW && aux->finite) {
+            // Runs of kRun consecutive start samples per thread, their
+            // kRun + 31 samples read into registers once.  The largest SNR of
+            // each kGroup widths is taken with max3; only the first group that
+            // raised the maximum is kept, as its number and the boxcar sum
+            // before it, and its SNRs are computed once more (the same
+            // operations) to find the width: 3.8 operations per width where
+            // keeping the width along with each maximum takes 5.
             constexpr int kRun = 4, kWin = kRun + kMaxW;   // 36 registers: s[j0 .. j0 + 35]
+            constexpr int kGroup = 4;
             static_assert(kTile % (kRun * kThreads) == 0, "whole runs per thread");
+            const bool vec_s = so && ((uintptr_t)so & 15) == 0, vec_w = wo && ((uintptr_t)wo & 7) == 0;
 #pragma unroll 1
             for (int k = 0; k < kTile / (kRun * kThreads); ++k) {
                 const int j0 = kRun * (tid + kThreads * k);
@@ -341,22 +445,59 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
                     v[4 * m + 2] = q.z;
                     v[4 * m + 3] = q.w;
                 }
+                f32x4 best;
+                u16x4 bw;
 #pragma unroll
                 for (int i = 0; i < kRun; ++i) {
-                    float B = v[i];
-                    float best = __builtin_fmaf(B, r[0], p[0]);
-                    int bw = 1;
+                    float B = 0.0f, top = 0.0f, before = 0.0f;
+                    int at = 0;   // first width - 1 of the group with the maximum
 #pragma unroll
-                    for (int w = 1; w < kMaxW; ++w) {
-                        B += v[i + w];
-                        const float x = __builtin_fmaf(B, r[w], p[w]);
-                        if (x > best) {
-                            best = x;
-                            bw = w + 1;
+                    for (int g = 0; g < kMaxW; g += kGroup) {
+                        const float start = B;
+                        float x[kGroup];
+#pragma unroll
+                        for (int w = 0; w < kGroup; ++w) {
+                            B += v[i + g + w];
+                            x[w] = __builtin_fmaf(B, r[g + w], p[g + w]);
+                        }
+                        float m = fmaxf(fmaxf(x[0], x[1]), x[2]);
+                        if (g == 0) {
+                            top = fmaxf(m, x[3]);
+                        } else {
+                            m = fmaxf(fmaxf(m, x[3]), top);
+                            const bool more = m > top;
+                            before = more ? start : before;
+                            at = more ? g : at;
+                            top = m;
                         }
                     }
-                    if (so) so[j0 + i] = best;
-                    if (wo) wo[j0 + i] = (uint16_t)bw;
+                    const float* y = s + j0 + i + at;
+                    const f32x4 rg = *reinterpret_cast<const f32x4*>(rsd + at);
+                    const f32x4 pg = *reinterpret_cast<const f32x4*>(prod + at);
+                    float x[kGroup];
+#pragma unroll
+                    for (int w = 0; w < kGroup; ++w) {
+                        before += y[w];
+                        x[w] = __builtin_fmaf(before, rg[w], pg[w]);
+                    }
+                    int n = 4;   // the first of the group that is the maximum
+                    n = x[2] == top ? 3 : n;
+                    n = x[1] == top ? 2 : n;
+                    n = x[0] == top ? 1 : n;
+                    best[i] = top;
+                    bw[i] = (uint16_t)(at + n);
+                }
+                if (vec_s) {
+                    *reinterpret_cast<f32x4*>(so + j0) = best;
+                } else if (so) {
+#pragma unroll
+                    for (int i = 0; i < kRun; ++i) so[j0 + i] = best[i];
+                }
+                if (vec_w) {
+                    *reinterpret_cast<u16x4*>(wo + j0) = bw;
+                } else if (wo) {
+#pragma unroll
+                    for (int i = 0; i < kRun; ++i) wo[j0 + i] = bw[i];
                 }
             }
             return;
