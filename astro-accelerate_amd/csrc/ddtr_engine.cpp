@@ -150,7 +150,7 @@ lds_params lds_params_of(const range_launch &rl) {
     p.out_pitch = rl.out_pitch;
     p.row_quads = rl.row_quads;
     p.pair_recs = rl.pair_recs;
-    if (rl.variant >= 0 && rl.variant != kShapeMatrix) lds_job_tiles(p, rl.variant);
+    if (rl.variant >= 0 && rl.variant < kLdsVariants) lds_job_tiles(p, rl.variant);
     return p;
 }
 
@@ -172,6 +172,7 @@ hipError_t launch_range(const range_launch &rl, hipStream_t s) {
                                             rl.mstartdm, rl.mdmstep, rl.inBin, rl.out, rl.out_pitch, s);
     }
     if (rl.variant == kShapeMatrix) return launch_dedisperse_matrix(lds_params_of(rl), rl.mat, s);
+    if (rl.variant == kShapeRows) return launch_dedisperse_rows(lds_params_of(rl), s);
     if (rl.variant >= 0) return launch_dedisperse_lds(lds_params_of(rl), rl.variant, s);
     return launch_dedisperse_direct_u8(rl.L, rl.pitch, rl.nchans, rl.d_dmshifts, rl.ndms, rl.t_processed,
                                        rl.mstartdm, rl.mdmstep, rl.inBin, rl.out, rl.out_pitch, s);
@@ -431,6 +432,10 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
     }
     if (m_lds.size() != m_ranges.size()) m_lds.assign(m_ranges.size(), lds_choice{-2, 0});
     lds_choice &c = m_lds[(size_t)r];
+    // A range that is small, or whose trials are far apart, goes straight from
+    // the rows (in a batch the beams' ranges fill the chip together).
+    const bool automatic = range_variant(r) < 0 && m_kernel == AA_HIP_KERNEL_AUTO && rd.ndms > 0;
+    const bool alone = automatic && !batched;
     // No shape asked for: the matrix kernel where its plan is the cheaper one.
     if (range_variant(r) < 0 && (m_kernel == AA_HIP_KERNEL_AUTO || m_kernel == AA_HIP_KERNEL_LDS) &&
         (!batched || matrix_tiles_at_most(rd.ndms, t_processed) >= kMatrixAloneTiles)) {
@@ -449,7 +454,8 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
         }
         const long tiles =
             mt.lay.tile_out > 0 ? (long)mt.lay.n_dm_tiles * ((t_processed + mt.lay.tile_out - 1) / mt.lay.tile_out) : 0;
-        if (tiles > 0 && (!batched || tiles >= kMatrixAloneTiles)) {
+        if (tiles > 0 && (!batched || tiles >= kMatrixAloneTiles) &&
+            !(alone && rows_beat_matrix(m_nchans, rd.ndms, t_processed, mt.lay))) {
             st = resolve_launch(m_kernel, lv.ptr, lv.pitch, m_nchans, m_d_dmshifts, m_dmshifts.data(), rd.ndms,
                                 t_processed, mstartdm, mdmstep, rd.inBin, d_out, out_pitch,
                                 lds_choice{kShapeMatrix, mt.lay.tile_out}, rl);
@@ -464,9 +470,12 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
         if (c.variant < 0 && want >= 0)  // preferred shape does not fit: any that does
             c = choose_lds(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, -1);
     }
+    const bool rows = (alone || (automatic && c.variant < 0)) &&
+                      rows_beat_shape(m_nchans, rd.ndms, t_processed, c.variant);
     st = resolve_launch(m_kernel, lv.ptr, lv.pitch, m_nchans, m_d_dmshifts, m_dmshifts.data(), rd.ndms,
-                        t_processed, mstartdm, mdmstep, rd.inBin, d_out, out_pitch, c, rl);
-    if (st != AA_HIP_SUCCESS || rl->variant < 2) return st;
+                        t_processed, mstartdm, mdmstep, rd.inBin, d_out, out_pitch,
+                        rows ? lds_choice{kShapeRows, 0} : c, rl);
+    if (st != AA_HIP_SUCCESS || rl->variant < 2 || rl->variant == kShapeRows) return st;
     // Chunk shapes from 2 on read plan tables; they depend on the range and
     // shape only, so they are built once (on the first call that needs them,
     // never while a later call is being captured into a graph).
@@ -610,13 +619,13 @@ int ddtr_engine::autotune_range(int r, int t_processed, float *d_out, size_t out
     if (e == hipSuccess) e = hipEventCreate(&e1);
     int st = AA_HIP_SUCCESS;
     float best_ms = 0.0f;
-    float auto_ms = -1.0f;   // the automatic choice where that is the matrix kernel
+    float auto_ms = -1.0f;   // the automatic choice where that is none of the shapes
     for (int v = -1; v < kLdsVariants && e == hipSuccess && st == AA_HIP_SUCCESS; ++v) {
         if (v >= 0) ms[v] = -1.0f;
         st = set_range_variant(r, v);
         range_launch rl;
         if (st == AA_HIP_SUCCESS) st = prepare_range(r, t_processed, d_out, out_pitch, s, &rl);
-        if (st != AA_HIP_SUCCESS || rl.variant != (v < 0 ? kShapeMatrix : v)) continue;
+        if (st != AA_HIP_SUCCESS || (v < 0 ? rl.variant < kLdsVariants : rl.variant != v)) continue;
         e = launch_range(rl, s);
         if (e == hipSuccess) e = hipEventRecord(e0, s);
         for (int i = 0; i < reps && e == hipSuccess; ++i) e = launch_range(rl, s);

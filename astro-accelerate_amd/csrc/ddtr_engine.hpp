@@ -20,6 +20,7 @@
 #include "ddtr_kernels.h"
 #include "ddtr_lds.h"
 #include "ddtr_matrix.h"
+#include "ddtr_rows.h"
 
 namespace aa_hip {
 
@@ -44,12 +45,12 @@ struct lds_choice {
     int row_quads;
 };
 // First shape (or only `variant` when >= 0) whose rows hold the range's
-// windows, tried in the order 4, 2 (pair pre-summation with 2048- and
-// 1024-sample tiles, the fastest on the 8-range 4096-channel plan), 3, 0, 1.
+// windows, tried in the order 4, 5, 2 (pair pre-summation with 2016-, 1512- and
+// 1008-sample tiles, the fastest where rows are shared through LDS), 3, 0, 1, 6.
 lds_choice choose_lds(const float *h_dmshifts, int nchans, int ndms, float mstartdm, float mdmstep, int variant);
 
-// One range, resolved to a kernel: variant >= 0 = LDS kernel with that chunk
-// shape, -1 = direct kernel.
+// One range, resolved to a kernel: variant 0-6 = LDS kernel with that chunk
+// shape, kShapeMatrix, kShapeRows, -1 = direct kernel.
 struct range_launch {
     const uint8_t *L = nullptr;
     size_t pitch = 0;
@@ -117,17 +118,18 @@ public:
     // the caller (launch_range, or a batched launch).
     // batched: the caller puts the launches of many ranges into shared ones;
     // the matrix kernel, which runs one launch per range, is then taken only
-    // by ranges that fill the GPU by themselves.
+    // by ranges that fill the GPU by themselves, the kernel that reads the
+    // rows directly only by ranges that fit no shape.
     int prepare_range(int r, int t_processed, float *d_out, size_t out_pitch, hipStream_t s, range_launch *rl,
                       bool batched = false);
-    // LDS chunk shape preferred for range r (-1 = first that fits, in the
-    // order of choose_lds); used when it fits the range's delay spread.
+    // LDS chunk shape preferred for range r (-1 = automatic, see prepare_range);
+    // used when it fits the range's delay spread.
     int set_range_variant(int r, int variant);
     int range_variant(int r) const;
     // Times every LDS chunk shape that fits range r (reps launches each, after
     // one untimed launch; output written to d_out) and keeps the fastest as
-    // the range's preference, or none where the matrix kernel is the automatic
-    // choice and faster than all of them.  ms[v] = average launch time of shape v, or -1
+    // the range's preference, or none where the automatic choice is none of them
+    // and faster than all.  ms[v] = average launch time of shape v, or -1
     // when it does not fit.  *best = -1 when no shape fits.
     int autotune_range(int r, int t_processed, float *d_out, size_t out_pitch, int reps, hipStream_t s,
                        int *best, float *ms);

@@ -17,6 +17,7 @@ constexpr int kShapeMatrix = kLdsVariants;
 struct matrix_layout {
     int n_dm_tiles = 0;
     int tile_out = 0;      // output samples per tile (0: the range does not take this kernel)
+    float tile_cost = 0;   // a tile's work in steps with wide slots
     int planes = 1;        // 2: 16-bit samples as two planes of byte rows, low bytes then high bytes
     size_t off_group = 0, off_step = 0, bytes = 0;
 };

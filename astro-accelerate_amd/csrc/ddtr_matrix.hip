@@ -608,6 +608,7 @@ matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float m
     auto align = [](size_t v) { return (v + 255) / 256 * 256; };
     lay.n_dm_tiles = ntiles;
     lay.tile_out = tile_out;
+    lay.tile_cost = (float)(cost / ntiles);
     lay.planes = planes;
     lay.off_group = align(tiles.size() * sizeof(mat_tile));
     lay.off_step = align(lay.off_group + groups.size() * sizeof(mat_group));

@@ -800,11 +800,12 @@ class DdtrPlan:
         """Preferred LDS chunk shape of range r (0: 32 channels, 1: 16 channels, 2: 16 channels in
         pre-summed pairs on 1008-sample tiles, 3: 16 channels in pre-summed groups of four, 4: shape 2
         on 2016-sample tiles, 5: shape 2 on 1512-sample tiles, 6: shape 2 with 32 DM trials per tile,
-        -1: first that fits)."""
+        -1: automatic: the matrix-core kernel, sums straight from the rows, or the first shape that fits)."""
         check(_lib_or_raise().aa_hip_ddtr_set_range_variant(self.handle, int(r), int(variant)), "set_range_variant")
 
     def autotune_range(self, r: int, t_processed: int, out, reps: int = 2, stream=None):
-        """Times each LDS chunk shape that fits range r; keeps the fastest.
+        """Times each LDS chunk shape that fits range r; keeps the fastest, or the automatic choice where
+        that is none of them and faster still.
         Returns (best variant or -1, [ms per variant, -1 = does not fit])."""
         best = ctypes.c_int()
         ms = (ctypes.c_float * LDS_SHAPES)()

@@ -44,7 +44,8 @@ typedef enum {
 /* Kernel variants for aa_hip_dedisperse_u8 / aa_hip_ddtr_set_kernel. */
 typedef enum {
     AA_HIP_KERNEL_AUTO = 0,     /* handles: tuned LDS shape if set, else the matrix-core kernel where it is the
-                                   cheaper one; else the LDS kernel when a chunk shape fits, else direct */
+                                   cheaper one, sums straight from the rows for small ranges and trials far
+                                   apart; else the LDS kernel when a chunk shape fits, else direct */
     AA_HIP_KERNEL_DIRECT = 1,   /* one thread per (DM, sample), global gathers */
     AA_HIP_KERNEL_LDS = 2,      /* LDS-staged windows, packed integer sums, first shape that fits */
     AA_HIP_KERNEL_LDS_C32 = 3,  /* LDS kernel, 32-channel chunks (rows up to 2432 bytes) */
@@ -277,11 +278,12 @@ int aa_hip_ddtr_run_range(aa_hip_ddtr *h, int range, int t_processed, float *d_o
  * same rows); shapes 2, 4, 5 and 6 read rows with 16-byte LDS reads.
  * set_range_variant records a preference for range r (-1 = automatic: the
  * matrix-core kernel where the range's plan makes it the cheaper one, else the
- * first shape that fits, in the order 4, 5, 2, 3, 0, 1, 6), used whenever it
- * fits.
+ * first shape that fits, in the order 4, 5, 2, 3, 0, 1, 6; sums straight from
+ * the rows where the range is too small to fill the GPU with tiles, or its
+ * trials too far apart for shared rows), used whenever it fits.
  * autotune_range times every shape that fits range r on `stream` (reps
  * launches each, writing d_out), keeps the fastest as the preference (or -1
- * where the matrix-core kernel is the automatic choice and faster still) and
+ * where the automatic choice is none of the shapes and faster still) and
  * reports the fastest shape: *best_variant (-1 if none fits) and variant_ms[0..6] (-1 =
  * does not fit; the array holds 7 floats).
  * The range's level must be resident (after ingest). */
