@@ -308,7 +308,7 @@ int ddtr_engine::ingest(const void *d_input_tc, int input_bits, int t_processed0
     }
     int fused = 0;
     const hipError_t e = launch_corner_turn_levels(d_input_tc, input_bits / 8, len0, m_nchans, ptrs, pitches, nlev,
-                                                   m_d_err, s, &fused);
+                                                   m_d_err, s, &fused, true);
     if (e != hipSuccess) return hip_fail(e, "corner turn");
     for (auto &lv : m_levels) lv.len = 0;
     for (int k = 0; k <= fused; ++k) m_levels[(size_t)k].len = len0 >> k;

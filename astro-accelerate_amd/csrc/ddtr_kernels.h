@@ -35,14 +35,14 @@ hipError_t launch_corner_turn_u16(const uint16_t* in_tc, int nsamp, int nchans,
 // [c][t] at ptrs[0], plus the x2 floor-average levels 1..nlev (nlev <= 3)
 // L_k[t] = (L_{k-1}[2t] + L_{k-1}[2t+1]) >> 1, t < nsamp >> k, in the same
 // pass.  Rows of level k are pitches[k] bytes apart.  *fused = the number of
-// binned levels written: nlev on the wide path (nchans a multiple of 16,
-// 16-byte aligned input, rows and pitches), else 0 (level 0 only).
+// binned levels written: nlev where nchans is a multiple of 16 and the input,
+// rows and pitches are 16-byte aligned (any_fused: at any nchans and input
+// address where rows and pitches are), else 0 (level 0 only).
 constexpr int kCtMaxLevels = 3;
 hipError_t launch_corner_turn_levels(const void* in_tc, int sample_bytes, long nsamp, int nchans,
                                      uint8_t* const* ptrs, const size_t* pitches, int nlev, int* d_err,
-                                     hipStream_t s, int* fused);
-// Whether launch_corner_turn_levels writes all nlev binned levels (its wide
-// path) for these buffers, and the work-groups that path launches.
+                                     hipStream_t s, int* fused, bool any_fused = false);
+// Whether launch_corner_turn_batch takes these buffers, and the work-groups that path launches.
 bool corner_turn_levels_wide(const void* in_tc, int nchans, uint8_t* const* ptrs, const size_t* pitches, int nlev);
 long corner_turn_tiles(long nsamp, int nchans);
 // One u8 chunk of a batched corner turn: as launch_corner_turn_levels on its
