@@ -1,11 +1,14 @@
 // extern "C" surface of libaa_ddtr_hip.so (declared in include/aa_ddtr_hip.h).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <memory>
 #include <new>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "aa_ddtr_hip.h"
@@ -482,6 +485,32 @@ int aa_hip_bandpass_average(const void *h_in_tc, int bytes_per_sample, size_t nc
     if (nsamp == 0) return bad("nsamp must be positive");
     if (!h_in_tc || !h_bandpass) return bad("NULL buffer");
     aa_hip::bandpass_average(h_in_tc, bytes_per_sample, nchans, nsamp, h_bandpass);
+    return AA_HIP_SUCCESS;
+}
+
+int aa_hip_host_copy(void *dst, const void *src, size_t bytes) {
+    if (bytes == 0) return AA_HIP_SUCCESS;
+    if (!dst || !src) return bad("NULL buffer");
+    constexpr size_t kMaxThreads = 8, kPart = (size_t)4 << 20;
+    const size_t n = std::min<size_t>({kMaxThreads, bytes / kPart, std::max(1u, std::thread::hardware_concurrency())});
+    if (n <= 1) {
+        std::memcpy(dst, src, bytes);
+        return AA_HIP_SUCCESS;
+    }
+    const size_t part = (bytes / n + 4095) / 4096 * 4096;
+    const auto copy = [=](size_t i) {
+        const size_t from = std::min(i * part, bytes), to = i + 1 == n ? bytes : std::min(from + part, bytes);
+        std::memcpy((char *)dst + from, (const char *)src + from, to - from);
+    };
+    std::thread threads[kMaxThreads];
+    size_t started = 1;   // part 0 is this thread's
+    try {
+        for (; started < n; ++started) threads[started] = std::thread(copy, started);
+    } catch (const std::system_error &) {   // no more threads: the rest is this thread's too
+    }
+    copy(0);
+    for (size_t i = started; i < n; ++i) copy(i);
+    for (size_t i = 1; i < started; ++i) threads[i].join();
     return AA_HIP_SUCCESS;
 }
 

@@ -203,6 +203,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "aa_hip_input_ddtr_normalization_u16": ([vp, ctypes.c_long, i, i, vp], i),
         "aa_hip_output_ddtr_normalization": ([vp, i, ctypes.c_long, vp], i),
         "aa_hip_bandpass_average": ([vp, i, ctypes.c_size_t, ctypes.c_size_t, vp], i),
+        "aa_hip_host_copy": ([vp, vp, ctypes.c_size_t], i),
         "aa_hip_sigproc_open": ([ctypes.c_char_p, ctypes.POINTER(vp), ctypes.POINTER(filterbank_header)], i),
         "aa_hip_sigproc_read_u8": ([vp, i, ctypes.POINTER(ctypes.POINTER(ctypes.c_ubyte)), ctypes.POINTER(sz)], i),
         "aa_hip_sigproc_read_u16": ([vp, ctypes.POINTER(ctypes.POINTER(ctypes.c_ushort)), ctypes.POINTER(sz)], i),
@@ -485,8 +486,10 @@ class aa_py_pipeline:
             total = sum(strategy.t_processed(r, k) for k in range(strategy.num_tchunks))
             nd = strategy.ndms(r)
             # rows of one range are contiguous in this library
-            base = np.ctypeslib.as_array(buf[r][0], shape=(nd * total,))
-            planes.append(base.reshape(nd, total).copy())
+            plane = np.empty((nd, total), dtype=np.float32)
+            check(_lib_or_raise().aa_hip_host_copy(plane.ctypes.data, ctypes.cast(buf[r][0], ctypes.c_void_p),
+                                                   plane.nbytes), "output_planes")
+            planes.append(plane)
         return planes
 
 

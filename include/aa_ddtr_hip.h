@@ -579,6 +579,11 @@ int aa_hip_output_ddtr_normalization(float *d_plane, int ndms, long nsamp, void 
 int aa_hip_bandpass_average(const void *h_in_tc, int bytes_per_sample, size_t nchans, size_t nsamp,
                             float *h_bandpass);
 
+/* Copies `bytes` bytes of host memory between buffers that do not overlap, with
+ * up to 8 threads from 4 MiB each on: for planes of host output, which one
+ * thread reads at 2 to 3 GB/s after the GPU has written them. */
+int aa_hip_host_copy(void *dst, const void *src, size_t bytes);
+
 /* SIGPROC filterbank input.  Replaces aa_sigproc_input::read_metadata /
  * read_signal (include/aa_sigproc_input.hpp:31-47, src/aa_sigproc_input.cpp:52-80,
  * 85-541) for callers over the C ABI; the C++ class of the same name is in
