@@ -51,25 +51,26 @@ CONFIGS = {
 ADD_ROOFLINE_T = 78.64   # T adds/s, packed FP32 VALU adds
 # HBM bytes moved by the dedisperse launches of one step, from rocprofv3
 # FETCH_SIZE (x2.000, calibrated on a 1 GiB device copy) + WRITE_SIZE (x1.000)
-# summed over the launches of chunk shape 4 (pair rows on 2016-sample
-# tiles, the automatic choice): the 8 launches of the 8-range plan
-# (profiles/dedisperse_wide_8range_4096ch_1048576_hbm_traffic.txt) and the
-# one of the single-range plan (519.3 MB read + 505.5 MB written,
-# profiles/dedisperse_wide_1range_512ch_131072_kernel_trace.txt).
-# Counters cannot be read live, so the figure is tied to the kernel it was
-# taken on.
-MEASURED_TRAFFIC = {2: {"bytes": 173.5e9, "kernel": "pair",
-                        "profile": "profiles/dedisperse_wide_8range_4096ch_1048576_hbm_traffic.txt"},
-                    1: {"bytes": 1.0248e9, "kernel": "pair",
-                        "profile": "profiles/dedisperse_wide_1range_512ch_131072_kernel_trace.txt"}}
-# The kernels add 8-bit samples with integer SWAR (packed 16-bit fields,
-# v_perm + v_add3_u32), not FP32 adds, so the FP32 figure above is a nominal
-# ratio.  Their own ceiling is the VALU issue rate: 256 CU x 4 SIMD x 16
-# lanes x 2.4 GHz = 39.32 T lane-ops/s, divided by the lane-ops the kernel
-# issues per channel-add (SQ_INSTS_VALU x 64 / channel-adds, rocprofv3).
+# summed over the launches, by (config, --kernel): the matrix kernel (the
+# automatic choice on the 8-range plan), and chunk shape 4 (pair rows on
+# 2016-sample tiles) on the 8-range and the single-range plan (519.3 MB read +
+# 505.5 MB written).  Counters cannot be read live, so the figure is tied to
+# the kernel it was taken on.
+MEASURED_TRAFFIC = {(2, "auto"): {"bytes": 133.6e9,
+                                  "profile": "profiles/dedisperse_matrix_8range_4096ch_1048576_counters.txt"},
+                    (2, "pair"): {"bytes": 173.5e9,
+                                  "profile": "profiles/dedisperse_wide_8range_4096ch_1048576_hbm_traffic.txt"},
+                    (1, "pair"): {"bytes": 1.0248e9,
+                                  "profile": "profiles/dedisperse_wide_1range_512ch_131072_kernel_trace.txt"}}
+# The kernels add 8-bit samples as integers (int8 matrix products, or packed
+# 16-bit fields with v_perm + v_add3_u32), not with FP32 adds, so the FP32
+# figure above is a nominal ratio.  The pair kernels' own ceiling is the VALU
+# issue rate: 256 CU x 4 SIMD x 16 lanes x 2.4 GHz = 39.32 T lane-ops/s, divided
+# by the lane-ops the kernel issues per channel-add (SQ_INSTS_VALU x 64 /
+# channel-adds, rocprofv3).
 VALU_LANE_OPS_T = 39.32
-MEASURED_ISSUE = {2: {"lane_ops_per_add": 0.401, "kernel": "pair",
-                      "profile": "profiles/dedisperse_wide_8range_4096ch_1048576_sq_counters.txt"}}
+MEASURED_ISSUE = {(2, "pair"): {"lane_ops_per_add": 0.401,
+                                "profile": "profiles/dedisperse_wide_8range_4096ch_1048576_sq_counters.txt"}}
 HBM_PEAK_GBS = 8000.0
 SEED = 20261202
 
@@ -250,8 +251,8 @@ def main():
         f"{achieved:.2f} T adds/s ({achieved / ADD_ROOFLINE_T * 100:.1f}% of {ADD_ROOFLINE_T})")
 
     value = dm_x_samples / (ms_step * 1e-3)
-    meas = MEASURED_TRAFFIC.get(args.config)
-    traffic = meas["bytes"] if meas and args.kernel in ("auto", meas["kernel"]) else None
+    meas = MEASURED_TRAFFIC.get((args.config, args.kernel))
+    traffic = meas["bytes"] if meas else None
     result = {
         "metric": "DM×sample/s bit-exact, % FP32 add roofline; batched vs per-beam speedup",
         "value": value,
@@ -276,10 +277,11 @@ def main():
                      "hbm_frac": hbm_bytes / (k_total_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
                      "hbm_algorithmic_bytes": hbm_bytes,
                      "traffic_source": meas["profile"] if traffic else None,
-                     "peak_note": "nominal: FP32 packed-add rate; the kernels add integers (SWAR)"},
+                     "peak_note": "nominal: FP32 packed-add rate; the kernels add integers (int8 matrix "
+                                  "products or SWAR)"},
     }
-    iss = MEASURED_ISSUE.get(args.config)
-    if iss and args.kernel in ("auto", iss["kernel"]):
+    iss = MEASURED_ISSUE.get((args.config, args.kernel))
+    if iss:
         bound = VALU_LANE_OPS_T / iss["lane_ops_per_add"]
         result["roofline"]["valu_issue_bound"] = {
             "lane_ops_per_add": iss["lane_ops_per_add"], "peak_lane_ops_T": VALU_LANE_OPS_T,
@@ -420,7 +422,7 @@ def bench_spd(args, cfg):
     the 8-range plan, seeded N(0, 1) noise.  Timed with HIP events on its
     stream; MSD only (one read of the plane) and MSD + SNR (the plane read
     twice, SNR written as float and the width as u16).  Work per start sample
-    and width: one LDS read and about four VALU operations, so the pass is
+    and width: two (MSD) and four (SNR) VALU operations, so the pass is
     VALU-bound; reported beside the algorithmic HBM bytes."""
     import torch
     import py_astro_accelerate as aa
