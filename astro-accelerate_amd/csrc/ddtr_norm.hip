@@ -11,8 +11,8 @@
 // row order; then p[y] += p[y+i] for i = 16, 8, 4, 2, 1; s = p[0]/rows -
 // factor; every value becomes x - s (integers: clamped to [0, 2^nbits - 1]
 // and truncated).  The float sums round, so the order is kept exactly:
-//   - normalize_strip_f32_kernel (float planes of at most 1536 rows) keeps
-//     each partial in its own lanes and the strip in registers between the
+//   - normalize_strip_f32_kernel (float planes of at most 1536 rows; 64 or 16
+//     columns per workgroup) keeps each partial in its own lanes and the strip in registers between the
 //     sums and the write: one read, one write.
 //   - normalize_columns_kernel keeps it literally (64 columns per
 //     workgroup, wave w owns partials w and w + 16), with a second read to
@@ -96,18 +96,19 @@ __global__ __launch_bounds__(1024) void normalize_columns_kernel(T* data, long r
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef f32x4 f32x4u __attribute__((aligned(4)));   // rows start at any float
 
-// Float planes of at most 32 NR rows: 64 columns per workgroup, 16 lanes of 4
-// columns by the 32 row partials.  The strip is read once and waits in
+// Float planes of at most 32 NR rows: 4 LANES columns per workgroup, LANES lanes
+// of 4 columns by the 32 row partials.  The strip is read once and waits in
 // registers (thread y of a lane's column holds rows y, y + 32, ..., which is
 // partial y's order) until its columns' offsets are known, then is written.
-constexpr int kStripCols = 64;
 constexpr int kStripMaxRows = 1536;
-template <int NR>
-__global__ __launch_bounds__(512) void normalize_strip_f32_kernel(float* data, long rows, long cols, float factor)
+template <int NR, int LANES>
+__global__ __launch_bounds__(32 * LANES) void normalize_strip_f32_kernel(float* data, long rows, long cols,
+                                                                         float factor)
 {
-    __shared__ f32x4 part[32][kStripCols / 4];
+    constexpr int kStripCols = 4 * LANES;
+    __shared__ f32x4 part[32][LANES];
     __shared__ __align__(16) float offs[kStripCols];
-    const int q = threadIdx.x & 15, y = threadIdx.x >> 4;
+    const int q = threadIdx.x & (LANES - 1), y = threadIdx.x / LANES;
     const long c = (long)blockIdx.x * kStripCols + 4 * q;
     const bool whole = (long)blockIdx.x * kStripCols + kStripCols <= cols;   // the strip's, for all threads
     float* col = data + y * cols + c;
@@ -393,6 +394,24 @@ hipError_t normalize_int(T* data, long rows, long cols, float factor, int nbits,
     return hipGetLastError();
 }
 
+template <int LANES>
+hipError_t launch_strips(float* data, long rows, long cols, float factor, hipStream_t s)
+{
+    const dim3 strips(blocks_of(cols, 4 * LANES)), threads(32 * LANES);
+    if (rows <= 128)
+        hipLaunchKernelGGL((normalize_strip_f32_kernel<4, LANES>), strips, threads, 0, s, data, rows, cols, factor);
+    else if (rows <= 256)
+        hipLaunchKernelGGL((normalize_strip_f32_kernel<8, LANES>), strips, threads, 0, s, data, rows, cols, factor);
+    else if (rows <= 512)
+        hipLaunchKernelGGL((normalize_strip_f32_kernel<16, LANES>), strips, threads, 0, s, data, rows, cols, factor);
+    else if (rows <= 1024)
+        hipLaunchKernelGGL((normalize_strip_f32_kernel<32, LANES>), strips, threads, 0, s, data, rows, cols, factor);
+    else
+        hipLaunchKernelGGL((normalize_strip_f32_kernel<kStripMaxRows / 32, LANES>), strips, threads, 0, s, data, rows,
+                           cols, factor);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 size_t normalize_columns_scratch_bytes(long cols) { return (size_t)(cols > 0 ? cols : 0) * 33u * sizeof(float); }
@@ -414,21 +433,14 @@ hipError_t launch_normalize_columns_f32(float* data, long rows, long cols, float
 {
     if (!data || rows < 0 || cols <= 0) return hipErrorInvalidValue;
     if (rows == 0) return hipSuccess;
-    const dim3 strips(blocks_of(cols, kStripCols));
-    if (rows <= 128)
-        hipLaunchKernelGGL(normalize_strip_f32_kernel<4>, strips, dim3(512), 0, s, data, rows, cols, factor);
-    else if (rows <= 256)
-        hipLaunchKernelGGL(normalize_strip_f32_kernel<8>, strips, dim3(512), 0, s, data, rows, cols, factor);
-    else if (rows <= 512)
-        hipLaunchKernelGGL(normalize_strip_f32_kernel<16>, strips, dim3(512), 0, s, data, rows, cols, factor);
-    else if (rows <= 1024)
-        hipLaunchKernelGGL(normalize_strip_f32_kernel<32>, strips, dim3(512), 0, s, data, rows, cols, factor);
-    else if (rows <= kStripMaxRows)
-        hipLaunchKernelGGL(normalize_strip_f32_kernel<kStripMaxRows / 32>, strips, dim3(512), 0, s, data, rows, cols,
-                           factor);
-    else
-        hipLaunchKernelGGL(normalize_columns_kernel<float>, dim3(blocks_of(cols, 64)), dim3(1024), 0, s, data,
-                           rows, cols, factor, 0.0f);
+    // Strips of 64 columns, or of 16 where those would be fewer than 64: 1152 x
+    // 3117 floats 34 us with 49 strips and 20 with 195, 1536 x 3000 46 and 20;
+    // above, the longer row segments win (512 x 8000 7.4 us against 16.8).
+    if (rows <= kStripMaxRows)
+        return cols >= 64 * 64 ? launch_strips<16>(data, rows, cols, factor, s)
+                               : launch_strips<4>(data, rows, cols, factor, s);
+    hipLaunchKernelGGL(normalize_columns_kernel<float>, dim3(blocks_of(cols, 64)), dim3(1024), 0, s, data, rows, cols,
+                       factor, 0.0f);
     return hipGetLastError();
 }
 
