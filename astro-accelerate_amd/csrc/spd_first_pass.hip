@@ -25,11 +25,12 @@
 // kernel centres on the plane mean c = mean_1 and divides
 // (B'_w - (mean_w - w c)) by sd_w.
 //
-// Cost per start sample and width: 2 VALU operations in the MSD pass at W =
-// 32, else 3; 3.8 in the SNR pass at W = 32, else 5.  At W = 32 both passes
-// read a run of consecutive start samples' samples into registers once (8 in
-// the MSD pass, 4 in the SNR pass), else one LDS read per start sample and
-// width.  VALU-bound; the plane is read twice from HBM.
+// Cost per start sample and width (W rounded up to 8, 16 or 32): 2 VALU
+// operations in the MSD pass, 3.8 in the SNR pass.  Both passes read a run of
+// consecutive start samples' samples into registers once (8 in the MSD pass, 4
+// in the SNR pass).  Tiles at a row's end, where not every width fits, take 3
+// and 5 operations and an LDS read.  VALU-bound at 32 widths; the plane is read
+// twice from HBM.
 //
 // Measured on 1536 x 890,624 samples at W = 32 (2.4e9 instructions of a wave
 // for the 2 and 3.8 operations, 7.1 ms at 4.34 cycles each and 2.4 GHz; 19.2 GB,
@@ -37,7 +38,9 @@
 // instructions were the sums over the lanes of 32 widths one at a time, the
 // tile's staging (LDS written, read and written again to centre it) and one
 // wave's serial sum over the tile's edges.  SNR 6.37 ms, with 5 operations per
-// width and stores of one float at a stride of four.
+// width and stores of one float at a stride of four.  Other limits, 512 x
+// 200,000 samples, both passes: W = 5 1114 -> 326 us, 8 1186 -> 330, 16 1362 ->
+// 380, 20 1466 -> 558.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -86,39 +89,51 @@ __device__ __forceinline__ float wave_sum_to_lane63(float v)
     return v;
 }
 
-// Sums over the wave's 64 lanes of 32 values, each lane keeping one: lane l
-// gets value spread_width(l)'s.  Half of the values go to the other half of the
-// lanes at each step (row swaps, then DPP with a select), so 70 instructions
-// where a sum to lane 63 per value takes 21 each.
+// Sums over the wave's 64 lanes of N (32, 16 or 8) values, each lane keeping
+// one: lane l gets value spread_width<N>(l)'s, of the lanes with the same value
+// those without a bit of spread_again<N>() are one each.  Half of the values go
+// to the other half of the lanes at each step (row swaps, then DPP with a
+// select): at N = 32 70 instructions where a sum to lane 63 per value takes 21
+// each.
+template <int N>
 __device__ __forceinline__ int spread_width(int lane)
 {
-    return (lane >> 5) * 16 + (lane >> 4 & 1) * 8 + (lane >> 2 & 1) * 4 + (lane >> 3 & 1) * 2 + (lane >> 1 & 1);
+    const int b5 = lane >> 5, b4 = lane >> 4 & 1, b3 = lane >> 3 & 1, b2 = lane >> 2 & 1, b1 = lane >> 1 & 1;
+    return N == 32 ? b5 * 16 + b4 * 8 + b2 * 4 + b3 * 2 + b1 : N == 16 ? b5 * 8 + b4 * 4 + b2 * 2 + b3
+                                                                      : b5 * 4 + b4 * 2 + b2;
 }
+template <int N>
+constexpr int spread_again() { return N == 32 ? 1 : N == 16 ? 3 : 11; }
 template <int CTRL>
 __device__ __forceinline__ float spread_add(float a, float b, bool second)
 {
     const float keep = second ? b : a, send = second ? a : b;
     return keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(send), CTRL, 0xf, 0xf, true));
 }
-__device__ __forceinline__ float wave_spread_sum(const float (&a)[32], int lane)
+template <int N>
+__device__ __forceinline__ float wave_spread_sum(const float (&a)[N], int lane)
 {
-    float v[16];
+    float v[N / 2];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[i]), __float_as_uint(a[i + 16]), false, false);
+    for (int i = 0; i < N / 2; ++i) {
+        const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[i]), __float_as_uint(a[i + N / 2]), false, false);
         v[i] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 8]), false, false);
+    for (int i = 0; i < N / 4; ++i) {
+        const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + N / 4]), false, false);
         v[i] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
     }
     // row_ror:4 pairs lanes of unlike bit 2 (and any bit 3), row_ror:8 of unlike bit 3
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = spread_add<0x124>(v[i], v[i + 4], lane & 4);
+    for (int i = 0; i < N / 8; ++i) v[i] = spread_add<0x124>(v[i], v[i + N / 8], lane & 4);
+    if constexpr (N >= 16) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) v[i] = spread_add<0x128>(v[i], v[i + 2], lane & 8);
-    v[0] = spread_add<0x4E>(v[0], v[1], lane & 2);
+        for (int i = 0; i < N / 16; ++i) v[i] = spread_add<0x128>(v[i], v[i + N / 16], lane & 8);
+    } else {
+        v[0] = dpp_add<0x128, 0xf>(v[0]);
+    }
+    v[0] = N == 32 ? spread_add<0x4E>(v[0], v[1], lane & 2) : dpp_add<0x4E, 0xf>(v[0]);
     return dpp_add<0xB1, 0xf>(v[0]);
 }
 
@@ -160,16 +175,17 @@ __device__ __forceinline__ void chan_merge(double& na, double& ma, double& m2a, 
 
 // Per-workgroup moments over its tiles: partial[blk][w] = (n_w, mean of B_w,
 // sum of squared deviations of B_w).
-// WC: the width limit when it is known at compile time (32, the default),
-// else 0 and W_arg.  A runtime limit costs a scalar condition per width
-// (32 of them live across the loops, spilled to vector lanes).
+// WC: the width limit W rounded up to 8, 16 or 32; widths past W are computed
+// and left out.  EXACT: W is WC, known at compile time (a runtime limit costs a
+// scalar condition per width in the tiles at a row's end, live across the loops:
+// 8 % of the whole pass at 32).
 // Four waves per SIMD (128 registers a lane): the persistent grid of
 // kBlocks work-groups is resident at once only at four work-groups per CU.
-template <int WC>
+template <int WC, bool EXACT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void spd_msd_kernel(
     const float* __restrict__ plane, long pitch, int ndms, int nsamp, int W_arg, double* __restrict__ partial)
 {
-    const int W = WC > 0 ? WC : W_arg;
+    const int W = EXACT ? WC : W_arg;
     __shared__ __align__(16) float s[kTile + kMaxW];
     __shared__ float red[kThreads / 64][2 * kMaxW];
     __shared__ float wsum[kThreads / 64];
@@ -184,8 +200,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
         const long rest = (long)nsamp - t0;
         const int nout = (int)(rest < kTile ? rest : kTile);                 // start samples in the tile
         const int nload = (int)(rest < kTile + W - 1 ? rest : kTile + W - 1);  // samples staged
-        // All 32 widths fit at every start sample (a wave-uniform case).
-        const bool fast = WC == kMaxW && nload == kTile + W - 1;
+        // All WC widths fit at every start sample (a wave-uniform case).
+        const bool fast = rest >= kTile + WC - 1;
         float c;
         if (fast) {
             // The tile waits in registers for its mean, so it is written to LDS
@@ -194,7 +210,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
 #pragma unroll
             for (int k = 0; k < kK / 4; ++k)
                 v[k] = *reinterpret_cast<const f32x4u*>(row + t0 + 4 * (tid + kThreads * k));
-            const float after = tid < kMaxW - 1 ? row[t0 + kTile + tid] : 0.0f;
+            const float after = tid < WC - 1 ? row[t0 + kTile + tid] : 0.0f;
             float part = 0.0f;
 #pragma unroll
             for (int k = 0; k < kK / 4; ++k) part += (v[k].x + v[k].y) + (v[k].z + v[k].w);
@@ -222,9 +238,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
             for (int i = tid; i < nload; i += kThreads) s[i] -= c;
             __syncthreads();
         }
-        float a1[kMaxW], a2[kMaxW];
+        float a1[WC], a2[WC];
 #pragma unroll
-        for (int w = 0; w < kMaxW; ++w) a1[w] = a2[w] = 0.0f;
+        for (int w = 0; w < WC; ++w) a1[w] = a2[w] = 0.0f;
         // With all widths at every start sample the sums of B_w over the tile follow from the tile's sum C_0 and its
         // edges (below), so the loop keeps only the running sum and the
         // square sums; runs of kRun consecutive start samples per thread,
@@ -232,7 +248,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
         // reads (instead of one LDS read per start sample and width).
         float cs = 0.0f;   // fast: this thread's part of C_0 = sum of s[0 .. kTile)
         if (fast) {
-            constexpr int kRun = 8, kWin = kRun + kMaxW;   // 40 registers: s[j0 .. j0 + 39]
+            constexpr int kRun = 8, kWin = kRun + WC;   // 40 registers: s[j0 .. j0 + 39]
             static_assert(kTile % (kRun * kThreads) == 0, "whole runs per thread");
 #pragma unroll 1
             for (int k = 0; k < kTile / (kRun * kThreads); ++k) {
@@ -251,7 +267,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
                     cs += v[i];
                     float B = 0.0f;
 #pragma unroll
-                    for (int w = 0; w < kMaxW; ++w) {
+                    for (int w = 0; w < WC; ++w) {
                         B += v[i + w];
                         a2[w] = __builtin_fmaf(B, B, a2[w]);
                     }
@@ -263,7 +279,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
                 const int j = tid + kThreads * k;
                 float B = 0.0f;
 #pragma unroll
-                for (int w = 0; w < kMaxW; ++w) {
+                for (int w = 0; w < WC; ++w) {
                     if (w < W) {
                         B += s[j + w];
                         a1[w] += B;
@@ -277,7 +293,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
                 if (j >= nout) break;
                 float B = 0.0f;
 #pragma unroll
-                for (int w = 0; w < kMaxW; ++w) {
+                for (int w = 0; w < WC; ++w) {
                     if (w < W && j + w < nload) {
                         B += s[j + w];
                         a1[w] += B;
@@ -288,8 +304,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
         }
         const float r2 = wave_spread_sum(a2, lane);
         const float r1 = fast ? wave_sum_to_lane63(cs) : wave_spread_sum(a1, lane);
-        if ((lane & 1) == 0) red[wv][kMaxW + spread_width(lane)] = r2;
-        if (fast ? lane == 63 : (lane & 1) == 0) red[wv][fast ? 0 : spread_width(lane)] = r1;
+        const bool keeps = (lane & spread_again<WC>()) == 0;
+        if (keeps) red[wv][kMaxW + spread_width<WC>(lane)] = r2;
+        if (fast ? lane == 63 : keeps) red[wv][fast ? 0 : spread_width<WC>(lane)] = r1;
         __syncthreads();
         if (tid < W) {
             const int w = tid + 1;
@@ -373,12 +390,12 @@ __global__ __launch_bounds__(kFinThreads) void spd_msd_finalize_kernel(const dou
     if (threadIdx.x == 0) aux->finite = finite;
 }
 
-template <int WC>
+template <int WC, bool EXACT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void spd_snr_kernel(
     const float* __restrict__ plane, long pitch, int nsamp, int W_arg, const spd_aux* __restrict__ aux,
     float* __restrict__ snr, long snr_pitch, uint16_t* __restrict__ width, long width_pitch)
 {
-    const int W = WC > 0 ? WC : W_arg;
+    const int W = EXACT ? WC : W_arg;
     __shared__ __align__(16) float s[kTile + kMaxW];
     __shared__ float off[kMaxW];
     __shared__ __align__(16) float rsd[kMaxW], prod[kMaxW];   // prod: -off * rsd
@@ -392,16 +409,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
     const int nload = (int)(rest < kTile + W - 1 ? rest : kTile + W - 1);
     const float c = aux->c;
     if (tid < kMaxW) {
-        off[tid] = aux->off[tid];
-        rsd[tid] = aux->rsd[tid];
-        prod[tid] = -off[tid] * rsd[tid];
+        // widths past W: an SNR below every other
+        off[tid] = tid < W ? aux->off[tid] : 0.0f;
+        rsd[tid] = tid < W ? aux->rsd[tid] : 0.0f;
+        prod[tid] = tid < W ? -off[tid] * rsd[tid] : -INFINITY;
     }
-    if (WC == kMaxW && nload == kTile + W - 1) {
+    const bool fast = rest >= kTile + WC - 1;   // all WC widths fit at every start sample
+    if (fast) {
         f32x4 v[kK / 4];
 #pragma unroll
         for (int k = 0; k < kK / 4; ++k)
             v[k] = *reinterpret_cast<const f32x4u*>(row + t0 + 4 * (tid + kThreads * k));
-        const float after = tid < kMaxW - 1 ? row[t0 + kTile + tid] : 0.0f;
+        const float after = tid < WC - 1 ? row[t0 + kTile + tid] : 0.0f;
 #pragma unroll
         for (int k = 0; k < kK / 4; ++k) *reinterpret_cast<f32x4*>(s + 4 * (tid + kThreads * k)) = v[k] - c;
         if (tid < kMaxW) s[kTile + tid] = after - c;
@@ -413,15 +432,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
     uint16_t* wo = width ? width + d * width_pitch + t0 : nullptr;
     if (nload == kTile + W - 1) {   // every width fits at every start sample
         // SNR_w = B'_w * rsd_w - off_w * rsd_w: one FMA per width
-        float p[kMaxW], r[kMaxW];
+        float p[WC], r[WC];
 #pragma unroll
-        for (int w = 0; w < kMaxW; ++w) {
+        for (int w = 0; w < WC; ++w) {
             r[w] = rsd[w];
-            p[w] = WC == kMaxW ? __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(prod[w]))) : prod[w];
+            p[w] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(prod[w])));
         }
         // Finite: no SNR is a NaN (the offsets hold the plane's mean, so every
         // sample is finite as well), which the maxima below would pass over.
-        if (WC == kMaxW && aux->finite) {
+        if (fast && aux->finite) {
             // Runs of kRun consecutive start samples per thread, their
             // kRun + 31 samples read into registers once.  The largest SNR of
             // each kGroup widths is taken with max3; only the first group that
@@ -429,7 +448,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
             // before it, and its SNRs are computed once more (the same
             // operations) to find the width: 3.8 operations per width where
             // keeping the width along with each maximum takes 5.
-            constexpr int kRun = 4, kWin = kRun + kMaxW;   // 36 registers: s[j0 .. j0 + 35]
+            constexpr int kRun = 4, kWin = kRun + WC;   // 36 registers: s[j0 .. j0 + 35]
             constexpr int kGroup = 4;
             static_assert(kTile % (kRun * kThreads) == 0, "whole runs per thread");
             const bool vec_s = so && ((uintptr_t)so & 15) == 0, vec_w = wo && ((uintptr_t)wo & 7) == 0;
@@ -452,7 +471,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
                     float B = 0.0f, top = 0.0f, before = 0.0f;
                     int at = 0;   // first width - 1 of the group with the maximum
 #pragma unroll
-                    for (int g = 0; g < kMaxW; g += kGroup) {
+                    for (int g = 0; g < WC; g += kGroup) {
                         const float start = B;
                         float x[kGroup];
 #pragma unroll
@@ -509,7 +528,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))
             float best = __builtin_fmaf(B, r[0], p[0]);
             int bw = 1;
 #pragma unroll
-            for (int w = 1; w < kMaxW; ++w) {
+            for (int w = 1; w < WC; ++w) {
                 if (w < W) {
                     B += s[j + w];
                     const float v = __builtin_fmaf(B, r[w], p[w]);
@@ -562,20 +581,27 @@ hipError_t launch_spd_first_pass(const float* plane, size_t pitch, int ndms, int
     const long per_row = ((long)nsamp + kTile - 1) / kTile;
     const long ntiles = (long)ndms * per_row;
     if (ntiles > 0x7fffffffL) return hipErrorInvalidValue;
-    if (W == kMaxW)
-        hipLaunchKernelGGL(spd_msd_kernel<kMaxW>, dim3(kBlocks), dim3(kThreads), 0, s, plane, (long)pitch, ndms, nsamp,
-                           W, partial);
-    else
-        hipLaunchKernelGGL(spd_msd_kernel<0>, dim3(kBlocks), dim3(kThreads), 0, s, plane, (long)pitch, ndms, nsamp, W,
-                           partial);
+#define AA_SPD_MSD(WC_, EXACT_) \
+    hipLaunchKernelGGL((spd_msd_kernel<WC_, EXACT_>), dim3(kBlocks), dim3(kThreads), 0, s, plane, (long)pitch, ndms, nsamp, W, partial)
+    if (W == kMaxW) AA_SPD_MSD(kMaxW, true);
+    else if (W > 16) AA_SPD_MSD(kMaxW, false);
+    else if (W == 16) AA_SPD_MSD(16, true);
+    else if (W > 8) AA_SPD_MSD(16, false);
+    else if (W == 8) AA_SPD_MSD(8, true);
+    else AA_SPD_MSD(8, false);
+#undef AA_SPD_MSD
     hipLaunchKernelGGL(spd_msd_finalize_kernel, dim3(1), dim3(kFinThreads), 0, s, (const double*)partial, kBlocks, W, msd, aux);
     if (snr || width) {
-        if (W == kMaxW)
-            hipLaunchKernelGGL(spd_snr_kernel<kMaxW>, dim3((unsigned)ntiles), dim3(kThreads), 0, s, plane, (long)pitch,
-                               nsamp, W, (const spd_aux*)aux, snr, (long)snr_pitch, width, (long)width_pitch);
-        else
-            hipLaunchKernelGGL(spd_snr_kernel<0>, dim3((unsigned)ntiles), dim3(kThreads), 0, s, plane, (long)pitch,
-                               nsamp, W, (const spd_aux*)aux, snr, (long)snr_pitch, width, (long)width_pitch);
+#define AA_SPD_SNR(WC_, EXACT_) \
+    hipLaunchKernelGGL((spd_snr_kernel<WC_, EXACT_>), dim3((unsigned)ntiles), dim3(kThreads), 0, s, plane, (long)pitch, nsamp, W, \
+                       (const spd_aux*)aux, snr, (long)snr_pitch, width, (long)width_pitch)
+        if (W == kMaxW) AA_SPD_SNR(kMaxW, true);
+        else if (W > 16) AA_SPD_SNR(kMaxW, false);
+        else if (W == 16) AA_SPD_SNR(16, true);
+        else if (W > 8) AA_SPD_SNR(16, false);
+        else if (W == 8) AA_SPD_SNR(8, true);
+        else AA_SPD_SNR(8, false);
+#undef AA_SPD_SNR
     }
     return hipGetLastError();
 }

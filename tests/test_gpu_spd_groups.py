@@ -60,3 +60,21 @@ def test_a_flat_plane(aa, cuda):
     msd, snr, width = aa.spd_first_pass(x, 32)
     assert bool((msd[:, 1] == 0).all())
     assert bool((snr == 0).all()) and bool((width == 1).all())
+
+
+@pytest.mark.parametrize("W", [1, 2, 5, 7, 8, 9, 15, 16, 17, 31])
+@pytest.mark.parametrize("nsamp", ["all widths of one tile", "one short", "two tiles and 8", "two tiles and 31"])
+def test_other_width_limits(aa, cuda, W, nsamp):
+    """Limits between the 8, 16 and 32 the kernels are compiled for."""
+    import torch
+    n = {"all widths of one tile": TILE + W - 1, "one short": TILE + max(W - 2, 0), "two tiles and 8": 2 * TILE + 8,
+         "two tiles and 31": 2 * TILE + 31}[nsamp]
+    rng = np.random.default_rng(100 * W + n)
+    x = rng.normal(40.0, 1.0, size=(5, n)).astype(np.float32)
+    x[3, 4000:4000 + W] += 9.0
+    x[4, TILE - 3:TILE - 3 + W] += 9.0
+    msd, snr, width = aa.spd_first_pass(torch.from_numpy(x).to(cuda), W)
+    check_first_pass(x, W, msd.cpu().numpy(), snr.cpu().numpy(), width.cpu().numpy().astype(np.int64))
+    x[1, 77] = np.nan
+    _, snr, width = aa.spd_first_pass(torch.from_numpy(x).to(cuda), W)
+    assert bool(torch.isnan(snr).all()) and bool((width == 1).all())
