@@ -446,8 +446,8 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
             const matrix_layout lay =
                 matrix_plan(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, lv.pitch, &bytes);
             if (lay.tile_out > 0) {
-                st = keep_tables(mt.t, kShapeMatrix, bytes);
-                if (st != AA_HIP_SUCCESS) return st;
+                const hipError_t e = keep_tables(mt.t, kShapeMatrix, bytes);
+                if (e != hipSuccess) return hip_fail(e, "plan tables");
             }
             mt.lay = lay;
             mt.planned = true;
@@ -486,8 +486,8 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
         if (lds_plan_tables(rl->variant, m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, lv.pitch, &bytes) !=
             rl->row_quads)
             return fail(AA_HIP_ERROR_UNSUPPORTED, "plan tables disagree with the chosen row width");
-        st = keep_tables(pt, rl->variant, bytes);
-        if (st != AA_HIP_SUCCESS) return st;
+        const hipError_t e = keep_tables(pt, rl->variant, bytes);
+        if (e != hipSuccess) return hip_fail(e, "plan tables");
     }
     rl->pair_recs = pt.ptr;
     return AA_HIP_SUCCESS;
@@ -507,7 +507,8 @@ int ddtr_engine::u16_window(int r) {
 
 // The automatic choice on u16 levels: the matrix kernel over the rows' byte
 // planes where its plan pays (dedisperse_u16 then computes the tiles it
-// flags).  Without the memory for its tables the range keeps dedisperse_u16.
+// flags).  Without the memory for its tables or the level's planes the range
+// keeps dedisperse_u16, from its first chunk on.
 bool ddtr_engine::u16_matrix(int r) {
     if (m_sample_bytes != 2 || m_kernel != AA_HIP_KERNEL_AUTO || u16_window(r) <= 0) return false;
     if (m_matrix.size() != m_ranges.size()) m_matrix.resize(m_ranges.size());
@@ -521,14 +522,16 @@ bool ddtr_engine::u16_matrix(int r) {
     std::vector<uint8_t> bytes;
     const matrix_layout lay = matrix_plan(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep,
                                           round_up((size_t)lv.capacity + kRowPad, kPitchAlign), &bytes, 2);
-    if (lay.tile_out <= 0 || keep_tables(mt.t, kShapeMatrix, bytes) != AA_HIP_SUCCESS) return false;
+    if (lay.tile_out <= 0 || keep_tables(mt.t, kShapeMatrix, bytes) != hipSuccess) return false;
     const size_t tiles =
         (size_t)lay.n_dm_tiles * (size_t)((lv.capacity + lay.tile_out - 1) / lay.tile_out) * sizeof(int);
     if (hipMalloc(&mt.flags, tiles) != hipSuccess) {
-        mt.flags = nullptr;
         (void)hipGetLastError();
+        mt.flags = nullptr;
+        drop_matrix(r);
         return false;
     }
+    mt.flag_bytes = tiles;
     m_device_bytes += tiles;
     mt.lay = lay;
     return true;
@@ -546,6 +549,9 @@ int ddtr_engine::level_planes(int k, hipStream_t s) {
     return AA_HIP_SUCCESS;
 }
 
+// Byte planes of level k for the current chunk.  Without the memory for them
+// no range of the level takes the matrix kernel: OUT_OF_MEMORY, no message set.
+
 int ddtr_engine::ensure_planes(int k, hipStream_t s) {
     level &lv = m_levels[(size_t)k];
     if (lv.planes_ok) return AA_HIP_SUCCESS;
@@ -555,6 +561,8 @@ int ddtr_engine::ensure_planes(int k, hipStream_t s) {
         if (hipMalloc(&p, 2 * pitch * (size_t)m_nchans) != hipSuccess || hipMalloc(&o, 64 * sizeof(int)) != hipSuccess) {
             (void)hipGetLastError();
             if (p) (void)hipFree(p);
+            for (int r = 0; r < (int)m_matrix.size(); ++r)
+                if (log2i(m_ranges[(size_t)r].inBin) == k) drop_matrix(r);
             return AA_HIP_ERROR_OUT_OF_MEMORY;
         }
         lv.planes = static_cast<uint8_t *>(p);
@@ -572,24 +580,37 @@ int ddtr_engine::ensure_planes(int k, hipStream_t s) {
     return AA_HIP_SUCCESS;
 }
 
-int ddtr_engine::keep_tables(plan_tables &pt, int variant, const std::vector<uint8_t> &bytes) {
-    if (pt.ptr) {
-        (void)hipFree(pt.ptr);
-        m_device_bytes -= pt.bytes;
-    }
-    pt = plan_tables{};
+hipError_t ddtr_engine::keep_tables(plan_tables &pt, int variant, const std::vector<uint8_t> &bytes) {
+    drop_tables(pt);
     void *t = nullptr;
     hipError_t e = hipMalloc(&t, bytes.size());
     if (e == hipSuccess) e = hipMemcpy(t, bytes.data(), bytes.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
+        (void)hipGetLastError();   // else the next launch reports it
         if (t) (void)hipFree(t);
-        return hip_fail(e, "plan tables");
+        return e;
     }
     pt.variant = variant;
     pt.ptr = t;
     pt.bytes = bytes.size();
     m_device_bytes += bytes.size();
-    return AA_HIP_SUCCESS;
+    return hipSuccess;
+}
+
+void ddtr_engine::drop_tables(plan_tables &pt) {
+    if (pt.ptr) (void)hipFree(pt.ptr);
+    m_device_bytes -= pt.bytes;
+    pt = plan_tables{};
+}
+
+// Range r is not the matrix kernel's after all; gives back what it held for it.
+void ddtr_engine::drop_matrix(int r) {
+    matrix_tables &mt = m_matrix[(size_t)r];
+    drop_tables(mt.t);
+    if (mt.flags) (void)hipFree(mt.flags);
+    m_device_bytes -= mt.flag_bytes;
+    mt = matrix_tables{};
+    mt.planned = true;
 }
 
 int ddtr_engine::set_range_variant(int r, int variant) {

@@ -158,8 +158,6 @@ private:
         int *over = nullptr;
         bool planes_ok = false;
     };
-    // Byte planes of level k for the current chunk; OUT_OF_MEMORY without a
-    // message set when they cannot be allocated.
     int ensure_planes(int k, hipStream_t s);
 
     int m_device = 0;
@@ -188,14 +186,18 @@ private:
         matrix_layout lay;
         plan_tables t;
         int *flags = nullptr;   // u16 levels: one entry per tile
+        size_t flag_bytes = 0;
     };
     std::vector<matrix_tables> m_matrix;  // per range: the matrix kernel's, kept beside the LDS shape's, which a
                                           // captured batch may still read
     int u16_window(int r);
     bool u16_matrix(int r);
     int level_planes(int k, hipStream_t s);
-    // Uploads tables of `variant` in place of what pt holds.
-    int keep_tables(plan_tables &pt, int variant, const std::vector<uint8_t> &bytes);
+    // Uploads tables of `variant` in place of what pt holds; on failure pt is
+    // empty and HIP's pending error taken.
+    hipError_t keep_tables(plan_tables &pt, int variant, const std::vector<uint8_t> &bytes);
+    void drop_tables(plan_tables &pt);
+    void drop_matrix(int r);
     size_t m_device_bytes = 0;
 };
 
