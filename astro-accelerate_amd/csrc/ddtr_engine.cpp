@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <new>
 
 #include "aa_ddtr_hip.h"
 #include "ddtr_lds.h"
@@ -439,19 +440,9 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
     // No shape asked for: the matrix kernel where its plan is the cheaper one.
     if (range_variant(r) < 0 && (m_kernel == AA_HIP_KERNEL_AUTO || m_kernel == AA_HIP_KERNEL_LDS) &&
         (!batched || matrix_tiles_at_most(rd.ndms, t_processed) >= kMatrixAloneTiles)) {
-        if (m_matrix.size() != m_ranges.size()) m_matrix.resize(m_ranges.size());
-        matrix_tables &mt = m_matrix[(size_t)r];
-        if (!mt.planned) {
-            std::vector<uint8_t> bytes;
-            const matrix_layout lay =
-                matrix_plan(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, lv.pitch, &bytes);
-            if (lay.tile_out > 0) {
-                const hipError_t e = keep_tables(mt.t, kShapeMatrix, bytes);
-                if (e != hipSuccess) return hip_fail(e, "plan tables");
-            }
-            mt.lay = lay;
-            mt.planned = true;
-        }
+        const hipError_t e = plan_matrix(r, lv.pitch, 1);
+        if (e != hipSuccess && e != hipErrorOutOfMemory) return hip_fail(e, "plan tables");
+        const matrix_tables &mt = m_matrix[(size_t)r];
         const long tiles =
             mt.lay.tile_out > 0 ? (long)mt.lay.n_dm_tiles * ((t_processed + mt.lay.tile_out - 1) / mt.lay.tile_out) : 0;
         if (tiles > 0 && (!batched || tiles >= kMatrixAloneTiles) &&
@@ -511,20 +502,12 @@ int ddtr_engine::u16_window(int r) {
 // keeps dedisperse_u16, from its first chunk on.
 bool ddtr_engine::u16_matrix(int r) {
     if (m_sample_bytes != 2 || m_kernel != AA_HIP_KERNEL_AUTO || u16_window(r) <= 0) return false;
-    if (m_matrix.size() != m_ranges.size()) m_matrix.resize(m_ranges.size());
+    const level &lv = m_levels[(size_t)log2i(m_ranges[(size_t)r].inBin)];
+    (void)plan_matrix(r, round_up((size_t)lv.capacity + kRowPad, kPitchAlign), 2);
     matrix_tables &mt = m_matrix[(size_t)r];
-    if (mt.planned) return mt.lay.tile_out > 0;
-    mt.planned = true;
-    const range_desc &rd = m_ranges[(size_t)r];
-    const level &lv = m_levels[(size_t)log2i(rd.inBin)];
-    float mstartdm, mdmstep;
-    range_scalars(r, &mstartdm, &mdmstep);
-    std::vector<uint8_t> bytes;
-    const matrix_layout lay = matrix_plan(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep,
-                                          round_up((size_t)lv.capacity + kRowPad, kPitchAlign), &bytes, 2);
-    if (lay.tile_out <= 0 || keep_tables(mt.t, kShapeMatrix, bytes) != hipSuccess) return false;
+    if (mt.lay.tile_out <= 0 || mt.flags) return mt.lay.tile_out > 0;
     const size_t tiles =
-        (size_t)lay.n_dm_tiles * (size_t)((lv.capacity + lay.tile_out - 1) / lay.tile_out) * sizeof(int);
+        (size_t)mt.lay.n_dm_tiles * (size_t)((lv.capacity + mt.lay.tile_out - 1) / mt.lay.tile_out) * sizeof(int);
     if (hipMalloc(&mt.flags, tiles) != hipSuccess) {
         (void)hipGetLastError();
         mt.flags = nullptr;
@@ -533,7 +516,6 @@ bool ddtr_engine::u16_matrix(int r) {
     }
     mt.flag_bytes = tiles;
     m_device_bytes += tiles;
-    mt.lay = lay;
     return true;
 }
 
@@ -601,6 +583,29 @@ void ddtr_engine::drop_tables(plan_tables &pt) {
     if (pt.ptr) (void)hipFree(pt.ptr);
     m_device_bytes -= pt.bytes;
     pt = plan_tables{};
+}
+
+// Range r's plan for the matrix kernel, made once, with its tables on the
+// device; tile_out 0 where the plan does not pay.  Without the memory for it
+// (host or device) the range is not the matrix kernel's either, from its first
+// call on: hipErrorOutOfMemory, once, for callers that have no other kernel.
+hipError_t ddtr_engine::plan_matrix(int r, size_t pitch, int planes) {
+    if (m_matrix.size() != m_ranges.size()) m_matrix.resize(m_ranges.size());
+    matrix_tables &mt = m_matrix[(size_t)r];
+    if (mt.planned) return hipSuccess;
+    mt.planned = true;
+    float mstartdm, mdmstep;
+    range_scalars(r, &mstartdm, &mdmstep);
+    try {
+        std::vector<uint8_t> bytes;
+        const matrix_layout lay =
+            matrix_plan(m_dmshifts.data(), m_nchans, m_ranges[(size_t)r].ndms, mstartdm, mdmstep, pitch, &bytes, planes);
+        const hipError_t e = lay.tile_out > 0 ? keep_tables(mt.t, kShapeMatrix, bytes) : hipSuccess;
+        if (e == hipSuccess) mt.lay = lay;
+        return e;
+    } catch (const std::bad_alloc &) {
+        return hipErrorOutOfMemory;
+    }
 }
 
 // Range r is not the matrix kernel's after all; gives back what it held for it.

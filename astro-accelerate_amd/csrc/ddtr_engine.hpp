@@ -197,6 +197,7 @@ private:
     // empty and HIP's pending error taken.
     hipError_t keep_tables(plan_tables &pt, int variant, const std::vector<uint8_t> &bytes);
     void drop_tables(plan_tables &pt);
+    hipError_t plan_matrix(int r, size_t pitch, int planes);
     void drop_matrix(int r);
     size_t m_device_bytes = 0;
 };

@@ -45,3 +45,32 @@ assert plan.device_bytes() == bytes_
 plan.close()
 assert fake.lib.fake_device_bytes() == 0
 ''', tmp_path)
+
+
+@pytest.mark.parametrize("where", ["device", "host"])
+def test_8_bit_plan_without_memory(tmp_path, where):
+    """Without the memory for the matrix kernel's tables an 8-bit range runs the
+    LDS shape that fits, from its first call on."""
+    host_library.run(GEOMETRY + f'''
+x = Tensor((tp + maxshift, 1024), 1)
+plan = make(8)
+created = len(fake.allocations())
+plan.execute_chunk(x, [tp], [out])
+assert fake.ran("dedisperse_matrix_kernel")
+tables, = fake.allocations()[created:]
+plan.close()
+plan = make(8)
+plan.ingest(x, tp)
+if "{where}" == "device":
+    fake.fail_allocations(tables, tables + 1)
+else:
+    fake.lib.fake_fail_host_allocations(tables)   # the tables are put together in host memory
+plan.run_range(0, tp, out)
+names = fake.kernels()
+assert any("dedisperse_wide_kernel" in n for n in names) and not any("matrix" in n for n in names), names
+fake.fail_allocations()
+fake.lib.fake_fail_host_allocations(2 ** 64 - 1)
+plan.run_range(0, tp, out)
+assert not fake.ran("matrix")
+assert plan.device_bytes() == fake.lib.fake_device_bytes()
+''', tmp_path)
