@@ -27,6 +27,11 @@ int hip_fail(hipError_t e, const char *what) {
                 std::string(what) + ": " + hipGetErrorString(e));
 }
 
+int no_matrix() {
+    return fail(AA_HIP_ERROR_UNSUPPORTED, "the matrix kernel does not take this range (its plan does not fit or does "
+                                          "not pay, or there is no memory for its tables)");
+}
+
 // A batched range with this many tiles fills the GPU's 256 work-groups twice
 // over and runs a matrix launch of its own; smaller ones stay in the shared
 // launches (96 beams of 64-256 channels: 1.98 ms batched, 4.27 ms with a
@@ -265,7 +270,7 @@ ddtr_engine::~ddtr_engine() {
 }
 
 int ddtr_engine::set_kernel(int kernel) {
-    if (kernel < AA_HIP_KERNEL_AUTO || kernel > AA_HIP_KERNEL_LDS_QUAD)
+    if (kernel < AA_HIP_KERNEL_AUTO || kernel > AA_HIP_KERNEL_MATRIX)
         return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "unknown kernel variant");
     m_kernel = kernel;
     return AA_HIP_SUCCESS;
@@ -417,9 +422,11 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
         rl->wide_win = m_kernel == AA_HIP_KERNEL_DIRECT ? -1 : u16_window(r);
         if (rl->wide_win < 0 && m_kernel != AA_HIP_KERNEL_AUTO && m_kernel != AA_HIP_KERNEL_DIRECT)
             return fail(AA_HIP_ERROR_UNSUPPORTED, "the 16-bit LDS kernel does not fit this range's delay spread");
-        if (rd.ndms <= 0 || !u16_matrix(r)) return AA_HIP_SUCCESS;
+        if (rd.ndms <= 0) return AA_HIP_SUCCESS;
+        const bool forced = m_kernel == AA_HIP_KERNEL_MATRIX;
+        if (!u16_matrix(r)) return forced ? no_matrix() : AA_HIP_SUCCESS;
         st = ensure_planes(k, s);   // (the kernel setting may have changed since the level was written)
-        if (st == AA_HIP_ERROR_OUT_OF_MEMORY) return AA_HIP_SUCCESS;
+        if (st == AA_HIP_ERROR_OUT_OF_MEMORY) return forced ? no_matrix() : AA_HIP_SUCCESS;
         if (st != AA_HIP_SUCCESS) return st;
         const matrix_tables &mt = m_matrix[(size_t)r];
         rl->variant = kShapeMatrix;
@@ -438,15 +445,16 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
     const bool automatic = range_variant(r) < 0 && m_kernel == AA_HIP_KERNEL_AUTO && rd.ndms > 0;
     const bool alone = automatic && !batched;
     // No shape asked for: the matrix kernel where its plan is the cheaper one.
-    if (range_variant(r) < 0 && (m_kernel == AA_HIP_KERNEL_AUTO || m_kernel == AA_HIP_KERNEL_LDS) &&
-        (!batched || matrix_tiles_at_most(rd.ndms, t_processed) >= kMatrixAloneTiles)) {
+    const bool forced = m_kernel == AA_HIP_KERNEL_MATRIX && rd.ndms > 0;
+    if (forced || (automatic && (!batched || matrix_tiles_at_most(rd.ndms, t_processed) >= kMatrixAloneTiles))) {
         const hipError_t e = plan_matrix(r, lv.pitch, 1);
-        if (e != hipSuccess && e != hipErrorOutOfMemory) return hip_fail(e, "plan tables");
+        if (e != hipSuccess && (forced || e != hipErrorOutOfMemory)) return hip_fail(e, "plan tables");
         const matrix_tables &mt = m_matrix[(size_t)r];
+        if (forced && mt.lay.tile_out <= 0) return no_matrix();
         const long tiles =
             mt.lay.tile_out > 0 ? (long)mt.lay.n_dm_tiles * ((t_processed + mt.lay.tile_out - 1) / mt.lay.tile_out) : 0;
-        if (tiles > 0 && (!batched || tiles >= kMatrixAloneTiles) &&
-            !(alone && rows_beat_matrix(m_nchans, rd.ndms, t_processed, mt.lay))) {
+        if (forced || (tiles > 0 && (!batched || tiles >= kMatrixAloneTiles) &&
+                       !(alone && rows_beat_matrix(m_nchans, rd.ndms, t_processed, mt.lay)))) {
             st = resolve_launch(m_kernel, lv.ptr, lv.pitch, m_nchans, m_d_dmshifts, m_dmshifts.data(), rd.ndms,
                                 t_processed, mstartdm, mdmstep, rd.inBin, d_out, out_pitch,
                                 lds_choice{kShapeMatrix, mt.lay.tile_out}, rl);
@@ -501,7 +509,9 @@ int ddtr_engine::u16_window(int r) {
 // flags).  Without the memory for its tables or the level's planes the range
 // keeps dedisperse_u16, from its first chunk on.
 bool ddtr_engine::u16_matrix(int r) {
-    if (m_sample_bytes != 2 || m_kernel != AA_HIP_KERNEL_AUTO || u16_window(r) <= 0) return false;
+    if (m_sample_bytes != 2 || (m_kernel != AA_HIP_KERNEL_AUTO && m_kernel != AA_HIP_KERNEL_MATRIX) ||
+        u16_window(r) <= 0)
+        return false;
     const level &lv = m_levels[(size_t)log2i(m_ranges[(size_t)r].inBin)];
     (void)plan_matrix(r, round_up((size_t)lv.capacity + kRowPad, kPitchAlign), 2);
     matrix_tables &mt = m_matrix[(size_t)r];

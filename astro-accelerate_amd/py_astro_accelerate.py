@@ -1029,5 +1029,6 @@ def inject_pulse_u8(d_data_tc, nsamp: int, nchans: int, d_dmshifts, dm: float, t
                                                  _stream_ptr(stream)), "inject_pulse_u8")
 
 
-KERNEL_AUTO, KERNEL_DIRECT, KERNEL_LDS, KERNEL_LDS_C32, KERNEL_LDS_C16, KERNEL_LDS_PAIR, KERNEL_LDS_QUAD = range(7)
+(KERNEL_AUTO, KERNEL_DIRECT, KERNEL_LDS, KERNEL_LDS_C32, KERNEL_LDS_C16, KERNEL_LDS_PAIR, KERNEL_LDS_QUAD,
+ KERNEL_MATRIX) = range(8)
 LDS_SHAPES = 7   # LDS chunk shapes 0-6 (set_range_variant, autotune_range)

@@ -53,7 +53,9 @@ typedef enum {
     AA_HIP_KERNEL_LDS_PAIR = 5, /* LDS kernel, 16-channel chunks pre-summed in channel pairs
                                    (the widest tile that fits: 2016, 1512 or 1008
                                    samples, read with 16-byte LDS reads) */
-    AA_HIP_KERNEL_LDS_QUAD = 6  /* LDS kernel, 16-channel chunks pre-summed in groups of four */
+    AA_HIP_KERNEL_LDS_QUAD = 6, /* LDS kernel, 16-channel chunks pre-summed in groups of four */
+    AA_HIP_KERNEL_MATRIX = 7    /* handles only: the matrix-core kernel at any size; unsupported for a range that
+                                   AUTO never gives it */
 } aa_hip_kernel;
 
 /* Message for the calling thread's most recent aa_hip_* failure ("" if none). */

@@ -45,7 +45,7 @@ def test_matrix_range(aa, oracle, cuda, geom, pitch_extra):
     want = oracle.dedisperse(rows[:, :tp + maxd].copy(), ds, ndms, tp, float(ms), float(st), ib)
     plan = aa.DdtrPlan(ds, [(low, step, ndms, ib)], tsamp, maxd * ib, tp * ib)
     d_in = torch.from_numpy(data).to(cuda)
-    for kernel in (aa.KERNEL_AUTO, aa.KERNEL_LDS):
+    for kernel in (aa.KERNEL_AUTO, aa.KERNEL_LDS, aa.KERNEL_MATRIX):
         plan.set_kernel(kernel)
         out = torch.full((ndms, tp + pitch_extra), -1.0, dtype=torch.float32, device=cuda)
         plan.ingest(d_in, tp * ib)
@@ -67,7 +67,7 @@ def test_matrix_choice_follows_the_kernel_setting(aa, oracle, cuda):
     want = oracle.dedisperse(oracle.corner_turn(data, tp + maxd, nchans), ds, ndms, tp, 0.0,
                              float(np.float32(0.5) / np.float32(tsamp)), 1)
     plan.ingest(d_in, tp)
-    for kernel, variant in ((0, -1), (5, -1), (0, -1), (0, 4), (0, 1), (0, -1), (1, -1), (2, -1)):
+    for kernel, variant in ((0, -1), (5, -1), (0, -1), (0, 4), (0, 1), (0, -1), (1, -1), (2, -1), (7, -1)):
         plan.set_kernel(kernel)
         plan.set_range_variant(0, variant)
         out = torch.full((ndms, tp), -1.0, dtype=torch.float32, device=cuda)

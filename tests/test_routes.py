@@ -1,0 +1,55 @@
+"""Which kernel a range's call launches (CPU: the library's host code on a HIP
+runtime without a GPU)."""
+import os
+import sys
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "host"))
+import host_library  # noqa: E402
+
+GEOMETRY = '''
+import ddtr_oracle as oracle
+ds = oracle.dmshifts(1024, 1500.0, -0.3)
+tp, maxshift = 60000, 3000
+x, out = Tensor((tp + maxshift, 1024), 1), Tensor((256, tp))
+def make(bits=8, nranges=1):
+    return aa.DdtrPlan(ds, [(0.0, 0.5, 256, 1)] * nranges, 64e-6, maxshift, tp, sample_bits=bits)
+'''
+
+
+def test_forced_lds_kernel_is_the_lds_kernel(tmp_path):
+    """AA_HIP_KERNEL_LDS on a handle, alone and in a batch, runs the first LDS
+    shape that fits, as the handle-free call does; AA_HIP_KERNEL_MATRIX the
+    matrix kernel, or nothing where it does not take the range."""
+    host_library.run(GEOMETRY + '''
+plan = make()
+plan.ingest(x, tp)
+plan.run_range(0, tp, out)
+assert fake.ran("dedisperse_matrix_kernel")
+plan.set_kernel(aa.KERNEL_LDS)
+plan.run_range(0, tp, out)
+assert fake.ran("dedisperse_wide_kernel")
+batch = aa.DdtrBatch([plan])
+batch.execute([x], [[tp]], [[out]], use_graph=False)
+names = fake.kernels()
+assert any("dedisperse_wide_batch_kernel" in n for n in names) and not any("matrix" in n for n in names), names
+plan.set_kernel(aa.KERNEL_MATRIX)
+plan.run_range(0, 600, out)      # small: the automatic choice would be the rows
+assert fake.ran("dedisperse_matrix_kernel")
+plan.set_kernel(aa.KERNEL_AUTO)
+plan.run_range(0, 600, out)
+assert fake.ran("dedisperse_rows_kernel")
+coarse = aa.DdtrPlan(ds, [(0.0, 40.0, 64, 1)], 64e-6, maxshift * 20, tp)
+xc = Tensor((tp + maxshift * 20, 1024), 1)
+coarse.set_kernel(aa.KERNEL_MATRIX)
+coarse.ingest(xc, tp)
+try:
+    coarse.run_range(0, tp, out)
+    raise SystemExit("the matrix kernel does not take this range")
+except aa.AAHipError as e:
+    assert e.status == aa.AA_HIP_ERROR_UNSUPPORTED
+try:
+    aa.dedisperse_u8(x, 63232, 63000, ds, x, 256, tp, 0.0, 1.0, 1, out, tp, kernel=aa.KERNEL_MATRIX)
+    raise SystemExit("the handle-free call has no matrix kernel")
+except aa.AAHipError as e:
+    assert e.status == aa.AA_HIP_ERROR_INVALID_ARGUMENT
+''', tmp_path)
