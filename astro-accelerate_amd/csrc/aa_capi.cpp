@@ -331,7 +331,21 @@ int aa_hip_ddtr_run_range(aa_hip_ddtr *h, int range, int t_processed, float *d_o
 
 int aa_hip_ddtr_set_range_variant(aa_hip_ddtr *h, int range, int variant) {
     if (!h || !h->engine) return bad("NULL handle");
-    return h->engine->set_range_variant(range, variant);
+    return h->engine->set_range_tuning(range, variant, false);
+}
+
+int aa_hip_ddtr_set_range_tuning(aa_hip_ddtr *h, int range, int variant, int automatic) {
+    if (!h || !h->engine) return bad("NULL handle");
+    return h->engine->set_range_tuning(range, variant, automatic != 0);
+}
+
+int aa_hip_ddtr_range_tuning(const aa_hip_ddtr *h, int range, int *variant, int *automatic) {
+    if (!h || !h->engine) return bad("NULL handle");
+    if (range < 0 || range >= h->engine->nranges()) return bad("bad range index");
+    const aa_hip::range_tuning t = h->engine->tuning(range);
+    if (variant) *variant = t.variant;
+    if (automatic) *automatic = t.automatic ? 1 : 0;
+    return AA_HIP_SUCCESS;
 }
 
 int aa_hip_ddtr_autotune_range(aa_hip_ddtr *h, int range, int t_processed, float *d_out, size_t out_pitch,

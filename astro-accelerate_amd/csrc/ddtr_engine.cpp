@@ -442,7 +442,8 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
     lds_choice &c = m_lds[(size_t)r];
     // A range that is small, or whose trials are far apart, goes straight from
     // the rows (in a batch the beams' ranges fill the chip together).
-    const bool automatic = range_variant(r) < 0 && m_kernel == AA_HIP_KERNEL_AUTO && rd.ndms > 0;
+    const range_tuning tuned = tuning(r);
+    const bool automatic = tuned.automatic && m_kernel == AA_HIP_KERNEL_AUTO && rd.ndms > 0;
     const bool alone = automatic && !batched;
     // No shape asked for: the matrix kernel where its plan is the cheaper one.
     const bool forced = m_kernel == AA_HIP_KERNEL_MATRIX && rd.ndms > 0;
@@ -464,9 +465,8 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
         }
     }
     if (c.variant == -2) {
-        const int want = r < (int)m_variant_pref.size() ? m_variant_pref[(size_t)r] : -1;
-        c = choose_lds(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, want);
-        if (c.variant < 0 && want >= 0)  // preferred shape does not fit: any that does
+        c = choose_lds(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, tuned.variant);
+        if (c.variant < 0 && tuned.variant >= 0)  // preferred shape does not fit: any that does
             c = choose_lds(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, -1);
     }
     const bool rows = (alone || (automatic && c.variant < 0)) &&
@@ -628,17 +628,17 @@ void ddtr_engine::drop_matrix(int r) {
     mt.planned = true;
 }
 
-int ddtr_engine::set_range_variant(int r, int variant) {
+int ddtr_engine::set_range_tuning(int r, int variant, bool automatic) {
     if (r < 0 || r >= (int)m_ranges.size()) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "bad range index");
     if (variant < -1 || variant >= kLdsVariants) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "bad LDS variant");
-    if (m_variant_pref.size() != m_ranges.size()) m_variant_pref.assign(m_ranges.size(), -1);
-    m_variant_pref[(size_t)r] = variant;
+    if (m_tuning.size() != m_ranges.size()) m_tuning.assign(m_ranges.size(), range_tuning{});
+    m_tuning[(size_t)r] = range_tuning{variant, automatic || variant < 0};
     if (m_lds.size() == m_ranges.size()) m_lds[(size_t)r] = lds_choice{-2, 0};
     return AA_HIP_SUCCESS;
 }
 
-int ddtr_engine::range_variant(int r) const {
-    return r >= 0 && r < (int)m_variant_pref.size() ? m_variant_pref[(size_t)r] : -1;
+range_tuning ddtr_engine::tuning(int r) const {
+    return r >= 0 && r < (int)m_tuning.size() ? m_tuning[(size_t)r] : range_tuning{};
 }
 
 int ddtr_engine::autotune_range(int r, int t_processed, float *d_out, size_t out_pitch, int reps, hipStream_t s,
@@ -658,7 +658,7 @@ int ddtr_engine::autotune_range(int r, int t_processed, float *d_out, size_t out
     float auto_ms = -1.0f;   // the automatic choice where that is none of the shapes
     for (int v = -1; v < kLdsVariants && e == hipSuccess && st == AA_HIP_SUCCESS; ++v) {
         if (v >= 0) ms[v] = -1.0f;
-        st = set_range_variant(r, v);
+        st = set_range_tuning(r, v, false);
         range_launch rl;
         if (st == AA_HIP_SUCCESS) st = prepare_range(r, t_processed, d_out, out_pitch, s, &rl);
         if (st != AA_HIP_SUCCESS || (v < 0 ? rl.variant < kLdsVariants : rl.variant != v)) continue;
@@ -680,8 +680,9 @@ int ddtr_engine::autotune_range(int r, int t_processed, float *d_out, size_t out
     if (e1) (void)hipEventDestroy(e1);
     m_kernel = saved_kernel;
     if (st == AA_HIP_SUCCESS && e != hipSuccess) st = hip_fail(e, "autotune");
-    const bool keep_auto = auto_ms >= 0.0f && (*best < 0 || auto_ms <= best_ms);
-    if (st == AA_HIP_SUCCESS) st = set_range_variant(r, keep_auto ? -1 : *best);
+    // The best shape is kept beside the automatic choice too: a batch leaves the
+    // matrix and row kernels out where its ranges share launches.
+    if (st == AA_HIP_SUCCESS) st = set_range_tuning(r, *best, auto_ms >= 0.0f && (*best < 0 || auto_ms <= best_ms));
     return st;
 }
 

@@ -44,6 +44,12 @@ struct lds_choice {
     int variant;
     int row_quads;
 };
+// A range's preference: an LDS chunk shape (-1: the first that fits), and whether
+// the automatic choice goes before it where that is none of the shapes.
+struct range_tuning {
+    int variant = -1;
+    bool automatic = true;
+};
 // First shape (or only `variant` when >= 0) whose rows hold the range's
 // windows, tried in the order 4, 5, 2 (pair pre-summation with 2016-, 1512- and
 // 1008-sample tiles, the fastest where rows are shared through LDS), 3, 0, 1, 6.
@@ -122,13 +128,13 @@ public:
     // rows directly only by ranges that fit no shape.
     int prepare_range(int r, int t_processed, float *d_out, size_t out_pitch, hipStream_t s, range_launch *rl,
                       bool batched = false);
-    // LDS chunk shape preferred for range r (-1 = automatic, see prepare_range);
-    // used when it fits the range's delay spread.
-    int set_range_variant(int r, int variant);
-    int range_variant(int r) const;
+    // Preference of range r: its shape is used where it fits the range's delay
+    // spread; variant -1 is always automatic (see prepare_range).
+    int set_range_tuning(int r, int variant, bool automatic);
+    range_tuning tuning(int r) const;
     // Times every LDS chunk shape that fits range r (reps launches each, after
     // one untimed launch; output written to d_out) and keeps the fastest as
-    // the range's preference, or none where the automatic choice is none of them
+    // the range's preference, behind the automatic choice where that is none of them
     // and faster than all.  ms[v] = average launch time of shape v, or -1
     // when it does not fit.  *best = -1 when no shape fits.
     int autotune_range(int r, int t_processed, float *d_out, size_t out_pitch, int reps, hipStream_t s,
@@ -173,7 +179,7 @@ private:
     std::vector<level> m_levels;
     int m_resident = -1;  // highest level valid for the current chunk
     std::vector<lds_choice> m_lds;     // per range: chosen LDS shape (-2 = not computed, -1 = direct)
-    std::vector<int> m_variant_pref;   // per range: preferred LDS shape, -1 = any
+    std::vector<range_tuning> m_tuning;  // per range (empty: all automatic)
     std::vector<int> m_wide_win;       // per range (u16 levels): dedisperse_u16 window, 0 = not computed
     struct plan_tables {
         int variant = -1;  // chunk shape the tables are for

@@ -126,9 +126,12 @@ def shape_class(beam: Beam, r: int):
 
 def autotune(beams: Sequence[Beam], cache_path: Optional[str] = None, reps: int = 2, stream=None,
              log=None) -> Dict[str, dict]:
-    """Picks the LDS chunk shape of every (beam, range) by timing each shape
-    that fits (aa_hip_ddtr_autotune_range) once per shape class; results are
-    kept in a JSON cache (`cache_path`) and applied to every beam."""
+    """Picks the kernel of every (beam, range) by timing each LDS chunk shape
+    that fits and the automatic choice (aa_hip_ddtr_autotune_range) once per
+    shape class; results are kept in a JSON cache (`cache_path`) and applied to
+    every beam of the class: "variant" the fastest shape, "automatic" whether
+    the automatic choice (the matrix-core kernel or the rows) beat it.  Entries
+    of a file without "automatic", made before it was timed, are timed again."""
     cache: Dict[str, dict] = {}
     if cache_path and os.path.exists(cache_path):
         with open(cache_path) as f:
@@ -138,17 +141,17 @@ def autotune(beams: Sequence[Beam], cache_path: Optional[str] = None, reps: int 
         ingested = False
         for r in range(len(b.ndms)):
             key = repr(shape_class(b, r))
-            if key in cache:
-                b.plan.set_range_variant(r, int(cache[key]["variant"]))
+            if "automatic" in cache.get(key, {}):
+                b.plan.set_range_tuning(r, int(cache[key]["variant"]), bool(cache[key]["automatic"]))
                 continue
             if not ingested:
                 b.plan.ingest(b.d_input, b.tps[0], stream=stream)
                 ingested = True
             best, ms = b.plan.autotune_range(r, b.tps[r], b.outs[r], reps=reps, stream=stream)
-            cache[key] = {"variant": best, "ms": ms}
+            cache[key] = {"variant": best, "ms": ms, "automatic": b.plan.range_tuning(r)[1]}
             tuned += 1
             if log:
-                log(f"[autotune] {key}: shape {best} ({ms})")
+                log(f"[autotune] {key}: shape {best} ({ms}){', automatic' if cache[key]['automatic'] else ''}")
     if cache_path:
         os.makedirs(os.path.dirname(os.path.abspath(cache_path)), exist_ok=True)
         with open(cache_path, "w") as f:

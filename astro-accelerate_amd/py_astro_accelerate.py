@@ -179,6 +179,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         "aa_hip_synth_noise_u8": ([u64, i64, d, d, vp, vp], i),
         "aa_hip_inject_pulse_u8": ([vp, i, i, vp, d, d, i, i, i, vp], i),
         "aa_hip_ddtr_set_range_variant": ([vp, i, i], i),
+        "aa_hip_ddtr_set_range_tuning": ([vp, i, i, i], i),
+        "aa_hip_ddtr_range_tuning": ([vp, i, pi, pi], i),
         "aa_hip_ddtr_autotune_range": ([vp, i, i, vp, sz, i, vp, pi, PFLOAT], i),
         "aa_hip_ddtr_batch_create": ([i, ctypes.POINTER(vp), ctypes.POINTER(vp)], i),
         "aa_hip_ddtr_batch_destroy": ([vp], i),
@@ -806,9 +808,22 @@ class DdtrPlan:
         -1: automatic: the matrix-core kernel, sums straight from the rows, or the first shape that fits)."""
         check(_lib_or_raise().aa_hip_ddtr_set_range_variant(self.handle, int(r), int(variant)), "set_range_variant")
 
+    def set_range_tuning(self, r: int, variant: int, automatic: bool):
+        """As set_range_variant; with ``automatic`` the automatic choice goes before the shape wherever that
+        is the matrix-core kernel or the rows."""
+        check(_lib_or_raise().aa_hip_ddtr_set_range_tuning(self.handle, int(r), int(variant), int(bool(automatic))),
+              "set_range_tuning")
+
+    def range_tuning(self, r: int):
+        """The preference of range r: (shape, automatic), as set_range_tuning takes it."""
+        variant, automatic = ctypes.c_int(), ctypes.c_int()
+        check(_lib_or_raise().aa_hip_ddtr_range_tuning(self.handle, int(r), ctypes.byref(variant),
+                                                       ctypes.byref(automatic)), "range_tuning")
+        return variant.value, bool(automatic.value)
+
     def autotune_range(self, r: int, t_processed: int, out, reps: int = 2, stream=None):
-        """Times each LDS chunk shape that fits range r; keeps the fastest, or the automatic choice where
-        that is none of them and faster still.
+        """Times each LDS chunk shape that fits range r; keeps the fastest, behind the automatic choice where
+        that is none of them and faster still (range_tuning).
         Returns (best variant or -1, [ms per variant, -1 = does not fit])."""
         best = ctypes.c_int()
         ms = (ctypes.c_float * LDS_SHAPES)()

@@ -629,7 +629,8 @@ def bench_multibeam(args):
     stream.synchronize()
     shapes = {}
     for v in cache.values():
-        shapes[v["variant"]] = shapes.get(v["variant"], 0) + 1
+        kept = "automatic" if v["automatic"] else v["variant"]
+        shapes[kept] = shapes.get(kept, 0) + 1
     log(f"[bench] autotune: {len(cache)} shape classes in {time.perf_counter() - t0:.1f} s, shapes chosen {shapes}")
     batch = aa.DdtrBatch([b.plan for b in beams])
     ins, tps, outs = [b.d_input for b in beams], [b.tps for b in beams], [b.outs for b in beams]
@@ -682,7 +683,8 @@ def bench_multibeam(args):
             f"{exact_bytes}) -> batched speedup {ms_per_beam_bytes / ms_batched:.3f}x")
         for b in beams:   # back to the tuned shapes
             for r in range(len(b.tps)):
-                b.plan.set_range_variant(r, int(cache[repr(mb.shape_class(b, r))]["variant"]))
+                v = cache[repr(mb.shape_class(b, r))]
+                b.plan.set_range_tuning(r, int(v["variant"]), bool(v["automatic"]))
     achieved = adds / (ms_batched * 1e-3) / 1e12
     result = {
         "metric": "DM×sample/s bit-exact, % FP32 add roofline; batched vs per-beam speedup",

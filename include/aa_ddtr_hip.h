@@ -283,13 +283,21 @@ int aa_hip_ddtr_run_range(aa_hip_ddtr *h, int range, int t_processed, float *d_o
  * first shape that fits, in the order 4, 5, 2, 3, 0, 1, 6; sums straight from
  * the rows where the range is too small to fill the GPU with tiles, or its
  * trials too far apart for shared rows), used whenever it fits.
+ * set_range_tuning records a shape too; with automatic != 0 the automatic
+ * choice goes before it wherever that is the matrix-core kernel or the rows, so
+ * that the shape is what the range falls back to (in a batch, where ranges of
+ * few tiles share launches).  range_tuning reads the preference back.
  * autotune_range times every shape that fits range r on `stream` (reps
- * launches each, writing d_out), keeps the fastest as the preference (or -1
- * where the automatic choice is none of the shapes and faster still) and
- * reports the fastest shape: *best_variant (-1 if none fits) and variant_ms[0..6] (-1 =
- * does not fit; the array holds 7 floats).
+ * launches each, writing d_out), keeps the fastest as the preference (with
+ * automatic set where the automatic choice is none of the shapes and faster
+ * still) and reports the fastest shape: *best_variant (-1 if none fits) and
+ * variant_ms[0..6] (-1 = does not fit; the array holds 7 floats).  What it
+ * found is handed to another handle of the same range by range_tuning and
+ * set_range_tuning.
  * The range's level must be resident (after ingest). */
 int aa_hip_ddtr_set_range_variant(aa_hip_ddtr *h, int range, int variant);
+int aa_hip_ddtr_set_range_tuning(aa_hip_ddtr *h, int range, int variant, int automatic);
+int aa_hip_ddtr_range_tuning(const aa_hip_ddtr *h, int range, int *variant, int *automatic);
 int aa_hip_ddtr_autotune_range(aa_hip_ddtr *h, int range, int t_processed, float *d_out,
                                size_t out_pitch, int reps, void *stream, int *best_variant,
                                float *variant_ms);

@@ -53,3 +53,74 @@ try:
 except aa.AAHipError as e:
     assert e.status == aa.AA_HIP_ERROR_INVALID_ARGUMENT
 ''', tmp_path)
+
+
+TUNING = GEOMETRY + '''
+import json
+import multibeam as mb
+
+class Strategy:
+    def dm(self, r):
+        return (0.0, 128.0, 0.5, 1, 1)
+
+def beam(plan, n=1):
+    return mb.Beam(dict(nchans=1024), Strategy(), plan, x, [out] * n, [tp] * n, [256] * n)
+
+def kernel_alone(plan):
+    plan.ingest(x, tp)
+    fake.kernels()
+    plan.run_range(0, tp, out)
+    return fake.kernels()
+
+def kernel_batched(plans, tp=tp):
+    batch = aa.DdtrBatch(plans)
+    batch.execute([x] * len(plans), [[tp]] * len(plans), [[out]] * len(plans), use_graph=False)
+    return [n for n in fake.kernels() if "dedisperse" in n]
+'''
+
+
+def test_autotuned_class_runs_one_kernel(tmp_path):
+    """Two beams of one class, and a third from the reloaded cache, keep what
+    the autotuner found fastest: here the matrix kernel."""
+    cache = tmp_path / "tune.json"
+    host_library.run(TUNING + f'''
+path = {str(cache)!r}
+fake.lib.fake_cost(b"dedisperse_matrix", 0.5)
+fake.lib.fake_cost(b"dedisperse_wide_kernelILi4ELi3E", 0.7)   # shape 5; the other shapes take 1 ms
+a, b, c = make(), make(), make()
+mb.autotune([beam(a), beam(b)], cache_path=path)
+mb.autotune([beam(c)], cache_path=path)
+for plan in (a, b, c):
+    assert plan.range_tuning(0) == (5, True)
+    assert any("dedisperse_matrix_kernel" in n for n in kernel_alone(plan))
+names = kernel_batched([a, b, c])
+assert len(names) == 3 and all("dedisperse_matrix_kernel" in n for n in names), names
+# in a batch a range too small for a matrix launch of its own takes the shape that was fastest
+names = kernel_batched([a, b, c], 9000)
+assert len(names) == 1 and "dedisperse_wide_batch_kernelILi4ELi3E" in names[0], names
+''', tmp_path)
+
+
+def test_autotuned_class_on_an_lds_shape(tmp_path):
+    """The same where a shape is fastest; and a cache file without the automatic
+    choice's time is timed again."""
+    cache = tmp_path / "tune.json"
+    host_library.run(TUNING + f'''
+path = {str(cache)!r}
+fake.lib.fake_cost(b"dedisperse_wide_kernelILi4ELi3E", 0.3)
+a, b, c = make(), make(), make()
+mb.autotune([beam(a), beam(b)], cache_path=path)
+mb.autotune([beam(c)], cache_path=path)
+for plan in (a, b, c):
+    assert plan.range_tuning(0) == (5, False)
+    assert any("dedisperse_wide_kernelILi4ELi3E" in n for n in kernel_alone(plan))
+old = json.load(open(path))
+for v in old.values():
+    del v["automatic"]
+json.dump(old, open(path, "w"))
+fake.lib.fake_cost(b"dedisperse_matrix", 0.2)
+d = make()
+mb.autotune([beam(d)], cache_path=path)
+assert d.range_tuning(0) == (5, True)
+assert all(v["automatic"] for v in json.load(open(path)).values())
+''', tmp_path)
