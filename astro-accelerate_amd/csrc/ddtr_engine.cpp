@@ -261,8 +261,9 @@ ddtr_engine::~ddtr_engine() {
     }
     if (m_d_dmshifts) (void)hipFree(m_d_dmshifts);
     if (m_d_err) (void)hipFree(m_d_err);
-    for (const plan_tables &t : m_tables)
-        if (t.ptr) (void)hipFree(t.ptr);
+    for (const auto &range : m_tables)
+        for (const plan_tables &t : range)
+            if (t.ptr) (void)hipFree(t.ptr);
     for (const matrix_tables &t : m_matrix) {
         if (t.t.ptr) (void)hipFree(t.t.ptr);
         if (t.flags) (void)hipFree(t.flags);
@@ -478,14 +479,14 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
     // Chunk shapes from 2 on read plan tables; they depend on the range and
     // shape only, so they are built once (on the first call that needs them,
     // never while a later call is being captured into a graph).
-    if (m_tables.size() != m_ranges.size()) m_tables.assign(m_ranges.size(), plan_tables{});
-    plan_tables &pt = m_tables[(size_t)r];
-    if (pt.variant != rl->variant) {
+    if (m_tables.size() != m_ranges.size()) m_tables.resize(m_ranges.size());
+    plan_tables &pt = m_tables[(size_t)r][(size_t)rl->variant];
+    if (!pt.ptr) {
         std::vector<uint8_t> bytes;
         if (lds_plan_tables(rl->variant, m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, lv.pitch, &bytes) !=
             rl->row_quads)
             return fail(AA_HIP_ERROR_UNSUPPORTED, "plan tables disagree with the chosen row width");
-        const hipError_t e = keep_tables(pt, rl->variant, bytes);
+        const hipError_t e = keep_tables(pt, bytes);
         if (e != hipSuccess) return hip_fail(e, "plan tables");
     }
     rl->pair_recs = pt.ptr;
@@ -572,8 +573,7 @@ int ddtr_engine::ensure_planes(int k, hipStream_t s) {
     return AA_HIP_SUCCESS;
 }
 
-hipError_t ddtr_engine::keep_tables(plan_tables &pt, int variant, const std::vector<uint8_t> &bytes) {
-    drop_tables(pt);
+hipError_t ddtr_engine::keep_tables(plan_tables &pt, const std::vector<uint8_t> &bytes) {
     void *t = nullptr;
     hipError_t e = hipMalloc(&t, bytes.size());
     if (e == hipSuccess) e = hipMemcpy(t, bytes.data(), bytes.size(), hipMemcpyHostToDevice);
@@ -582,7 +582,6 @@ hipError_t ddtr_engine::keep_tables(plan_tables &pt, int variant, const std::vec
         if (t) (void)hipFree(t);
         return e;
     }
-    pt.variant = variant;
     pt.ptr = t;
     pt.bytes = bytes.size();
     m_device_bytes += bytes.size();
@@ -610,7 +609,7 @@ hipError_t ddtr_engine::plan_matrix(int r, size_t pitch, int planes) {
         std::vector<uint8_t> bytes;
         const matrix_layout lay =
             matrix_plan(m_dmshifts.data(), m_nchans, m_ranges[(size_t)r].ndms, mstartdm, mdmstep, pitch, &bytes, planes);
-        const hipError_t e = lay.tile_out > 0 ? keep_tables(mt.t, kShapeMatrix, bytes) : hipSuccess;
+        const hipError_t e = lay.tile_out > 0 ? keep_tables(mt.t, bytes) : hipSuccess;
         if (e == hipSuccess) mt.lay = lay;
         return e;
     } catch (const std::bad_alloc &) {
@@ -650,6 +649,8 @@ int ddtr_engine::autotune_range(int r, int t_processed, float *d_out, size_t out
     const int saved_kernel = m_kernel;
     m_kernel = AA_HIP_KERNEL_AUTO;
     *best = -1;
+    bool had[kLdsVariants];
+    for (int v = 0; v < kLdsVariants; ++v) had[v] = !m_tables.empty() && m_tables[(size_t)r][(size_t)v].ptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     hipError_t e = hipEventCreate(&e0);
     if (e == hipSuccess) e = hipEventCreate(&e1);
@@ -680,6 +681,8 @@ int ddtr_engine::autotune_range(int r, int t_processed, float *d_out, size_t out
     if (e1) (void)hipEventDestroy(e1);
     m_kernel = saved_kernel;
     if (st == AA_HIP_SUCCESS && e != hipSuccess) st = hip_fail(e, "autotune");
+    for (int v = 0; !m_tables.empty() && v < kLdsVariants; ++v)   // tables made for this, in no graph
+        if (v != *best && !had[v]) drop_tables(m_tables[(size_t)r][(size_t)v]);
     // The best shape is kept beside the automatic choice too: a batch leaves the
     // matrix and row kernels out where its ranges share launches.
     if (st == AA_HIP_SUCCESS) st = set_range_tuning(r, *best, auto_ms >= 0.0f && (*best < 0 || auto_ms <= best_ms));

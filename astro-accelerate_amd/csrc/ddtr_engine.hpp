@@ -13,6 +13,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -182,11 +183,12 @@ private:
     std::vector<range_tuning> m_tuning;  // per range (empty: all automatic)
     std::vector<int> m_wide_win;       // per range (u16 levels): dedisperse_u16 window, 0 = not computed
     struct plan_tables {
-        int variant = -1;  // chunk shape the tables are for
         void *ptr = nullptr;
         size_t bytes = 0;
     };
-    std::vector<plan_tables> m_tables;  // per range: plan tables (device), built on first use
+    // Per range and shape: plan tables (device), built on first use and kept: a
+    // captured batch may still read the tables of a shape the range has left.
+    std::vector<std::array<plan_tables, kLdsVariants>> m_tables;
     struct matrix_tables {
         bool planned = false;   // lay is known (tile_out 0: not this kernel)
         matrix_layout lay;
@@ -194,14 +196,13 @@ private:
         int *flags = nullptr;   // u16 levels: one entry per tile
         size_t flag_bytes = 0;
     };
-    std::vector<matrix_tables> m_matrix;  // per range: the matrix kernel's, kept beside the LDS shape's, which a
-                                          // captured batch may still read
+    std::vector<matrix_tables> m_matrix;  // per range: the matrix kernel's
     int u16_window(int r);
     bool u16_matrix(int r);
     int level_planes(int k, hipStream_t s);
-    // Uploads tables of `variant` in place of what pt holds; on failure pt is
-    // empty and HIP's pending error taken.
-    hipError_t keep_tables(plan_tables &pt, int variant, const std::vector<uint8_t> &bytes);
+    // Uploads tables into an empty pt; on failure it stays empty and HIP's
+    // pending error is taken.
+    hipError_t keep_tables(plan_tables &pt, const std::vector<uint8_t> &bytes);
     void drop_tables(plan_tables &pt);
     hipError_t plan_matrix(int r, size_t pitch, int planes);
     void drop_matrix(int r);

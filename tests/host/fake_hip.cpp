@@ -4,6 +4,7 @@
 // hipGetLastError takes it), and a stream under capture refuses allocations and
 // synchronous copies.  Host allocations (operator new) can be made to fail too.
 // Loaded before the library under HIP's own soname.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -22,7 +23,8 @@ struct event { size_t at = 0; };
 std::map<const void*, std::string> g_kernels;
 std::vector<launch> g_launches;
 std::map<std::string, float> g_cost;      // ms per launch, by part of the kernel's name
-std::map<void*, size_t> g_blocks;
+struct block { size_t bytes, number; };
+std::map<void*, block> g_blocks;
 std::vector<size_t> g_allocated;          // every allocation's bytes, in order
 size_t g_fail_from = ~(size_t)0, g_fail_to = ~(size_t)0, g_bytes = 0;
 size_t g_host_from = ~(size_t)0;
@@ -53,6 +55,13 @@ void fake_capture(void* stream) { g_capturing = stream; g_capture_broken = false
 int fake_capture_broken() { return g_capture_broken; }
 size_t fake_device_bytes() { return g_bytes; }
 size_t fake_blocks() { return g_blocks.size(); }
+size_t fake_block(size_t i)   // number of the i-th block in use, in the order of their allocation
+{
+    std::vector<size_t> n;
+    for (const auto& b : g_blocks) n.push_back(b.second.number);
+    std::sort(n.begin(), n.end());
+    return n[i];
+}
 void fake_cost(const char* part, float ms) { g_cost[part] = ms; }
 void fake_clear_launches() { g_launches.clear(); }
 int fake_launches() { return (int)g_launches.size(); }
@@ -98,7 +107,7 @@ err_t hipMalloc(void** p, size_t n)
     if (n >= g_fail_from && n < g_fail_to) return set(oom);
     *p = std::malloc(n ? n : 1);
     if (!*p) return set(oom);
-    g_blocks[*p] = n;
+    g_blocks[*p] = {n, g_allocated.size()};
     g_bytes += n;
     return ok;
 }
@@ -106,7 +115,7 @@ err_t hipFree(void* p)
 {
     const auto it = g_blocks.find(p);
     if (it == g_blocks.end()) return p ? set(invalid) : ok;
-    g_bytes -= it->second;
+    g_bytes -= it->second.bytes;
     g_blocks.erase(it);
     std::free(p);
     return ok;

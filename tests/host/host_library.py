@@ -55,7 +55,8 @@ class Tensor:
 class Fake:
     def __init__(self, lib):
         self.lib = lib
-        lib.fake_device_bytes.restype = lib.fake_blocks.restype = ctypes.c_size_t
+        lib.fake_device_bytes.restype = lib.fake_blocks.restype = lib.fake_block.restype = ctypes.c_size_t
+        lib.fake_block.argtypes = [ctypes.c_size_t]
         lib.fake_launch_name.restype = ctypes.c_char_p
         lib.fake_launch_stream.restype = ctypes.c_void_p
         lib.fake_fail_allocations.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
@@ -72,6 +73,10 @@ class Fake:
 
     def ran(self, part):
         return any(part in n for n in self.kernels())
+
+    def blocks(self):
+        """Numbers of the device blocks in use."""
+        return [self.lib.fake_block(i) for i in range(self.lib.fake_blocks())]
 
     def allocations(self):
         return [self.lib.fake_allocated(i) for i in range(self.lib.fake_allocations())]

@@ -79,6 +79,27 @@ def kernel_batched(plans, tp=tp):
 '''
 
 
+def test_captured_tables_outlive_a_change_of_shape(tmp_path):
+    """A captured batch reads the plan tables of its ranges' shapes: another
+    shape's call on the handle, or autotuning it, leaves them in place."""
+    host_library.run(TUNING + '''
+plan = make()
+plan.set_range_variant(0, 4)
+batch = aa.DdtrBatch([plan])
+batch.execute([x], [[tp]], [[out]], use_graph=True)
+captured = set(fake.blocks())
+for variant in (5, 6, 4, 2):
+    plan.set_range_variant(0, variant)
+    plan.run_range(0, tp, out)
+    assert captured <= set(fake.blocks()), variant
+had = len(fake.blocks())
+plan.autotune_range(0, tp, out, 1)
+assert captured <= set(fake.blocks())
+assert len(fake.blocks()) <= had + 2          # keeps the best shape's and the automatic choice's, no others
+plan.close()
+''', tmp_path)
+
+
 def test_autotuned_class_runs_one_kernel(tmp_path):
     """Two beams of one class, and a third from the reloaded cache, keep what
     the autotuner found fastest: here the matrix kernel."""
