@@ -27,6 +27,15 @@ int hip_fail(hipError_t e, const char *what) {
                 std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// Whether s is being captured into a graph, or cannot be asked because another
+// stream is: allocations and synchronous copies would break the capture.
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 int no_matrix() {
     return fail(AA_HIP_ERROR_UNSUPPORTED, "the matrix kernel does not take this range (its plan does not fit or does "
                                           "not pay, or there is no memory for its tables)");
@@ -425,7 +434,7 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
             return fail(AA_HIP_ERROR_UNSUPPORTED, "the 16-bit LDS kernel does not fit this range's delay spread");
         if (rd.ndms <= 0) return AA_HIP_SUCCESS;
         const bool forced = m_kernel == AA_HIP_KERNEL_MATRIX;
-        if (!u16_matrix(r)) return forced ? no_matrix() : AA_HIP_SUCCESS;
+        if (!u16_matrix(r, s)) return forced ? no_matrix() : AA_HIP_SUCCESS;
         st = ensure_planes(k, s);   // (the kernel setting may have changed since the level was written)
         if (st == AA_HIP_ERROR_OUT_OF_MEMORY) return forced ? no_matrix() : AA_HIP_SUCCESS;
         if (st != AA_HIP_SUCCESS) return st;
@@ -449,7 +458,7 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
     // No shape asked for: the matrix kernel where its plan is the cheaper one.
     const bool forced = m_kernel == AA_HIP_KERNEL_MATRIX && rd.ndms > 0;
     if (forced || (automatic && (!batched || matrix_tiles_at_most(rd.ndms, t_processed) >= kMatrixAloneTiles))) {
-        const hipError_t e = plan_matrix(r, lv.pitch, 1);
+        const hipError_t e = plan_matrix(r, lv.pitch, 1, s);
         if (e != hipSuccess && (forced || e != hipErrorOutOfMemory)) return hip_fail(e, "plan tables");
         const matrix_tables &mt = m_matrix[(size_t)r];
         if (forced && mt.lay.tile_out <= 0) return no_matrix();
@@ -475,21 +484,33 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
     st = resolve_launch(m_kernel, lv.ptr, lv.pitch, m_nchans, m_d_dmshifts, m_dmshifts.data(), rd.ndms,
                         t_processed, mstartdm, mdmstep, rd.inBin, d_out, out_pitch,
                         rows ? lds_choice{kShapeRows, 0} : c, rl);
-    if (st != AA_HIP_SUCCESS || rl->variant < 2 || rl->variant == kShapeRows) return st;
-    // Chunk shapes from 2 on read plan tables; they depend on the range and
-    // shape only, so they are built once (on the first call that needs them,
-    // never while a later call is being captured into a graph).
+    if (st != AA_HIP_SUCCESS || rl->variant < 2) return st;
+    if (rl->variant != kShapeRows) return shape_tables(r, rl->variant, rl->row_quads, &rl->pair_recs);
+    // A longer chunk of this range may take the shape, and under capture: its
+    // tables are made now.  This call does without them.
+    const void *unused;
+    if (c.variant >= 2 && !capturing(s)) (void)shape_tables(r, c.variant, c.row_quads, &unused);
+    return AA_HIP_SUCCESS;
+}
+
+// Chunk shapes from 2 on read plan tables, which depend on the range and shape
+// only: made on the range's first eager call that is not the matrix kernel's,
+// whatever its length, so that a later one can be captured into a graph.
+int ddtr_engine::shape_tables(int r, int variant, int row_quads, const void **tables) {
     if (m_tables.size() != m_ranges.size()) m_tables.resize(m_ranges.size());
-    plan_tables &pt = m_tables[(size_t)r][(size_t)rl->variant];
+    plan_tables &pt = m_tables[(size_t)r][(size_t)variant];
     if (!pt.ptr) {
+        const range_desc &rd = m_ranges[(size_t)r];
+        float mstartdm, mdmstep;
+        range_scalars(r, &mstartdm, &mdmstep);
         std::vector<uint8_t> bytes;
-        if (lds_plan_tables(rl->variant, m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, lv.pitch, &bytes) !=
-            rl->row_quads)
+        if (lds_plan_tables(variant, m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep,
+                            m_levels[(size_t)log2i(rd.inBin)].pitch, &bytes) != row_quads)
             return fail(AA_HIP_ERROR_UNSUPPORTED, "plan tables disagree with the chosen row width");
         const hipError_t e = keep_tables(pt, bytes);
         if (e != hipSuccess) return hip_fail(e, "plan tables");
     }
-    rl->pair_recs = pt.ptr;
+    *tables = pt.ptr;
     return AA_HIP_SUCCESS;
 }
 
@@ -508,13 +529,14 @@ int ddtr_engine::u16_window(int r) {
 // The automatic choice on u16 levels: the matrix kernel over the rows' byte
 // planes where its plan pays (dedisperse_u16 then computes the tiles it
 // flags).  Without the memory for its tables or the level's planes the range
-// keeps dedisperse_u16, from its first chunk on.
-bool ddtr_engine::u16_matrix(int r) {
+// keeps dedisperse_u16, from its first chunk on; captured before they are there,
+// a call takes dedisperse_u16 this time.
+bool ddtr_engine::u16_matrix(int r, hipStream_t s) {
     if (m_sample_bytes != 2 || (m_kernel != AA_HIP_KERNEL_AUTO && m_kernel != AA_HIP_KERNEL_MATRIX) ||
         u16_window(r) <= 0)
         return false;
     const level &lv = m_levels[(size_t)log2i(m_ranges[(size_t)r].inBin)];
-    (void)plan_matrix(r, round_up((size_t)lv.capacity + kRowPad, kPitchAlign), 2);
+    (void)plan_matrix(r, round_up((size_t)lv.capacity + kRowPad, kPitchAlign), 2, s);
     matrix_tables &mt = m_matrix[(size_t)r];
     if (mt.lay.tile_out <= 0 || mt.flags) return mt.lay.tile_out > 0;
     const size_t tiles =
@@ -535,7 +557,7 @@ bool ddtr_engine::u16_matrix(int r) {
 int ddtr_engine::level_planes(int k, hipStream_t s) {
     m_levels[(size_t)k].planes_ok = false;
     for (int r = 0; r < (int)m_ranges.size(); ++r)
-        if (log2i(m_ranges[(size_t)r].inBin) == k && m_ranges[(size_t)r].ndms > 0 && u16_matrix(r)) {
+        if (log2i(m_ranges[(size_t)r].inBin) == k && m_ranges[(size_t)r].ndms > 0 && u16_matrix(r, s)) {
             const int st = ensure_planes(k, s);
             return st == AA_HIP_ERROR_OUT_OF_MEMORY ? AA_HIP_SUCCESS : st;
         }
@@ -543,12 +565,14 @@ int ddtr_engine::level_planes(int k, hipStream_t s) {
 }
 
 // Byte planes of level k for the current chunk.  Without the memory for them
-// no range of the level takes the matrix kernel: OUT_OF_MEMORY, no message set.
+// no range of the level takes the matrix kernel (captured before they are there,
+// this time): OUT_OF_MEMORY, no message set.
 
 int ddtr_engine::ensure_planes(int k, hipStream_t s) {
     level &lv = m_levels[(size_t)k];
     if (lv.planes_ok) return AA_HIP_SUCCESS;
     if (!lv.planes) {
+        if (capturing(s)) return AA_HIP_ERROR_OUT_OF_MEMORY;
         const size_t pitch = round_up((size_t)lv.capacity + kRowPad, kPitchAlign);
         void *p = nullptr, *o = nullptr;
         if (hipMalloc(&p, 2 * pitch * (size_t)m_nchans) != hipSuccess || hipMalloc(&o, 64 * sizeof(int)) != hipSuccess) {
@@ -598,10 +622,11 @@ void ddtr_engine::drop_tables(plan_tables &pt) {
 // device; tile_out 0 where the plan does not pay.  Without the memory for it
 // (host or device) the range is not the matrix kernel's either, from its first
 // call on: hipErrorOutOfMemory, once, for callers that have no other kernel.
-hipError_t ddtr_engine::plan_matrix(int r, size_t pitch, int planes) {
+// Under capture nothing is planned; the next eager call does.
+hipError_t ddtr_engine::plan_matrix(int r, size_t pitch, int planes, hipStream_t s) {
     if (m_matrix.size() != m_ranges.size()) m_matrix.resize(m_ranges.size());
     matrix_tables &mt = m_matrix[(size_t)r];
-    if (mt.planned) return hipSuccess;
+    if (mt.planned || capturing(s)) return hipSuccess;
     mt.planned = true;
     float mstartdm, mdmstep;
     range_scalars(r, &mstartdm, &mdmstep);

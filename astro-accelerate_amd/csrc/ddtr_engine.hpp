@@ -198,13 +198,14 @@ private:
     };
     std::vector<matrix_tables> m_matrix;  // per range: the matrix kernel's
     int u16_window(int r);
-    bool u16_matrix(int r);
+    bool u16_matrix(int r, hipStream_t s);
     int level_planes(int k, hipStream_t s);
     // Uploads tables into an empty pt; on failure it stays empty and HIP's
     // pending error is taken.
     hipError_t keep_tables(plan_tables &pt, const std::vector<uint8_t> &bytes);
     void drop_tables(plan_tables &pt);
-    hipError_t plan_matrix(int r, size_t pitch, int planes);
+    hipError_t plan_matrix(int r, size_t pitch, int planes, hipStream_t s);
+    int shape_tables(int r, int variant, int row_quads, const void **tables);
     void drop_matrix(int r);
     size_t m_device_bytes = 0;
 };

@@ -145,3 +145,73 @@ mb.autotune([beam(d)], cache_path=path)
 assert d.range_tuning(0) == (5, True)
 assert all(v["automatic"] for v in json.load(open(path)).values())
 ''', tmp_path)
+
+
+CAPTURE = GEOMETRY + '''
+capture = Stream(4096)
+def captured(call):
+    """The kernels of a call under capture, which it must not break."""
+    fake.kernels()
+    fake.lib.fake_capture(4096)
+    call()
+    broken = fake.lib.fake_capture_broken()
+    fake.lib.fake_capture(None)
+    assert not broken, "the call allocated or synchronised under capture"
+    return fake.kernels()
+'''
+
+
+def test_16_bit_chunk_captured_at_first(tmp_path):
+    """A 16-bit chunk may be captured without an eager call before it: what the
+    matrix kernel needs is not there, so dedisperse_u16 runs; eager calls and
+    captures after one take the matrix kernel."""
+    host_library.run(CAPTURE + '''
+maxshift *= 3
+x16, half = Tensor((tp + maxshift, 1024), 2), tp // 2
+plan = aa.DdtrPlan(ds, [(0.0, 0.5, 256, 1), (128.0, 1.0, 128, 2)], 64e-6, maxshift, tp, sample_bits=16)
+outs = [out, Tensor((128, half))]
+def chunk():
+    plan.execute_chunk(x16, [tp, half], outs, stream=capture)
+names = captured(chunk)
+assert sum("dedisperse_u16_kernel" in n for n in names) == 2 and not any("matrix" in n for n in names), names
+# eager up to the first range: the second one's level has no planes yet
+plan.ingest(x16, tp)
+plan.run_range(0, tp, out)
+assert fake.ran("dedisperse_matrix_kernel")
+names = captured(lambda: plan.run_range(1, half, outs[1], stream=capture))
+assert any("dedisperse_u16_kernel" in n for n in names) and not any("matrix" in n for n in names), names
+chunk()
+assert sum("dedisperse_matrix_kernel" in n for n in fake.kernels()) == 2
+assert sum("dedisperse_matrix_kernel" in n for n in captured(chunk)) == 2
+''', tmp_path)
+
+
+def test_captured_chunk_longer_than_the_eager_one(tmp_path):
+    """A short eager chunk goes from the rows; a longer one captured after it
+    takes an LDS shape, whose tables are there."""
+    host_library.run(CAPTURE + '''
+ds = oracle.dmshifts(128, 1500.0, -5.0)   # a range that the matrix kernel does not take
+shift = int(ds[-1] * 256.0 / 64e-6) + 10
+plan = aa.DdtrPlan(ds, [(0.0, 0.5, 512, 1)], 64e-6, shift, tp)
+xl, ol = Tensor((tp + shift, 128), 1), Tensor((512, tp))
+plan.ingest(xl, 100)
+plan.run_range(0, 100, ol)
+assert fake.ran("dedisperse_rows_kernel")
+plan.ingest(xl, tp)
+names = captured(lambda: plan.run_range(0, tp, ol, stream=capture))
+assert any("dedisperse_wide_kernel" in n for n in names), names
+''', tmp_path)
+
+
+def test_8_bit_range_captured_at_first(tmp_path):
+    """A range that can do without tables may be captured at once, although the
+    matrix kernel, which cannot, would be the automatic choice."""
+    host_library.run(CAPTURE + '''
+plan = make()
+plan.ingest(x, tp)
+plan.set_range_tuning(0, 0, True)
+names = captured(lambda: plan.run_range(0, tp, out, stream=capture))
+assert any("dedisperse_lds_kernel" in n or "dedisperse_rows_kernel" in n for n in names), names
+plan.run_range(0, tp, out)
+assert fake.ran("dedisperse_matrix_kernel")
+''', tmp_path)
