@@ -165,7 +165,11 @@ int aa_hip_frac_create(int device, int nchans, const float* delay_per_dm, int nt
     if (e == hipSuccess) e = hipMalloc(&p->d_ds, sizeof(float) * nchans);
     if (e == hipSuccess) e = hipMalloc(&p->d_trials, sizeof(float) * ntrials);
     if (e == hipSuccess) e = hipMalloc(&p->d_part, sizeof(double) * p->part_entries);
-    if (e == hipSuccess && ypart) e = hipMalloc(&p->d_ypart, sizeof(float) * ypart);
+    if (e == hipSuccess && ypart && hipMalloc(&p->d_ypart, sizeof(float) * ypart) != hipSuccess) {
+        (void)hipGetLastError();   // no memory for it: forward calls are not split
+        p->d_ypart = nullptr;
+        ypart = 0;
+    }
     if (e == hipSuccess) e = hipMemcpy(p->d_ds, ds.data(), sizeof(float) * nchans, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->d_trials, tr.data(), sizeof(float) * ntrials, hipMemcpyHostToDevice);
     (void)hipSetDevice(cur);
@@ -202,7 +206,8 @@ int aa_hip_frac_forward(aa_hip_frac* h, const float* d_x, int nbatch, const floa
     a.y = d_y;
     a.group_q = h->trials_per_wave;
     a.n_groups = (h->ntrials + 16 * a.group_q - 1) / (16 * a.group_q);
-    a.n_split = aa_hip::frac_channel_split((size_t)nbatch * a.n_ttiles * a.n_groups, h->nchans);
+    a.n_split =
+        h->d_ypart ? aa_hip::frac_channel_split((size_t)nbatch * a.n_ttiles * a.n_groups, h->nchans) : 1;
     a.y_part = h->d_ypart;
     return from_hip(aa_hip::launch_frac_forward(a, (hipStream_t)stream), "frac forward");
 }

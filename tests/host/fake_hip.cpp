@@ -18,7 +18,7 @@ enum { ok = 0, invalid = 1, oom = 2, capture_unsupported = 900 };
 struct dim { unsigned x, y, z; };
 
 namespace {
-struct launch { std::string name; void* stream; unsigned grid; };
+struct launch { std::string name; void* stream; unsigned grid; unsigned long long words[14]; };   // words: of its first argument
 struct event { size_t at = 0; };
 std::map<const void*, std::string> g_kernels;
 std::vector<launch> g_launches;
@@ -67,6 +67,7 @@ void fake_clear_launches() { g_launches.clear(); }
 int fake_launches() { return (int)g_launches.size(); }
 const char* fake_launch_name(int i) { return g_launches[(size_t)i].name.c_str(); }
 void* fake_launch_stream(int i) { return g_launches[(size_t)i].stream; }
+unsigned long long fake_launch_word(int i, int k) { return g_launches[(size_t)i].words[k]; }
 unsigned fake_launch_grid(int i) { return g_launches[(size_t)i].grid; }
 
 // ---- the runtime
@@ -83,9 +84,11 @@ err_t __hipPopCallConfiguration(dim* g, dim* b, size_t* lds, void** s)
     *g = g_call.grid; *b = g_call.block; *lds = g_call.lds; *s = g_call.stream;
     return ok;
 }
-err_t hipLaunchKernel(const void* f, dim g, dim, void**, size_t, void* s)
+err_t hipLaunchKernel(const void* f, dim g, dim, void** args, size_t, void* s)
 {
-    g_launches.push_back({g_kernels[f], s, g.x});
+    launch l{g_kernels[f], s, g.x, {}};
+    std::memcpy(l.words, args[0], sizeof(l.words));
+    g_launches.push_back(l);
     return ok;
 }
 err_t hipGetLastError() { const err_t e = g_last; g_last = ok; return e; }

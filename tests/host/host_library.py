@@ -33,14 +33,21 @@ class Stream:
 
 class Tensor:
     """Memory with the few tensor methods that the library's Python side reads."""
+    is_cuda, device = True, "cuda:0"
 
-    def __init__(self, shape, size=4):
-        self.shape, self.size = tuple(shape), size
+    def __init__(self, shape, size=4, dtype="float32"):
+        self.shape, self.size, self.dtype = tuple(shape), size, dtype
         n = size
         for s in shape:
             n *= s
         self.buffer = ctypes.create_string_buffer(n + 256)
         self.at = (ctypes.addressof(self.buffer) + 255) // 256 * 256
+
+    def is_contiguous(self):
+        return True
+
+    def dim(self):
+        return len(self.shape)
 
     def data_ptr(self):
         return self.at
@@ -59,6 +66,7 @@ class Fake:
         lib.fake_block.argtypes = [ctypes.c_size_t]
         lib.fake_launch_name.restype = ctypes.c_char_p
         lib.fake_launch_stream.restype = ctypes.c_void_p
+        lib.fake_launch_word.restype = ctypes.c_uint64
         lib.fake_fail_allocations.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
         lib.fake_fail_host_allocations.argtypes = [ctypes.c_size_t]
         lib.fake_allocated.restype = ctypes.c_size_t
@@ -70,6 +78,11 @@ class Fake:
         names = [self.lib.fake_launch_name(i).decode() for i in range(self.lib.fake_launches())]
         self.lib.fake_clear_launches()
         return names
+
+    def argument_words(self, part, word):
+        """The given 8-byte word of the first argument of every launch of `part` since kernels()."""
+        return [self.lib.fake_launch_word(i, word) for i in range(self.lib.fake_launches())
+                if part in self.lib.fake_launch_name(i).decode()]
 
     def ran(self, part):
         return any(part in n for n in self.kernels())
@@ -89,6 +102,10 @@ class Fake:
 def load(so):
     fake = ctypes.CDLL(so, mode=ctypes.RTLD_GLOBAL)
     torch = types.ModuleType("torch")   # the real one would load the real runtime
+    for name, size in (("uint8", 1), ("float32", 4), ("float64", 8)):
+        setattr(torch, name, name)
+    torch.empty = lambda shape, dtype, device: Tensor(shape if isinstance(shape, tuple) else (shape,),
+                                                      {"uint8": 1, "float32": 4, "float64": 8}[dtype], dtype)
     torch.cuda = types.SimpleNamespace(current_stream=lambda *a: Stream())
     sys.modules["torch"] = torch
     for p in ("astro-accelerate_amd", "oracle"):
