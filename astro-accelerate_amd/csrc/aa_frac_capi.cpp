@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <new>
 #include <string>
 #include <vector>
@@ -96,6 +97,20 @@ aa_hip::frac_args base_args(const aa_hip_frac* p, int nbatch, const float* d_dm)
     a.K = p->ntrials;
     a.n_ttiles = (p->nsamp + aa_hip::kFracTile - 1) / aa_hip::kFracTile;
     return a;
+}
+
+// Work-groups of an unsplit pass over the channels, the channel parts of a split
+// one, and the bytes of its partial profiles.
+size_t row_groups(const aa_hip_frac* p, int nbatch) {
+    const int per_group = 16 * p->trials_per_wave;
+    return (size_t)nbatch * ((p->nsamp + aa_hip::kFracTile - 1) / aa_hip::kFracTile) *
+           ((p->ntrials + per_group - 1) / per_group);
+}
+int row_split(const aa_hip_frac* p, int nbatch) {
+    return aa_hip::frac_channel_split(row_groups(p, nbatch), p->nchans);
+}
+size_t forward_bytes(const aa_hip_frac* p, int nbatch) {
+    return sizeof(float) * row_split(p, nbatch) * (size_t)nbatch * p->ntrials * p->nsamp;
 }
 
 bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
@@ -195,8 +210,8 @@ int aa_hip_frac_grouping(const aa_hip_frac* h, int* trials_per_wave, int* chans_
     return AA_HIP_SUCCESS;
 }
 
-int aa_hip_frac_forward(aa_hip_frac* h, const float* d_x, int nbatch, const float* d_dm, float* d_y,
-                        void* stream) {
+static int frac_forward(aa_hip_frac* h, const float* d_x, int nbatch, const float* d_dm, float* d_y, float* y_part,
+                        size_t work_bytes, void* stream) {
     if (!h || !d_x || !d_dm || !d_y) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "NULL argument");
     if (nbatch < 0 || nbatch > h->max_batch) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "batch exceeds the plan's");
     if (!aligned16(d_x) || !aligned16(d_y)) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "buffers must be 16-byte aligned");
@@ -206,14 +221,33 @@ int aa_hip_frac_forward(aa_hip_frac* h, const float* d_x, int nbatch, const floa
     a.y = d_y;
     a.group_q = h->trials_per_wave;
     a.n_groups = (h->ntrials + 16 * a.group_q - 1) / (16 * a.group_q);
-    a.n_split =
-        h->d_ypart ? aa_hip::frac_channel_split((size_t)nbatch * a.n_ttiles * a.n_groups, h->nchans) : 1;
-    a.y_part = h->d_ypart;
+    a.n_split = y_part ? row_split(h, nbatch) : 1;
+    a.y_part = y_part;
+    if (a.n_split > 1 && (work_bytes < forward_bytes(h, nbatch) || !aligned16(y_part)))
+        return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "workspace too small for the batch, or not 16-byte aligned");
     return from_hip(aa_hip::launch_frac_forward(a, (hipStream_t)stream), "frac forward");
 }
 
-int aa_hip_frac_adjoint(aa_hip_frac* h, const float* d_x, const float* d_gy, int nbatch, const float* d_dm,
-                        float* d_gx, double* d_gdm, void* stream) {
+int aa_hip_frac_forward(aa_hip_frac* h, const float* d_x, int nbatch, const float* d_dm, float* d_y,
+                        void* stream) {
+    return frac_forward(h, d_x, nbatch, d_dm, d_y, h ? h->d_ypart : nullptr, SIZE_MAX, stream);
+}
+
+int aa_hip_frac_forward_ws(aa_hip_frac* h, const float* d_x, int nbatch, const float* d_dm, float* d_y, void* d_work,
+                           size_t work_bytes, void* stream) {
+    return frac_forward(h, d_x, nbatch, d_dm, d_y, (float*)d_work, work_bytes, stream);
+}
+
+int aa_hip_frac_workspace_bytes(const aa_hip_frac* h, int nbatch, size_t* forward, size_t* adjoint) {
+    if (!h || !forward || !adjoint) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "NULL argument");
+    if (nbatch < 0 || nbatch > h->max_batch) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "batch exceeds the plan's");
+    *forward = nbatch > 0 && row_split(h, nbatch) > 1 ? forward_bytes(h, nbatch) : 0;
+    *adjoint = nbatch > 0 ? sizeof(double) * row_groups(h, nbatch) * (size_t)row_split(h, nbatch) : 0;
+    return AA_HIP_SUCCESS;
+}
+
+static int frac_adjoint(aa_hip_frac* h, const float* d_x, const float* d_gy, int nbatch, const float* d_dm,
+                        float* d_gx, double* d_gdm, double* gdm_part, size_t work_bytes, void* stream) {
     if (!h || !d_gy || !d_dm) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "NULL argument");
     if (d_gdm && !d_x) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "the DM adjoint needs the input");
     if (nbatch < 0 || nbatch > h->max_batch) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "batch exceeds the plan's");
@@ -235,16 +269,27 @@ int aa_hip_frac_adjoint(aa_hip_frac* h, const float* d_x, const float* d_gy, int
         a.x = d_x;
         a.gy = d_gy;
         a.gdm = d_gdm;
-        a.gdm_part = h->d_part;
+        a.gdm_part = gdm_part;
         a.group_q = h->trials_per_wave;
         a.n_groups = (h->ntrials + 16 * a.group_q - 1) / (16 * a.group_q);
-        a.n_split = aa_hip::frac_channel_split((size_t)nbatch * a.n_ttiles * a.n_groups, h->nchans);
-        if (aa_hip::frac_grad_dm_parts(a) > h->part_entries)
-            return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "workspace too small for the batch");
+        a.n_split = row_split(h, nbatch);
+        if (!gdm_part || !aligned16(gdm_part) || work_bytes < sizeof(double) * aa_hip::frac_grad_dm_parts(a))
+            return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "workspace too small for the batch, or not 16-byte aligned");
         const int st = from_hip(aa_hip::launch_frac_grad_dm(a, s), "frac DM adjoint");
         if (st != AA_HIP_SUCCESS) return st;
     }
     return AA_HIP_SUCCESS;
+}
+
+int aa_hip_frac_adjoint(aa_hip_frac* h, const float* d_x, const float* d_gy, int nbatch, const float* d_dm,
+                        float* d_gx, double* d_gdm, void* stream) {
+    return frac_adjoint(h, d_x, d_gy, nbatch, d_dm, d_gx, d_gdm, h ? h->d_part : nullptr,
+                        h ? sizeof(double) * h->part_entries : 0, stream);
+}
+
+int aa_hip_frac_adjoint_ws(aa_hip_frac* h, const float* d_x, const float* d_gy, int nbatch, const float* d_dm,
+                           float* d_gx, double* d_gdm, void* d_work, size_t work_bytes, void* stream) {
+    return frac_adjoint(h, d_x, d_gy, nbatch, d_dm, d_gx, d_gdm, (double*)d_work, work_bytes, stream);
 }
 
 int aa_hip_refine_create(int device, int ncand, const int64_t* x_offsets, const int64_t* ds_offsets,

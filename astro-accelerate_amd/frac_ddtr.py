@@ -52,7 +52,9 @@ def _stream_handle():
 
 
 class FracPlan:
-    """Device plan (aa_hip_frac handle): delay table, trial offsets, window length."""
+    """Device plan (aa_hip_frac handle): delay table, trial offsets, window length.
+    Calls may overlap (streams, threads): each allocates its own scratch memory
+    on the current stream."""
 
     def __init__(self, delay_per_dm: np.ndarray, trials: Sequence[float], nsamp: int, max_batch: int,
                  dm_absmax: float = 16.0, device: int = 0):
@@ -104,6 +106,15 @@ class FracPlan:
             raise ValueError("dm must be a contiguous float32 CUDA tensor of shape [B]")
         return b
 
+    def _work(self, b: int, device, adjoint: bool):
+        """Scratch memory of one call (a tensor of the current stream) and its bytes."""
+        import torch
+        fwd, adj = ctypes.c_size_t(), ctypes.c_size_t()
+        aa.check(aa.load_library().aa_hip_frac_workspace_bytes(self.handle, b, ctypes.byref(fwd), ctypes.byref(adj)),
+                 "aa_hip_frac_workspace_bytes")
+        n = adj.value if adjoint else fwd.value
+        return (torch.empty(n, dtype=torch.uint8, device=device) if n else None), n
+
     def forward(self, x, dm, out=None):
         """y[B, K, T] for windows x[B, C, T] at continuous DM offsets dm[B]."""
         import torch
@@ -112,10 +123,12 @@ class FracPlan:
         y = out if out is not None else torch.empty((b, self.ntrials, self.nsamp), dtype=torch.float32,
                                                     device=x.device)
         self._check_x(y, "out")
-        aa.check(aa.load_library().aa_hip_frac_forward(self.handle, ctypes.c_void_p(x.data_ptr()), b,
-                                                        ctypes.c_void_p(dm.data_ptr()),
-                                                        ctypes.c_void_p(y.data_ptr()), _stream_handle()),
-                 "aa_hip_frac_forward")
+        work, n = self._work(b, x.device, adjoint=False)
+        aa.check(aa.load_library().aa_hip_frac_forward_ws(self.handle, ctypes.c_void_p(x.data_ptr()), b,
+                                                          ctypes.c_void_p(dm.data_ptr()),
+                                                          ctypes.c_void_p(y.data_ptr()),
+                                                          ctypes.c_void_p(work.data_ptr() if n else 0), n,
+                                                          _stream_handle()), "aa_hip_frac_forward")
         return y
 
     def adjoint(self, x, gy, dm, want_x: bool = True, want_dm: bool = True):
@@ -129,10 +142,12 @@ class FracPlan:
             self._check_x(x)
             if tuple(x.shape) != (b, self.nchans, self.nsamp):
                 raise ValueError("x does not match gy")
-        aa.check(aa.load_library().aa_hip_frac_adjoint(
+        work, n = self._work(b, gy.device, adjoint=True) if want_dm else (None, 0)
+        aa.check(aa.load_library().aa_hip_frac_adjoint_ws(
             self.handle, ctypes.c_void_p(x.data_ptr() if x is not None else 0), ctypes.c_void_p(gy.data_ptr()), b,
             ctypes.c_void_p(dm.data_ptr()), ctypes.c_void_p(gx.data_ptr() if gx is not None else 0),
-            ctypes.c_void_p(gdm.data_ptr() if gdm is not None else 0), _stream_handle()), "aa_hip_frac_adjoint")
+            ctypes.c_void_p(gdm.data_ptr() if gdm is not None else 0), ctypes.c_void_p(work.data_ptr() if n else 0), n,
+            _stream_handle()), "aa_hip_frac_adjoint")
         return gx, gdm
 
 

@@ -197,6 +197,9 @@ def _declare(lib: ctypes.CDLL) -> None:
         "aa_hip_frac_grouping": ([vp, pi, pi], i),
         "aa_hip_frac_forward": ([vp, vp, i, vp, vp, vp], i),
         "aa_hip_frac_adjoint": ([vp, vp, vp, i, vp, vp, vp, vp], i),
+        "aa_hip_frac_workspace_bytes": ([vp, i, ctypes.POINTER(sz), ctypes.POINTER(sz)], i),
+        "aa_hip_frac_forward_ws": ([vp, vp, i, vp, vp, vp, sz, vp], i),
+        "aa_hip_frac_adjoint_ws": ([vp, vp, vp, i, vp, vp, vp, vp, sz, vp], i),
         "aa_hip_zero_dm_u8": ([vp, i, i, vp, i, vp], i),
         "aa_hip_zero_dm_u16": ([vp, i, i, vp, i, vp], i),
         "aa_hip_zero_dm_outliers_u8": ([vp, ctypes.c_long, i, vp, i, vp], i),

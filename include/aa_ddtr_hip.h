@@ -475,7 +475,8 @@ int aa_hip_inject_pulse_u8(uint8_t *d_data_tc, int nsamp, int nchans, const floa
  *   i0 = floor(tau), f = (float)(tau - i0), x = 0 outside [0, T).
  * The adjoint gives gx = (dy/dx)^T gy and gdm[b] = sum_{k,t} gy * dy/d(dm[b])
  * (accumulated in double).  Device buffers are caller-owned, 16-byte
- * aligned; calls on one handle must not overlap.
+ * aligned.  Calls on one handle must not overlap, except those that bring
+ * workspaces of their own (_ws).
  * ---------------------------------------------------------------------- */
 typedef struct aa_hip_frac aa_hip_frac;
 /* dm_absmax bounds |dm[b]| for sizing the input adjoint's channel groups
@@ -495,6 +496,17 @@ int aa_hip_frac_forward(aa_hip_frac *h, const float *d_x, int nbatch, const floa
  * from x: nothing from the forward pass is stored. */
 int aa_hip_frac_adjoint(aa_hip_frac *h, const float *d_x, const float *d_gy, int nbatch,
                         const float *d_dm, float *d_gx, double *d_gdm, void *stream);
+/* The same with scratch memory of the call's own, so that calls on one handle
+ * may overlap (streams, host threads): d_work is device memory, 16-byte
+ * aligned, of at least the bytes that workspace_bytes gives for the batch, and
+ * free for other use once the call's work on `stream` is done.  The forward
+ * call takes NULL where it needs none, and without one is not split over the
+ * channels (slower on small batches); the adjoint needs one for gdm only. */
+int aa_hip_frac_workspace_bytes(const aa_hip_frac *h, int nbatch, size_t *forward, size_t *adjoint);
+int aa_hip_frac_forward_ws(aa_hip_frac *h, const float *d_x, int nbatch, const float *d_dm, float *d_y,
+                           void *d_work, size_t work_bytes, void *stream);
+int aa_hip_frac_adjoint_ws(aa_hip_frac *h, const float *d_x, const float *d_gy, int nbatch, const float *d_dm,
+                           float *d_gx, double *d_gdm, void *d_work, size_t work_bytes, void *stream);
 
 /* Batched DM refinement of candidate windows of uneven size (no reference
  * counterpart).  Candidate b's window is float [nchans[b]][nsamp[b]] at

@@ -35,3 +35,32 @@ def test_split_channels_match_reference(cuda, shape):
     assert float((y.double() - y64).abs().max()) <= 2e-6 * scale * max(1.0, (C / 256) ** 0.5)
     assert float((gx.double() - gx64).abs().max()) <= 2e-6 * float(gx64.abs().max())
     assert float((gdm.double() - gdm64).abs().max()) <= 1e-5 * max(float(gdm64.abs().max()), scale)
+
+
+def test_two_streams_share_a_plan(cuda):
+    """Forward and backward of one plan on two streams at once give, bit for bit,
+    what they give alone."""
+    import torch
+    import frac_ddtr
+    B, C, T, K = 2, 2048, 1024, 32
+    g = torch.Generator(device=cuda).manual_seed(3)
+    plan = frac_ddtr.FracPlan(np.linspace(0.0, 3.7, C).astype(np.float32), np.linspace(-2.0, 2.0, K), T, B)
+    xs = [torch.randn((B, C, T), generator=g, device=cuda, requires_grad=True) for _ in range(2)]
+    dms = [(torch.rand(B, generator=g, device=cuda) - 0.5).requires_grad_(True) for _ in range(2)]
+
+    def step(i):
+        y = frac_ddtr.frac_dedisperse(xs[i], dms[i], plan)
+        return [y.detach()] + list(torch.autograd.grad(y.square().sum(), (xs[i], dms[i])))
+
+    want = [step(i) for i in range(2)]
+    torch.cuda.synchronize()
+    streams, got = [torch.cuda.Stream() for _ in range(2)], [[], []]
+    for _ in range(10):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                got[i].append(step(i))
+    torch.cuda.synchronize()
+    for i in range(2):
+        for result in got[i]:
+            for a, b in zip(result, want[i]):
+                assert torch.equal(a, b)
