@@ -176,7 +176,7 @@ hipError_t launch_range(const range_launch &rl, hipStream_t s) {
             lds_params p = lds_params_of(rl);
             p.L = rl.planes;
             p.pitch = rl.plane_pitch;
-            const hipError_t e = launch_dedisperse_matrix(p, rl.mat, s, rl.over, rl.flags);
+            const hipError_t e = launch_dedisperse_matrix(p, rl.mat, s, rl.over, rl.flags, rl.t_flags);
             if (e != hipSuccess) return e;
         }
         if (rl.wide_win > 0)
@@ -446,6 +446,7 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
         rl->plane_pitch = lv.plane_pitch;
         rl->over = lv.over;
         rl->flags = mt.flags;
+        rl->t_flags = (int)std::min(lv.len - m_maxshift / rd.inBin, 0x7fffffffL);
         return AA_HIP_SUCCESS;
     }
     if (m_lds.size() != m_ranges.size()) m_lds.assign(m_ranges.size(), lds_choice{-2, 0});

@@ -80,6 +80,7 @@ struct range_launch {
     size_t plane_pitch = 0;
     const int *over = nullptr;
     int *flags = nullptr;
+    int t_flags = 0;
 };
 
 class ddtr_engine {

@@ -41,8 +41,10 @@ matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float m
 // tile with a sum above 2^24, where the reference's float adds round, sets its
 // entry of flags (n_dm_tiles x time tiles, time tile major; else 0) and has to
 // be computed in channel order; more than half of over's 64 entries set flags
-// every tile and computes none.
+// every tile and computes none.  t_flags: the most samples (at least
+// t_processed) that the rows hold for this range; the flags depend on them and
+// not on t_processed.
 hipError_t launch_dedisperse_matrix(const lds_params& p, const matrix_layout& lay, hipStream_t s,
-                                    const int* over = nullptr, int* flags = nullptr);
+                                    const int* over = nullptr, int* flags = nullptr, int t_flags = 0);
 
 }  // namespace aa_hip

@@ -110,6 +110,7 @@ struct mat_args {
     int tile_out;
     const int* over;       // 64 entries: more than half of them set: flag every tile
     int* flags;
+    int t_flags;           // samples that can set a tile's flag
 };
 
 __shared__ uint32_t m_rows[2 * kMatDms * kMatRow + 512];   // the tail: reads past the last row's window
@@ -317,7 +318,11 @@ __global__ __launch_bounds__(kMatThreads, 2) void dedisperse_matrix_kernel(mat_a
 
     const long t_end = t0 + a.tile_out < p.t_processed ? t0 + a.tile_out : (long)p.t_processed;
     const int bias = 128 * p.nchans * (PLANES ? 257 : 1);   // what the sign flips took off every sum
-    bool above = false;   // a sum whose float adds round
+    // A sum whose float adds round.  Looked for in all samples that the rows hold,
+    // also those past t_processed: calls of different lengths that overlap on
+    // other streams then write the same flags.
+    const long f_end = PLANES ? (t0 + a.tile_out < a.t_flags ? t0 + a.tile_out : (long)a.t_flags) : 0;
+    bool above = false;
 #pragma unroll
     for (int dd = 0; dd < 2; ++dd) {
         const int d = dm_tile * kMatDms + 2 * wave + dd;
@@ -328,7 +333,7 @@ __global__ __launch_bounds__(kMatThreads, 2) void dedisperse_matrix_kernel(mat_a
         for (int j = 0; j < kMatOut; ++j) {
             const long t = t0 + 2 * (lane + 64 * j);
             const uint32_t s0 = (uint32_t)(lo[dd][j] + bias), s1 = (uint32_t)(hi[dd][j] + bias);
-            if (PLANES) above |= (t < t_end && s0 > (1u << 24)) || (t + 1 < t_end && s1 > (1u << 24));
+            if (PLANES) above |= (t < f_end && s0 > (1u << 24)) || (t + 1 < f_end && s1 > (1u << 24));
             const float v0 = out_value(s0, p), v1 = out_value(s1, p);
             if (aligned && t + 1 < t_end) {
                 *reinterpret_cast<float2*>(orow + t) = make_float2(v0, v1);
@@ -623,10 +628,10 @@ matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float m
 }
 
 hipError_t launch_dedisperse_matrix(const lds_params& p, const matrix_layout& lay, hipStream_t s, const int* over,
-                                    int* flags)
+                                    int* flags, int t_flags)
 {
     if (p.ndms <= 0 || p.t_processed <= 0) return hipSuccess;
-    if ((lay.planes == 2) != (over && flags)) return hipErrorInvalidValue;
+    if ((lay.planes == 2) != (over && flags) || (flags && t_flags < p.t_processed)) return hipErrorInvalidValue;
     if (!p.pair_recs || lay.tile_out <= 0 || lay.n_dm_tiles != (p.ndms + kMatDms - 1) / kMatDms)
         return hipErrorInvalidValue;
     mat_args a{};
@@ -636,6 +641,7 @@ hipError_t launch_dedisperse_matrix(const lds_params& p, const matrix_layout& la
     a.tile_out = lay.tile_out;
     a.over = over;
     a.flags = flags;
+    a.t_flags = t_flags;
     const char* t = static_cast<const char*>(p.pair_recs);
     a.tiles = reinterpret_cast<const mat_tile*>(t);
     a.groups = reinterpret_cast<const mat_group*>(t + lay.off_group);

@@ -115,3 +115,43 @@ def test_u16_byte_planes(aa, oracle, cuda, kind, nchans):
         got = outs[r].cpu().numpy()
         np.testing.assert_array_equal(got[:, :tps[r]], want[r], err_msg=f"range {r}")
         assert np.all(got[:, tps[r]:] == -1.0)
+
+
+def test_u16_lengths_on_two_streams(aa, oracle, cuda):
+    """Two lengths of one 16-bit range on two streams at once: the shorter call's
+    samples sum exactly, the longer one's round from the middle of a tile on."""
+    import torch
+    nchans, tsamp, nsamp, ndms, lengths = 1024, 64e-6, 16000, 64, (600, 4000)
+    ds = oracle.dmshifts(nchans, 1500.0, -300.0 / nchans)
+    maxd = int(ds[-1] * (0.4 * ndms / tsamp)) + 2
+    assert 600 + maxd < 1500
+    rng = np.random.default_rng(8)
+    x = rng.integers(0, 2001, size=(nsamp, nchans))
+    x[1500:4000 + maxd] = rng.integers(0, 40001, size=(2500 + maxd, nchans))   # sums about 2e7
+    d_in = torch.from_numpy(x.astype(np.uint16).view(np.int16)).to(cuda)
+    plan = aa.DdtrPlan(ds, [(0.0, 0.4, ndms, 1)], tsamp, maxd, nsamp - maxd, sample_bits=16)
+    plan.ingest(d_in, nsamp - maxd)
+    want = []
+    for tp in lengths:
+        out = torch.empty((ndms, tp), dtype=torch.float32, device=cuda)
+        plan.run_range(0, tp, out)
+        want.append(out)
+    direct = aa.DdtrPlan(ds, [(0.0, 0.4, ndms, 1)], tsamp, maxd, nsamp - maxd, sample_bits=16)
+    direct.set_kernel(aa.KERNEL_DIRECT)      # in channel order, whatever the sums
+    direct.ingest(d_in, nsamp - maxd)
+    for tp, w in zip(lengths, want):
+        out = torch.empty((ndms, tp), dtype=torch.float32, device=cuda)
+        direct.run_range(0, tp, out)
+        assert torch.equal(out, w)
+    torch.cuda.synchronize()
+    streams, got = [torch.cuda.Stream() for _ in lengths], [[], []]
+    for _ in range(20):
+        for i, (tp, s) in enumerate(zip(lengths, streams)):
+            with torch.cuda.stream(s):
+                out = torch.empty((ndms, tp), dtype=torch.float32, device=cuda)
+                plan.run_range(0, tp, out, stream=s)
+                got[i].append(out)
+    torch.cuda.synchronize()
+    for outs, w in zip(got, want):
+        for out in outs:
+            assert torch.equal(out, w)
