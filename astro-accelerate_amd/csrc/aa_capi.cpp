@@ -521,6 +521,7 @@ int aa_hip_host_copy(void *dst, const void *src, size_t bytes) {
     try {
         for (; started < n; ++started) threads[started] = std::thread(copy, started);
     } catch (const std::system_error &) {   // no more threads: the rest is this thread's too
+    } catch (const std::bad_alloc &) {
     }
     copy(0);
     for (size_t i = started; i < n; ++i) copy(i);
