@@ -30,6 +30,8 @@
 
 #include <cmath>
 
+#include "linear_grid.h"
+
 namespace aa_hip {
 
 namespace {
@@ -70,8 +72,9 @@ __global__ __launch_bounds__(kRowThreads) void dedisperse_rows_kernel(lds_params
     const int n_t = (p.t_processed + kRowTile - 1) / kRowTile;
     const int ntiles = p.ndms * n_t;
     const int per = (ntiles + 7) / 8;
-    const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per || tile >= ntiles) return;   // whole work-group, before the barrier
+    const int g = (int)linear_block();
+    const int tile = (g & 7) * per + (g >> 3);
+    if ((g >> 3) >= per || tile >= ntiles) return;   // whole work-group, before the barrier
     const int d = tile % p.ndms;
     const long t0 = (long)(tile / p.ndms) * kRowTile;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -184,7 +187,8 @@ hipError_t launch_dedisperse_rows(const lds_params& p, hipStream_t s)
     if (p.ndms <= 0 || p.t_processed <= 0) return hipSuccess;
     const long tiles = (long)p.ndms * ((p.t_processed + kRowTile - 1) / kRowTile);
     if (tiles > 0x0fffffffL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(dedisperse_rows_kernel, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(kRowThreads), 0, s, p);
+    hipLaunchKernelGGL(dedisperse_rows_kernel, linear_grid(8 * ((tiles + 7) / 8), kRowThreads), dim3(kRowThreads), 0, s,
+                       p);
     return hipGetLastError();
 }
 

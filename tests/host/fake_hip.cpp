@@ -1,9 +1,10 @@
 // A HIP runtime without a GPU, for tests of the library's host code: device
 // memory is host memory, kernels are recorded by name and not run, an
 // allocation can be made to fail (leaving its error behind, as HIP does, until
-// hipGetLastError takes it), and a stream under capture refuses allocations and
-// synchronous copies.  Host allocations (operator new) can be made to fail too.
-// Loaded before the library under HIP's own soname.
+// hipGetLastError takes it), launches of 2^32 threads or more along a dimension
+// are refused (HIP runs a part of them), and a stream under capture refuses
+// allocations and synchronous copies.  Host allocations (operator new) can be
+// made to fail too.  Loaded before the library under HIP's own soname.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -14,7 +15,7 @@
 #include <vector>
 
 typedef int err_t;   // hipError_t
-enum { ok = 0, invalid = 1, oom = 2, capture_unsupported = 900 };
+enum { ok = 0, invalid = 1, oom = 2, invalid_configuration = 9, capture_unsupported = 900 };
 struct dim { unsigned x, y, z; };
 
 namespace {
@@ -84,8 +85,9 @@ err_t __hipPopCallConfiguration(dim* g, dim* b, size_t* lds, void** s)
     *g = g_call.grid; *b = g_call.block; *lds = g_call.lds; *s = g_call.stream;
     return ok;
 }
-err_t hipLaunchKernel(const void* f, dim g, dim, void** args, size_t, void* s)
+err_t hipLaunchKernel(const void* f, dim g, dim b, void** args, size_t, void* s)
 {
+    if ((size_t)g.x * b.x >> 32 || (size_t)g.y * b.y >> 32 || (size_t)g.z * b.z >> 32) return set(invalid_configuration);
     launch l{g_kernels[f], s, g.x, {}};
     std::memcpy(l.words, args[0], sizeof(l.words));
     g_launches.push_back(l);
