@@ -480,39 +480,33 @@ int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_
         if (c.variant < 0 && tuned.variant >= 0)  // preferred shape does not fit: any that does
             c = choose_lds(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, -1);
     }
-    const bool rows = (alone || (automatic && c.variant < 0)) &&
-                      rows_beat_shape(m_nchans, rd.ndms, t_processed, c.variant);
+    // Under capture a shape whose tables are not there yet (the calls before went
+    // another way) would break the capture; the rows need none.
+    const bool rows = ((alone || (automatic && c.variant < 0)) &&
+                       rows_beat_shape(m_nchans, rd.ndms, t_processed, c.variant)) ||
+                      (automatic && c.variant >= 2 && !has_tables(r, c.variant) && capturing(s));
     st = resolve_launch(m_kernel, lv.ptr, lv.pitch, m_nchans, m_d_dmshifts, m_dmshifts.data(), rd.ndms,
                         t_processed, mstartdm, mdmstep, rd.inBin, d_out, out_pitch,
                         rows ? lds_choice{kShapeRows, 0} : c, rl);
-    if (st != AA_HIP_SUCCESS || rl->variant < 2) return st;
-    if (rl->variant != kShapeRows) return shape_tables(r, rl->variant, rl->row_quads, &rl->pair_recs);
-    // A longer chunk of this range may take the shape, and under capture: its
-    // tables are made now.  This call does without them.
-    const void *unused;
-    if (c.variant >= 2 && !capturing(s)) (void)shape_tables(r, c.variant, c.row_quads, &unused);
-    return AA_HIP_SUCCESS;
-}
-
-// Chunk shapes from 2 on read plan tables, which depend on the range and shape
-// only: made on the range's first eager call that is not the matrix kernel's,
-// whatever its length, so that a later one can be captured into a graph.
-int ddtr_engine::shape_tables(int r, int variant, int row_quads, const void **tables) {
+    if (st != AA_HIP_SUCCESS || rl->variant < 2 || rl->variant == kShapeRows) return st;
+    // Chunk shapes from 2 on read plan tables; they depend on the range and
+    // shape only, so they are built once, on the first call that needs them.
     if (m_tables.size() != m_ranges.size()) m_tables.resize(m_ranges.size());
-    plan_tables &pt = m_tables[(size_t)r][(size_t)variant];
+    plan_tables &pt = m_tables[(size_t)r][(size_t)rl->variant];
     if (!pt.ptr) {
-        const range_desc &rd = m_ranges[(size_t)r];
-        float mstartdm, mdmstep;
-        range_scalars(r, &mstartdm, &mdmstep);
         std::vector<uint8_t> bytes;
-        if (lds_plan_tables(variant, m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep,
-                            m_levels[(size_t)log2i(rd.inBin)].pitch, &bytes) != row_quads)
+        if (lds_plan_tables(rl->variant, m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, lv.pitch, &bytes) !=
+            rl->row_quads)
             return fail(AA_HIP_ERROR_UNSUPPORTED, "plan tables disagree with the chosen row width");
         const hipError_t e = keep_tables(pt, bytes);
         if (e != hipSuccess) return hip_fail(e, "plan tables");
     }
-    *tables = pt.ptr;
+    rl->pair_recs = pt.ptr;
     return AA_HIP_SUCCESS;
+}
+
+bool ddtr_engine::has_tables(int r, int variant) const {
+    return !m_tables.empty() && m_tables[(size_t)r][(size_t)variant].ptr;
 }
 
 // The window of dedisperse_u16 for range r of a u16 plan (-1: direct kernel).
@@ -676,7 +670,7 @@ int ddtr_engine::autotune_range(int r, int t_processed, float *d_out, size_t out
     m_kernel = AA_HIP_KERNEL_AUTO;
     *best = -1;
     bool had[kLdsVariants];
-    for (int v = 0; v < kLdsVariants; ++v) had[v] = !m_tables.empty() && m_tables[(size_t)r][(size_t)v].ptr;
+    for (int v = 0; v < kLdsVariants; ++v) had[v] = has_tables(r, v);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     hipError_t e = hipEventCreate(&e0);
     if (e == hipSuccess) e = hipEventCreate(&e1);

@@ -206,7 +206,7 @@ private:
     hipError_t keep_tables(plan_tables &pt, const std::vector<uint8_t> &bytes);
     void drop_tables(plan_tables &pt);
     hipError_t plan_matrix(int r, size_t pitch, int planes, hipStream_t s);
-    int shape_tables(int r, int variant, int row_quads, const void **tables);
+    bool has_tables(int r, int variant) const;
     void drop_matrix(int r);
     size_t m_device_bytes = 0;
 };

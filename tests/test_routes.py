@@ -187,8 +187,9 @@ assert sum("dedisperse_matrix_kernel" in n for n in captured(chunk)) == 2
 
 
 def test_captured_chunk_longer_than_the_eager_one(tmp_path):
-    """A short eager chunk goes from the rows; a longer one captured after it
-    takes an LDS shape, whose tables are there."""
+    """A short eager chunk goes from the rows, and so does a longer one captured
+    after it, whose shape's tables are not there; after an eager one it takes
+    the shape."""
     host_library.run(CAPTURE + '''
 ds = oracle.dmshifts(128, 1500.0, -5.0)   # a range that the matrix kernel does not take
 shift = int(ds[-1] * 256.0 / 64e-6) + 10
@@ -198,17 +199,22 @@ plan.ingest(xl, 100)
 plan.run_range(0, 100, ol)
 assert fake.ran("dedisperse_rows_kernel")
 plan.ingest(xl, tp)
-names = captured(lambda: plan.run_range(0, tp, ol, stream=capture))
-assert any("dedisperse_wide_kernel" in n for n in names), names
+def chunk():
+    plan.run_range(0, tp, ol, stream=capture)
+assert any("dedisperse_rows_kernel" in n for n in captured(chunk))
+chunk()
+assert fake.ran("dedisperse_wide_kernel")
+assert any("dedisperse_wide_kernel" in n for n in captured(chunk))
 ''', tmp_path)
 
 
 def test_8_bit_range_captured_at_first(tmp_path):
-    """A range that can do without tables may be captured at once, although the
-    matrix kernel, which cannot, would be the automatic choice."""
+    """A range left to the automatic choice may be captured at once: it goes from
+    the rows or on a shape that reads no tables."""
     host_library.run(CAPTURE + '''
 plan = make()
 plan.ingest(x, tp)
+assert any("dedisperse_rows_kernel" in n for n in captured(lambda: plan.run_range(0, tp, out, stream=capture)))
 plan.set_range_tuning(0, 0, True)
 names = captured(lambda: plan.run_range(0, tp, out, stream=capture))
 assert any("dedisperse_lds_kernel" in n or "dedisperse_rows_kernel" in n for n in names), names
