@@ -38,6 +38,7 @@
 #include <type_traits>
 
 #include "ddtr_kernels.h"
+#include "linear_grid.h"
 
 namespace aa_hip {
 namespace {
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(1024) void normalize_columns_kernel(T* data, long r
     __shared__ float part[16][64];
     __shared__ float offs[64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const long c = (long)blockIdx.x * 64 + lane;
+    const long c = linear_block() * 64 + lane;
     const bool on = c < cols;
     float a0 = 0.0f, a1 = 0.0f;
     if (on) {
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(1024) void normalize_columns_f32x4_kernel(float* da
     __shared__ float4 offs[64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const long nq = cols >> 2;
-    const long q = (long)blockIdx.x * 64 + lane;
+    const long q = linear_block() * 64 + lane;
     const bool on = q < nq;
     float4* d = reinterpret_cast<float4*>(data);
     float4 a0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), a1 = a0;
@@ -169,8 +170,8 @@ __global__ __launch_bounds__(32 * LANES) void normalize_strip_f32_kernel(float* 
     __shared__ f32x4 part[32][LANES];
     __shared__ __align__(16) float offs[kStripCols];
     const int q = threadIdx.x & (LANES - 1), y = threadIdx.x / LANES;
-    const long c = (long)blockIdx.x * kStripCols + 4 * q;
-    const bool whole = (long)blockIdx.x * kStripCols + kStripCols <= cols;   // the strip's, for all threads
+    const long c0 = linear_block() * kStripCols, c = c0 + 4 * q;
+    const bool whole = c0 + kStripCols <= cols;   // the strip's, for all threads
     float* col = data + y * cols + c;
     const int mine = rows > y ? (int)((rows - y + 31) / 32) : 0;
     const int left = c < cols ? (int)(cols - c < 4 ? cols - c : 4) : 0;   // columns of this thread
@@ -457,7 +458,7 @@ hipError_t normalize_int(T* data, long rows, long cols, float factor, int nbits,
 template <int LANES>
 hipError_t launch_strips(float* data, long rows, long cols, float factor, hipStream_t s)
 {
-    const dim3 strips(blocks_of(cols, 4 * LANES)), threads(32 * LANES);
+    const dim3 strips = linear_grid((cols + 4 * LANES - 1) / (4 * LANES), 32 * LANES), threads(32 * LANES);
     if (rows <= 128)
         hipLaunchKernelGGL((normalize_strip_f32_kernel<4, LANES>), strips, threads, 0, s, data, rows, cols, factor);
     else if (rows <= 256)
@@ -504,11 +505,11 @@ hipError_t launch_normalize_columns_f32(float* data, long rows, long cols, float
     // per lane, 6080 x 111,328 1.68 ms against 1.86; 3072 x 32,768 256 us against
     // 244, 1600 x 20,000 65 against 62.
     if (cols % 4 == 0 && (uintptr_t)data % 16 == 0 && cols >= 160 * 256)
-        hipLaunchKernelGGL(normalize_columns_f32x4_kernel, dim3(blocks_of(cols / 4, 64)), dim3(1024), 0, s, data,
-                           rows, cols, factor);
+        hipLaunchKernelGGL(normalize_columns_f32x4_kernel, linear_grid((cols / 4 + 63) / 64, 1024), dim3(1024), 0, s,
+                           data, rows, cols, factor);
     else
-        hipLaunchKernelGGL(normalize_columns_kernel<float>, dim3(blocks_of(cols, 64)), dim3(1024), 0, s, data, rows,
-                           cols, factor, 0.0f);
+        hipLaunchKernelGGL(normalize_columns_kernel<float>, linear_grid((cols + 63) / 64, 1024), dim3(1024), 0, s, data,
+                           rows, cols, factor, 0.0f);
     return hipGetLastError();
 }
 

@@ -56,6 +56,8 @@
 
 #include <cmath>
 
+#include "linear_grid.h"
+
 namespace aa_hip {
 
 namespace {
@@ -135,7 +137,9 @@ __global__ __launch_bounds__(kThreads) void refine_partial_kernel(refine_args a,
     __shared__ float dsv[kChunk];
     __shared__ double r_y[kSeg], r_p[NK ? 1 : kSeg + 8];
     __shared__ double r_b[2][kThreads / 64];
-    const refine_item it = a.items[blockIdx.x];
+    const long item = linear_block();
+    if (item >= a.nitems) return;   // whole work-group, before any barrier
+    const refine_item it = a.items[item];
     const refine_cand cd = a.cands[it.cand];
     const int tid = threadIdx.x, T = cd.T, C = it.nc, t_first = it.seg * kSeg;
     const int nt = min(kSeg, T - t_first);
@@ -293,7 +297,9 @@ __device__ __forceinline__ void noise_part(const refine_args& a, const refine_ca
 __global__ __launch_bounds__(kCombineThreads) void refine_scan_loss_kernel(refine_args a, int k0)
 {
     __shared__ double red[kCombineThreads / 64];
-    const int b = blockIdx.x, k = blockIdx.y, tid = threadIdx.x;
+    const long b = linear_block();
+    if (b >= a.ncand) return;   // whole work-group, before any barrier
+    const int k = blockIdx.y, tid = threadIdx.x;
     const refine_cand cd = a.cands[b];
     const int row = cd.T + (cd.T - 1) / kSeg, nchunk = (cd.C + kChunk - 1) / kChunk;
     const double* part = a.part + cd.part_off + (size_t)k * row;
@@ -333,7 +339,9 @@ __global__ void refine_start_kernel(refine_args a, int k0, int nk)
 __global__ __launch_bounds__(kCombineThreads) void refine_combine_kernel(refine_args a, int last)
 {
     __shared__ double red[kCombineThreads / 64];
-    const int b = blockIdx.x, tid = threadIdx.x;
+    const long b = linear_block();
+    if (b >= a.ncand) return;   // whole work-group, before any barrier
+    const int tid = threadIdx.x;
     const refine_cand cd = a.cands[b];
     const int row = cd.T + (cd.T - 1) / kSeg, nchunk = (cd.C + kChunk - 1) / kChunk;
     const double* part = a.part + cd.part_off;
@@ -412,20 +420,23 @@ hipError_t launch_refine(const refine_args& a, hipStream_t s)
 {
     if (a.ncand <= 0) return hipSuccess;
     if (a.nitems <= 0 || (a.loss_kind != 0 && a.loss_kind != 1)) return hipErrorInvalidValue;
-    const unsigned n = (unsigned)a.ncand, ni = (unsigned)a.nitems;
+    const unsigned n = (unsigned)a.ncand;
+    const dim3 items = linear_grid(a.nitems, kThreads);
     if (a.loss_kind == 1)
         hipLaunchKernelGGL(refine_power_kernel, dim3(n, kPowerBlocksY), dim3(256), 0, s, a);
     for (int k0 = 0; k0 == 0 || k0 < a.scan_n; k0 += kScan) {
         const int nk = a.scan_n - k0 < kScan ? a.scan_n - k0 : kScan;
         if (nk > 0) {
-            hipLaunchKernelGGL(refine_partial_kernel<kScan>, dim3(ni), dim3(kThreads), 0, s, a, k0, nk);
-            hipLaunchKernelGGL(refine_scan_loss_kernel, dim3(n, (unsigned)nk), dim3(kCombineThreads), 0, s, a, k0);
+            hipLaunchKernelGGL(refine_partial_kernel<kScan>, items, dim3(kThreads), 0, s, a, k0, nk);
+            hipLaunchKernelGGL(refine_scan_loss_kernel, linear_grid(a.ncand, kCombineThreads, nk),
+                               dim3(kCombineThreads), 0, s, a, k0);
         }
         hipLaunchKernelGGL(refine_start_kernel, dim3((n + 63) / 64), dim3(64), 0, s, a, k0, nk);
     }
     for (int i = 0; i <= a.nsteps; ++i) {
-        hipLaunchKernelGGL(refine_partial_kernel<0>, dim3(ni), dim3(kThreads), 0, s, a, 0, 0);
-        hipLaunchKernelGGL(refine_combine_kernel, dim3(n), dim3(kCombineThreads), 0, s, a, i == a.nsteps ? 1 : 0);
+        hipLaunchKernelGGL(refine_partial_kernel<0>, items, dim3(kThreads), 0, s, a, 0, 0);
+        hipLaunchKernelGGL(refine_combine_kernel, linear_grid(a.ncand, kCombineThreads), dim3(kCombineThreads), 0, s, a,
+                           i == a.nsteps ? 1 : 0);
     }
     return hipGetLastError();
 }

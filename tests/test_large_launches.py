@@ -23,3 +23,31 @@ plan.run_range(0, tp, out)
 names = fake.kernels()
 assert len(names) == 1 and "dedisperse_rows_kernel" in names[0], names
 ''', tmp_path)
+
+
+def test_output_normalisation_of_a_long_plane(tmp_path):
+    """600 million columns."""
+    host_library.run('''
+fake.kernels()
+for rows in (3, 2000):
+    aa.check(aa.load_library().aa_hip_output_ddtr_normalization(Tensor((1, 1)).data_ptr(), rows, 600000001, None))
+    assert len(fake.kernels()) == 1
+''', tmp_path)
+
+
+def test_refinement_of_many_windows(tmp_path):
+    """Five million windows of one channel and eight samples, energy loss."""
+    host_library.run('''
+n = 5000000
+lib = aa.load_library()
+i64, i32 = ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int)
+xo, do = np.arange(n, dtype=np.int64) * 8, np.zeros(n, dtype=np.int64)
+nc, ns = np.full(n, 1, dtype=np.int32), np.full(n, 8, dtype=np.int32)
+h = ctypes.c_void_p()
+aa.check(lib.aa_hip_refine_create(0, n, xo.ctypes.data_as(i64), do.ctypes.data_as(i64), nc.ctypes.data_as(i32),
+                                  ns.ctypes.data_as(i32), ctypes.byref(h)))
+p = Tensor((1, 1)).data_ptr()   # never read: no kernel runs
+fake.kernels()
+aa.check(lib.aa_hip_refine_run(h, p, p, p, p, p, p, p, 3, -1.0, 0.5, 2, 0.5, 1e-4, None))
+assert len(fake.kernels()) == 3 + 2 * 3      # a scan pass and three evaluations
+''', tmp_path)
