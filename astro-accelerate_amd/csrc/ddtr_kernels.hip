@@ -651,10 +651,15 @@ hipError_t launch_corner_turn_levels(const void* in_tc, int sample_bytes, long n
     }
     const bool aligned = ct_wide_fits(in_tc, nchans, ptrs, pitches, nlev);
     if (!aligned && !any_fused) nlev = 0;
-    // The byte kernel keeps what the wide one cannot store, and level 0 alone
-    // of a few tiles (5000 samples x 65 channels: 9.0 us against 11.6).
+    // The byte kernel keeps what the wide one cannot store, and level 0 alone of
+    // unaligned rows in few tiles, each of which takes 8 to 11 us: u8 1000 x 4000
+    // samples (32 tiles) 7.3 us against 9.1 on the wide path, 2001 x 500 (16 tiles)
+    // 7.0 against 11.0, 40 x 100,000 (98 part-filled tiles) 7.3 against 8.0; 500 x
+    // 24,000 (96 tiles) 15.3 against 11.3.  With binned levels the wide path wins
+    // at every size (17 x 500 to 4097 x 24,000: 0.23 to 0.82 of the time).
+    const bool few = corner_turn_tiles(nsamp, nchans) <= 64 || nsamp * nchans < 6L << 20;
     if (!ct_rows_fit(ptrs, pitches, nlev) || (uintptr_t)in_tc % (uintptr_t)sample_bytes != 0 ||
-        (!aligned && nlev == 0 && corner_turn_tiles(nsamp, nchans) < 16)) {
+        (!aligned && nlev == 0 && few)) {
         const dim3 grid(ceil_div(nsamp, kTile), ceil_div(nchans, kTile));
         if (sample_bytes == 1)
             hipLaunchKernelGGL(corner_turn_kernel<uint8_t>, grid, dim3(256), 0, s, (const uint8_t*)in_tc, (int)nsamp,

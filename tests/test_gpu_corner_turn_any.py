@@ -7,7 +7,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nsamp,nchans", [(16384, 1), (16385, 15), (17000, 33), (2049, 1003), (16400, 127), (8193, 257)])
+@pytest.mark.parametrize("nsamp,nchans", [(16384, 1), (16385, 15), (17000, 33), (2049, 1003), (16400, 127), (8193, 257),
+                                          (66561, 100), (33001, 257), (8195, 1003)])   # the wide path
 @pytest.mark.parametrize("sample_bytes,offset", [(1, 0), (1, 1), (1, 2), (1, 3), (2, 0), (2, 2)])
 def test_turn(aa, oracle, cuda, nsamp, nchans, sample_bytes, offset):
     """offset: bytes from an aligned address.  The samples around the chunk

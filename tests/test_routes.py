@@ -238,3 +238,25 @@ assert "normalize_columns_f32x4_kernel" in kernel(6080, 40960)
 for rows, cols, at in ((6080, 40956, plane), (1537, 222657, plane), (1537, 222656, plane + 4)):
     assert "normalize_columns_kernel" in kernel(rows, cols, at)
 ''', tmp_path)
+
+
+def test_level_0_of_unaligned_rows(tmp_path):
+    """The wide corner turn where it has tiles enough; the byte kernel for less,
+    and the wide one at any size where binned levels follow or rows are aligned."""
+    host_library.run('''
+at = Tensor((1, 1)).data_ptr()
+def kernel(nsamp, nchans, levels=1):
+    fake.kernels()
+    pitch = (nsamp + 255) // 256 * 256
+    aa.corner_turn_levels(Tensor((1, 1)), 1, nsamp, nchans, [Tensor((1, 1))] * levels, [pitch] * levels)
+    return fake.kernels()[0]
+for nsamp, nchans in ((500, 2001), (4000, 1000), (100000, 40), (24000, 200), (8000, 1000)):
+    assert "18corner_turn_kernel" in kernel(nsamp, nchans), (nsamp, nchans)
+for nsamp, nchans in ((24000, 500), (100000, 65), (4000, 4097), (500, 2000), (200, 16)):
+    assert "corner_turn_wide_kernel" in kernel(nsamp, nchans), (nsamp, nchans)
+ds = np.linspace(0, 1e-3, 99).astype(np.float32)
+plan = aa.DdtrPlan(ds, [(0.0, 0.5, 16, 1), (8.0, 1.0, 16, 2)], 64e-6, 400, 1400)
+fake.kernels()
+plan.ingest(Tensor((1800, 99), 1), 1400)
+assert fake.ran("corner_turn_wide_kernel")
+''', tmp_path)
