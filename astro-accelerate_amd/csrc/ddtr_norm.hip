@@ -243,6 +243,19 @@ __device__ __forceinline__ lane_rows rows_of_lane(long i, long r0, long r1, long
     return lane_rows{(int)((r1 - r0) / 32), ((r1 - r0) % 32) * cols - 16 * i};
 }
 
+// The last 1 to 15 bytes of a lane, zero past them; all loads go out together
+// (a loop of loads took 5 us of a 30 us call of one row).
+__device__ __forceinline__ u32x4 tail_bytes(const uint8_t* d, int tail)
+{
+    uint32_t v[16];
+#pragma unroll
+    for (int b = 0; b < 16; ++b) v[b] = d[b < tail ? b : tail - 1];
+    u32x4 x = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int b = 0; b < 16; ++b) x[b >> 2] |= b < tail ? v[b] << (8 * (b & 3)) : 0u;
+    return x;
+}
+
 // Integer partial sums of one row segment of u8 data: lanes numbered through
 // the bytes of 32 consecutive rows, 16 bytes each (32 rows are a whole number
 // of them at any column count; a lane's bytes may cross rows), so that every
@@ -257,6 +270,7 @@ __global__ __launch_bounds__(256) void norm_partial_u8_kernel(const uint8_t* dat
     const long i0 = (long)blockIdx.x * 256, i = i0 + threadIdx.x;
     const long r0 = (long)blockIdx.y * seg_rows;
     const long r1 = rows < r0 + seg_rows ? rows : r0 + seg_rows;
+    if (16 * i0 >= (r1 - r0) * cols) return;   // whole work-group: fewer than 32 rows, none of them its
     uint32_t even[4] = {0u, 0u, 0u, 0u}, odd[4] = {0u, 0u, 0u, 0u};
     auto add = [&](u32x4 x) {
 #pragma unroll
@@ -273,14 +287,8 @@ __global__ __launch_bounds__(256) void norm_partial_u8_kernel(const uint8_t* dat
         d += (long)n.blocks * 32 * cols;
         if (n.tail >= 16) {
             add(*reinterpret_cast<const u32x4u*>(d));
-        } else {
-            for (int b = 0; b < (int)n.tail; ++b) {
-                u32x4 x = {0u, 0u, 0u, 0u};
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (j == b >> 2) x[j] = (uint32_t)d[b] << (8 * (b & 3));
-                add(x);
-            }
+        } else if (n.tail > 0) {
+            add(tail_bytes(d, (int)n.tail));
         }
     }
 #pragma unroll
@@ -352,6 +360,7 @@ __global__ __launch_bounds__(256) void norm_apply_u8_kernel(uint8_t* data, long 
     const long r0 = (long)blockIdx.y * seg_rows;
     const long r1 = rows < r0 + seg_rows ? rows : r0 + seg_rows;
     const lane_rows n = rows_of_lane(i, r0, r1, cols);
+    if (n.blocks == 0 && n.tail <= 0) return;
     uint8_t* d = data + r0 * cols + 16 * i;
     float s[16];
     long c = 16 * i % cols;
@@ -379,10 +388,11 @@ __global__ __launch_bounds__(256) void norm_apply_u8_kernel(uint8_t* data, long 
         *reinterpret_cast<u32x4u*>(d) = apply(*reinterpret_cast<const u32x4u*>(d));
     if (n.tail >= 16) {
         *reinterpret_cast<u32x4u*>(d) = apply(*reinterpret_cast<const u32x4u*>(d));
-    } else {
+    } else if (n.tail > 0) {
+        const u32x4 x = apply(tail_bytes(d, (int)n.tail));
 #pragma unroll
-        for (int b = 0; b < 16; ++b)
-            if (b < n.tail) d[b] = (uint8_t)norm_value((float)d[b], s[b], maxval);
+        for (int b = 0; b < 15; ++b)
+            if (b < n.tail) d[b] = (uint8_t)(x[b >> 2] >> (8 * (b & 3)));
     }
 }
 
@@ -497,14 +507,18 @@ hipError_t launch_normalize_columns_f32(float* data, long rows, long cols, float
     // Strips of 64 columns, or of 16 where those would be fewer than 64: 1152 x
     // 3117 floats 34 us with 49 strips and 20 with 195, 1536 x 3000 46 and 20;
     // above, the longer row segments win (512 x 8000 7.4 us against 16.8).
-    if (rows <= kStripMaxRows)
+    // Of up to 4 rows most of a strip's threads have none: 1 x 500,000 9.9 us by
+    // columns of 4 against 11.2, 4 x 500,000 11.0 against 11.9; 6 rows 12.8
+    // against 12.4.
+    const bool columns4 = cols % 4 == 0 && (uintptr_t)data % 16 == 0 && cols >= 160 * 256;
+    if (rows <= kStripMaxRows && !(rows <= 4 && columns4))
         return cols >= 64 * 64 ? launch_strips<16>(data, rows, cols, factor, s)
                                : launch_strips<4>(data, rows, cols, factor, s);
     // Taller planes are read twice, 4 columns per lane where that leaves enough
     // workgroups of 256 columns: 1600 x 50,000 177 us against 218 with one column
     // per lane, 6080 x 111,328 1.68 ms against 1.86; 3072 x 32,768 256 us against
     // 244, 1600 x 20,000 65 against 62.
-    if (cols % 4 == 0 && (uintptr_t)data % 16 == 0 && cols >= 160 * 256)
+    if (columns4)
         hipLaunchKernelGGL(normalize_columns_f32x4_kernel, linear_grid((cols / 4 + 63) / 64, 1024), dim3(1024), 0, s,
                            data, rows, cols, factor);
     else

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 PLANES = [(r, c) for r, c in [(1, 64), (31, 3), (32, 128), (33, 65), (128, 66), (129, 127), (256, 191), (257, 64),
                               (512, 130), (513, 61), (1024, 190), (1025, 129), (1535, 63), (1536, 257), (1537, 70),
                               (65, 4095), (65, 4096), (1100, 4131), (700, 16391),
-                              (1537, 40960), (1601, 41003)]]   # 4 columns per lane, where words are aligned
+                              (1537, 40960), (1601, 41003), (4, 40964)]]   # 4 columns per lane, where words are aligned
 
 
 @pytest.mark.parametrize("ndms,nsamp", PLANES)

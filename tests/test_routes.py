@@ -224,8 +224,8 @@ assert fake.ran("dedisperse_matrix_kernel")
 
 
 def test_output_normalisation_of_tall_planes(tmp_path):
-    """Planes of more rows than a strip keeps in registers: 4 columns per lane
-    where the plane is wide and its words are aligned."""
+    """Planes of more rows than a strip keeps in registers, or of next to none: 4
+    columns per lane where the plane is wide and its words are aligned."""
     host_library.run('''
 plane = Tensor((1, 1)).data_ptr()
 def kernel(rows, cols, at=plane):
@@ -233,6 +233,10 @@ def kernel(rows, cols, at=plane):
     aa.check(aa.load_library().aa_hip_output_ddtr_normalization(at, rows, cols, None))
     return fake.kernels()[0]
 assert "normalize_strip_f32_kernel" in kernel(1536, 222656)
+assert "normalize_strip_f32_kernel" in kernel(5, 222656)
+assert "normalize_strip_f32_kernel" in kernel(4, 222657)
+assert "normalize_strip_f32_kernel" in kernel(4, 4096)
+assert "normalize_columns_f32x4_kernel" in kernel(4, 222656)
 assert "normalize_columns_f32x4_kernel" in kernel(1537, 222656)
 assert "normalize_columns_f32x4_kernel" in kernel(6080, 40960)
 for rows, cols, at in ((6080, 40956, plane), (1537, 222657, plane), (1537, 222656, plane + 4)):
