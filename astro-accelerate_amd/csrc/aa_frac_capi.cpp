@@ -32,6 +32,7 @@ struct aa_hip_refine {
     int device = 0;
     int ncand = 0;
     int nitems = 0;
+    int chunk = 0;
     int loss_kind = 0;
     aa_hip::refine_cand* d_cands = nullptr;
     aa_hip::refine_item* d_items = nullptr;
@@ -301,6 +302,7 @@ int aa_hip_refine_create(int device, int ncand, const int64_t* x_offsets, const 
     std::vector<aa_hip::refine_cand> cands((size_t)ncand);
     int64_t power_entries = 0, part_entries = 0;
     std::vector<aa_hip::refine_item> items;
+    const int chunk = aa_hip::refine_chunk(ncand, nchans, nsamp);
     for (int b = 0; b < ncand; ++b) {
         if (nchans[b] <= 0 || nchans[b] > aa_hip::kRefineMaxChannels || nsamp[b] <= 0 ||
             nsamp[b] > aa_hip::kRefineMaxSamples || x_offsets[b] < 0 || ds_offsets[b] < 0)
@@ -311,11 +313,10 @@ int aa_hip_refine_create(int device, int ncand, const int64_t* x_offsets, const 
         cands[(size_t)b] =
             aa_hip::refine_cand{x_offsets[b], ds_offsets[b], power_entries, part_entries, nchans[b], nsamp[b]};
         power_entries += nchans[b];
-        part_entries += aa_hip::refine_part_entries(nchans[b], nsamp[b]);
-        for (int c = 0; c < nchans[b]; c += aa_hip::kRefineChunk)
+        part_entries += aa_hip::refine_part_entries(nchans[b], nsamp[b], chunk);
+        for (int c = 0; c < nchans[b]; c += chunk)
             for (int g = 0; g * aa_hip::kRefineSeg < nsamp[b]; ++g)
-                items.push_back(aa_hip::refine_item{b, c / aa_hip::kRefineChunk, c,
-                                                    std::min(aa_hip::kRefineChunk, nchans[b] - c), g});
+                items.push_back(aa_hip::refine_item{b, c / chunk, c, std::min(chunk, nchans[b] - c), g});
     }
     if (items.size() > 0x7fffffffu) return fail(AA_HIP_ERROR_UNSUPPORTED, "too many windows");
     // longest items first: the tail is made of short ones
@@ -336,6 +337,7 @@ int aa_hip_refine_create(int device, int ncand, const int64_t* x_offsets, const 
     (void)hipGetDevice(&cur);
     hipError_t e = hipSetDevice(device);
     p->nitems = (int)items.size();
+    p->chunk = chunk;
     if (e == hipSuccess) e = hipMalloc(&p->d_cands, sizeof(aa_hip::refine_cand) * (size_t)ncand);
     if (e == hipSuccess) e = hipMalloc(&p->d_items, sizeof(aa_hip::refine_item) * items.size());
     if (e == hipSuccess) e = hipMalloc(&p->d_state, sizeof(aa_hip::refine_state) * (size_t)ncand);
@@ -391,6 +393,7 @@ int aa_hip_refine_run(aa_hip_refine* h, const float* d_x, const float* d_delay_p
     a.items = h->d_items;
     a.ncand = h->ncand;
     a.nitems = h->nitems;
+    a.chunk = h->chunk;
     a.u = d_u;
     a.step = d_step;
     a.prev_grad = d_prev_grad;

@@ -10,7 +10,8 @@ constexpr int kRefineMaxSamples = 4096;    // per window
 constexpr int kRefineMaxChannels = 4096;   // per window
 constexpr int kRefineThreads = 256;
 constexpr int kRefineSeg = 1024;           // samples of an item
-constexpr int kRefineChunk = 256;          // channels of an item
+constexpr int kRefineChunk = 256;          // channels of an item at most
+constexpr int kRefineChunkMin = 16;        // (a plan's own number: refine_chunk)
 constexpr int kRefineScan = 3;             // scan points of a pass
 
 struct refine_cand {
@@ -21,18 +22,23 @@ struct refine_cand {
     int C, T;
 };
 
-// Part of one window: channels c0 .. c0 + nc - 1 (chunk number c0 /
-// kRefineChunk), samples seg * kRefineSeg on.
+// Part of one window: channels c0 .. c0 + nc - 1 (chunk number c0 / the plan's
+// chunk), samples seg * kRefineSeg on.
 struct refine_item {
     int cand, chunk, c0, nc, seg;
 };
 
 // Partial profiles of one window: a chunk holds up to kRefineScan rows of
 // T + (T - 1) / kRefineSeg entries.
-inline int64_t refine_part_entries(int C, int T)
+inline int64_t refine_part_entries(int C, int T, int chunk)
 {
-    return (int64_t)((C + kRefineChunk - 1) / kRefineChunk) * kRefineScan * (T + (T - 1) / kRefineSeg);
+    return (int64_t)((C + chunk - 1) / chunk) * kRefineScan * (T + (T - 1) / kRefineSeg);
 }
+
+// Channels per item for a plan's windows: kRefineChunk, halved while the items
+// are fewer than four per CU and an item's channels (each lane's serial loop)
+// still outweigh the chunks that the combine pass then adds.
+int refine_chunk(int ncand, const int* nchans, const int* nsamp);
 
 // A candidate between evaluations.
 struct refine_state {
@@ -46,6 +52,7 @@ struct refine_args {
     const refine_cand* cands;   // [ncand]
     const refine_item* items;   // [nitems], longest first
     int ncand, nitems;
+    int chunk;                  // channels of an item
     float* u;                   // [ncand] residual DM, updated in place
     float* step;                // [ncand] Rprop step, updated in place
     double* prev_grad;          // [ncand] previous dL/du, updated in place

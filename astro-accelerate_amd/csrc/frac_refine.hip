@@ -29,9 +29,9 @@
 // dy/du together and dE/du = 2 sum_t y dy/du follows from them.  The scan's
 // points (kScan at a time) share one pass too.
 //
-// Work split: an item is up to kChunk channels x kSeg samples of one window, a
-// 256-thread work-group each, so that windows of any number and size spread
-// over the whole GPU.  A group of S lanes covers the item's samples, 4
+// Work split: an item is up to kChunk channels (fewer where the windows are few,
+// refine_chunk) x kSeg samples of one window, a 256-thread work-group each, so
+// that windows of any number and size spread over the whole GPU.  A group of S lanes covers the item's samples, 4
 // consecutive ones per lane, and the work-group holds G = 256 / S such groups,
 // each summing every G-th channel.  A lane reads its 4 samples x[c][t0 + i_c ..
 // t0 + i_c + 3] as one 16-byte load; the second tap of the sample before them
@@ -301,7 +301,7 @@ __global__ __launch_bounds__(kCombineThreads) void refine_scan_loss_kernel(refin
     if (b >= a.ncand) return;   // whole work-group, before any barrier
     const int k = blockIdx.y, tid = threadIdx.x;
     const refine_cand cd = a.cands[b];
-    const int row = cd.T + (cd.T - 1) / kSeg, nchunk = (cd.C + kChunk - 1) / kChunk;
+    const int row = cd.T + (cd.T - 1) / kSeg, nchunk = (cd.C + a.chunk - 1) / a.chunk;
     const double* part = a.part + cd.part_off + (size_t)k * row;
     double l2 = 0.0, n, dn;
     for (int t = tid; t < cd.T; t += kCombineThreads) {
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(kCombineThreads) void refine_combine_kernel(refine_
     if (b >= a.ncand) return;   // whole work-group, before any barrier
     const int tid = threadIdx.x;
     const refine_cand cd = a.cands[b];
-    const int row = cd.T + (cd.T - 1) / kSeg, nchunk = (cd.C + kChunk - 1) / kChunk;
+    const int row = cd.T + (cd.T - 1) / kSeg, nchunk = (cd.C + a.chunk - 1) / a.chunk;
     const double* part = a.part + cd.part_off;
     refine_state st = a.cur[b];
     double l2 = 0.0, gs = 0.0, n, dn;
@@ -416,10 +416,24 @@ __global__ __launch_bounds__(256) void refine_power_kernel(refine_args a)
 
 }  // namespace
 
+int refine_chunk(int ncand, const int* nchans, const int* nsamp)
+{
+    int chunk = kChunk, most = 0;
+    for (int b = 0; b < ncand; ++b) most = nchans[b] > most ? nchans[b] : most;
+    auto items = [&] {
+        long n = 0;
+        for (int b = 0; b < ncand && n < 1024; ++b)
+            n += (long)((nchans[b] + chunk - 1) / chunk) * ((nsamp[b] + kSeg - 1) / kSeg);
+        return n;
+    };
+    while (chunk > kRefineChunkMin && chunk * chunk > 2 * most && items() < 1024) chunk /= 2;
+    return chunk;
+}
+
 hipError_t launch_refine(const refine_args& a, hipStream_t s)
 {
     if (a.ncand <= 0) return hipSuccess;
-    if (a.nitems <= 0 || (a.loss_kind != 0 && a.loss_kind != 1)) return hipErrorInvalidValue;
+    if (a.nitems <= 0 || a.chunk < 1 || a.chunk > kChunk || (a.loss_kind != 0 && a.loss_kind != 1)) return hipErrorInvalidValue;
     const unsigned n = (unsigned)a.ncand;
     const dim3 items = linear_grid(a.nitems, kThreads);
     if (a.loss_kind == 1)

@@ -1,6 +1,7 @@
 """Batched refinement at the edges of its work split: windows whose samples end
 just before, at and after a segment (1024 samples), whose channels end around
-a chunk (256), and scans whose points end around a pass (3 points)."""
+a chunk (32 for these windows alone, 256 for a plan of many), and scans whose
+points end around a pass (3 points)."""
 import numpy as np
 import pytest
 
@@ -32,21 +33,25 @@ def _state(n, cuda, u):
     return u.clone(), torch.full((n,), 0.1, device=cuda), torch.zeros(n, **z), torch.empty(n, **z), torch.empty(n, **z)
 
 
+@pytest.mark.parametrize("copies", [1, 60])
 @pytest.mark.parametrize("loss_kind", ["energy", "excess"])
-def test_evaluation_at_split_edges(cuda, loss_kind):
+def test_evaluation_at_split_edges(cuda, loss_kind, copies):
     """Loss and gradient against the float64 reference; the kernels round the
     interpolation weight to float32 (6e-8), so 1e-5 of the terms' size."""
     import torch
     import frac_ddtr
     x, ds, off, ds_off, tables = _windows(cuda, 3)
-    n = len(WINDOWS)
-    plan = frac_ddtr.RefinePlan([w[0] for w in WINDOWS], [w[1] for w in WINDOWS], off, ds_off, loss=loss_kind)
+    n = len(WINDOWS) * copies
+    plan = frac_ddtr.RefinePlan([w[0] for w in WINDOWS] * copies, [w[1] for w in WINDOWS] * copies, off * copies,
+                                ds_off * copies, loss=loss_kind)
     for u_val in (0.0, 0.37, -0.81):
         print(f"refine split edges {loss_kind} u={u_val}", flush=True)
         u0 = torch.full((n,), u_val, device=cuda)
         u, step, prev, loss, grad = _state(n, cuda, u0)
         plan.run(x, ds, u, step, prev, loss, grad, nsteps=0)
         torch.cuda.synchronize()
+        for v in (loss, grad):   # the copies agree
+            assert torch.equal(v.view(copies, -1), v[:len(WINDOWS)].expand(copies, -1))
         for b, (C, T) in enumerate(WINDOWS):
             w = x[off[b]:off[b] + C * T].view(1, C, T).double()
             ub = u0[b:b + 1].double().requires_grad_(True)

@@ -264,3 +264,25 @@ fake.kernels()
 plan.ingest(Tensor((1800, 99), 1), 1400)
 assert fake.ran("corner_turn_wide_kernel")
 ''', tmp_path)
+
+
+def test_refinement_items(tmp_path):
+    """Few windows are split into smaller items; many keep 256 channels each."""
+    host_library.run('''
+import frac_ddtr
+def items(n, C, T):
+    plan = frac_ddtr.RefinePlan([C] * n, [T] * n, [0] * n, [0] * n, loss="energy")
+    p, h = Tensor((1, 1)).data_ptr(), plan.handle
+    fake.kernels()
+    aa.check(aa.load_library().aa_hip_refine_run(h, p, p, p, p, p, p, p, 0, 0.0, 0.0, 0, 0.5, 1e-4, None))
+    return [fake.lib.fake_launch_grid(i) for i in range(fake.lib.fake_launches())
+            if b"refine_partial" in fake.lib.fake_launch_name(i)][0]
+assert items(1, 64, 64) == 4
+assert items(32, 256, 256) == 32 * 16
+assert items(64, 256, 256) == 64 * 16
+assert items(256, 256, 256) == 256 * 4
+assert items(1, 4096, 1024) == 64
+assert items(16, 4096, 2048) == 16 * 2 * 32
+assert items(100, 4096, 1024) == 100 * 16
+assert items(5000, 16, 2000) == 5000 * 2
+''', tmp_path)
