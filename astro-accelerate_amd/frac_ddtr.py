@@ -71,6 +71,7 @@ class FracPlan:
                                         self.trials.ctypes.data_as(aa.PFLOAT), self.nsamp, self.max_batch,
                                         float(dm_absmax), ctypes.byref(h)), "aa_hip_frac_create")
         self.handle = h
+        self._work_bytes = {}   # batch -> scratch bytes of (forward, adjoint)
 
     def grouping(self):
         tq, cq = ctypes.c_int(), ctypes.c_int()
@@ -109,10 +110,13 @@ class FracPlan:
     def _work(self, b: int, device, adjoint: bool):
         """Scratch memory of one call (a tensor of the current stream) and its bytes."""
         import torch
-        fwd, adj = ctypes.c_size_t(), ctypes.c_size_t()
-        aa.check(aa.load_library().aa_hip_frac_workspace_bytes(self.handle, b, ctypes.byref(fwd), ctypes.byref(adj)),
-                 "aa_hip_frac_workspace_bytes")
-        n = adj.value if adjoint else fwd.value
+        n = self._work_bytes.get(b)
+        if n is None:
+            fwd, adj = ctypes.c_size_t(), ctypes.c_size_t()
+            aa.check(aa.load_library().aa_hip_frac_workspace_bytes(self.handle, b, ctypes.byref(fwd),
+                                                                   ctypes.byref(adj)), "aa_hip_frac_workspace_bytes")
+            n = self._work_bytes[b] = (fwd.value, adj.value)
+        n = n[adjoint]
         return (torch.empty(n, dtype=torch.uint8, device=device) if n else None), n
 
     def forward(self, x, dm, out=None):
@@ -124,11 +128,9 @@ class FracPlan:
                                                     device=x.device)
         self._check_x(y, "out")
         work, n = self._work(b, x.device, adjoint=False)
-        aa.check(aa.load_library().aa_hip_frac_forward_ws(self.handle, ctypes.c_void_p(x.data_ptr()), b,
-                                                          ctypes.c_void_p(dm.data_ptr()),
-                                                          ctypes.c_void_p(y.data_ptr()),
-                                                          ctypes.c_void_p(work.data_ptr() if n else 0), n,
-                                                          _stream_handle()), "aa_hip_frac_forward")
+        aa.check(aa.load_library().aa_hip_frac_forward_ws(self.handle, x.data_ptr(), b, dm.data_ptr(), y.data_ptr(),
+                                                          work.data_ptr() if n else None, n, _stream_handle()),
+                 "aa_hip_frac_forward")
         return y
 
     def adjoint(self, x, gy, dm, want_x: bool = True, want_dm: bool = True):
@@ -144,10 +146,9 @@ class FracPlan:
                 raise ValueError("x does not match gy")
         work, n = self._work(b, gy.device, adjoint=True) if want_dm else (None, 0)
         aa.check(aa.load_library().aa_hip_frac_adjoint_ws(
-            self.handle, ctypes.c_void_p(x.data_ptr() if x is not None else 0), ctypes.c_void_p(gy.data_ptr()), b,
-            ctypes.c_void_p(dm.data_ptr()), ctypes.c_void_p(gx.data_ptr() if gx is not None else 0),
-            ctypes.c_void_p(gdm.data_ptr() if gdm is not None else 0), ctypes.c_void_p(work.data_ptr() if n else 0), n,
-            _stream_handle()), "aa_hip_frac_adjoint")
+            self.handle, x.data_ptr() if x is not None else None, gy.data_ptr(), b, dm.data_ptr(),
+            gx.data_ptr() if gx is not None else None, gdm.data_ptr() if gdm is not None else None,
+            work.data_ptr() if n else None, n, _stream_handle()), "aa_hip_frac_adjoint")
         return gx, gdm
 
 
