@@ -530,10 +530,16 @@ bool ddtr_engine::u16_matrix(int r, hipStream_t s) {
     if (m_sample_bytes != 2 || (m_kernel != AA_HIP_KERNEL_AUTO && m_kernel != AA_HIP_KERNEL_MATRIX) ||
         u16_window(r) <= 0)
         return false;
-    const level &lv = m_levels[(size_t)log2i(m_ranges[(size_t)r].inBin)];
+    const bool forced = m_kernel == AA_HIP_KERNEL_MATRIX;
+    if (!forced && m_nchans < kU16MatrixMinChannels) return false;
+    const range_desc &rd = m_ranges[(size_t)r];
+    const level &lv = m_levels[(size_t)log2i(rd.inBin)];
     (void)plan_matrix(r, round_up((size_t)lv.capacity + kRowPad, kPitchAlign), 2, s);
     matrix_tables &mt = m_matrix[(size_t)r];
-    if (mt.lay.tile_out <= 0 || mt.flags) return mt.lay.tile_out > 0;
+    // The chunk's length decides, not the call's: its planes are made at ingest.
+    if (mt.lay.tile_out <= 0 || !(forced || matrix_beats_u16(m_nchans, lv.len - m_maxshift / rd.inBin, mt.lay)))
+        return false;
+    if (mt.flags) return true;
     const size_t tiles =
         (size_t)mt.lay.n_dm_tiles * (size_t)((lv.capacity + mt.lay.tile_out - 1) / mt.lay.tile_out) * sizeof(int);
     if (hipMalloc(&mt.flags, tiles) != hipSuccess) {

@@ -37,6 +37,11 @@ inline long matrix_tiles_at_most(int ndms, int t_processed)
 matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float mstartdm, float mdmstep, size_t pitch,
                           std::vector<uint8_t>* bytes, int planes = 1);
 
+// Whether a 16-bit range of t samples is done sooner by the matrix kernel over
+// byte planes (this layout) than by dedisperse_u16.
+constexpr int kU16MatrixMinChannels = 24;
+bool matrix_beats_u16(int nchans, long t, const matrix_layout& lay);
+
 // p.pair_recs: the tables on the device.  planes 2: the sums are integers; a
 // tile with a sum above 2^24, where the reference's float adds round, sets its
 // entry of flags (n_dm_tiles x time tiles, time tile major; else 0) and has to

@@ -627,6 +627,26 @@ matrix_layout matrix_plan(const float* h_dmshifts, int nchans, int ndms, float m
     return lay;
 }
 
+// Time model in us, fitted on 800 ranges of 8 to 2000 channels, 1 to 1000 trials
+// of fine and coarse steps, 200 to 200,000 samples (both kernels with all their
+// passes, 12 % standard error each): the matrix kernel's tiles one per CU, 12 us
+// to start and end one and 0.86 per step, after the byte planes are made;
+// dedisperse_u16's tiles of 512 samples about two per CU, 0.79 us per channel.
+// With it no range of those is more than 7 % slower than by the other kernel;
+// without, 40 channels x 1000 trials 2 DM units apart x 200,000 samples took 2.38
+// ms in place of 1.61, 16 x 64 x 4000 39 us in place of 21.  Below 24 channels the
+// matrix kernel gains 5 % at most.
+bool matrix_beats_u16(int nchans, long t, const matrix_layout& lay)
+{
+    if (nchans < kU16MatrixMinChannels || lay.tile_out <= 0 || t <= 0) return false;
+    const double tiles = (double)lay.n_dm_tiles * (double)((t + lay.tile_out - 1) / lay.tile_out) / 256.0;
+    const double rounds = tiles <= 1.0 ? 1.0 : tiles < 2.0 ? 2.0 : tiles;
+    const double matrix = 4.0 + rounds * (12.0 + 0.86 * lay.tile_cost) + 1.75e-6 * nchans * t;
+    const double u16_tiles = (double)lay.n_dm_tiles * (double)((t + 511) / 512) / (1.9 * 256.0);
+    const double u16 = 8.0 + std::max(1.0, u16_tiles) * 0.79 * nchans + 1.9e-6 * nchans * t;
+    return matrix < u16;
+}
+
 hipError_t launch_dedisperse_matrix(const lds_params& p, const matrix_layout& lay, hipStream_t s, const int* over,
                                     int* flags, int t_flags)
 {

@@ -286,3 +286,25 @@ assert items(16, 4096, 2048) == 16 * 2 * 32
 assert items(100, 4096, 1024) == 100 * 16
 assert items(5000, 16, 2000) == 5000 * 2
 ''', tmp_path)
+
+
+def test_16_bit_ranges_on_the_faster_kernel(tmp_path):
+    """Few channels, or trials far apart, keep dedisperse_u16, and no byte planes
+    are made for them."""
+    host_library.run('''
+import ddtr_oracle as oracle
+def kernels(nchans, ndms, tp, step, kernel=0):
+    ds = oracle.dmshifts(nchans, 1500.0, -300.0 / nchans)
+    shift = int(ds[-1] * step * ndms / 64e-6) + 16
+    plan = aa.DdtrPlan(ds, [(0.0, step, ndms, 1)], 64e-6, shift, tp, sample_bits=16)
+    plan.set_kernel(kernel)
+    fake.kernels()
+    plan.execute_chunk(Tensor((tp + shift, nchans), 2), [tp], [Tensor((ndms, tp))])
+    return " ".join(fake.kernels())
+for case in ((16, 64, 4000, 0.5), (40, 1000, 200000, 2.0), (56, 64, 16000, 2.0), (32, 16, 200, 0.5)):
+    names = kernels(*case)
+    assert "dedisperse_u16_kernel" in names and "matrix" not in names and "split_u16" not in names, case
+for case in ((40, 256, 60000, 0.25), (64, 64, 60000, 0.25), (128, 16, 1000, 0.5), (1024, 256, 60000, 0.5)):
+    assert "dedisperse_matrix_kernel" in kernels(*case), case
+assert "dedisperse_matrix_kernel" in kernels(16, 64, 4000, 0.5, aa.KERNEL_MATRIX)
+''', tmp_path)
