@@ -32,7 +32,7 @@ struct aa_hip_refine {
     int device = 0;
     int ncand = 0;
     int nitems = 0;
-    int chunk = 0;
+    int chunk = 0, longest = 0;
     int loss_kind = 0;
     aa_hip::refine_cand* d_cands = nullptr;
     aa_hip::refine_item* d_items = nullptr;
@@ -338,6 +338,7 @@ int aa_hip_refine_create(int device, int ncand, const int64_t* x_offsets, const 
     hipError_t e = hipSetDevice(device);
     p->nitems = (int)items.size();
     p->chunk = chunk;
+    p->longest = *std::max_element(nsamp, nsamp + ncand);
     if (e == hipSuccess) e = hipMalloc(&p->d_cands, sizeof(aa_hip::refine_cand) * (size_t)ncand);
     if (e == hipSuccess) e = hipMalloc(&p->d_items, sizeof(aa_hip::refine_item) * items.size());
     if (e == hipSuccess) e = hipMalloc(&p->d_state, sizeof(aa_hip::refine_state) * (size_t)ncand);
@@ -394,6 +395,7 @@ int aa_hip_refine_run(aa_hip_refine* h, const float* d_x, const float* d_delay_p
     a.ncand = h->ncand;
     a.nitems = h->nitems;
     a.chunk = h->chunk;
+    a.longest = h->longest;
     a.u = d_u;
     a.step = d_step;
     a.prev_grad = d_prev_grad;

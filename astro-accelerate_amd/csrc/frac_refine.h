@@ -53,6 +53,7 @@ struct refine_args {
     const refine_item* items;   // [nitems], longest first
     int ncand, nitems;
     int chunk;                  // channels of an item
+    int longest;                // most samples of a window
     float* u;                   // [ncand] residual DM, updated in place
     float* step;                // [ncand] Rprop step, updated in place
     double* prev_grad;          // [ncand] previous dL/du, updated in place

@@ -68,7 +68,8 @@ constexpr int kU = 4;                         // channels in flight per lane
 constexpr int kSeg = kRefineSeg;
 constexpr int kChunk = kRefineChunk;
 constexpr int kScan = kRefineScan;
-constexpr int kCombineThreads = 1024;
+constexpr int kCombineThreads = 1024;         // threads of a window's combine pass; 256 for short windows,
+constexpr int kCombineShort = 256;            // whose samples would leave most of them idle
 static_assert(kSeg == kThreads * kSpt, "a segment's samples fit one lane span each");
 
 // w[m] = row[j + m], m = 0..3, zero outside [0, T).
@@ -265,6 +266,7 @@ __global__ __launch_bounds__(kThreads) void refine_partial_kernel(refine_args a,
     }
 }
 
+template <int NT>
 __device__ __forceinline__ double block_sum(double v, double* red, int tid)
 {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
@@ -272,17 +274,18 @@ __device__ __forceinline__ double block_sum(double v, double* red, int tid)
     if ((tid & 63) == 0) red[tid >> 6] = v;
     __syncthreads();
     double s = 0.0;
-    for (int i = 0; i < kCombineThreads / 64; ++i) s += red[i];
+    for (int i = 0; i < NT / 64; ++i) s += red[i];
     return s;
 }
 
 // This thread's channels of the noise energy N (loss 1) and dN/du at u.
+template <int NT>
 __device__ __forceinline__ void noise_part(const refine_args& a, const refine_cand& cd, float u, int tid, double* n,
                                            double* dn)
 {
     *n = *dn = 0.0;
     if (a.loss_kind != 1) return;
-    for (int c = tid; c < cd.C; c += kCombineThreads) {
+    for (int c = tid; c < cd.C; c += NT) {
         const float ds = a.ds[cd.ds_off + c];
         const int2 e = delay_of(ds, u);
         const double f = (double)__int_as_float(e.y);       // the weight the passes use
@@ -294,9 +297,10 @@ __device__ __forceinline__ void noise_part(const refine_args& a, const refine_ca
 }
 
 // Loss at scan point k0 + blockIdx.y of candidate blockIdx.x.
-__global__ __launch_bounds__(kCombineThreads) void refine_scan_loss_kernel(refine_args a, int k0)
+template <int NT>
+__global__ __launch_bounds__(NT) void refine_scan_loss_kernel(refine_args a, int k0)
 {
-    __shared__ double red[kCombineThreads / 64];
+    __shared__ double red[NT / 64];
     const long b = linear_block();
     if (b >= a.ncand) return;   // whole work-group, before any barrier
     const int k = blockIdx.y, tid = threadIdx.x;
@@ -304,13 +308,13 @@ __global__ __launch_bounds__(kCombineThreads) void refine_scan_loss_kernel(refin
     const int row = cd.T + (cd.T - 1) / kSeg, nchunk = (cd.C + a.chunk - 1) / a.chunk;
     const double* part = a.part + cd.part_off + (size_t)k * row;
     double l2 = 0.0, n, dn;
-    for (int t = tid; t < cd.T; t += kCombineThreads) {
+    for (int t = tid; t < cd.T; t += NT) {
         double v[1];
         profile_at(part, (size_t)kScan * row, row, nchunk, t, cd.T, v);
         l2 = __builtin_fma(v[0], v[0], l2);
     }
-    noise_part(a, cd, a.u[b] + a.scan_lo + a.scan_step * (float)(k0 + k), tid, &n, &dn);
-    const double l = block_sum(l2 - n, red, tid);
+    noise_part<NT>(a, cd, a.u[b] + a.scan_lo + a.scan_step * (float)(k0 + k), tid, &n, &dn);
+    const double l = block_sum<NT>(l2 - n, red, tid);
     if (tid == 0) a.scan_loss[(size_t)b * kScan + k] = l;
 }
 
@@ -336,9 +340,10 @@ __global__ void refine_start_kernel(refine_args a, int k0, int nk)
 }
 
 // One candidate's loss and gradient from the partial profiles, and its step.
-__global__ __launch_bounds__(kCombineThreads) void refine_combine_kernel(refine_args a, int last)
+template <int NT>
+__global__ __launch_bounds__(NT) void refine_combine_kernel(refine_args a, int last)
 {
-    __shared__ double red[kCombineThreads / 64];
+    __shared__ double red[NT / 64];
     const long b = linear_block();
     if (b >= a.ncand) return;   // whole work-group, before any barrier
     const int tid = threadIdx.x;
@@ -347,15 +352,15 @@ __global__ __launch_bounds__(kCombineThreads) void refine_combine_kernel(refine_
     const double* part = a.part + cd.part_off;
     refine_state st = a.cur[b];
     double l2 = 0.0, gs = 0.0, n, dn;
-    for (int t = tid; t < cd.T; t += kCombineThreads) {
+    for (int t = tid; t < cd.T; t += NT) {
         double v[2];   // y, dy/du
         profile_at(part, 2 * (size_t)row, row, nchunk, t, cd.T, v);
         l2 = __builtin_fma(v[0], v[0], l2);
         gs = __builtin_fma(v[0], v[1], gs);
     }
-    noise_part(a, cd, st.u, tid, &n, &dn);
-    const double loss = block_sum(l2 - n, red, tid);
-    const double grad = block_sum(2.0 * gs - dn, red, tid);
+    noise_part<NT>(a, cd, st.u, tid, &n, &dn);
+    const double loss = block_sum<NT>(l2 - n, red, tid);
+    const double grad = block_sum<NT>(2.0 * gs - dn, red, tid);
     if (tid != 0) return;
     if (loss > st.best_l) {  // the result is the best point visited
         st.best_l = loss;
@@ -385,7 +390,9 @@ __global__ __launch_bounds__(kCombineThreads) void refine_combine_kernel(refine_
 constexpr int kPowerBlocksY = 16;
 __global__ __launch_bounds__(256) void refine_power_kernel(refine_args a)
 {
-    const refine_cand cd = a.cands[blockIdx.x];
+    const long b = linear_block();
+    if (b >= a.ncand) return;
+    const refine_cand cd = a.cands[b];
     const float* __restrict__ x = a.x + cd.x_off;
     double* __restrict__ v = a.power + cd.power_off;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -430,29 +437,34 @@ int refine_chunk(int ncand, const int* nchans, const int* nsamp)
     return chunk;
 }
 
-hipError_t launch_refine(const refine_args& a, hipStream_t s)
+template <int NT>
+static hipError_t launch_refine_passes(const refine_args& a, hipStream_t s)
 {
-    if (a.ncand <= 0) return hipSuccess;
-    if (a.nitems <= 0 || a.chunk < 1 || a.chunk > kChunk || (a.loss_kind != 0 && a.loss_kind != 1)) return hipErrorInvalidValue;
-    const unsigned n = (unsigned)a.ncand;
     const dim3 items = linear_grid(a.nitems, kThreads);
     if (a.loss_kind == 1)
-        hipLaunchKernelGGL(refine_power_kernel, dim3(n, kPowerBlocksY), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(refine_power_kernel, linear_grid(a.ncand, 256, kPowerBlocksY), dim3(256), 0, s, a);
     for (int k0 = 0; k0 == 0 || k0 < a.scan_n; k0 += kScan) {
         const int nk = a.scan_n - k0 < kScan ? a.scan_n - k0 : kScan;
         if (nk > 0) {
             hipLaunchKernelGGL(refine_partial_kernel<kScan>, items, dim3(kThreads), 0, s, a, k0, nk);
-            hipLaunchKernelGGL(refine_scan_loss_kernel, linear_grid(a.ncand, kCombineThreads, nk),
-                               dim3(kCombineThreads), 0, s, a, k0);
+            hipLaunchKernelGGL(refine_scan_loss_kernel<NT>, linear_grid(a.ncand, NT, nk), dim3(NT), 0, s, a, k0);
         }
-        hipLaunchKernelGGL(refine_start_kernel, dim3((n + 63) / 64), dim3(64), 0, s, a, k0, nk);
+        hipLaunchKernelGGL(refine_start_kernel, dim3(((unsigned)a.ncand + 63) / 64), dim3(64), 0, s, a, k0, nk);
     }
     for (int i = 0; i <= a.nsteps; ++i) {
         hipLaunchKernelGGL(refine_partial_kernel<0>, items, dim3(kThreads), 0, s, a, 0, 0);
-        hipLaunchKernelGGL(refine_combine_kernel, linear_grid(a.ncand, kCombineThreads), dim3(kCombineThreads), 0, s, a,
-                           i == a.nsteps ? 1 : 0);
+        hipLaunchKernelGGL(refine_combine_kernel<NT>, linear_grid(a.ncand, NT), dim3(NT), 0, s, a, i == a.nsteps ? 1 : 0);
     }
     return hipGetLastError();
+}
+
+hipError_t launch_refine(const refine_args& a, hipStream_t s)
+{
+    if (a.ncand <= 0) return hipSuccess;
+    if (a.nitems <= 0 || a.chunk < 1 || a.chunk > kChunk || (a.loss_kind != 0 && a.loss_kind != 1))
+        return hipErrorInvalidValue;
+    return a.longest <= 2 * kCombineShort ? launch_refine_passes<kCombineShort>(a, s)
+                                          : launch_refine_passes<kCombineThreads>(a, s);
 }
 
 }  // namespace aa_hip
