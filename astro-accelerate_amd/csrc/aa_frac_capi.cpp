@@ -114,6 +114,10 @@ size_t forward_bytes(const aa_hip_frac* p, int nbatch) {
     return sizeof(float) * row_split(p, nbatch) * (size_t)nbatch * p->ntrials * p->nsamp;
 }
 
+size_t adjoint_bytes(const aa_hip_frac* p, int nbatch) {
+    return sizeof(double) * aa_hip::frac_grad_dm_parts(row_groups(p, nbatch) * row_split(p, nbatch), nbatch);
+}
+
 bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 
 }  // namespace
@@ -243,7 +247,7 @@ int aa_hip_frac_workspace_bytes(const aa_hip_frac* h, int nbatch, size_t* forwar
     if (!h || !forward || !adjoint) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "NULL argument");
     if (nbatch < 0 || nbatch > h->max_batch) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "batch exceeds the plan's");
     *forward = nbatch > 0 && row_split(h, nbatch) > 1 ? forward_bytes(h, nbatch) : 0;
-    *adjoint = nbatch > 0 ? sizeof(double) * row_groups(h, nbatch) * (size_t)row_split(h, nbatch) : 0;
+    *adjoint = nbatch > 0 ? adjoint_bytes(h, nbatch) : 0;
     return AA_HIP_SUCCESS;
 }
 
@@ -274,7 +278,8 @@ static int frac_adjoint(aa_hip_frac* h, const float* d_x, const float* d_gy, int
         a.group_q = h->trials_per_wave;
         a.n_groups = (h->ntrials + 16 * a.group_q - 1) / (16 * a.group_q);
         a.n_split = row_split(h, nbatch);
-        if (!gdm_part || !aligned16(gdm_part) || work_bytes < sizeof(double) * aa_hip::frac_grad_dm_parts(a))
+        const size_t need = adjoint_bytes(h, nbatch);
+        if (need && (!gdm_part || !aligned16(gdm_part) || work_bytes < need))
             return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "workspace too small for the batch, or not 16-byte aligned");
         const int st = from_hip(aa_hip::launch_frac_grad_dm(a, s), "frac DM adjoint");
         if (st != AA_HIP_SUCCESS) return st;

@@ -61,7 +61,8 @@ hipError_t launch_frac_forward(const frac_args& a, hipStream_t s);
 hipError_t launch_frac_grad_dm(const frac_args& a, hipStream_t s);   // writes gdm_part then gdm
 hipError_t launch_frac_grad_x(const frac_args& a, hipStream_t s);
 
-// Work-groups (hence gdm_part entries) of launch_frac_grad_dm.
-size_t frac_grad_dm_parts(const frac_args& a);
+// gdm_part entries of launch_frac_grad_dm for its work-groups (batch x time tiles
+// x trial groups x channel parts); one work-group per candidate needs none.
+size_t frac_grad_dm_parts(size_t groups, int B);
 
 }  // namespace aa_hip

@@ -577,13 +577,15 @@ hipError_t launch_frac_forward(const frac_args& a, hipStream_t s)
     return hipGetLastError();
 }
 
-size_t frac_grad_dm_parts(const frac_args& a) { return (size_t)a.B * a.n_ttiles * a.n_groups * a.n_split; }
+size_t frac_grad_dm_parts(size_t groups, int B) { return groups > (size_t)B ? groups : 0; }
 
-hipError_t launch_frac_grad_dm(const frac_args& a, hipStream_t s)
+hipError_t launch_frac_grad_dm(const frac_args& in, hipStream_t s)
 {
-    const hipError_t e = launch_rows<true>(a, s);
-    if (e != hipSuccess) return e;
+    frac_args a = in;
     const int per_b = a.n_ttiles * a.n_groups * a.n_split;
+    if (per_b == 1) a.gdm_part = a.gdm;   // one work-group's sum is the result
+    const hipError_t e = launch_rows<true>(a, s);
+    if (e != hipSuccess || per_b == 1) return e;
     hipLaunchKernelGGL(frac_gdm_finalize, dim3((a.B + 255) / 256), dim3(256), 0, s, a.gdm_part, per_b, a.B, a.gdm);
     return hipGetLastError();
 }

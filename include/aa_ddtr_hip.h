@@ -501,7 +501,8 @@ int aa_hip_frac_adjoint(aa_hip_frac *h, const float *d_x, const float *d_gy, int
  * aligned, of at least the bytes that workspace_bytes gives for the batch, and
  * free for other use once the call's work on `stream` is done.  The forward
  * call takes NULL where it needs none, and without one is not split over the
- * channels (slower on small batches); the adjoint needs one for gdm only. */
+ * channels (slower on small batches); the adjoint needs one, of the bytes given,
+ * for gdm only. */
 int aa_hip_frac_workspace_bytes(const aa_hip_frac *h, int nbatch, size_t *forward, size_t *adjoint);
 int aa_hip_frac_forward_ws(aa_hip_frac *h, const float *d_x, int nbatch, const float *d_dm, float *d_y,
                            void *d_work, size_t work_bytes, void *stream);

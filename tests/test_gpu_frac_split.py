@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 # batch, channels, samples, trials
 @pytest.mark.parametrize("shape", [(1, 191, 64, 5), (1, 192, 128, 33), (2, 193, 1028, 16), (1, 1541, 256, 16),
-                                   (3, 1548, 64, 64), (1, 4096, 4, 1)])
+                                   (3, 1548, 64, 64), (1, 4096, 4, 1), (5, 40, 64, 3)])
 def test_split_channels_match_reference(cuda, shape):
     """Forward within 2e-6 and DM gradient within 1e-5 of the result's size:
     float32 sums of up to 4096 channels, as for the unsplit kernels."""
