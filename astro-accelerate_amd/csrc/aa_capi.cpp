@@ -348,6 +348,13 @@ int aa_hip_ddtr_range_tuning(const aa_hip_ddtr *h, int range, int *variant, int 
     return AA_HIP_SUCCESS;
 }
 
+int aa_hip_ddtr_range_kernel(const aa_hip_ddtr *h, int range, int *kernel) {
+    if (!h || !h->engine || !kernel) return bad("NULL argument");
+    if (range < 0 || range >= h->engine->nranges()) return bad("bad range index");
+    *kernel = h->engine->range_kernel(range);
+    return AA_HIP_SUCCESS;
+}
+
 int aa_hip_ddtr_autotune_range(aa_hip_ddtr *h, int range, int t_processed, float *d_out, size_t out_pitch,
                                int reps, void *stream, int *best_variant, float *variant_ms) {
     if (!h || !h->engine) return bad("NULL handle");

@@ -395,6 +395,23 @@ int ddtr_engine::ensure_level(int k, hipStream_t s) {
 
 int ddtr_engine::prepare_range(int r, int t_processed, float *d_out, size_t out_pitch, hipStream_t s,
                                range_launch *rl, bool batched) {
+    const int st = choose_launch(r, t_processed, d_out, out_pitch, s, rl, batched);
+    if (st == AA_HIP_SUCCESS) {
+        if (m_ran.size() != m_ranges.size()) m_ran.assign(m_ranges.size(), AA_HIP_RANGE_NONE);
+        m_ran[(size_t)r] = rl->sample_bytes == 1 || rl->variant == kShapeMatrix ? rl->variant
+                           : rl->wide_win > 0                                   ? (int)AA_HIP_RANGE_U16
+                                                                                : (int)AA_HIP_RANGE_DIRECT;
+    }
+    return st;
+}
+
+int ddtr_engine::range_kernel(int r) const {
+    static_assert(kShapeMatrix == AA_HIP_RANGE_MATRIX && kShapeRows == AA_HIP_RANGE_ROWS, "numbers of the kernels");
+    return r >= 0 && r < (int)m_ran.size() ? m_ran[(size_t)r] : (int)AA_HIP_RANGE_NONE;
+}
+
+int ddtr_engine::choose_launch(int r, int t_processed, float *d_out, size_t out_pitch, hipStream_t s,
+                               range_launch *rl, bool batched) {
     if (r < 0 || r >= (int)m_ranges.size()) return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "bad range index");
     if (!d_out || out_pitch < (size_t)std::max(t_processed, 0))
         return fail(AA_HIP_ERROR_INVALID_ARGUMENT, "bad output buffer");

@@ -130,6 +130,8 @@ public:
     // rows directly only by ranges that fit no shape.
     int prepare_range(int r, int t_processed, float *d_out, size_t out_pitch, hipStream_t s, range_launch *rl,
                       bool batched = false);
+    // The kernel that range r's last call took (aa_hip_range_kernel).
+    int range_kernel(int r) const;
     // Preference of range r: its shape is used where it fits the range's delay
     // spread; variant -1 is always automatic (see prepare_range).
     int set_range_tuning(int r, int variant, bool automatic);
@@ -198,6 +200,9 @@ private:
         size_t flag_bytes = 0;
     };
     std::vector<matrix_tables> m_matrix;  // per range: the matrix kernel's
+    std::vector<int> m_ran;  // per range: the kernel of its last call
+    int choose_launch(int r, int t_processed, float *d_out, size_t out_pitch, hipStream_t s, range_launch *rl,
+                      bool batched);
     int u16_window(int r);
     bool u16_matrix(int r, hipStream_t s);
     int level_planes(int k, hipStream_t s);

@@ -181,6 +181,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "aa_hip_ddtr_set_range_variant": ([vp, i, i], i),
         "aa_hip_ddtr_set_range_tuning": ([vp, i, i, i], i),
         "aa_hip_ddtr_range_tuning": ([vp, i, pi, pi], i),
+        "aa_hip_ddtr_range_kernel": ([vp, i, pi], i),
         "aa_hip_ddtr_autotune_range": ([vp, i, i, vp, sz, i, vp, pi, PFLOAT], i),
         "aa_hip_ddtr_batch_create": ([i, ctypes.POINTER(vp), ctypes.POINTER(vp)], i),
         "aa_hip_ddtr_batch_destroy": ([vp], i),
@@ -824,6 +825,12 @@ class DdtrPlan:
                                                        ctypes.byref(automatic)), "range_tuning")
         return variant.value, bool(automatic.value)
 
+    def range_kernel(self, r: int) -> int:
+        """The kernel that range r's last call took: an LDS chunk shape 0-6 or a RANGE_ constant."""
+        kernel = ctypes.c_int()
+        check(_lib_or_raise().aa_hip_ddtr_range_kernel(self.handle, int(r), ctypes.byref(kernel)), "range_kernel")
+        return kernel.value
+
     def autotune_range(self, r: int, t_processed: int, out, reps: int = 2, stream=None):
         """Times each LDS chunk shape that fits range r; keeps the fastest, behind the automatic choice where
         that is none of them and faster still (range_tuning).
@@ -1049,4 +1056,5 @@ def inject_pulse_u8(d_data_tc, nsamp: int, nchans: int, d_dmshifts, dm: float, t
 
 (KERNEL_AUTO, KERNEL_DIRECT, KERNEL_LDS, KERNEL_LDS_C32, KERNEL_LDS_C16, KERNEL_LDS_PAIR, KERNEL_LDS_QUAD,
  KERNEL_MATRIX) = range(8)
+RANGE_NONE, RANGE_DIRECT, RANGE_MATRIX, RANGE_ROWS, RANGE_U16 = -2, -1, 7, 8, 9   # range_kernel
 LDS_SHAPES = 7   # LDS chunk shapes 0-6 (set_range_variant, autotune_range)

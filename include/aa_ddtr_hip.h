@@ -298,6 +298,16 @@ int aa_hip_ddtr_run_range(aa_hip_ddtr *h, int range, int t_processed, float *d_o
 int aa_hip_ddtr_set_range_variant(aa_hip_ddtr *h, int range, int variant);
 int aa_hip_ddtr_set_range_tuning(aa_hip_ddtr *h, int range, int variant, int automatic);
 int aa_hip_ddtr_range_tuning(const aa_hip_ddtr *h, int range, int *variant, int *automatic);
+/* The kernel that the last call of a range took on this handle, alone or in a
+ * batch: an LDS chunk shape 0-6, or one of these. */
+typedef enum {
+    AA_HIP_RANGE_NONE = -2,     /* no call yet */
+    AA_HIP_RANGE_DIRECT = -1,
+    AA_HIP_RANGE_MATRIX = 7,    /* 16-bit ranges: with dedisperse_u16 for the tiles whose sums round */
+    AA_HIP_RANGE_ROWS = 8,
+    AA_HIP_RANGE_U16 = 9        /* the 16-bit LDS kernel */
+} aa_hip_range_kernel;
+int aa_hip_ddtr_range_kernel(const aa_hip_ddtr *h, int range, int *kernel);
 int aa_hip_ddtr_autotune_range(aa_hip_ddtr *h, int range, int t_processed, float *d_out,
                                size_t out_pitch, int reps, void *stream, int *best_variant,
                                float *variant_ms);

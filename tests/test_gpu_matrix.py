@@ -1,6 +1,7 @@
 """The matrix-core dedispersion kernel (the automatic choice of a DdtrPlan
-range whose channel groups fit it), bit for bit against the CPU oracle at the
-edges of its tiles, groups and steps."""
+range whose channel groups fit it, unless it is as small as these), bit for bit
+against the CPU oracle at the edges of its tiles, groups and steps; in a batch;
+and over the byte planes of 16-bit samples."""
 import numpy as np
 import pytest
 
@@ -50,6 +51,8 @@ def test_matrix_range(aa, oracle, cuda, geom, pitch_extra):
         out = torch.full((ndms, tp + pitch_extra), -1.0, dtype=torch.float32, device=cuda)
         plan.ingest(d_in, tp * ib)
         plan.run_range(0, tp, out)
+        ran = plan.range_kernel(0)
+        assert ran == aa.RANGE_MATRIX if kernel == aa.KERNEL_MATRIX else ran != aa.RANGE_MATRIX
         got = out.cpu().numpy()
         np.testing.assert_array_equal(got[:, :tp], want)
         assert np.all(got[:, tp:] == -1.0)   # nothing written past a row's samples
@@ -73,6 +76,40 @@ def test_matrix_choice_follows_the_kernel_setting(aa, oracle, cuda):
         out = torch.full((ndms, tp), -1.0, dtype=torch.float32, device=cuda)
         plan.run_range(0, tp, out)
         np.testing.assert_array_equal(out.cpu().numpy(), want, err_msg=f"kernel {kernel} variant {variant}")
+
+
+def test_matrix_launches_of_a_batch(aa, oracle, cuda):
+    """Ranges of at least 512 tiles run matrix launches of their own in a batch,
+    eager and replayed with other inputs, beside ranges that share launches."""
+    import torch
+    nchans, tsamp, tp, small = 256, 64e-6, 33000, 3000
+    ds = oracle.dmshifts(nchans, 1550.0, -1.17)
+    ranges = [(0.0, 0.25, 512, 1), (128.0, 0.5, 64, 2)]
+    maxd = (int(ds[-1] * (160.0 / tsamp)) + 4) // 2 * 2
+    plans = [aa.DdtrPlan(ds, ranges, tsamp, maxd, tp) for _ in range(2)]
+    tps = [tp, small]
+    ins = [torch.empty((tp + maxd, nchans), dtype=torch.uint8, device=cuda) for _ in plans]
+    outs = [[torch.empty((r[2], t), dtype=torch.float32, device=cuda) for r, t in zip(ranges, tps)] for _ in plans]
+    batch = aa.DdtrBatch(plans)
+    for call, graph in enumerate((False, True, True, True)):   # eager, captured, replayed twice
+        datas = [oracle.gen_noise(10 * call + b, tp + maxd, nchans) for b in range(2)]
+        for b in range(2):
+            ins[b].copy_(torch.from_numpy(datas[b]))
+            for o in outs[b]:
+                o.fill_(-1.0)
+        torch.cuda.synchronize()
+        batch.execute(ins, [tps] * 2, outs, use_graph=graph)
+        torch.cuda.synchronize()
+        assert [p.range_kernel(0) for p in plans] == [aa.RANGE_MATRIX] * 2
+        assert all(0 <= p.range_kernel(1) < aa.LDS_SHAPES for p in plans)
+        for b in range(2):
+            rows = oracle.corner_turn(datas[b], tp + maxd, nchans)
+            for r, (low, step, nd, ib) in enumerate(ranges):
+                rows = rows if ib == 1 else oracle.bin2(rows, rows.shape[1] // 2)
+                tsr = np.float32(np.float32(tsamp) * np.float32(ib))
+                want = oracle.dedisperse(rows[:, :tps[r] + maxd // ib].copy(), ds, nd, tps[r],
+                                         float(np.float32(low) / tsr), float(np.float32(step) / tsr), ib)
+                np.testing.assert_array_equal(outs[b][r].cpu().numpy(), want, err_msg=f"call {call} beam {b} range {r}")
 
 
 def _u16_fill(kind, nsamp, nchans, rng):
@@ -112,6 +149,7 @@ def test_u16_byte_planes(aa, oracle, cuda, kind, nchans):
         outs = [torch.full((s.ndms[r], tps[r] + 3), -1.0, dtype=torch.float32, device=cuda) for r in range(s.nranges)]
         plan.execute_chunk(d_in if chunk else torch.flip(d_in, (0,)).contiguous(), tps, outs)
     for r in range(s.nranges):
+        assert plan.range_kernel(r) == aa.RANGE_MATRIX
         got = outs[r].cpu().numpy()
         np.testing.assert_array_equal(got[:, :tps[r]], want[r], err_msg=f"range {r}")
         assert np.all(got[:, tps[r]:] == -1.0)
@@ -135,6 +173,7 @@ def test_u16_lengths_on_two_streams(aa, oracle, cuda):
     for tp in lengths:
         out = torch.empty((ndms, tp), dtype=torch.float32, device=cuda)
         plan.run_range(0, tp, out)
+        assert plan.range_kernel(0) == aa.RANGE_MATRIX
         want.append(out)
     direct = aa.DdtrPlan(ds, [(0.0, 0.4, ndms, 1)], tsamp, maxd, nsamp - maxd, sample_bits=16)
     direct.set_kernel(aa.KERNEL_DIRECT)      # in channel order, whatever the sums

@@ -53,6 +53,7 @@ def test_range(aa, oracle, cuda, geom, pitch_extra):
     out = torch.full((ndms, tp + pitch_extra), -1.0, dtype=torch.float32, device=cuda)
     plan.ingest(torch.from_numpy(data).to(cuda), tp * ib)
     plan.run_range(0, tp, out)
+    assert plan.range_kernel(0) == aa.RANGE_ROWS
     got = out.cpu().numpy()
     np.testing.assert_array_equal(got[:, :tp], want)
     assert np.all(got[:, tp:] == -1.0)   # nothing written past a row's samples
@@ -80,6 +81,7 @@ def test_autotune_and_batch(aa, oracle, cuda):
         for o in outs:
             o.fill_(-1.0)
         batch.execute([d_in] * 3, [[tp]] * 3, [[o] for o in outs], use_graph=graph)
+        assert all(p.range_kernel(0) == aa.RANGE_ROWS for p in plans)
         torch.cuda.synchronize()
         for o in outs:
             np.testing.assert_array_equal(o.cpu().numpy(), want)
