@@ -42,9 +42,9 @@ int no_matrix() {
 }
 
 // A batched range with this many tiles fills the GPU's 256 work-groups twice
-// over and runs a matrix launch of its own; smaller ones stay in the shared
-// launches (96 beams of 64-256 channels: 1.98 ms batched, 4.27 ms with a
-// matrix launch per range).
+// over and may run a matrix launch of its own (matrix_beats_shared); smaller ones
+// stay in the shared launches (96 beams of 64-256 channels: 1.98 ms batched, 4.27
+// ms with a matrix launch per range).
 constexpr long kMatrixAloneTiles = 512;
 
 bool is_pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
@@ -473,6 +473,14 @@ int ddtr_engine::choose_launch(int r, int t_processed, float *d_out, size_t out_
     const range_tuning tuned = tuning(r);
     const bool automatic = tuned.automatic && m_kernel == AA_HIP_KERNEL_AUTO && rd.ndms > 0;
     const bool alone = automatic && !batched;
+    const auto shape = [&]() {   // the range's LDS shape: c, chosen on first use
+        if (c.variant == -2) {
+            c = choose_lds(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, tuned.variant);
+            if (c.variant < 0 && tuned.variant >= 0)  // preferred shape does not fit: any that does
+                c = choose_lds(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, -1);
+        }
+        return c.variant;
+    };
     // No shape asked for: the matrix kernel where its plan is the cheaper one.
     const bool forced = m_kernel == AA_HIP_KERNEL_MATRIX && rd.ndms > 0;
     if (forced || (automatic && (!batched || matrix_tiles_at_most(rd.ndms, t_processed) >= kMatrixAloneTiles))) {
@@ -482,8 +490,11 @@ int ddtr_engine::choose_launch(int r, int t_processed, float *d_out, size_t out_
         if (forced && mt.lay.tile_out <= 0) return no_matrix();
         const long tiles =
             mt.lay.tile_out > 0 ? (long)mt.lay.n_dm_tiles * ((t_processed + mt.lay.tile_out - 1) / mt.lay.tile_out) : 0;
-        if (forced || (tiles > 0 && (!batched || tiles >= kMatrixAloneTiles) &&
-                       !(alone && rows_beat_matrix(m_nchans, rd.ndms, t_processed, mt.lay)))) {
+        const bool takes =
+            forced || (tiles > 0 && (batched ? tiles >= kMatrixAloneTiles &&
+                                                   matrix_beats_shared(m_nchans, rd.ndms, t_processed, mt.lay, shape())
+                                             : !rows_beat_matrix(m_nchans, rd.ndms, t_processed, mt.lay)));
+        if (takes) {
             st = resolve_launch(m_kernel, lv.ptr, lv.pitch, m_nchans, m_d_dmshifts, m_dmshifts.data(), rd.ndms,
                                 t_processed, mstartdm, mdmstep, rd.inBin, d_out, out_pitch,
                                 lds_choice{kShapeMatrix, mt.lay.tile_out}, rl);
@@ -492,11 +503,7 @@ int ddtr_engine::choose_launch(int r, int t_processed, float *d_out, size_t out_
             return st;
         }
     }
-    if (c.variant == -2) {
-        c = choose_lds(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, tuned.variant);
-        if (c.variant < 0 && tuned.variant >= 0)  // preferred shape does not fit: any that does
-            c = choose_lds(m_dmshifts.data(), m_nchans, rd.ndms, mstartdm, mdmstep, -1);
-    }
+    shape();
     // Under capture a shape whose tables are not there yet (the calls before went
     // another way) would break the capture; the rows need none.
     const bool rows = ((alone || (automatic && c.variant < 0)) &&

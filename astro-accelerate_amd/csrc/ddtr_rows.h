@@ -15,6 +15,9 @@ constexpr int kShapeRows = kShapeMatrix + 1;
 // from the rows than by the kernel it would have otherwise: the matrix kernel
 // with this layout, or the chunk shape `variant` (-1: the direct kernel).
 bool rows_beat_matrix(int nchans, int ndms, int t_processed, const matrix_layout& lay);
+// Whether a range of a batch is done sooner by a matrix launch of its own than in
+// the launch that its chunk shape `variant` shares with other ranges.
+bool matrix_beats_shared(int nchans, int ndms, int t_processed, const matrix_layout& lay, int variant);
 bool rows_beat_shape(int nchans, int ndms, int t_processed, int variant);
 
 // Rows as for the LDS kernels (at whole dwords, 4 KiB readable past each row's

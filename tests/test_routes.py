@@ -308,3 +308,24 @@ for case in ((40, 256, 60000, 0.25), (64, 64, 60000, 0.25), (128, 16, 1000, 0.5)
     assert "dedisperse_matrix_kernel" in kernels(*case), case
 assert "dedisperse_matrix_kernel" in kernels(16, 64, 4000, 0.5, aa.KERNEL_MATRIX)
 ''', tmp_path)
+
+
+def test_matrix_launches_in_a_batch(tmp_path):
+    """Ranges of many tiles take matrix launches of their own in a batch where
+    that is faster than the shared launch: not with few channels."""
+    host_library.run('''
+import ddtr_oracle as oracle
+def ran(nchans, ndms, tp, step, band, fch1):
+    ds = oracle.dmshifts(nchans, fch1, -band / nchans)
+    shift = int(ds[-1] * step * ndms / 64e-6) + 16
+    plan = aa.DdtrPlan(ds, [(0.0, step, ndms, 1)], 64e-6, shift, tp)
+    batch = aa.DdtrBatch([plan])
+    batch.execute([Tensor((tp + shift, nchans), 1)], [[tp]], [[Tensor((ndms, tp))]], use_graph=False)
+    return plan.range_kernel(0)
+for case in ((64, 512, 30000, 0.25, 300.0, 1500.0), (192, 512, 30000, 0.5, 810.0, 1760.0),
+             (256, 128, 120000, 0.5, 810.0, 1760.0), (64, 128, 120000, 0.25, 300.0, 1500.0)):
+    assert 0 <= ran(*case) < aa.LDS_SHAPES, case
+for case in ((1024, 512, 30000, 0.25, 300.0, 1500.0), (512, 256, 60000, 0.25, 300.0, 1500.0),
+             (1024, 1000, 60000, 0.5, 810.0, 1760.0), (128, 1000, 60000, 0.25, 300.0, 1500.0)):
+    assert ran(*case) == aa.RANGE_MATRIX, case
+''', tmp_path)
