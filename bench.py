@@ -13,8 +13,10 @@ value = DM x samples per second = sum_r ndms_r * t_processed_r / step time.
 Also reported:
   roofline     the dedisperse kernel alone, HIP events on its stream:
                algorithmic channel-adds (nchans * ndms_r * t_processed_r per
-               launch) / kernel time, against MI355X's FP32 VALU add roofline
-               (78.64 T adds/s = 256 CU x 128 packed adds/clk x 2.4 GHz);
+               launch) / kernel time, against the rate of int8 products where
+               the matrix-core kernel runs (279 T adds/s), and against MI355X's
+               FP32 VALU add roofline (78.64 T adds/s = 256 CU x 128 packed
+               adds/clk x 2.4 GHz; fp32_add_frac, and frac of other kernels);
   cpu_baseline the CPU oracle (OpenMP C) on the host cores, timed on the
                whole hot path over 1/24 of the chunk's output samples (every
                DM row of every range; --cpu-slice 1 runs the whole plane, the
@@ -49,6 +51,10 @@ CONFIGS = {
                     (2000, 3000, 2.0, 8, 8)], pulses="config2"),
 }
 ADD_ROOFLINE_T = 78.64   # T adds/s, packed FP32 VALU adds
+# The matrix kernel's channel-adds as int8 products, 8 operations each (one of
+# four bytes of a slot is selected), at twice the bf16 rate that an 8192^3 product
+# reaches on this card (1115 TFLOP/s).
+MATRIX_ROOFLINE_T = 2 * 1115.0 / 8
 # HBM bytes moved by the dedisperse launches of one step, from rocprofv3
 # FETCH_SIZE (x2.000, calibrated on a 1 GiB device copy) + WRITE_SIZE (x1.000)
 # summed over the launches, by (config, --kernel): the matrix kernel (the
@@ -88,7 +94,7 @@ def main():
                     help="untimed steps first (default 2; 200 on the single-range plan, so the clocks have "
                          "risen before the timed region)")
     ap.add_argument("--config", type=int, default=2, choices=[1, 2, 3, 4, 5])
-    ap.add_argument("--tune-cache", default=None, help="config 4: JSON file of autotuned chunk shapes")
+    ap.add_argument("--tune-cache", default=None, help="config 4: JSON file of autotuned choices")
     ap.add_argument("--beam-set", default="standard", choices=["standard", "small"],
                     help="config 4: the 48 beams (standard), or 256 small beams (64-256 channels, "
                          "2^14-2^15 samples, DM max 100/200 in 1-2 ranges) whose launches do not fill the GPU")
@@ -250,6 +256,8 @@ def main():
     log(f"[bench] dedisperse kernel per range (ms): {[round(x, 3) for x in kt]} total {k_total_ms:.3f} ms -> "
         f"{achieved:.2f} T adds/s ({achieved / ADD_ROOFLINE_T * 100:.1f}% of {ADD_ROOFLINE_T})")
 
+    matrix = all(ddtr.range_kernel(r) == aa.RANGE_MATRIX for r in range(nr))
+    peak = MATRIX_ROOFLINE_T if matrix else ADD_ROOFLINE_T
     value = dm_x_samples / (ms_step * 1e-3)
     meas = MEASURED_TRAFFIC.get((args.config, args.kernel))
     traffic = meas["bytes"] if meas else None
@@ -270,15 +278,17 @@ def main():
                    "dm_trials": sum(ndms), "dm_x_samples": dm_x_samples, "channel_adds": adds,
                    "kernel": args.kernel, "parallelism": "single GPU"},
         "channel_adds_per_s": adds / (ms_step * 1e-3),
-        "roofline": {"bound": "valu", "achieved": achieved, "peak": ADD_ROOFLINE_T, "unit": "Tadd/s",
-                     "frac": achieved / ADD_ROOFLINE_T, "traffic": traffic,
+        "roofline": {"bound": "mfma" if matrix else "valu", "achieved": achieved, "peak": peak, "unit": "Tadd/s",
+                     "frac": achieved / peak, "fp32_add_peak": ADD_ROOFLINE_T,
+                     "fp32_add_frac": achieved / ADD_ROOFLINE_T, "traffic": traffic,
                      "kernel": "dedisperse (all ranges)", "kernel_ms": k_total_ms,
                      "hbm_algorithmic_GBs": hbm_bytes / (k_total_ms * 1e-3) / 1e9,
                      "hbm_frac": hbm_bytes / (k_total_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
                      "hbm_algorithmic_bytes": hbm_bytes,
                      "traffic_source": meas["profile"] if traffic else None,
-                     "peak_note": "nominal: FP32 packed-add rate; the kernels add integers (int8 matrix "
-                                  "products or SWAR)"},
+                     "peak_note": ("int8 products of the matrix kernel at the rate a large matrix product reaches; "
+                                   "fp32_add: the nominal packed-add rate" if matrix else
+                                   "nominal: FP32 packed-add rate; the kernels add integers (SWAR)")},
     }
     iss = MEASURED_ISSUE.get((args.config, args.kernel))
     if iss:
@@ -601,9 +611,11 @@ def bench_multibeam(args):
     3000 in 1-4 AA-style ranges, seeded u8 noise + 2 pulses each): all beams
     batched and replayed from a hipGraph (DdtrBatch: one launch per kernel
     instantiation over all beams' ranges), against the same beams launched
-    one after another (execute_chunk per beam) on the same tuned shapes
-    (speedup_vs_per_beam_same_kernels, beside the 1.5x target), and on the
-    byte-row shapes.  Chunk shapes are autotuned per shape class first.
+    one after another (execute_chunk per beam) as tuned
+    (speedup_vs_per_beam_same_kernels, beside the 1.5x target; alone a range may
+    take the matrix or the row kernel where the batch shares a launch, see
+    per_beam_range_kernels), and on the byte-row shapes.  Shapes and the automatic
+    choice are autotuned per shape class first.
     --beam-set small: 256 beams of 64-256 channels whose launches hold a few
     dozen tiles each, fewer than the GPU's 256 CUs."""
     import torch
@@ -664,7 +676,12 @@ def bench_multibeam(args):
         ms_per_beam = timed(per_beam, args.steps)
         log(f"[bench] per-beam launches: {ms_per_beam:.2f} ms/step")
         ms_batched = timed(batched, args.steps)
-        log(f"[bench] batched (graph, persistent): {ms_batched:.2f} ms/step -> speedup {ms_per_beam / ms_batched:.3f}x")
+        kernels = {}
+        for b in beams:
+            for r in range(len(b.tps)):
+                k = b.plan.range_kernel(r)
+                kernels[k] = kernels.get(k, 0) + 1
+        log(f"[bench] batched (graph): {ms_batched:.2f} ms/step -> speedup {ms_per_beam / ms_batched:.3f}x")
         # The same per-beam launches on the byte-row shapes (each range's
         # faster of the 32- and 16-channel shapes where one fits; ranges no
         # byte-row shape fits keep the automatic choice): the path a port of
@@ -703,6 +720,7 @@ def bench_multibeam(args):
         "speedup_target": 1.5,
         "bit_exact_vs_per_beam": exact,
         "batch_stats": batch.stats(),
+        "per_beam_range_kernels": kernels,
         "per_beam_byte_rows_ms_per_step": ms_per_beam_bytes,
         "speedup_vs_per_beam_byte_rows": ms_per_beam_bytes / ms_batched,
         "bit_exact_vs_per_beam_byte_rows": exact_bytes,
