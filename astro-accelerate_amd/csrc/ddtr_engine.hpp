@@ -126,7 +126,8 @@ public:
     // the caller (launch_range, or a batched launch).
     // batched: the caller puts the launches of many ranges into shared ones;
     // the matrix kernel, which runs one launch per range, is then taken only
-    // by ranges that fill the GPU by themselves, the kernel that reads the
+    // by ranges that fill the GPU by themselves and where that launch is faster
+    // than their part of a shared one (matrix_beats_shared), the kernel that reads the
     // rows directly only by ranges that fit no shape.
     int prepare_range(int r, int t_processed, float *d_out, size_t out_pitch, hipStream_t s, range_launch *rl,
                       bool batched = false);

@@ -35,7 +35,7 @@ struct lds_params {
     float* out;
     size_t out_pitch;        // floats between output rows
     int row_quads;           // staged row width in uint4 (from lds_row_quads)
-    const void* pair_recs;   // chunk shapes 2-4: device plan tables (from lds_plan_tables)
+    const void* pair_recs;   // chunk shapes 2-6: device plan tables (from lds_plan_tables)
     int n_dm_tiles, n_t_tiles;  // filled by the launcher / lds_job_tiles
 };
 

@@ -17,7 +17,7 @@
 // and the even sums follow at the end modulo 2^16; 256 channels of 255 fit.
 //
 // Bound: latency at the smallest sizes, then the vector memory path (a byte
-// from L2 per add) and the 24 instructions per 16 adds and lane: 22 to 25 T
+// from L2 per add) and the 23 instructions per 16 adds and lane: 22 to 25 T
 // adds/s.  Sharing rows pays from there on, unless the trials are so far apart
 // that the shared windows are mostly unused, or too wide for LDS: then the byte
 // row shapes run at 8 to 20 T adds/s and the direct kernel at 1.4.

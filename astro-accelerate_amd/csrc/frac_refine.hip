@@ -31,9 +31,9 @@
 //
 // Work split: an item is up to kChunk channels (fewer where the windows are few,
 // refine_chunk) x kSeg samples of one window, a 256-thread work-group each, so
-// that windows of any number and size spread over the whole GPU.  A group of S lanes covers the item's samples, 4
-// consecutive ones per lane, and the work-group holds G = 256 / S such groups,
-// each summing every G-th channel.  A lane reads its 4 samples x[c][t0 + i_c ..
+// that windows of any number and size spread over the whole GPU.  A group of S
+// lanes covers the item's samples, 4 consecutive ones per lane, and the work-group
+// holds G = 256 / S such groups, each summing every G-th channel.  A lane reads its 4 samples x[c][t0 + i_c ..
 // t0 + i_c + 3] as one 16-byte load; the second tap of the sample before them
 // is kept apart and added to it after the pass.  Sums are double; the groups'
 // are added in LDS and the items' by one work-group per candidate
@@ -44,7 +44,7 @@
 //
 // Bound: HBM (each pass reads every window once; the partial profiles add 2 to
 // 3 % of that).  Measured on 256 windows (1024-4096 channels x 256-4096
-// samples, 3.64 GB; 9-point scan and 20 steps): 22.2 ms, of which a gradient
+// samples, 3.64 GB; 9-point scan and 20 steps): 21.7 ms, of which a gradient
 // pass takes 0.75 ms (4.85 TB/s; a 4 GiB device copy does 4.77), its combine
 // 0.04, a scan pass of 3 points 1.45, the channel powers 1.05.  With one
 // work-group per window, two passes per evaluation and one per scan point it

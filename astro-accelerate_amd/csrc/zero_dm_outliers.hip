@@ -32,8 +32,9 @@
 // that of an integer, the pass is repeated with the reference's own
 // accumulators (a few rows in 1000 on noise).  Measured on 4096 channels x
 // 262,144 samples of noise with 64 loud channels: 0.95 ms (2.3 TB/s; the
-// accumulators in every pass took 4.7); bound by vector issue, about 2200
-// instructions a row: 450 for the output values, 10 per dword and pass.
+// accumulators in every pass took 4.7); bound by vector issue, 1360
+// instructions a row (counted) at two thirds of the issue rate, the rest waits
+// between dependent passes at 5 waves per SIMD (86 registers).
 //
 // Other rows (zero_dm_outliers_kernel: 16-bit samples, whose sums may round,
 // and more channels) always run those accumulators: lane l holds accumulators

@@ -236,10 +236,14 @@ int aa_hip_ddtr_create(int device, int nchans, const float *dmshifts, int nrange
  * the cascade levels stay u16 and each output is the float channel sum in
  * channel order, as the reference's cache kernel forms it
  * (src/aa_device_dedispersion_kernel.cu:422-450; it rounds once a sum passes
- * 2^24).  Ingest takes input_bits 16 only; the kernel choice is the 16-bit
- * LDS kernel (AA_HIP_KERNEL_AUTO) or the direct kernel (DIRECT, and AUTO
- * where a tile's delay spread exceeds the LDS rows).  Not usable in
- * batches. */
+ * 2^24).  Ingest takes input_bits 16 only.  AA_HIP_KERNEL_AUTO runs the
+ * matrix-core kernel over the rows' low and high bytes where a time model says
+ * that it is faster, with the 16-bit LDS kernel for tiles whose sums round, else
+ * the 16-bit LDS kernel, or the direct kernel where a tile's delay spread exceeds
+ * the LDS rows; DIRECT is always the direct kernel.  The byte planes take a
+ * level's size again in device memory, and the tables some MB, allocated on first
+ * use and not under capture; without them the 16-bit LDS kernel runs.  Not usable
+ * in batches. */
 int aa_hip_ddtr_create_u16(int device, int nchans, const float *dmshifts, int nranges,
                            const float *dm_low, const float *dm_step, const int *ndms,
                            const int *inBin, double tsamp, int maxshift, int max_t_processed0,
@@ -323,8 +327,8 @@ int aa_hip_ddtr_autotune_range(aa_hip_ddtr *h, int range, int t_processed, float
  * LDS shapes in one persistent launch, the pair pre-summation shapes in one
  * launch per tile width and row width; ranges on the quad shape, or that no
  * chunk shape fits, run launches of their own after them (in the same
- * graph), as do ranges of at least 512 tiles that take the matrix-core kernel.
- * With use_graph != 0 the
+ * graph), as do ranges of at least 512 tiles for which a matrix-core launch is
+ * faster than their part of the shared one.  With use_graph != 0 the
  * sequence is captured into a hipGraph on the first call for a given set of
  * buffers and replayed by later calls with the same buffers.  Results are
  * bit-identical to aa_hip_ddtr_execute_chunk per beam.  Calls on one batch
@@ -336,7 +340,7 @@ int aa_hip_ddtr_batch_execute(aa_hip_ddtr_batch *h, const void *const *d_inputs_
                               const int *t_processed, float *const *d_out,
                               const size_t *out_pitch, int use_graph, void *stream);
 /* Jobs (ranges) in the batched launches, their tiles, and ranges launched
- * on their own (quad shape or direct kernel) in the last execute. */
+ * on their own (matrix-core kernel, quad shape, rows or direct kernel) in the last execute. */
 int aa_hip_ddtr_batch_stats(const aa_hip_ddtr_batch *h, int *njobs, long *ntiles, int *ndirect);
 /* Corner turns of the last execute: *batched = launches that turned many
  * beams at once (one per number of binned levels written), *own = beams
